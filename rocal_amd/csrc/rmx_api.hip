@@ -42,7 +42,9 @@ enum OpKind {
     OP_SATURATION, OP_WARP_AFFINE, OP_ROTATE, OP_TO_TENSOR, OP_GAMMA, OP_EXPOSURE, OP_COLOR_TEMPERATURE, OP_BLEND, OP_NORMALIZE, OP_TRANSPOSE
 };
 
-constexpr int TABLE_RING = 4;  // updates in flight before the host has to wait on an old upload
+// Table slots. One event per half of the ring, recorded behind the upload of its last slot and waited for before its first
+// slot is filled again: recording and asking an event costs the host about 5 us, which every update paid while each slot had its own.
+constexpr int TABLE_RING = 8, RING_HALF = TABLE_RING / 2;
 
 }  // namespace
 
@@ -74,6 +76,7 @@ __global__ void __launch_bounds__(256) rmx_table_upload_kernel(const uint4 *__re
 static std::mutex g_life_lock;  // creation and destruction of ops against the destruction of their context
 
 struct rmx_ctx {
+    int compact = 1;              // 1: rows that fit the kernel's arguments travel there (compact_rows)
     int upload_kernel = 1;        // 1: tables are uploaded by rmx_table_upload_kernel, 0: by hipMemcpyAsync
     // (both under g_life_lock: a garbage collector may destroy ops and their context from different threads)
     int live_ops = 0;             // ops made on this context and not yet destroyed: they use its streams until their own end
@@ -116,8 +119,15 @@ struct rmx_op {
     bool slot_ragged[TABLE_RING] = {};    // what the table slot was committed with
     uint64_t slot_src_bytes[TABLE_RING] = {};
     RmxSample *d_table[TABLE_RING] = {};
-    hipEvent_t uploaded[TABLE_RING] = {};
-    int cur = -1;  // slot of the last update, -1 before the first
+    hipEvent_t uploaded[2] = {};      // per half of the ring: its last upload has completed
+    bool half_pending[2] = {};        // ... was recorded and not yet waited for
+    int cur = -1;  // slot of the last update that went through the table, -1 before the first
+    bool updated = false;
+    // the rows of the last update in the form that travels in the kernel's arguments (compact 0: they are in table slot `cur`)
+    uint32_t compact = 0, compact_words = 0;
+    RmxSample shared{};
+    uint32_t rec[RMX_C_WORDS];
+    uint64_t compact_src_bytes = 0;   // extent of the ragged source the records name
     // A launch of this op was recorded into a HIP graph: the graph's kernel node holds the address of the table slot of the
     // last update, which the ring would hand out again four updates later. Such an op keeps its parameters: updates are refused.
     bool captured = false;
@@ -194,33 +204,46 @@ int make_op(rmx_ctx *ctx, int kind, const rmx_tensor_desc *src, const rmx_tensor
     op->extra_per_sample = extra_per_sample;
     // (the upload kernel moves whole 16-byte pieces: a slot is a whole number of them)
     const size_t bytes = slot_bytes(op);
-    for (int i = 0; i < TABLE_RING; i++) {
-        hipError_t e = hipHostMalloc((void **)&op->h_table[i], bytes, hipHostMallocDefault);
-        if (e == hipSuccess) e = hipMalloc((void **)&op->d_table[i], bytes);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&op->uploaded[i], hipEventDisableTiming);
-        if (e != hipSuccess) {
-            rmx_op_destroy(op);
-            return fail(RMX_ERR_HIP, "allocating the parameter table failed: %d (%s)", (int)e, hipGetErrorString(e));
-        }
-        memset(op->h_table[i], 0, bytes);
+    // (one block per side for the whole ring, slots at multiples of 128 bytes)
+    const size_t pitch = (bytes + 127) & ~(size_t)127;
+    hipError_t e = hipHostMalloc((void **)&op->h_table[0], pitch * TABLE_RING, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipMalloc((void **)&op->d_table[0], pitch * TABLE_RING);
+    for (int i = 0; i < 2 && e == hipSuccess; i++) e = hipEventCreateWithFlags(&op->uploaded[i], hipEventDisableTiming);
+    if (e != hipSuccess) {
+        rmx_op_destroy(op);
+        return fail(RMX_ERR_HIP, "allocating the parameter table failed: %d (%s)", (int)e, hipGetErrorString(e));
+    }
+    memset(op->h_table[0], 0, pitch * TABLE_RING);
+    for (int i = 1; i < TABLE_RING; i++) {
+        op->h_table[i] = reinterpret_cast<RmxSample *>(reinterpret_cast<char *>(op->h_table[0]) + pitch * i);
+        op->d_table[i] = reinterpret_cast<RmxSample *>(reinterpret_cast<char *>(op->d_table[0]) + pitch * i);
     }
     *out = op;
     return RMX_OK;
 }
 
-// Next table slot; waits until the upload that last used it has completed.
+// Next table slot; waits until the uploads that last used its half of the ring have completed.
 int next_slot(rmx_op *op, RmxSample **row) {
     if (op->captured)
         return fail(RMX_ERR_INVALID, "a launch of this op was recorded into a HIP graph, whose replays read the parameter rows of the update before the capture: "
                                      "the op keeps those parameters (create another op for new ones, or record rmx_resize_cmn_noalloc, which carries its rows in the graph)"), -2;
     int slot = (op->cur + 1) % TABLE_RING;
-    HIP_TRY(hipSetDevice(op->ctx->device));
-    HIP_TRY(hipEventSynchronize(op->uploaded[slot]));
+    const int half = slot / RING_HALF;
+    if (slot % RING_HALF == 0 && op->half_pending[half]) {
+        HIP_TRY(hipSetDevice(op->ctx->device));
+        HIP_TRY(hipEventSynchronize(op->uploaded[half]));
+        op->half_pending[half] = false;
+    }
     *row = op->h_table[slot];
     return slot;
 }
 
+bool compact_rows(rmx_op *op, const RmxSample *t);
+
 int commit_slot(rmx_op *op, int slot) {
+    op->updated = true;
+    if (compact_rows(op, op->h_table[slot])) return RMX_OK;  // (the slot stays free: nothing on the device reads it)
+    HIP_TRY(hipSetDevice(op->ctx->device));
     size_t bytes = sizeof(RmxSample) * (size_t)op->n;
     if (!op->layout.empty()) {
         memcpy(reinterpret_cast<char *>(op->h_table[slot]) + bytes, op->layout.data(), sizeof(RmxSrcLayout) * (size_t)op->n);
@@ -243,9 +266,135 @@ int commit_slot(rmx_op *op, int slot) {
     } else {
         HIP_TRY(hipMemcpyAsync(op->d_table[slot], op->h_table[slot], bytes, hipMemcpyHostToDevice, us));
     }
-    HIP_TRY(hipEventRecord(op->uploaded[slot], us));
+    if (slot % RING_HALF == RING_HALF - 1) {
+        HIP_TRY(hipEventRecord(op->uploaded[slot / RING_HALF], us));
+        op->half_pending[slot / RING_HALF] = true;
+    }
     op->cur = slot;
     return RMX_OK;
+}
+
+// Brings the rows `t` into the form that travels in the kernel's arguments (RMX_C_*, rmx_common.h) when they allow it: every
+// field outside the ones a record can hold is the same in all rows, and n records fit. False: the rows go through the table.
+bool compact_rows(rmx_op *op, const RmxSample *t) {
+    op->compact = 0;
+    if (!op->ctx->compact || op->extra_per_sample || op->n > RMX_C_WORDS) return false;
+    constexpr int W = (int)(sizeof(RmxSample) / 4);
+    enum { SRC = 0, DST = 4, FLAGS = 10, STRIP_ROWS = 11, RX = 12, COLOR = 22, M = 26 };  // dword of a field
+    // bits in which the rows differ, per dword
+    uint32_t diff[W] = {};
+    const uint32_t *first = reinterpret_cast<const uint32_t *>(t);
+    for (int i = 1; i < op->n; i++) {
+        const uint32_t *row = first + (size_t)i * W;
+        for (int k = 0; k < W; k++) diff[k] |= row[k] ^ first[k];
+    }
+    uint32_t c = RMX_C_ON, window = 0;
+    for (int k = 0; k < 4; k++) window |= diff[SRC + k];
+    window |= diff[FLAGS];
+    bool tiles[2] = {false, false};
+    switch (op->kind) {
+        case OP_TRANSPOSE:
+            if (op->aux1) return false;  // (height and width change places: a kernel of its own)
+            [[fallthrough]];
+        case OP_CMN: case OP_CROP: case OP_FLIP: case OP_TO_TENSOR: case OP_COLOR_TEMPERATURE:
+        case OP_COLOR_TWIST: case OP_BRIGHTNESS: case OP_CONTRAST: case OP_HUE: case OP_SATURATION: case OP_EXPOSURE: case OP_BLEND: {
+            const bool k1 = op->kind == OP_CMN || op->kind == OP_CROP || op->kind == OP_FLIP || op->kind == OP_TO_TENSOR || op->kind == OP_COLOR_TEMPERATURE || op->kind == OP_TRANSPOSE;
+            // (these kernels read the window's origin and the written size, which is the window's)
+            for (int i = 0; i < op->n; i++)
+                if (t[i].src_w != t[i].dst_w || t[i].src_h != t[i].dst_h) return false;
+            if (window) c |= RMX_C_WINDOW | RMX_C_DST;
+            diff[DST] = diff[DST + 1] = 0;
+            if (!k1)
+                for (int k = 0; k < 4; k++)
+                    if (diff[COLOR + k]) {
+                        c |= RMX_C_COLOR0 << k;
+                        diff[COLOR + k] = 0;
+                    }
+            break;
+        }
+        case OP_RESIZE: {
+            if (t[0].dst_w <= 0 || t[0].dst_h <= 0) return false;
+            const bool tri = op->interp == RMX_INTERP_TRIANGULAR;
+            tiles[0] = !tri && op->fn_fast && op->fast_aux1 == 0;            // the staged kernel's x-tiles
+            tiles[1] = !tri && (op->fn_mid || (op->fn_fast && !tiles[0]));  // the streaming kernel's
+            if (!tri && op->fn_mid) diff[STRIP_ROWS] = 0;  // (the general kernel, which reads it, is not reached)
+            bool order = false;
+            for (int i = 0; i < op->n; i++) order = order || t[i].plan[2] != i;
+            for (int k = 0; k < 2; k++)
+                if (tiles[k]) window |= diff[COLOR + k];
+            if (window) {
+                c |= RMX_C_WINDOW | RMX_C_RATIO;
+                for (int k = 0; k < 4; k++) diff[RX + k] = 0;
+            }
+            if (order) c |= RMX_C_ORDER;
+            diff[COLOR] = diff[COLOR + 1] = diff[COLOR + 2] = 0;
+            if (op->flags & (RMX_F_COLOR_LINEAR | RMX_F_COLOR_TWIST)) {
+                if (diff[M] | diff[M + 1] | diff[M + 2] | diff[M + 3]) c |= RMX_C_M4;
+                for (int k = 0; k < 4; k++) diff[M + k] = 0;
+            }
+            break;
+        }
+        case OP_WARP_AFFINE: case OP_ROTATE: {
+            uint32_t m = 0;
+            for (int k = 0; k < 6; k++) {
+                m |= diff[M + k];
+                diff[M + k] = 0;
+            }
+            if (window) c |= RMX_C_WINDOW;
+            if (m) c |= RMX_C_M6;
+            break;
+        }
+        default: return false;
+    }
+    if (c & RMX_C_WINDOW) {
+        for (int k = 0; k < 4; k++) diff[SRC + k] = 0;
+        diff[FLAGS] &= ~(uint32_t)(RMX_S_HFLIP | RMX_S_VFLIP);
+    }
+    uint32_t rest = 0;
+    for (int k = 0; k < W; k++) rest |= diff[k];
+    if (rest) return false;
+    if (!op->layout.empty()) c |= RMX_C_LAYOUT;
+    uint32_t words = ((c & RMX_C_WINDOW) ? 2u : 0u) + ((c & RMX_C_M4) ? 4u : 0u) + ((c & RMX_C_M6) ? 6u : 0u) + ((c & RMX_C_ORDER) ? 1u : 0u) + ((c & RMX_C_LAYOUT) ? 2u : 0u);
+    for (int k = 0; k < 4; k++) words += (c & (RMX_C_COLOR0 << k)) ? 1u : 0u;
+    if ((uint64_t)words * op->n > (uint64_t)RMX_C_WORDS) return false;
+    // an x-tile width as its code: 0 the whole row, k: RMX_C_TILE_WHOLE >> k
+    const int whole = std::min(std::max((int)t[0].dst_w, 8), RMX_C_TILE_WHOLE);
+    auto tile_code = [&](int tw) -> uint32_t {
+        if (tw == whole) return 0u;
+        for (uint32_t k = 1; k < 8; k++)
+            if (tw == RMX_C_TILE_WHOLE >> k) return k;
+        return 8u;
+    };
+    for (int i = 0; i < op->n; i++) {
+        uint32_t *r = op->rec + (size_t)i * words;
+        const RmxSample &s = t[i];
+        if (c & RMX_C_WINDOW) {
+            if ((uint32_t)(s.src_x | s.src_y | s.src_w | s.src_h) > 0x3fffu) return false;
+            if ((c & RMX_C_RATIO) && (s.src_w <= 0 || s.src_h <= 0)) return false;
+            const uint32_t t0 = tiles[0] ? tile_code(s.plan[0]) : 0u, t1 = tiles[1] ? tile_code(s.plan[1]) : 0u;
+            if (t0 > 7 || t1 > 7) return false;
+            *r++ = (uint32_t)s.src_x | (uint32_t)s.src_y << 14 | (s.flags & (RMX_S_HFLIP | RMX_S_VFLIP)) << 28 | (t0 & 3u) << 30;
+            *r++ = (uint32_t)s.src_w | (uint32_t)s.src_h << 14 | t1 << 28 | (t0 >> 2) << 31;
+        }
+        for (int k = 0; k < 4; k++)
+            if (c & (RMX_C_COLOR0 << k)) memcpy(r++, &s.color[k], 4);
+        const int nm = (c & RMX_C_M6) ? 6 : (c & RMX_C_M4) ? 4 : 0;
+        memcpy(r, s.m, 4 * (size_t)nm);
+        r += nm;
+        if (c & RMX_C_ORDER) *r++ = (uint32_t)s.plan[2];
+        if (c & RMX_C_LAYOUT) {
+            const RmxSrcLayout &l = op->layout[i];
+            if (l.offset >> 40 || l.row_stride >> 24) return false;
+            *r++ = (uint32_t)l.offset;
+            *r++ = (uint32_t)(l.offset >> 32) << 24 | l.row_stride;
+        }
+    }
+    op->shared = t[0];
+    if (c & RMX_C_WINDOW) op->shared.flags &= ~(uint32_t)(RMX_S_HFLIP | RMX_S_VFLIP);
+    op->compact = c;
+    op->compact_words = words;
+    op->compact_src_bytes = op->ragged_bytes;
+    return true;
 }
 
 // image size of sample i: its own when the source is ragged, the padded tensor's otherwise
@@ -398,6 +547,7 @@ int rmx_ctx_create(int device, void *stream, int own_stream, rmx_ctx **out) {
         ctx->fast_rows = tune_env("RMX_TUNE_FAST_ROWS", ctx->fast_rows, 1, 64);
         ctx->fast_lds = tune_env("RMX_TUNE_FAST_LDS", ctx->fast_lds, 2048, 48 * 1024);
         ctx->fast_wpb = tune_env("RMX_TUNE_FAST_WPB", ctx->fast_wpb, 1, 4);
+        ctx->compact = tune_env("RMX_TUNE_COMPACT", ctx->compact, 0, 1);  // 0: parameter rows always go through a table in device memory
         ctx->upload_kernel = tune_env("RMX_TUNE_UPLOAD_KERNEL", ctx->upload_kernel, 0, 1);
         ctx->dma = tune_env("RMX_TUNE_DMA", ctx->dma, 0, 1);  // 0: the bilinear fast path always stages through registers
         ctx->dma_lds = tune_env("RMX_TUNE_DMA_LDS", ctx->dma_lds, 2048, 32 * 1024) & ~15;  // LDS window of a wavefront
@@ -451,11 +601,10 @@ int rmx_op_destroy(rmx_op *op) {
     if (!op) return RMX_OK;
     (void)hipSetDevice(op->ctx->device);
     (void)hipStreamSynchronize(op->ctx->stream);
-    for (int i = 0; i < TABLE_RING; i++) {
-        if (op->uploaded[i]) (void)hipEventDestroy(op->uploaded[i]);
-        if (op->h_table[i]) (void)hipHostFree(op->h_table[i]);
-        if (op->d_table[i]) (void)hipFree(op->d_table[i]);
-    }
+    for (hipEvent_t ev : op->uploaded)
+        if (ev) (void)hipEventDestroy(ev);
+    if (op->h_table[0]) (void)hipHostFree(op->h_table[0]);
+    if (op->d_table[0]) (void)hipFree(op->d_table[0]);
     rmx_ctx *ctx = op->ctx;
     delete op;
     bool last;
@@ -513,7 +662,8 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
                         const void *src, const void *src2, void *dst);
 
 static int launch_impl(rmx_op *op, const void *src, const void *src2, void *dst) {
-    if (op->cur < 0 || !op->fn) return fail(RMX_ERR_INVALID, "op launched before its first update");
+    if (!op->updated || !op->fn) return fail(RMX_ERR_INVALID, "op launched before its first update");
+    if (op->compact) return launch_table(op, nullptr, nullptr, nullptr, (op->compact & RMX_C_LAYOUT) ? op->compact_src_bytes : 0, src, src2, dst);
     const bool ragged = op->slot_ragged[op->cur];
     return launch_table(op, op->d_table[op->cur], ragged ? reinterpret_cast<const RmxSrcLayout *>(op->d_table[op->cur] + op->n) : nullptr,
                         op->extra_per_sample ? slot_extra(op, op->d_table[op->cur]) : nullptr, ragged ? op->slot_src_bytes[op->cur] : 0, src, src2, dst);
@@ -523,13 +673,20 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
                         const void *src, const void *src2, void *dst) {
     if (!src || !dst) return fail(RMX_ERR_INVALID, "source/destination buffer is NULL");
     if (!op->fn) return fail(RMX_ERR_INVALID, "op launched before its first update");
-    RmxKArgs a{};
+    RmxKArgs a;
+    memset(&a, 0, offsetof(RmxKArgs, shared));
+    a.compact = op->compact;
+    if (op->compact) {
+        a.compact_words = op->compact_words;
+        a.shared = op->shared;
+        memcpy(a.rec, op->rec, 4 * (size_t)op->compact_words * op->n);
+    }
     a.src = (const uint8_t *)src;
     a.src2 = (const uint8_t *)src2;
     a.extra = extra;
     a.dst = dst;
     a.table = table;
-    a.src_bytes = layout ? ragged_bytes : (uint64_t)op->src.n * op->src.h * op->src.w * op->src.c;
+    a.src_bytes = ragged_bytes ? ragged_bytes : (uint64_t)op->src.n * op->src.h * op->src.w * op->src.c;
     a.layout = layout;
     a.n = op->n;
     a.src_h = (int)op->src.h;
@@ -597,8 +754,8 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
                           op->stats_shift, op->stats_mode != 0);
         HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(wpb * RMX_WAVE), lds, op->ctx->stream, a);
-    HIP_TRY(hipGetLastError());
+    void *kargs[1] = {&a};
+    HIP_TRY(hipLaunchKernel(reinterpret_cast<const void *>(fn), dim3((unsigned)blocks), dim3(wpb * RMX_WAVE), kargs, lds, op->ctx->stream));
     if (!op->captured) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(op->ctx->stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusActive) op->captured = true;
@@ -1827,6 +1984,7 @@ int rmx_resize_cmn_noalloc(rmx_ctx *ctx, const rmx_tensor_desc *src_desc, const 
     memset(rows, 0, sizeof(RmxSample) * (size_t)op.n);
     rc = fill_resize_rows(&op, rows, src_roi, dst_w, dst_h, crop_roi, scale, bias, nullptr, nullptr, mirror, nullptr);
     if (rc) return rc;
+    if (compact_rows(&op, rows)) return launch_table(&op, nullptr, nullptr, nullptr, 0, src, nullptr, dst);
     RmxSample *table = static_cast<RmxSample *>(ctx->scratch_ptr);  // the address asked of the runtime, never the array's name
     for (int first = 0; first < op.n; first += 16) {
         RmxRowPack pack;

@@ -43,6 +43,26 @@ enum : uint32_t {
     RMX_S_EDGE_REF = 8u  // bilinear: both neighbours clamp to the window's last-but-one column / row (RMX_F_EDGE_REF)
 };
 
+// A batch whose rows differ in little (crop windows and mirror flags, colour factors, a matrix) travels in the kernel's
+// arguments: one row of what all samples share and a few dwords per sample, from which load_sample() (rmx_device.h) makes the
+// row again. A table in device memory costs a launch of its own in front of every batch's kernel (the upload, 3 - 4 us on the
+// GPU and, with the event that guards its slot, 8 us of the host), the arguments 0.3 us and 1 us: measured for 2 KB of them
+// read by 14 336 wavefronts. Whole batches, one update and launch after the other: 256 RandomResizedCrop windows to 224 x 224 fp16
+// 37.4 -> 31.5 us, 128 crops of 224 x 224 to fp32 planes 22.2 -> 16.8 us, 14 small crops 16.9 -> 11.0 us. What a sample's dwords hold, in this order:
+enum : uint32_t {
+    RMX_C_ON = 1u,        // the rows are in the arguments
+    RMX_C_WINDOW = 2u,    // two dwords: x, y, w, h in 14 bits each, mirror flags, x-tile widths (see compact_rows, rmx_api.hip)
+    RMX_C_DST = 4u,       // (nothing stored) the written size is the window's
+    RMX_C_RATIO = 8u,     // (nothing stored) rx, ry, fsx, fsy are quotients of the sizes
+    RMX_C_COLOR0 = 16u,   // color[0..3], one dword each, those that differ between samples (four bits from here)
+    RMX_C_M4 = 256u,      // m[0..3]
+    RMX_C_M6 = 512u,      // m[0..5]
+    RMX_C_ORDER = 1024u,  // the sample this row belongs to (plan[2])
+    RMX_C_LAYOUT = 2048u  // two dwords, of the sample and not of the row: source offset (40 bits) and row stride (24 bits)
+};
+constexpr int RMX_C_WORDS = 768;  // 3 KB: 256 windows with their order, 192 colour twists, 128 matrices
+constexpr int RMX_C_TILE_WHOLE = 512;  // code k of an x-tile width: 0 the whole row (up to this many pixels), else this >> k
+
 struct RmxKArgs {
     const uint8_t *src;      // batch base, u8 NHWC
     void *dst;               // batch base
@@ -62,7 +82,12 @@ struct RmxKArgs {
     // wavefront -> (sample, strip) without a division, and samples dealt round-robin to the XCDs (see wave_to_sample)
     uint32_t inv_strips;         // ceil(2^32 / strips), or 0: divide
     uint32_t per_xcd, inv_per_xcd;  // samples per XCD (n / 8) and ceil(2^32 / per_xcd); per_xcd 0: samples in batch order
+    uint32_t compact;            // RMX_C_*: 0 when the rows are in `table`
+    uint32_t compact_words;      // dwords per sample in `rec`
+    RmxSample shared;            // what every sample's row holds
+    uint32_t rec[RMX_C_WORDS];
 };
+static_assert(sizeof(RmxKArgs) <= 4096, "kernel arguments are limited to 4 KB");
 
 #define RMX_WAVE 64
 

@@ -3,6 +3,8 @@
 #pragma once
 #include "rmx_common.h"
 
+#include <stddef.h>
+
 #define RMX_DEV __device__ __forceinline__
 
 namespace rmx {
@@ -24,8 +26,73 @@ RMX_DEV float round_u8(float v) {
     return __builtin_fminf(__builtin_fmaxf(v, 0.0f), 255.0f);
 }
 
+// The compact records of the kernel's arguments, read where the hardware put them (indexed as a member of the by-value struct,
+// they would be copied to scratch memory first).
+typedef const __attribute__((address_space(4))) uint32_t *karg_u32;
+RMX_DEV karg_u32 compact_record(const RmxKArgs &a, int i) {
+    return (karg_u32)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(RmxKArgs, rec)) +
+           (uint32_t)i * a.compact_words;
+}
+
+// Row i of the batch's parameter table: from device memory, or made again from the kernel's arguments (RMX_C_*). CAN: what a
+// record of this kernel's ops can hold. Everything is wave-uniform. The quotients are the host's (both IEEE divisions).
+template <uint32_t CAN>
+RMX_DEV RmxSample load_sample(const RmxKArgs &a, int i) {
+    if (!(a.compact & RMX_C_ON)) return a.table[i];
+    RmxSample P = a.shared;
+    karg_u32 r = compact_record(a, i);
+    if constexpr (CAN & RMX_C_WINDOW) {
+        if (a.compact & RMX_C_WINDOW) {
+            const uint32_t w0 = r[0], w1 = r[1];
+            r += 2;
+            P.src_x = (int32_t)(w0 & 0x3fffu);
+            P.src_y = (int32_t)((w0 >> 14) & 0x3fffu);
+            P.src_w = (int32_t)(w1 & 0x3fffu);
+            P.src_h = (int32_t)((w1 >> 14) & 0x3fffu);
+            P.flags |= (w0 >> 28) & (RMX_S_HFLIP | RMX_S_VFLIP);
+            if constexpr (CAN & RMX_C_DST) {
+                P.dst_w = P.src_w;
+                P.dst_h = P.src_h;
+            }
+            if constexpr (CAN & RMX_C_RATIO) {
+                const int whole = min(max(P.dst_w, 8), RMX_C_TILE_WHOLE);
+                const uint32_t t0 = (w0 >> 30) | ((w1 >> 31) << 2), t1 = (w1 >> 28) & 7u;
+                P.plan[0] = t0 ? RMX_C_TILE_WHOLE >> t0 : whole;
+                P.plan[1] = t1 ? RMX_C_TILE_WHOLE >> t1 : whole;
+                P.rx = (float)P.src_w / (float)P.rs_w;
+                P.ry = (float)P.src_h / (float)P.rs_h;
+                P.fsx = P.rx > 1.0f ? 1.0f / P.rx : 1.0f;
+                P.fsy = P.ry > 1.0f ? 1.0f / P.ry : 1.0f;
+            }
+        }
+    }
+    if constexpr (CAN & RMX_C_COLOR0) {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (a.compact & (RMX_C_COLOR0 << k)) P.color[k] = __builtin_bit_cast(float, *r++);
+    }
+    if constexpr (CAN & (RMX_C_M4 | RMX_C_M6)) {
+        if (a.compact & (RMX_C_M4 | RMX_C_M6)) {
+#pragma unroll
+            for (int k = 0; k < ((CAN & RMX_C_M6) ? 6 : 4); k++) P.m[k] = __builtin_bit_cast(float, r[k]);
+            r += (CAN & RMX_C_M6) ? 6 : 4;
+        }
+    }
+    if constexpr (CAN & RMX_C_RATIO) P.plan[2] = i;
+    if constexpr (CAN & RMX_C_ORDER) {
+        if (a.compact & RMX_C_ORDER) P.plan[2] = (int32_t)*r++;
+    }
+    return P;
+}
+
 // First pixel and row stride (bytes) of sample s: from the layout table of a ragged source, else the padded batch.
 RMX_DEV const uint8_t *sample_base(const RmxKArgs &a, int s, uint32_t &row_stride) {
+    if (a.compact & RMX_C_LAYOUT) {
+        karg_u32 r = compact_record(a, s) + a.compact_words - 2;
+        const uint32_t lo = r[0], hi = r[1];
+        row_stride = hi & 0xffffffu;
+        return a.src + (((uint64_t)(hi >> 24) << 32) | lo);
+    }
     if (a.layout) {
         const RmxSrcLayout L = a.layout[s];
         row_stride = L.row_stride;

@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
     int s, strip;
     wave_to_sample(a, wave, s, strip);
     // whole table row in one round trip (the empty statement keeps the fetch above the early exit)
-    const RmxSample P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_DST>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.flags), "s"(P.scale[0]), "s"(P.bias[2]));
 
     const int cw = P.dst_w, ch = P.dst_h;

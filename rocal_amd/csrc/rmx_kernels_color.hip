@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(256) rmx_color_kernel(RmxKArgs a) {
     // (a wavefront beyond the batch fetches the last wavefront's row: it stays for the workgroup's barrier and leaves then)
     wave_to_sample(a, min(wave, nwaves - 1), s, strip, false);
     // whole table row in one round trip (the empty statement keeps the fetch above the barrier and the early exit)
-    const RmxSample P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_DST | RMX_C_COLOR0>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.flags), "s"(P.color[0]), "s"(P.color[3]));
     if constexpr (KIND == COLOR_TWIST) {
         uint4 *ram = reinterpret_cast<uint4 *>(&tabs);

@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(256) rmx_point_kernel(RmxKArgs a) {
     // workgroups in launch order (no XCD renumbering): the whole device walks the batch as one contiguous address stream,
     // and dealing the samples would only break that stream up (measured: 11-16 % slower)
     wave_to_sample(a, wave, s, strip, false);
-    const RmxSample P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_DST | RMX_C_COLOR0>(a, s);
     const int w = P.dst_w, h = P.dst_h;
     const int srows = a.aux0;
     const int r0 = strip * srows;

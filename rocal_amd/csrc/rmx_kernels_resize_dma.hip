@@ -90,7 +90,7 @@ __global__ void __launch_bounds__(256) rmx_resize_dma_kernel(RmxKArgs a) {
     if (wave >= nwaves) return;
     int s, grp;
     wave_to_sample(a, wave, s, grp);
-    const RmxSample P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | (CHAIN == CHAIN_NONE ? 0u : RMX_C_M4)>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.pc_x), "s"(P.flags), "s"(P.rx), "s"(P.scale[0]), "s"(P.bias[2]), "s"(P.plan[1]));
 
     const int dw = P.dst_w, dh = P.dst_h;

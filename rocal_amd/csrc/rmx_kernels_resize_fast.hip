@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(256) rmx_resize_fast_kernel(RmxKArgs a) {
     // the whole 128-byte row at once: one memory round trip before the first use, not one per field group
     // (the empty statement "uses" fields from every part of the row, which keeps the compiler from sinking
     // part of the fetch below the early exit)
-    const RmxSample P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | (CHAIN == CHAIN_NONE ? 0u : RMX_C_M4)>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.pc_x), "s"(P.flags), "s"(P.rx), "s"(P.scale[0]), "s"(P.bias[2]), "s"(P.plan[0]));
 
     const int dw = P.dst_w, dh = P.dst_h;

@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(256) rmx_resize_kernel(RmxKArgs a) {
     if (wave >= nwaves) return;
     int s, strip;
     wave_to_sample(a, wave, s, strip);
-    const RmxSample &P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | (CHAIN == CHAIN_NONE ? 0u : RMX_C_M4)>(a, s);
 
     const int dw = P.dst_w, dh = P.dst_h;
     const int srows = a.aux0;

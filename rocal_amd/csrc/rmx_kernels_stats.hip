@@ -24,7 +24,7 @@ __global__ void __launch_bounds__(256) rmx_stats_reduce_kernel(RmxKArgs a, unsig
     if (wave >= nwaves) return;
     int s, strip;
     wave_to_sample(a, wave, s, strip, false);  // no XCD renumbering in this kernel: batch order keeps the address stream contiguous
-    const RmxSample &P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_DST>(a, s);
     const int w = P.dst_w, h = P.dst_h, x1 = P.src_x, y1 = P.src_y;
     const int r0 = strip * a.aux0;
     if (r0 >= h || w <= 0) return;

@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
     const int tiles_x = a.aux1;
     const int strip = part / tiles_x, tx = part - strip * tiles_x;
     // the whole table row in one round trip
-    const RmxSample P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | RMX_C_ORDER>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.pc_x), "s"(P.flags), "s"(P.rx), "s"(P.scale[0]), "s"(P.bias[2]), "s"(P.fsx));
     s = P.plan[2];  // (the host may have put the rows in another order: the row names its sample)
 

@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     const bool packed_ok = (a.aux1 & 1) != 0;
     const int ty = tile / tiles_x, tx = tile - ty * tiles_x;
     // the whole table row in one round trip
-    const RmxSample P = a.table[s];
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_M6>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.flags), "s"(P.m[0]), "s"(P.m[5]));
     const int dw = P.dst_w, dh = P.dst_h;
     const int X0 = tx * WTW, Y0 = ty * (WTH * passes);
