@@ -153,8 +153,8 @@ struct rmx_op {
     // shape): the batch is handed to the kernel as flat_h rows of 512 pixels per sample, so that all 64 lanes work whatever the
     // image width is (224 pixels are 28 groups of 8: two rows per step keep 56 lanes busy). 0: the images' own rows.
     int flat_h = 0;
-    int stats_mode = 0, stats_per_channel = 1;  // Normalize: what is computed on the device (bit 0 mean, bit 1 standard deviation)
-    float stats_scale = 1.0f, stats_shift = 0.0f;
+    bool own_moments = false;          // Normalize: the mean or the deviation of the last update is computed on the device
+    unsigned long long *moments = nullptr;  // ... from these shares (device workspace of the op, written in front of every streaming pass)
     rmx::KernelFn lds_fn[3] = {};  // kernels whose static LDS size has been asked of the runtime ([0] general, [1] fast, [2] mid)
     int lds_static[3] = {};
 };
@@ -296,9 +296,9 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
         case OP_TRANSPOSE:
             if (op->aux1) return false;  // (height and width change places: a kernel of its own)
             [[fallthrough]];
-        case OP_CMN: case OP_CROP: case OP_FLIP: case OP_TO_TENSOR: case OP_COLOR_TEMPERATURE:
+        case OP_CMN: case OP_CROP: case OP_FLIP: case OP_TO_TENSOR: case OP_COLOR_TEMPERATURE: case OP_NORMALIZE:
         case OP_COLOR_TWIST: case OP_BRIGHTNESS: case OP_CONTRAST: case OP_HUE: case OP_SATURATION: case OP_EXPOSURE: case OP_BLEND: {
-            const bool k1 = op->kind == OP_CMN || op->kind == OP_CROP || op->kind == OP_FLIP || op->kind == OP_TO_TENSOR || op->kind == OP_COLOR_TEMPERATURE || op->kind == OP_TRANSPOSE;
+            const bool k1 = op->kind == OP_CMN || op->kind == OP_CROP || op->kind == OP_FLIP || op->kind == OP_TO_TENSOR || op->kind == OP_COLOR_TEMPERATURE || op->kind == OP_NORMALIZE || op->kind == OP_TRANSPOSE;
             // (these kernels read the window's origin and the written size, which is the window's)
             for (int i = 0; i < op->n; i++)
                 if (t[i].src_w != t[i].dst_w || t[i].src_h != t[i].dst_h) return false;
@@ -605,6 +605,7 @@ int rmx_op_destroy(rmx_op *op) {
         if (ev) (void)hipEventDestroy(ev);
     if (op->h_table[0]) (void)hipHostFree(op->h_table[0]);
     if (op->d_table[0]) (void)hipFree(op->d_table[0]);
+    if (op->moments) (void)hipFree(op->moments);
     rmx_ctx *ctx = op->ctx;
     delete op;
     bool last;
@@ -745,13 +746,9 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
         a.inv_per_xcd = a.per_xcd > 1 ? recip(a.per_xcd) : 0u;
         if (a.per_xcd == 1) a.per_xcd = 0;  // (8..15 samples: nothing to deal)
     }
-    if (op->kind == OP_NORMALIZE) {
-        // moments of every sample's window (when asked for), then the FMA constants into the rows the streaming pass reads;
-        // the side table of the slot holds the given statistics (6 floats per sample) and, behind them, the 64-bit counters
-        const float *given = reinterpret_cast<const float *>(extra);
-        unsigned long long *counters = reinterpret_cast<unsigned long long *>(const_cast<uint8_t *>(extra) + (size_t)op->n * 24);
-        rmx::launch_stats(op->ctx->stream, a, counters, const_cast<RmxSample *>(table), given, op->stats_mode, op->stats_per_channel, op->stats_scale,
-                          op->stats_shift, op->stats_mode != 0);
+    if (op->own_moments) {  // shares of every sample's moments, which the streaming pass makes its constants from
+        a.extra = reinterpret_cast<const uint8_t *>(op->moments);
+        rmx::launch_moments(op->ctx->stream, a, op->moments);
         HIP_TRY(hipGetLastError());
     }
     void *kargs[1] = {&a};
@@ -942,10 +939,15 @@ int rmx_update_to_tensor(rmx_op *op, const float *multiplier, const float *offse
 /* ------------------------------------------------------------------ Normalize */
 
 int rmx_create_normalize(rmx_ctx *ctx, const rmx_tensor_desc *src, const rmx_tensor_desc *dst, int roi_type, rmx_op **out) {
-    // side table per sample: 6 floats of given statistics + 6 counters of 8 bytes
-    int rc = make_op(ctx, OP_NORMALIZE, src, dst, roi_type, out, 72);
+    int rc = make_op(ctx, OP_NORMALIZE, src, dst, roi_type, out);
     if (rc) return rc;
     (*out)->norm = true;
+    hipError_t e = hipMalloc((void **)&(*out)->moments, (size_t)src->n * 6 * RMX_MOMENT_PARTS * sizeof(unsigned long long));
+    if (e != hipSuccess) {
+        rmx_op_destroy(*out);
+        *out = nullptr;
+        return fail(RMX_ERR_HIP, "allocating the moments failed: %d (%s)", (int)e, hipGetErrorString(e));
+    }
     (*out)->fn = rmx::select_cmn_kernel(dst->dtype, dst->layout, true, 0, &(*out)->kernel_name);
     return RMX_OK;
 }
@@ -962,18 +964,26 @@ int rmx_update_normalize(rmx_op *op, const uint32_t *src_roi, uint32_t axis_mask
     int slot = -1;
     int rc = update_k1(op, src_roi, nullptr, nullptr, nullptr, nullptr, true, false, &slot);
     if (rc) return rc;
-    float *given = reinterpret_cast<float *>(slot_extra(op, op->h_table[slot]));
-    for (int i = 0; i < op->n; i++)
+    // given statistics, or neutral ones; with both given the constants are made here and the streaming pass runs alone
+    op->own_moments = !mean || !stddev;
+    for (int i = 0; i < op->n; i++) {
+        RmxSample &s = op->h_table[slot][i];
         for (int c = 0; c < 3; c++) {
-            given[(size_t)i * 6 + c] = mean ? mean[n_stats == 3 ? c : 0] : 0.0f;
-            given[(size_t)i * 6 + 3 + c] = stddev ? stddev[n_stats == 3 ? c : 0] : 1.0f;
+            s.m[c] = mean ? mean[n_stats == 3 ? c : 0] : 0.0f;
+            s.m[3 + c] = stddev ? stddev[n_stats == 3 ? c : 0] : 1.0f;
+            s.scale[c] = scale / s.m[3 + c];
+            s.bias[c] = std::fmaf(-s.m[c], s.scale[c], shift);
         }
-    op->stats_mode = (mean ? 0 : 1) | (stddev ? 0 : 2);
-    op->stats_per_channel = axis_mask == 3u ? 1 : 0;
-    op->stats_scale = scale;
-    op->stats_shift = shift;
+        s.color[0] = scale;
+        s.color[1] = shift;
+        s.flags |= (mean ? 0u : RMX_S_OWN_MEAN) | (stddev ? 0u : RMX_S_OWN_STD) | (axis_mask == 3u ? RMX_S_PER_CHANNEL : 0u);
+    }
+    const int knorm = op->own_moments ? 2 : 1;
+    op->fn = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, 0, &op->kernel_name);
+    if (op->fn_fast) op->fn_fast = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, 1, &op->fast_name);
+    if (op->fn_mid) op->fn_mid = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, 2, &op->mid_name);
     // the moments pass reads every source byte once more when something is computed
-    if (op->stats_mode) op->algo_bytes += op->algo_bytes / (1 + dtype_size(op->dst.dtype));
+    if (op->own_moments) op->algo_bytes += op->algo_bytes / (1 + dtype_size(op->dst.dtype));
     return commit_slot(op, slot);
 }
 

@@ -40,6 +40,9 @@ enum : uint32_t {
     RMX_S_HFLIP = 1u,
     RMX_S_VFLIP = 2u,
     RMX_S_CHREV = 4u,    // output channel k reads source channel 2-k
+    RMX_S_OWN_MEAN = 16u,  // Normalize: the mean / the deviation is the window's own (else m[0..2] / m[3..5]), one per channel or one
+    RMX_S_OWN_STD = 32u,   // for all three; color[0] and color[1] are scale and shift
+    RMX_S_PER_CHANNEL = 64u,
     RMX_S_EDGE_REF = 8u  // bilinear: both neighbours clamp to the window's last-but-one column / row (RMX_F_EDGE_REF)
 };
 
@@ -90,6 +93,7 @@ struct RmxKArgs {
 static_assert(sizeof(RmxKArgs) <= 4096, "kernel arguments are limited to 4 KB");
 
 #define RMX_WAVE 64
+#define RMX_MOMENT_PARTS 8  // workgroups per sample of the moments pass (Normalize): 6 x 8 shares, one per lane of a streaming wavefront
 
 // Hue shift of a sample in sextants (ColorTwist, Hue, Saturation). A pixel's hue before it is brought back into [0, 6] lies in
 // [shift - 1.0000002, shift + 5.0000002]; below RMX_HUE_SHIFT_LOW it can never reach 6, from RMX_HUE_SHIFT_HIGH on never fall

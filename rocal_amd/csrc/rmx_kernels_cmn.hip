@@ -28,8 +28,52 @@
 namespace rmx {
 
 enum { CMN_GENERAL = 0, CMN_FAST = 1, CMN_FAST_ANY = 2 };
+enum { NORM_NONE = 0, NORM_ROW = 1, NORM_OWN = 2 };
 
-template <typename T, int LAYOUT, bool NORM, int MODE>
+// FMA constants of a Normalize sample from the shares of its moments (rmx_kernels_stats.hip): lane 8 k + p holds share p of moment
+// k (three sums, three sums of squares), eight lanes add up, lane c makes channel c's constants. The double arithmetic runs
+// once per wavefront, in three lanes.
+struct OwnStats {
+    uint32_t flags;
+    float w, h, mean0, mean1, mean2, std0, std1, std2, scale, shift;
+};
+RMX_DEV void own_constants(const OwnStats o, const uint8_t *shares, int s, int lane, float (&sc)[3], float (&bi)[3]) {
+    static_assert(RMX_MOMENT_PARTS == 8, "eight lanes per moment");
+    const unsigned long long *mine = reinterpret_cast<const unsigned long long *>(shares) + (size_t)s * 6 * RMX_MOMENT_PARTS;
+    unsigned long long v = lane < 6 * RMX_MOMENT_PARTS ? mine[lane] : 0ull;
+#pragma unroll
+    for (int off = 1; off < RMX_MOMENT_PARTS; off <<= 1) v += __shfl_xor(v, off, RMX_WAVE);
+    const bool per_channel = (o.flags & RMX_S_PER_CHANNEL) != 0;
+    const int c = min(lane, 2);
+    double cnt = (double)o.w * (double)o.h;
+    unsigned long long isum = __shfl(v, 8 * c, RMX_WAVE), isq = __shfl(v, 24 + 8 * c, RMX_WAVE);
+    if (!per_channel) {
+        cnt *= 3.0;
+        isum = __shfl(isum, 0, RMX_WAVE) + __shfl(isum, 1, RMX_WAVE) + __shfl(isum, 2, RMX_WAVE);
+        isq = __shfl(isq, 0, RMX_WAVE) + __shfl(isq, 1, RMX_WAVE) + __shfl(isq, 2, RMX_WAVE);
+    }
+    const double sum = (double)isum, sq = (double)isq;
+    float mean = c == 0 ? o.mean0 : (c == 1 ? o.mean1 : o.mean2), sigma = c == 0 ? o.std0 : (c == 1 ? o.std1 : o.std2);
+    if (cnt > 0.0) {
+        const double m = (o.flags & RMX_S_OWN_MEAN) ? sum / cnt : (double)mean;
+        if (o.flags & RMX_S_OWN_MEAN) mean = (float)m;
+        if (o.flags & RMX_S_OWN_STD) {
+            // sum of (x - m)^2 = sq - 2 m sum + cnt m^2, every term exact or correctly rounded in double
+            double var = (sq - 2.0 * m * sum + cnt * m * m) / cnt;
+            if (var < 0.0) var = 0.0;
+            sigma = (float)__builtin_sqrt(var);
+        }
+    }
+    const float sa = sigma != 0.0f ? o.scale / sigma : 0.0f;
+    const float sb = __builtin_fmaf(-mean, sa, o.shift);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        sc[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sa), k));
+        bi[k] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sb), k));
+    }
+}
+
+template <typename T, int LAYOUT, int NORM, int MODE>
 __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
     constexpr bool FAST = MODE != CMN_GENERAL;
     constexpr bool ANY = MODE == CMN_FAST_ANY;
@@ -73,6 +117,14 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
         sc[c] = P.scale[c];
         bi[c] = P.bias[c];
     }
+    // (made behind the start of the first pixel loads where there is a pipeline, so that the two round trips and the double
+    // arithmetic run while those are on their way)
+    const OwnStats stats = {P.flags, (float)P.dst_w, (float)P.dst_h, P.m[0], P.m[1], P.m[2], P.m[3], P.m[4], P.m[5], P.color[0], P.color[1]};
+    auto own = [&](int xt) {
+        if constexpr (NORM == NORM_OWN) {
+            if (xt == 0) own_constants(stats, a.extra, s, lane, sc, bi);
+        }
+    };
 
     for (int xt = 0; xt < cw; xt += RMX_WAVE * PX) {
         const int tw = min(cw - xt, RMX_WAVE * PX);
@@ -105,7 +157,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
                         v[2][k] = t;
                     }
                 }
-                if constexpr (NORM) {
+                if constexpr (NORM != NORM_NONE) {
 #pragma unroll
                     for (int c = 0; c < 3; c++)
 #pragma unroll
@@ -159,6 +211,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
                 issue(r0, ta, ua, pa);
                 for (int base = r0; base < r1; base += 2 * step) {
                     if (base + step < r1) issue(base + step, tb, ub, pb);
+                    if (NORM == NORM_OWN && base == r0) own(xt);
                     consume(base, ta, ua, pa);
                     if (base + step < r1) {
                         if (base + 2 * step < r1) issue(base + 2 * step, ta, ua, pa);
@@ -167,6 +220,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
                 }
             } else {
                 // last bytes of the batch buffer: the bounds-checked loader, row by row
+                own(xt);
                 for (int r = r0 + lr; r < r1 && active; r += G) {
                     uint32_t ph, w[6];
                     const uint32_t *q = row_ptr(r, ph);
@@ -175,6 +229,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
                 }
             }
         } else {
+            own(xt);
             for (int r = r0 + lr; r < r1 && active; r += G) {
                 const int sy = y1 + (vf ? (ch - 1 - r) : r);
                 const uint8_t *p = simg + (size_t)sy * row_stride + (size_t)sx0 * 3;
@@ -190,7 +245,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
                         v[2][k] = t;
                     }
                 }
-                if constexpr (NORM) {
+                if constexpr (NORM != NORM_NONE) {
 #pragma unroll
                     for (int c = 0; c < 3; c++)
 #pragma unroll
@@ -202,21 +257,21 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
     }
 }
 
-template <typename T, int LAYOUT>
-static KernelFn pick_variant(bool norm, int mode) {
-    if (mode == CMN_FAST) return norm ? (KernelFn)rmx_cmn_kernel<T, LAYOUT, true, CMN_FAST> : (KernelFn)rmx_cmn_kernel<T, LAYOUT, false, CMN_FAST>;
-    if (mode == CMN_FAST_ANY) return norm ? (KernelFn)rmx_cmn_kernel<T, LAYOUT, true, CMN_FAST_ANY> : (KernelFn)rmx_cmn_kernel<T, LAYOUT, false, CMN_FAST_ANY>;
-    return norm ? (KernelFn)rmx_cmn_kernel<T, LAYOUT, true, CMN_GENERAL> : (KernelFn)rmx_cmn_kernel<T, LAYOUT, false, CMN_GENERAL>;
+template <typename T, int LAYOUT, int NORM>
+static KernelFn pick_mode(int mode) {
+    if (mode == CMN_FAST) return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_FAST>;
+    if (mode == CMN_FAST_ANY) return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_FAST_ANY>;
+    return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_GENERAL>;
 }
 
 template <typename T>
-static KernelFn pick_layout(int layout, bool norm, int mode) {
-    if (layout == RMX_NCHW) return pick_variant<T, RMX_NCHW>(norm, mode);
-    return pick_variant<T, RMX_NHWC>(norm, mode);
+static KernelFn pick_layout(int layout, int norm, int mode) {
+    if (layout == RMX_NCHW) return norm == NORM_OWN ? pick_mode<T, RMX_NCHW, NORM_OWN>(mode) : (norm ? pick_mode<T, RMX_NCHW, NORM_ROW>(mode) : pick_mode<T, RMX_NCHW, NORM_NONE>(mode));
+    return norm == NORM_OWN ? pick_mode<T, RMX_NHWC, NORM_OWN>(mode) : (norm ? pick_mode<T, RMX_NHWC, NORM_ROW>(mode) : pick_mode<T, RMX_NHWC, NORM_NONE>(mode));
 }
 
 // mode: 0 the general kernel, 1 whole groups and 16-byte aligned destination rows, 2 rows of 8 pixels and more at any alignment
-KernelFn select_cmn_kernel(int dtype, int layout, bool norm, int mode, const char **name) {
+KernelFn select_cmn_kernel(int dtype, int layout, int norm, int mode, const char **name) {
     static const char *names[3] = {"rmx_cmn_kernel<float", "rmx_cmn_kernel<__half", "rmx_cmn_kernel<unsigned char"};
     *name = names[dtype];
     switch (dtype) {

@@ -6,7 +6,8 @@
 namespace rmx {
 typedef void (*KernelFn)(RmxKArgs);
 
-KernelFn select_cmn_kernel(int dtype, int layout, bool norm, int mode, const char **name);
+// norm: 0 plain values, 1 the row's scale and bias, 2 constants from the sample's own moments (Normalize)
+KernelFn select_cmn_kernel(int dtype, int layout, int norm, int mode, const char **name);
 KernelFn select_resize_linear_kernel(int dtype, int layout, bool norm, bool quant, int chain, const char **name);
 KernelFn select_resize_fast_kernel(int dtype, int layout, bool norm, bool quant, int chain, const char **name);
 KernelFn select_resize_dma_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool aligned, const char **name);
@@ -23,9 +24,8 @@ KernelFn select_warp_kernel(int interp, int dtype, int layout, bool raw, const c
 #define RMX_WARP_RAW_PIECES 11
 #endif
 constexpr int kWarpRawPieces = RMX_WARP_RAW_PIECES;
-// Normalize: (reduce: zero + per-sample integer moments,) then the FMA constants into the rows of `table` (device memory)
-void launch_stats(hipStream_t stream, const RmxKArgs &a, unsigned long long *counters, RmxSample *table, const float *given, int mode, int per_channel,
-                  float scale, float shift, bool reduce);
+// Normalize: integer moments of every sample's window, RMX_MOMENT_PARTS shares of six 64-bit numbers per sample
+void launch_moments(hipStream_t stream, const RmxKArgs &a, unsigned long long *parts);
 void launch_copy(hipStream_t stream, const void *src, void *dst, size_t nbytes, int num_cus);
 // mode 0 copy, 1 read only, 2 write only; groups_per_cu 0 = the default (16)
 void launch_stream(hipStream_t stream, int mode, const void *src, void *dst, size_t nbytes, int num_cus, int groups_per_cu);
