@@ -150,8 +150,8 @@ struct rmx_op {
     uint64_t algo_bytes = 0;
     int tri_rows_in_flight = 0;  // streaming triangular kernel: accumulator sets (2 or 4), 0 for every other kernel
     // Point operations on whole frames (every sample's window is the whole padded image, source and destination of one
-    // shape): the batch is handed to the kernel as flat_h rows of 512 pixels per sample, so that all 64 lanes work whatever the
-    // image width is (224 pixels are 28 groups of 8: two rows per step keep 56 lanes busy). 0: the images' own rows.
+    // shape): the kernel walks a frame as flat_h rows of 512 pixels, so that all 64 lanes work whatever the image width is
+    // (224 pixels are 28 groups of 8: two rows per step keep 56 lanes busy; 299 pixels keep 38). 0: the images' own rows.
     int flat_h = 0;
     bool own_moments = false;          // Normalize: the mean or the deviation of the last update is computed on the device
     unsigned long long *moments = nullptr;  // ... from these shares (device workspace of the op, written in front of every streaming pass)
@@ -468,25 +468,21 @@ int pick_tile_width(int w, const TileCost &tc, long cap, NeedOf need_of, long *n
     return best;
 }
 
-// Whole-frame point operations as rows of kFlatRow pixels: true (and the rows of `t` rewritten) when every sample's window
-// is the whole padded source image, the destination has the source's shape, the pixels of a sample divide into whole rows
-// of kFlatRow, and the source is the dense tensor. The kernel then sees flat_h rows of kFlatRow pixels per sample.
+// Whole-frame point operations as rows of kFlatRow pixels (FlatRows, rmx_device.h): true when every sample's window is the whole
+// padded source image, the destination has the source's shape, and the source is the dense tensor. A frame that is as wide
+// as such a row is one already.
 constexpr int kFlatRow = 512;  // one step of 64 lanes x 8 pixels
-bool flatten_whole_frames(rmx_op *op, RmxSample *t) {
+bool flatten_whole_frames(rmx_op *op, const RmxSample *t) {
     op->flat_h = 0;
     if (!op->ctx->flat_frames || !op->layout.empty()) return false;
     if (op->src.w != op->dst.w || op->src.h != op->dst.h) return false;
     const uint64_t px = (uint64_t)op->src.w * op->src.h;
-    if (px % kFlatRow != 0 || px / kFlatRow > 0x7fffff || op->src.w == (uint32_t)kFlatRow) return false;
+    if (px < 8 || px > 0x7fffff00ull / 3 || op->src.w == (uint32_t)kFlatRow) return false;
     for (int i = 0; i < op->n; i++) {
         const RmxSample &s = t[i];
         if (s.src_x != 0 || s.src_y != 0 || s.src_w != (int32_t)op->src.w || s.src_h != (int32_t)op->src.h || s.dst_w != s.src_w || s.dst_h != s.src_h) return false;
     }
-    op->flat_h = (int)(px / kFlatRow);
-    for (int i = 0; i < op->n; i++) {
-        t[i].src_w = t[i].dst_w = kFlatRow;
-        t[i].src_h = t[i].dst_h = op->flat_h;
-    }
+    op->flat_h = (int)((px + kFlatRow - 1) / kFlatRow);
     return true;
 }
 
@@ -694,10 +690,6 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
     a.src_w = (int)op->src.w;
     a.dst_h = (int)op->dst.h;
     a.dst_w = (int)op->dst.w;
-    if (op->flat_h) {
-        a.src_h = a.dst_h = op->flat_h;
-        a.src_w = a.dst_w = kFlatRow;
-    }
     a.strips = op->strips;
     a.lds_bytes = op->lds_per_wave;
     a.aux0 = op->aux0;
@@ -866,11 +858,11 @@ static int update_k1(rmx_op *op, const uint32_t *roi, const float *scale, const 
     }
     plan_streaming(op, max_rows, rows);
     // aligned specialisation: whole 8-pixel groups everywhere and 16-byte aligned destination rows
-    bool aligned = op->flat_h ? true : op->dst.w % 8 == 0;
-    for (int i = 0; i < op->n && aligned; i++) aligned = (t[i].dst_w % 8 == 0);
+    bool aligned = op->flat_h ? ((uint64_t)op->dst.w * op->dst.h) % 16 == 0 : op->dst.w % 8 == 0;
+    for (int i = 0; i < op->n && aligned && !op->flat_h; i++) aligned = (t[i].dst_w % 8 == 0);
     op->fn_fast = nullptr;
     if (aligned) {
-        op->fn_fast = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, op->norm, 1, &op->fast_name);
+        op->fn_fast = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, op->norm, op->flat_h ? 3 : 1, &op->fast_name);
         op->fast_strips = op->strips;
         op->fast_lds = 0;
         op->fast_rows = op->aux0;
@@ -880,10 +872,10 @@ static int update_k1(rmx_op *op, const uint32_t *roi, const float *scale, const 
     // the same pipeline for rows of any width from 8 pixels on and a destination at any element (also what an aligned plan
     // falls back to when the destination base it is launched on is not 16-byte aligned)
     bool wide8 = true;
-    for (int i = 0; i < op->n && wide8; i++) wide8 = t[i].dst_w >= 8 || t[i].dst_w <= 0 || t[i].dst_h <= 0;
+    for (int i = 0; i < op->n && wide8 && !op->flat_h; i++) wide8 = t[i].dst_w >= 8 || t[i].dst_w <= 0 || t[i].dst_h <= 0;
     op->fn_mid = nullptr;
     if (wide8) {
-        op->fn_mid = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, op->norm, 2, &op->mid_name);
+        op->fn_mid = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, op->norm, op->flat_h ? 4 : 2, &op->mid_name);
         op->mid_strips = op->strips;
         op->mid_lds = 0;
         op->mid_rows = op->aux0;
@@ -980,8 +972,8 @@ int rmx_update_normalize(rmx_op *op, const uint32_t *src_roi, uint32_t axis_mask
     }
     const int knorm = op->own_moments ? 2 : 1;
     op->fn = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, 0, &op->kernel_name);
-    if (op->fn_fast) op->fn_fast = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, 1, &op->fast_name);
-    if (op->fn_mid) op->fn_mid = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, 2, &op->mid_name);
+    if (op->fn_fast) op->fn_fast = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, op->flat_h ? 3 : 1, &op->fast_name);
+    if (op->fn_mid) op->fn_mid = rmx::select_cmn_kernel(op->dst.dtype, op->dst.layout, knorm, op->flat_h ? 4 : 2, &op->mid_name);
     // the moments pass reads every source byte once more when something is computed
     if (op->own_moments) op->algo_bytes += op->algo_bytes / (1 + dtype_size(op->dst.dtype));
     return commit_slot(op, slot);
@@ -1650,8 +1642,8 @@ static int update_color(rmx_op *op, const uint32_t *roi, const float *p0, const 
     }
     plan_streaming(op, max_rows, rows);
     // aligned specialisation: whole 8-pixel groups everywhere and 16-byte aligned destination rows
-    bool aligned = op->flat_h ? true : op->dst.w % 8 == 0;
-    for (int i = 0; i < op->n && aligned; i++) aligned = (t[i].dst_w % 8 == 0);
+    bool aligned = op->flat_h ? ((uint64_t)op->dst.w * op->dst.h) % 16 == 0 : op->dst.w % 8 == 0;
+    for (int i = 0; i < op->n && aligned && !op->flat_h; i++) aligned = (t[i].dst_w % 8 == 0);
     op->fn_fast = nullptr;
     // kernel kind: 0 linear, 1 twist, 2 twist with one comparison for the hue's way back into range (no shift near one sextant)
     int kkind = 0;
@@ -1661,7 +1653,7 @@ static int update_color(rmx_op *op, const uint32_t *roi, const float *p0, const 
             if (!(t[i].color[2] < RMX_HUE_SHIFT_LOW || t[i].color[2] >= RMX_HUE_SHIFT_HIGH)) kkind = 1;
     }
     if (aligned) {
-        op->fn_fast = rmx::select_color_kernel(kkind, op->dst.dtype, op->dst.layout, 1, &op->fast_name);
+        op->fn_fast = rmx::select_color_kernel(kkind, op->dst.dtype, op->dst.layout, op->flat_h ? 3 : 1, &op->fast_name);
         op->fast_strips = op->strips;
         op->fast_lds = 0;
         op->fast_rows = op->aux0;
@@ -1670,10 +1662,10 @@ static int update_color(rmx_op *op, const uint32_t *roi, const float *p0, const 
     }
     // the same pipeline for rows of any width from 8 pixels on and a destination at any element
     bool wide8 = true;
-    for (int i = 0; i < op->n && wide8; i++) wide8 = t[i].dst_w >= 8 || t[i].dst_w <= 0 || t[i].dst_h <= 0;
+    for (int i = 0; i < op->n && wide8 && !op->flat_h; i++) wide8 = t[i].dst_w >= 8 || t[i].dst_w <= 0 || t[i].dst_h <= 0;
     op->fn_mid = nullptr;
     if (wide8) {
-        op->fn_mid = rmx::select_color_kernel(kkind, op->dst.dtype, op->dst.layout, 2, &op->mid_name);
+        op->fn_mid = rmx::select_color_kernel(kkind, op->dst.dtype, op->dst.layout, op->flat_h ? 4 : 2, &op->mid_name);
         op->mid_strips = op->strips;
         op->mid_lds = 0;
         op->mid_rows = op->aux0;
@@ -1810,11 +1802,11 @@ static int update_point(rmx_op *op, const uint32_t *roi, const float *p0, const 
         rows = op->ctx->k3_flat_rows ? op->ctx->k3_flat_rows : (op->kind == OP_GAMMA ? 1 : 2);
     }
     plan_streaming(op, max_rows, rows);
-    bool aligned = op->flat_h ? true : op->dst.w % 8 == 0;
-    for (int i = 0; i < op->n && aligned; i++) aligned = (t[i].dst_w % 8 == 0);
+    bool aligned = op->flat_h ? ((uint64_t)op->dst.w * op->dst.h) % 16 == 0 : op->dst.w % 8 == 0;
+    for (int i = 0; i < op->n && aligned && !op->flat_h; i++) aligned = (t[i].dst_w % 8 == 0);
     op->fn_fast = nullptr;
     if (aligned) {
-        op->fn_fast = rmx::select_point_kernel(op->kind == OP_BLEND ? 1 : 0, op->dst.dtype, op->dst.layout, 1, &op->fast_name);
+        op->fn_fast = rmx::select_point_kernel(op->kind == OP_BLEND ? 1 : 0, op->dst.dtype, op->dst.layout, op->flat_h ? 3 : 1, &op->fast_name);
         op->fast_strips = op->strips;
         op->fast_lds = 0;
         op->fast_rows = op->aux0;
@@ -1823,10 +1815,10 @@ static int update_point(rmx_op *op, const uint32_t *roi, const float *p0, const 
     }
     // the same pipeline for rows of any width from 8 pixels on and a destination at any element
     bool wide8 = true;
-    for (int i = 0; i < op->n && wide8; i++) wide8 = t[i].dst_w >= 8 || t[i].dst_w <= 0 || t[i].dst_h <= 0;
+    for (int i = 0; i < op->n && wide8 && !op->flat_h; i++) wide8 = t[i].dst_w >= 8 || t[i].dst_w <= 0 || t[i].dst_h <= 0;
     op->fn_mid = nullptr;
     if (wide8) {
-        op->fn_mid = rmx::select_point_kernel(op->kind == OP_BLEND ? 1 : 0, op->dst.dtype, op->dst.layout, 2, &op->mid_name);
+        op->fn_mid = rmx::select_point_kernel(op->kind == OP_BLEND ? 1 : 0, op->dst.dtype, op->dst.layout, op->flat_h ? 4 : 2, &op->mid_name);
         op->mid_strips = op->strips;
         op->mid_lds = 0;
         op->mid_rows = op->aux0;

@@ -212,6 +212,40 @@ RMX_DEV uint32_t load_raw4(const uint8_t *p, const uint8_t *buf_end, uint32_t (&
     return phase;
 }
 
+// A whole frame as rows of FLAT_ROW pixels, for operations that do not know the image's own rows: every lane of a wavefront takes
+// 8 pixels whatever the image is wide (a 299-pixel row fills 38 lanes), and a wavefront's loads and stores are contiguous
+// kilobytes. Frames are contiguous in source and destination (no crop, no padding); the last row takes what is left, and where
+// that is fewer than 8 pixels, 8 of the row before: no group reaches into pixels of another wavefront.
+constexpr int FLAT_ROW = RMX_WAVE * PX;
+struct FlatRows {
+    int px, n, adj;
+    RMX_DEV explicit FlatRows(int pixels) : px(pixels), n((pixels + FLAT_ROW - 1) / FLAT_ROW) {
+        const int rest = pixels - (n - 1) * FLAT_ROW;
+        adj = (rest < PX && n > 1) ? PX : 0;
+    }
+    RMX_DEV int start(int r) const { return r * FLAT_ROW - (r == n - 1 ? adj : 0); }
+    RMX_DEV int end(int r) const { return r >= n - 1 ? px : start(r + 1); }
+};
+
+// 8 pixels from pixel x of a frame on; `inside`: 28 bytes from the dword below them lie in the batch buffer (wave-uniform)
+RMX_DEV void flat_load(const uint8_t *simg, int x, const uint8_t *buf_end, bool inside, uint32_t (&d)[7], uint32_t &ph) {
+    const uint8_t *p = simg + (size_t)x * 3;
+    ph = (uint32_t)((uintptr_t)p & 3u);
+    const uint32_t *q = reinterpret_cast<const uint32_t *>(p - ph);
+    if (inside) {
+        const u32x4_a4 t = *reinterpret_cast<const u32x4_a4 *>(q);
+        const u32x3_a4 u = *reinterpret_cast<const u32x3_a4 *>(q + 4);
+        d[0] = t.x; d[1] = t.y; d[2] = t.z; d[3] = t.w; d[4] = u.x; d[5] = u.y; d[6] = u.z;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 7; i++) d[i] = ((const uint8_t *)(q + i) < buf_end) ? q[i] : 0u;
+    }
+}
+RMX_DEV void realign6(const uint32_t (&d)[7], uint32_t ph, uint32_t (&w)[6]) {
+#pragma unroll
+    for (int j = 0; j < 6; j++) w[j] = __builtin_amdgcn_alignbyte(d[j + 1], d[j], ph);
+}
+
 // raw dwords + byte phase -> 4 packed pixels expanded to one dword each (top byte is don't-care)
 RMX_DEV uint4 expand4(const uint32_t (&d)[4], uint32_t phase) {
     uint32_t w0 = __builtin_amdgcn_alignbyte(d[1], d[0], phase);
@@ -605,6 +639,19 @@ RMX_DEV void store_packed_coalesced_any(uint32_t *slab, int grp0, int l, int L, 
         T *seg = sample + ((size_t)y * W + xs) * 3;
         store_run_coalesced_any<PX * 3, NT>(slab, reinterpret_cast<uint8_t *>(seg), grp0, l, L, 3 * (x0 - xs), 3 * tw, g.w);
     }
+}
+
+// A lane's group of a flat row (FlatRows): pixels x .. x + 7 of a frame of px pixels, `start` the row's first pixel, len its length.
+// ALIGNED: frames of whole groups at 16-byte aligned addresses. Called by the L lanes of the row together.
+template <typename T, int LAYOUT, bool NT, bool ALIGNED>
+RMX_DEV void flat_store(uint32_t *slab, T *dimg, int px, int start, int len, int lane, int L, int x, const PackedGroup<T> &g) {
+    if constexpr (ALIGNED && coalesce_pays<T, LAYOUT>()) store_packed_coalesced<T, LAYOUT, NT>(slab, 0, lane, L, dimg, 1, px, 0, x, g);
+    else if constexpr (sizeof(T) == 4) store_packed_coalesced_any<T, LAYOUT, NT>(slab, 0, lane, L, start, len, dimg, 1, px, 0, x, g);
+    else store_packed<T, LAYOUT, NT, !ALIGNED>(dimg, 1, px, 0, x, g);
+}
+template <typename T, int LAYOUT, bool ALIGNED>
+constexpr bool flat_coalesces() {
+    return (ALIGNED && coalesce_pays<T, LAYOUT>()) || sizeof(T) == 4;
 }
 
 // Write one lane's group of N horizontally adjacent pixels (v[c][k], k-th pixel of the group)

@@ -27,7 +27,8 @@
 
 namespace rmx {
 
-enum { CMN_GENERAL = 0, CMN_FAST = 1, CMN_FAST_ANY = 2 };
+// CMN_FLAT, CMN_FLAT_ANY: whole frames that are not mirrored, as rows of FLAT_ROW pixels (with aligned groups, or any)
+enum { CMN_GENERAL = 0, CMN_FAST = 1, CMN_FAST_ANY = 2, CMN_FLAT = 3, CMN_FLAT_ANY = 4 };
 enum { NORM_NONE = 0, NORM_ROW = 1, NORM_OWN = 2 };
 
 // FMA constants of a Normalize sample from the shares of its moments (rmx_kernels_stats.hip): lane 8 k + p holds share p of moment
@@ -75,10 +76,11 @@ RMX_DEV void own_constants(const OwnStats o, const uint8_t *shares, int s, int l
 
 template <typename T, int LAYOUT, int NORM, int MODE>
 __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
-    constexpr bool FAST = MODE != CMN_GENERAL;
+    constexpr bool FAST = MODE == CMN_FAST || MODE == CMN_FAST_ANY;
     constexpr bool ANY = MODE == CMN_FAST_ANY;
     // LDS slab through which the lanes of a row exchange their runs before storing (see store_packed_coalesced)
-    constexpr bool COALESCE = (MODE == CMN_FAST && coalesce_pays<T, LAYOUT>()) || (ANY && sizeof(T) == 4);
+    constexpr bool FLAT = MODE == CMN_FLAT || MODE == CMN_FLAT_ANY;
+    constexpr bool COALESCE = FLAT ? flat_coalesces<T, LAYOUT, MODE == CMN_FLAT>() : (MODE == CMN_FAST && coalesce_pays<T, LAYOUT>()) || (ANY && sizeof(T) == 4);
     uint32_t *slab = nullptr;
     if constexpr (COALESCE) {
         __shared__ __attribute__((aligned(16))) uint32_t slabs[4 * RMX_WAVE * coalesce_slab_dwords<T, LAYOUT>()];
@@ -98,7 +100,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
     const int cw = P.dst_w, ch = P.dst_h;
     const int srows = a.aux0;
     const int r0 = strip * srows;
-    if (r0 >= ch) return;
+    if (r0 >= (FLAT ? FlatRows(a.dst_h * a.dst_w).n : ch)) return;
     const int r1 = min(r0 + srows, ch);
     const bool hf = (P.flags & RMX_S_HFLIP) != 0;
     const bool vf = (P.flags & RMX_S_VFLIP) != 0;
@@ -126,6 +128,54 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
         }
     };
 
+    auto epilogue = [&](float (&v)[3][PX]) {
+        if (chrev) {
+#pragma unroll
+            for (int k = 0; k < PX; k++) {
+                const float t = v[0][k];
+                v[0][k] = v[2][k];
+                v[2][k] = t;
+            }
+        }
+        if constexpr (NORM != NORM_NONE) {
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+#pragma unroll
+                for (int k = 0; k < PX; k++) v[c][k] = __builtin_fmaf(v[c][k], sc[c], bi[c]);
+        }
+    };
+
+    if constexpr (FLAT) {
+        const FlatRows rows(a.dst_h * a.dst_w);
+        const int f1 = min(r0 + srows, rows.n);
+        const bool inside = simg + (size_t)rows.end(f1 - 1) * 3 + 4 <= buf_end;
+        constexpr int NI = 2;
+        for (int rb = r0; rb < f1; rb += NI) {
+            uint32_t d[NI][7], ph[NI];
+#pragma unroll
+            for (int i = 0; i < NI; i++) {  // (a row beyond the strip repeats its last one and is not stored; so do lanes beyond a row)
+                const int r = min(rb + i, f1 - 1), start = rows.start(r), len = rows.end(r) - start;
+                flat_load(simg, start + min(lane * PX, len - PX), buf_end, inside, d[i], ph[i]);
+            }
+            if (NORM == NORM_OWN && rb == r0) own(0);
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int r = rb + i, start = rows.start(r), len = rows.end(r) - start, L = (len + PX - 1) / PX;
+                if (r < f1 && lane < L) {
+                    uint32_t w[6];
+                    realign6(d[i], ph[i], w);
+                    float v[3][PX];
+                    unpack8(w, v);
+                    epilogue(v);
+                    PackedGroup<T> packed;
+                    pack_group_dir<T, LAYOUT, false>(v, packed);
+                    flat_store<T, LAYOUT, RMX_K1_NT, MODE == CMN_FLAT>(slab, dimg, rows.px, start, len, lane, L, start + min(lane * PX, len - PX), packed);
+                }
+            }
+        }
+        return;
+    }
+
     for (int xt = 0; xt < cw; xt += RMX_WAVE * PX) {
         const int tw = min(cw - xt, RMX_WAVE * PX);
         const int L = (tw + PX - 1) / PX;  // lanes per row, <= 64
@@ -149,20 +199,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
             auto finish = [&](int r, const uint32_t (&w)[6]) {
                 float v[3][PX];
                 unpack8(w, v);
-                if (chrev) {
-#pragma unroll
-                    for (int k = 0; k < PX; k++) {
-                        const float t = v[0][k];
-                        v[0][k] = v[2][k];
-                        v[2][k] = t;
-                    }
-                }
-                if constexpr (NORM != NORM_NONE) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++)
-#pragma unroll
-                        for (int k = 0; k < PX; k++) v[c][k] = __builtin_fmaf(v[c][k], sc[c], bi[c]);
-                }
+                epilogue(v);
                 PackedGroup<T> packed;
                 pack_group<T, LAYOUT>(v, hf, packed);
                 if constexpr (COALESCE && ANY) store_packed_coalesced_any<T, LAYOUT, RMX_K1_NT>(slab, lane - g, g, L, min(xt, cw - PX), xt + tw - min(xt, cw - PX), dimg, a.dst_h, a.dst_w, r, gx, packed);  // (a tile narrower than 8 pixels: its one group reaches back into the tile before)
@@ -237,20 +274,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
                 load_realigned<7>(p, buf_end, w);
                 float v[3][PX];
                 unpack8(w, v);
-                if (chrev) {
-#pragma unroll
-                    for (int k = 0; k < PX; k++) {
-                        const float t = v[0][k];
-                        v[0][k] = v[2][k];
-                        v[2][k] = t;
-                    }
-                }
-                if constexpr (NORM != NORM_NONE) {
-#pragma unroll
-                    for (int c = 0; c < 3; c++)
-#pragma unroll
-                        for (int k = 0; k < PX; k++) v[c][k] = __builtin_fmaf(v[c][k], sc[c], bi[c]);
-                }
+                epilogue(v);
                 store_group<T, LAYOUT>(dimg, a.dst_h, a.dst_w, r, gx, cnt, v, hf);
             }
         }
@@ -261,6 +285,8 @@ template <typename T, int LAYOUT, int NORM>
 static KernelFn pick_mode(int mode) {
     if (mode == CMN_FAST) return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_FAST>;
     if (mode == CMN_FAST_ANY) return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_FAST_ANY>;
+    if (mode == CMN_FLAT) return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_FLAT>;
+    if (mode == CMN_FLAT_ANY) return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_FLAT_ANY>;
     return (KernelFn)rmx_cmn_kernel<T, LAYOUT, NORM, CMN_GENERAL>;
 }
 
@@ -270,7 +296,8 @@ static KernelFn pick_layout(int layout, int norm, int mode) {
     return norm == NORM_OWN ? pick_mode<T, RMX_NHWC, NORM_OWN>(mode) : (norm ? pick_mode<T, RMX_NHWC, NORM_ROW>(mode) : pick_mode<T, RMX_NHWC, NORM_NONE>(mode));
 }
 
-// mode: 0 the general kernel, 1 whole groups and 16-byte aligned destination rows, 2 rows of 8 pixels and more at any alignment
+// mode: 0 the general kernel, 1 whole groups and 16-byte aligned destination rows, 2 rows of 8 pixels and more at any alignment,
+// 3 / 4 whole frames as rows of 512 pixels, with whole aligned groups / any
 KernelFn select_cmn_kernel(int dtype, int layout, int norm, int mode, const char **name) {
     static const char *names[3] = {"rmx_cmn_kernel<float", "rmx_cmn_kernel<__half", "rmx_cmn_kernel<unsigned char"};
     *name = names[dtype];

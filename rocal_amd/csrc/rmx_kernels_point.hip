@@ -20,15 +20,17 @@ RMX_DEV void unpack8_table(const uint32_t (&w)[6], const uint8_t *lut, float (&v
 
 // MODE: 0 the general form; 1 whole 8-pixel groups and 16-byte aligned destination rows; 2 rows of 8 pixels and more at any
 // alignment: the pipeline of 1, the short last group of a row moved left until it is whole (it recomputes up to seven pixels of
-// its neighbour and stores the same values to the same places), groups stored at the element's own alignment.
+// its neighbour and stores the same values to the same places), groups stored at the element's own alignment; 3 / 4 whole frames
+// as rows of FLAT_ROW pixels (FlatRows), with whole aligned groups / any.
 template <typename T, int LAYOUT, int KIND, int MODE>
 __global__ void __launch_bounds__(256) rmx_point_kernel(RmxKArgs a) {
-    constexpr bool FAST = MODE != 0;
+    constexpr bool FAST = MODE == 1 || MODE == 2;
     constexpr bool ANY = MODE == 2;
+    constexpr bool FLAT = MODE >= 3;
     __shared__ uint32_t lut_words[4][64];  // one 256-byte table per wavefront of the workgroup
     const int lane = threadIdx.x & (RMX_WAVE - 1);
     // fp32 and interleaved fp16 outputs: the lanes of a row exchange their runs through LDS before storing (store_packed_coalesced)
-    constexpr bool COALESCE = MODE == 1 && coalesce_pays<T, LAYOUT>();
+    constexpr bool COALESCE = FLAT ? flat_coalesces<T, LAYOUT, MODE == 3>() : MODE == 1 && coalesce_pays<T, LAYOUT>();
     uint32_t *slab = nullptr;
     if constexpr (COALESCE) {
         __shared__ __attribute__((aligned(16))) uint32_t slabs[4 * RMX_WAVE * coalesce_slab_dwords<T, LAYOUT>()];
@@ -47,7 +49,7 @@ __global__ void __launch_bounds__(256) rmx_point_kernel(RmxKArgs a) {
     const int w = P.dst_w, h = P.dst_h;
     const int srows = a.aux0;
     const int r0 = strip * srows;
-    if (r0 >= h) return;
+    if (r0 >= (FLAT ? FlatRows(a.dst_h * a.dst_w).n : h)) return;
     const int r1 = min(r0 + srows, h);
     const int x1 = P.src_x, y1 = P.src_y;
     const float ratio = P.color[0];
@@ -80,6 +82,37 @@ __global__ void __launch_bounds__(256) rmx_point_kernel(RmxKArgs a) {
                 for (int c = 0; c < 3; c++) v[c][k] = __builtin_fmaf(v[c][k] - u[c][k], ratio, u[c][k]);
         }
     };
+
+    if constexpr (FLAT) {
+        const FlatRows rows(a.dst_h * a.dst_w);
+        const int f1 = min(r0 + srows, rows.n);
+        const bool inside = simg + (size_t)rows.end(f1 - 1) * 3 + 4 <= buf_end;
+        constexpr int NI = 2;
+        for (int rb = r0; rb < f1; rb += NI) {
+            uint32_t da[NI][7], db[NI][7], pha[NI], phb[NI];
+#pragma unroll
+            for (int i = 0; i < NI; i++) {  // (a row beyond the strip repeats its last one and is not stored; so do lanes beyond a row)
+                const int r = min(rb + i, f1 - 1), start = rows.start(r), len = rows.end(r) - start, x = start + min(lane * PX, len - PX);
+                flat_load(simg, x, buf_end, inside, da[i], pha[i]);
+                if constexpr (KIND == POINT_BLEND) flat_load(simg2, x, buf_end2, inside, db[i], phb[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < NI; i++) {
+                const int r = rb + i, start = rows.start(r), len = rows.end(r) - start, L = (len + PX - 1) / PX;
+                if (r < f1 && lane < L) {
+                    uint32_t wa[6], wb[6];
+                    realign6(da[i], pha[i], wa);
+                    if constexpr (KIND == POINT_BLEND) realign6(db[i], phb[i], wb);
+                    float v[3][PX];
+                    finish(wa, wb, v);
+                    PackedGroup<T> packed;
+                    pack_group_dir<T, LAYOUT, false>(v, packed);
+                    flat_store<T, LAYOUT, sizeof(T) == 1, MODE == 3>(slab, dimg, rows.px, start, len, lane, L, start + min(lane * PX, len - PX), packed);
+                }
+            }
+        }
+        return;
+    }
 
     for (int xt = 0; xt < w; xt += RMX_WAVE * PX) {
         const int tw = min(w - xt, RMX_WAVE * PX);
@@ -147,7 +180,13 @@ static KernelFn pick_point(int dtype, int layout) {
 
 template <int KIND>
 static KernelFn pick_point_mode(int mode, int dtype, int layout) {
-    return mode == 1 ? pick_point<KIND, 1>(dtype, layout) : (mode == 2 ? pick_point<KIND, 2>(dtype, layout) : pick_point<KIND, 0>(dtype, layout));
+    switch (mode) {
+        case 1: return pick_point<KIND, 1>(dtype, layout);
+        case 2: return pick_point<KIND, 2>(dtype, layout);
+        case 3: return pick_point<KIND, 3>(dtype, layout);
+        case 4: return pick_point<KIND, 4>(dtype, layout);
+        default: return pick_point<KIND, 0>(dtype, layout);
+    }
 }
 
 KernelFn select_point_kernel(int kind, int dtype, int layout, int mode, const char **name) {
