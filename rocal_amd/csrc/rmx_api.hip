@@ -90,7 +90,7 @@ struct rmx_ctx {
     // Launch-plan tunables (rows per wavefront strip, LDS budget of the resize fast path). Defaults are the
     // values measured best on MI355X; RMX_TUNE_* environment variables, read once when the context is
     // created and clamped to safe ranges, override them for sweeps. They change plans, never results.
-    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_lds = 10 * 1024, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, warp_passes = 2, warp_wpb = 4;
+    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, warp_passes = 2, warp_wpb = 4;
 };
 
 static int tune_env(const char *name, int def, int lo, int hi) {
@@ -291,7 +291,7 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
     uint32_t c = RMX_C_ON, window = 0;
     for (int k = 0; k < 4; k++) window |= diff[SRC + k];
     window |= diff[FLAGS];
-    bool tiles[2] = {false, false};
+    bool tiles = false;
     switch (op->kind) {
         case OP_TRANSPOSE:
             if (op->aux1) return false;  // (height and width change places: a kernel of its own)
@@ -315,13 +315,11 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
         case OP_RESIZE: {
             if (t[0].dst_w <= 0 || t[0].dst_h <= 0) return false;
             const bool tri = op->interp == RMX_INTERP_TRIANGULAR;
-            tiles[0] = !tri && op->fn_fast && op->fast_aux1 == 0;            // the staged kernel's x-tiles
-            tiles[1] = !tri && (op->fn_mid || (op->fn_fast && !tiles[0]));  // the streaming kernel's
+            tiles = !tri && (op->fn_mid || op->fn_fast);  // the streaming kernels' x-tiles
             if (!tri && op->fn_mid) diff[STRIP_ROWS] = 0;  // (the general kernel, which reads it, is not reached)
             bool order = false;
             for (int i = 0; i < op->n; i++) order = order || t[i].plan[2] != i;
-            for (int k = 0; k < 2; k++)
-                if (tiles[k]) window |= diff[COLOR + k];
+            if (tiles) window |= diff[COLOR + 1];
             if (window) {
                 c |= RMX_C_WINDOW | RMX_C_RATIO;
                 for (int k = 0; k < 4; k++) diff[RX + k] = 0;
@@ -371,10 +369,10 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
         if (c & RMX_C_WINDOW) {
             if ((uint32_t)(s.src_x | s.src_y | s.src_w | s.src_h) > 0x3fffu) return false;
             if ((c & RMX_C_RATIO) && (s.src_w <= 0 || s.src_h <= 0)) return false;
-            const uint32_t t0 = tiles[0] ? tile_code(s.plan[0]) : 0u, t1 = tiles[1] ? tile_code(s.plan[1]) : 0u;
-            if (t0 > 7 || t1 > 7) return false;
-            *r++ = (uint32_t)s.src_x | (uint32_t)s.src_y << 14 | (s.flags & (RMX_S_HFLIP | RMX_S_VFLIP)) << 28 | (t0 & 3u) << 30;
-            *r++ = (uint32_t)s.src_w | (uint32_t)s.src_h << 14 | t1 << 28 | (t0 >> 2) << 31;
+            const uint32_t code = tiles ? tile_code(s.plan[1]) : 0u;
+            if (code > 7) return false;
+            *r++ = (uint32_t)s.src_x | (uint32_t)s.src_y << 14 | (s.flags & (RMX_S_HFLIP | RMX_S_VFLIP)) << 28;
+            *r++ = (uint32_t)s.src_w | (uint32_t)s.src_h << 14 | code << 28;
         }
         for (int k = 0; k < 4; k++)
             if (c & (RMX_C_COLOR0 << k)) memcpy(r++, &s.color[k], 4);
@@ -541,11 +539,10 @@ int rmx_ctx_create(int device, void *stream, int own_stream, rmx_ctx **out) {
         ctx->tri_rows = tune_env("RMX_TUNE_TRI_ROWS", ctx->tri_rows, 0, 64);  // 0: chosen per batch
         ctx->gen_rows = tune_env("RMX_TUNE_RESIZE_ROWS", ctx->gen_rows, 1, 64);
         ctx->fast_rows = tune_env("RMX_TUNE_FAST_ROWS", ctx->fast_rows, 1, 64);
-        ctx->fast_lds = tune_env("RMX_TUNE_FAST_LDS", ctx->fast_lds, 2048, 48 * 1024);
         ctx->fast_wpb = tune_env("RMX_TUNE_FAST_WPB", ctx->fast_wpb, 1, 4);
         ctx->compact = tune_env("RMX_TUNE_COMPACT", ctx->compact, 0, 1);  // 0: parameter rows always go through a table in device memory
         ctx->upload_kernel = tune_env("RMX_TUNE_UPLOAD_KERNEL", ctx->upload_kernel, 0, 1);
-        ctx->dma = tune_env("RMX_TUNE_DMA", ctx->dma, 0, 1);  // 0: the bilinear fast path always stages through registers
+        ctx->dma = tune_env("RMX_TUNE_DMA", ctx->dma, 0, 1);  // 0: resizes of whole groups use the form for any byte phase, all others the general kernel; triangular and warp kernels stage through registers
         ctx->dma_lds = tune_env("RMX_TUNE_DMA_LDS", ctx->dma_lds, 2048, 32 * 1024) & ~15;  // LDS window of a wavefront
         ctx->dma_group = tune_env("RMX_TUNE_DMA_GROUP", ctx->dma_group, 0, 16);  // windows per wavefront, 0: chosen per batch
         ctx->flat_frames = tune_env("RMX_TUNE_FLAT_FRAMES", ctx->flat_frames, 0, 1);  // 0: point operations always walk the images' own rows
@@ -1366,118 +1363,73 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
     op->strip_rows = grows;
     op->aux0 = grows;
     op->strips = std::max(1, (max_dh + grows - 1) / grows);
-    // fast path: every written width a multiple of 8 and aligned destination rows. Its wavefronts stage
-    // the whole source window of a strip of `rows` destination rows at once; the x-tile of a sample is
-    // narrowed until that window fits the LDS budget of one wavefront.
+    // Streaming kernels (source rows straight into LDS). A wavefront loads the whole source window of `rows` destination rows at
+    // once; the x-tile of a sample is narrowed until that window fits the LDS budget of one wavefront. What they leave to the
+    // general kernel: windows too tall for it, and (RMX_TUNE_DMA=0, the kernels' cross-check) all but whole groups.
     op->fn_fast = nullptr;
     op->fn_mid = nullptr;
-    if (op->interp == RMX_INTERP_LINEAR) {
-        // (the kernels multiply row indices and the row stride with 24-bit multiplies)
-        const bool base_ok = op->src.w * 3u < (1u << 23) && op->src.h < (1u << 23);
-        bool widths8 = op->dst.w % 8 == 0;
-        for (int i = 0; i < op->n && widths8; i++) widths8 = t[i].dst_w % 8 == 0;
-        bool ok = base_ok && widths8;
-        // 4 rows and a 10 KB slice measured best on MI355X (more, shorter-lived wavefronts per CU)
-        const int rows = op->ctx->fast_rows, cap = op->ctx->fast_lds;
-        const TileCost tile_cost(rows);
-        int need_max = 64;
-        for (int i = 0; i < op->n && ok; i++) {
-            RmxSample &s = t[i];
-            s.plan[0] = 8;
-            if (s.dst_w % 8 != 0) {
-                ok = false;
-                break;
-            }
-            if (s.dst_w <= 0 || s.dst_h <= 0) continue;
-            const float magx = (float)(s.src_x + s.src_w + 2), magy = (float)(s.src_y + s.src_h + 2);
-            const int nrows = std::max(2, span_bound(std::min<int>(rows, s.dst_h) - 1, s.ry, magy) + 2);
-            long need = 0;
-            const int tw = pick_tile_width((int)s.dst_w, tile_cost, cap, [&](int w) {
-                const int nc = std::min<int>(s.src_w, span_bound(w - 1, s.rx, magx) + 2);
-                return (long)nrows * (8 + ((nc + 3) >> 2) * 4) * 4;  // bytes: one dword per pixel + replicas
-            }, &need);
-            if (tw == 0) {
-                ok = false;  // a window this tall does not fit: the general kernel takes the batch
-                break;
-            }
-            s.plan[0] = tw;
-            need_max = std::max<int>(need_max, (int)need);
-        }
-        if (ok) {
-            op->fn_fast = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, &op->fast_name);
-            op->fast_lds = (need_max + 15) / 16 * 16;
-            // interleaved fp32 output: room for the slab through which the lanes of a row exchange their runs before storing
-            // (64 lanes x the 24 dwords of one lane's run; the kernel takes it from the tail of the slice)
-            if (op->dst.dtype == RMX_FP32 && op->dst.layout == RMX_NHWC) op->fast_lds += 64 * 4 * 24;
-            op->fast_rows = rows;
-            op->fast_strips = std::max(1, (max_dh + rows - 1) / rows);
-            // (default 1: a workgroup's LDS is released only when its last wavefront ends, one-wave groups keep the CU full)
-            op->fast_wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, op->fast_lds)));
-            op->fast_needs_src16 = false;  // its loads only need dword alignment
-            op->fast_aux1 = 0;
-            if (op->fast_lds > op->ctx->max_lds_per_block - kStaticLdsMax) op->fn_fast = nullptr;
-        }
-        // Streaming kernel (source rows straight into LDS): needs every source row to start at the same byte phase (row stride
-        // a multiple of 4). Its any-width form serves every destination; the form for whole groups and aligned rows replaces
-        // the staged kernel above where that applies.
-        bool dma = base_ok && op->ctx->dma;
-        if (dma) {
-            if (op->layout.empty()) dma = (op->src.w * 3u) % 4u == 0;
-            else
-                for (int i = 0; i < op->n && dma; i++) dma = op->layout[i].row_stride % 4u == 0;
-        }
-        if (dma) {
-            // 10 KB measured best on MI355X: smaller caps cut more rows into two tiles, and the kernel's registers allow 16
-            // wavefronts per CU, which 10 KB each still fit
-            const int bufcap = op->ctx->dma_lds;
-            int need_max = 64;
-            for (int i = 0; i < op->n && dma; i++) {
-                RmxSample &s = t[i];
-                s.plan[1] = 8;
-                if (s.dst_w <= 0 || s.dst_h <= 0) continue;
-                const float magx = (float)(s.src_x + s.src_w + 2), magy = (float)(s.src_y + s.src_h + 2);
-                const int nrows = std::max(2, span_bound(std::min<int>(rows, s.dst_h) - 1, s.ry, magy) + 2);
-                long need = 0;
-                const int tw = pick_tile_width((int)s.dst_w, tile_cost, bufcap, [&](int w) {
-                    const int nc = std::min<int>(s.src_w, span_bound(w - 1, s.rx, magx) + 2);
-                    return (long)nrows * (1 + ((3 + 3 * (nc + 2) + 8 + 15) >> 4)) * 16;  // margin piece + data + replicas
-                }, &need);
-                if (tw == 0) {
-                    dma = false;
-                    break;
-                }
-                s.plan[1] = tw;
-                need_max = std::max<int>(need_max, (int)need);
-            }
-            if (dma && need_max <= op->ctx->max_lds_per_block - kStaticLdsMax) {
-                // A wavefront works through `group` windows (of `rows` destination rows) below each other per x-tile, so that the
-                // tile's x taps are computed once for all of them (1 measured best: more leave too few wavefronts to fill the chip evenly).
-                const long windows = (long)op->n * ((max_dh + rows - 1) / rows);
-                const int group = op->ctx->dma_group ? op->ctx->dma_group : (int)std::max<long>(1, std::min<long>(8, windows / 4096));
-                const int lds = (need_max + 15) / 16 * 16;
-                const int strips = std::max(1, (max_dh + rows * group - 1) / (rows * group));
-                const int wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, lds)));
-                op->fn_mid = rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, false, &op->mid_name);
-                op->mid_lds = lds;
-                op->mid_rows = rows;
-                op->mid_strips = strips;
-                op->mid_wpb = wpb;
-                op->mid_aux1 = group;
-                const char *dname = nullptr;
-                rmx::KernelFn dfn = widths8 ? rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &dname) : nullptr;
-                if (dfn) {
-                    op->fn_fast = dfn;
-                    op->fast_name = dname;
-                    op->fast_lds = lds;
-                    op->fast_rows = rows;
-                    op->fast_strips = strips;
-                    op->fast_wpb = wpb;
-                    op->fast_aux1 = group;
-                    op->fast_needs_src16 = false;
-                }
-            }
-        }
+    const bool nearest = op->interp == RMX_INTERP_NEAREST;
+    // (the kernels multiply row indices and the row stride with 24-bit multiplies)
+    bool ok = op->src.w * 3u < (1u << 23) && op->src.h < (1u << 23);
+    bool widths8 = op->dst.w % 8 == 0;
+    for (int i = 0; i < op->n && widths8; i++) widths8 = t[i].dst_w % 8 == 0;
+    if (!op->ctx->dma) ok = ok && widths8 && !nearest;
+    // every source row starts at one byte phase
+    bool one_phase = op->ctx->dma != 0 && !nearest;
+    if (one_phase) {
+        if (op->layout.empty()) one_phase = (op->src.w * 3u) % 4u == 0;
+        else
+            for (int i = 0; i < op->n && one_phase; i++) one_phase = op->layout[i].row_stride % 4u == 0;
     }
+    // 4 rows and a 10 KB slice measured best on MI355X: smaller caps cut more rows into two tiles, and the kernel's registers
+    // allow 16 wavefronts per CU, which 10 KB each still fit
+    const int rows = op->ctx->fast_rows, bufcap = op->ctx->dma_lds;
+    const TileCost tile_cost(rows);
+    int need_max = 64;
+    for (int i = 0; i < op->n && ok; i++) {
+        RmxSample &s = t[i];
+        s.plan[1] = 8;
+        if (s.dst_w <= 0 || s.dst_h <= 0) continue;
+        const float magx = (float)(s.src_x + s.src_w + 2), magy = (float)(s.src_y + s.src_h + 2);
+        const int wrows = std::min<int>(rows, s.dst_h);
+        const int nrows = nearest ? wrows : std::max(2, span_bound(wrows - 1, s.ry, magy) + 2);
+        long need = 0;
+        const int tw = pick_tile_width((int)s.dst_w, tile_cost, bufcap, [&](int w) {
+            const int nc = std::min<int>(s.src_w, span_bound(w - 1, s.rx, magx) + 2);
+            return (long)nrows * (1 + ((3 + 3 * (nc + 2) + 8 + 15) >> 4)) * 16;  // margin piece + data + replicas
+        }, &need);
+        if (tw == 0) ok = false;
+        s.plan[1] = tw;
+        need_max = std::max<int>(need_max, (int)need);
+    }
+    int slice = (need_max + 15) / 16 * 16;
+    // interleaved fp32 output: room for the slab through which the lanes of a row exchange their runs before storing (64 lanes x the
+    // 24 dwords of one lane's run; the kernel takes it from the tail of the slice)
+    if (op->dst.dtype == RMX_FP32 && op->dst.layout == RMX_NHWC) slice += 64 * 4 * 24;
+    if (!ok || slice > op->ctx->max_lds_per_block - kStaticLdsMax) return RMX_OK;
+    // A wavefront works through `group` windows (of `rows` destination rows) below each other per x-tile, so that the
+    // tile's x taps are computed once for all of them (1 measured best: more leave too few wavefronts to fill the chip evenly).
+    const long windows = (long)op->n * ((max_dh + rows - 1) / rows);
+    const int group = op->ctx->dma_group ? op->ctx->dma_group : (int)std::max<long>(1, std::min<long>(8, windows / 4096));
+    op->mid_lds = op->fast_lds = slice;
+    op->mid_rows = op->fast_rows = rows;
+    op->mid_strips = op->fast_strips = std::max(1, (max_dh + rows * group - 1) / (rows * group));
+    // (default 1: a workgroup's LDS is released only when its last wavefront ends, one-wave groups keep the CU full)
+    op->mid_wpb = op->fast_wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, slice)));
+    op->mid_aux1 = op->fast_aux1 = group;
+    op->fast_needs_src16 = false;
+    if (nearest) {
+        op->fn_mid = rmx::select_resize_near_kernel(op->dst.dtype, op->dst.layout, op->norm, &op->mid_name);
+        return RMX_OK;
+    }
+    if (one_phase) {
+        op->fn_mid = rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, false, &op->mid_name);
+        if (widths8) op->fn_fast = rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &op->fast_name);
+    } else if (op->ctx->dma) {
+        op->fn_mid = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, &op->mid_name);
+    }
+    // (also interleaved fp32 of whole groups)
+    if (widths8 && !op->fn_fast) op->fn_fast = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, &op->fast_name);
     return RMX_OK;
 }
 

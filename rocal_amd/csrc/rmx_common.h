@@ -21,7 +21,7 @@ struct __attribute__((aligned(16))) RmxSample {
     float scale[3], bias[3];             // normalisation: out = v*scale + bias
     union {
         float color[4];                  // colour twist: alpha, beta, hue shift in sextants [0,6], saturation
-        int32_t plan[4];                 // bilinear fast paths: x-tile width for this sample, [0] staged kernel, [1] streaming kernel
+        int32_t plan[4];                 // [1] x-tile width of the streaming resize kernels, [2] the row's sample (triangular)
     };
     float m[6];                          // warp: destination -> source affine about the centres
 };
@@ -54,7 +54,7 @@ enum : uint32_t {
 // 37.4 -> 31.5 us, 128 crops of 224 x 224 to fp32 planes 22.2 -> 16.8 us, 14 small crops 16.9 -> 11.0 us. What a sample's dwords hold, in this order:
 enum : uint32_t {
     RMX_C_ON = 1u,        // the rows are in the arguments
-    RMX_C_WINDOW = 2u,    // two dwords: x, y, w, h in 14 bits each, mirror flags, x-tile widths (see compact_rows, rmx_api.hip)
+    RMX_C_WINDOW = 2u,    // two dwords: x, y, w, h in 14 bits each, mirror flags, the x-tile width's code (see compact_rows, rmx_api.hip)
     RMX_C_DST = 4u,       // (nothing stored) the written size is the window's
     RMX_C_RATIO = 8u,     // (nothing stored) rx, ry, fsx, fsy are quotients of the sizes
     RMX_C_COLOR0 = 16u,   // color[0..3], one dword each, those that differ between samples (four bits from here)

@@ -56,9 +56,8 @@ RMX_DEV RmxSample load_sample(const RmxKArgs &a, int i) {
             }
             if constexpr (CAN & RMX_C_RATIO) {
                 const int whole = min(max(P.dst_w, 8), RMX_C_TILE_WHOLE);
-                const uint32_t t0 = (w0 >> 30) | ((w1 >> 31) << 2), t1 = (w1 >> 28) & 7u;
-                P.plan[0] = t0 ? RMX_C_TILE_WHOLE >> t0 : whole;
-                P.plan[1] = t1 ? RMX_C_TILE_WHOLE >> t1 : whole;
+                const uint32_t code = (w1 >> 28) & 7u;
+                P.plan[1] = code ? RMX_C_TILE_WHOLE >> code : whole;
                 P.rx = (float)P.src_w / (float)P.rs_w;
                 P.ry = (float)P.src_h / (float)P.rs_h;
                 P.fsx = P.rx > 1.0f ? 1.0f / P.rx : 1.0f;
@@ -638,6 +637,24 @@ RMX_DEV void store_packed_coalesced_any(uint32_t *slab, int grp0, int l, int L, 
     } else {
         T *seg = sample + ((size_t)y * W + xs) * 3;
         store_run_coalesced_any<PX * 3, NT>(slab, reinterpret_cast<uint8_t *>(seg), grp0, l, L, 3 * (x0 - xs), 3 * tw, g.w);
+    }
+}
+
+// Pixels first .. first + cnt - 1 of a packed group, element by element, the first of them to column x0.
+template <typename T, int LAYOUT>
+RMX_DEV void store_packed_part(T *sample, int H, int W, int y, int x0, int first, int cnt, const PackedGroup<T> &g) {
+    T e[PX * 3];
+    __builtin_memcpy(e, g.w, sizeof(e));
+#pragma unroll
+    for (int k = 0; k < PX; k++) {
+        if (k >= first && k < first + cnt) {
+            const int x = x0 + k - first;
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                if constexpr (LAYOUT == RMX_NCHW) sample[((size_t)c * H + y) * W + x] = e[c * PX + k];
+                else sample[((size_t)y * W + x) * 3 + c] = e[k * 3 + c];
+            }
+        }
     }
 }
 

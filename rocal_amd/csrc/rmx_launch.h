@@ -11,6 +11,7 @@ KernelFn select_cmn_kernel(int dtype, int layout, int norm, int mode, const char
 KernelFn select_resize_linear_kernel(int dtype, int layout, bool norm, bool quant, int chain, const char **name);
 KernelFn select_resize_fast_kernel(int dtype, int layout, bool norm, bool quant, int chain, const char **name);
 KernelFn select_resize_dma_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool aligned, const char **name);
+KernelFn select_resize_near_kernel(int dtype, int layout, bool norm, const char **name);
 KernelFn select_resize_nearest_kernel(int dtype, int layout, bool norm, bool quant, const char **name);
 KernelFn select_resize_tri_kernel(int dtype, int layout, bool norm, bool quant, const char **name);
 KernelFn select_resize_tri_down_kernel(int dtype, int layout, bool norm, bool quant, int columns_per_lane, const char **name);
