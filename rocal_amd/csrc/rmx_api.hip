@@ -542,7 +542,7 @@ int rmx_ctx_create(int device, void *stream, int own_stream, rmx_ctx **out) {
         ctx->fast_wpb = tune_env("RMX_TUNE_FAST_WPB", ctx->fast_wpb, 1, 4);
         ctx->compact = tune_env("RMX_TUNE_COMPACT", ctx->compact, 0, 1);  // 0: parameter rows always go through a table in device memory
         ctx->upload_kernel = tune_env("RMX_TUNE_UPLOAD_KERNEL", ctx->upload_kernel, 0, 1);
-        ctx->dma = tune_env("RMX_TUNE_DMA", ctx->dma, 0, 1);  // 0: resizes of whole groups use the form for any byte phase, all others the general kernel; triangular and warp kernels stage through registers
+        ctx->dma = tune_env("RMX_TUNE_DMA", ctx->dma, 0, 1);  // 0: resizes of whole groups use the form for any byte phase, all others the general kernel; the triangular kernel stages through registers, the warp kernel uses its form for any byte phase
         ctx->dma_lds = tune_env("RMX_TUNE_DMA_LDS", ctx->dma_lds, 2048, 32 * 1024) & ~15;  // LDS window of a wavefront
         ctx->dma_group = tune_env("RMX_TUNE_DMA_GROUP", ctx->dma_group, 0, 16);  // windows per wavefront, 0: chosen per batch
         ctx->flat_frames = tune_env("RMX_TUNE_FLAT_FRAMES", ctx->flat_frames, 0, 1);  // 0: point operations always walk the images' own rows
@@ -692,7 +692,6 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
     a.aux0 = op->aux0;
     a.aux1 = op->aux1;
     if ((((uintptr_t)src) | ((uintptr_t)src2)) & 3u) return fail(RMX_ERR_INVALID, "the source batch must start at a 4-byte aligned address");
-    if ((op->kind == OP_WARP_AFFINE || op->kind == OP_ROTATE) && (((uintptr_t)dst) & 15u)) a.aux1 &= ~1;  // packed stores need an aligned base
     // the fast specialisation wants 16-byte aligned batch bases (rows of both sides are then aligned too)
     const bool fast = op->fn_fast && (((uintptr_t)dst) & 15u) == 0 && (!op->fast_needs_src16 || (((uintptr_t)src) & 15u) == 0);
     const bool mid = !fast && op->fn_mid;
@@ -1819,8 +1818,8 @@ static int update_warp(rmx_op *op, const uint32_t *roi, const float *affine, con
     uint64_t bytes = 0;
     int max_dw = 1, max_dh = 1;
     double worst_box = 0;
-    // The form that loads the source box straight into LDS as packed bytes needs every source row to start at the same byte
-    // phase (row stride a multiple of 4).
+    // Row strides that are all multiples of 4: every source row starts at the same byte phase and the kernel keeps two
+    // instructions per pixel for the phase of the lower row out of its loop.
     bool raw = op->ctx->dma != 0;
     if (raw) {
         if (op->layout.empty()) raw = (op->src.w * 3u) % 4u == 0;
@@ -1858,32 +1857,22 @@ static int update_warp(rmx_op *op, const uint32_t *roi, const float *affine, con
         if (std::isfinite(bw) && std::isfinite(bh)) {
             bw = std::min(bw, (double)s.src_w + 1);
             bh = std::min(bh, (double)s.src_h + 1);
-            if (raw) {
-                // (packed bytes: rows of whole 16-byte pieces from the dword that holds the box's first pixel; boxes of up to
-                // kWarpRawPieces pieces per row are staged at that pitch; in dwords, like the other form)
-                const double pieces = std::ceil((3.0 + 3.0 * (bw + 1.0)) / 16.0);
-                worst_box = std::max(worst_box, (pieces <= rmx::kWarpRawPieces ? (double)rmx::kWarpRawPieces : pieces) * 4.0 * bh);
-            } else {
-                // (boxes of up to 60 dwords per row are staged at a pitch of 60, see the kernel)
-                const double pitch = std::ceil(bw / 4) * 4 + 4;
-                worst_box = std::max(worst_box, (pitch <= 60.0 ? 60.0 : pitch) * bh);
-            }
+            // (packed bytes: rows of whole 16-byte pieces from the dword that holds the box's first pixel, at least kWarpRawPieces
+            // of them; the form for any phase leaves 16 bytes between rows and up to 3 for the stride's remainder)
+            const double pieces = std::max<double>(std::ceil(((raw ? 3.0 : 22.0) + 3.0 * (bw + 1.0)) / 16.0), rmx::kWarpRawPieces);
+            worst_box = std::max(worst_box, (pieces * 16.0 + (raw ? 0.0 : 3.0)) * bh);
         }
     }
     op->algo_bytes = bytes;
     const int cap = 16 * 1024;  // per wave (16 loads per lane); bigger boxes fall back to global gathers inside the kernel
-    int need = (int)std::min<double>(worst_box * 4 + (raw ? 16 : 0), (double)cap);
+    int need = (int)std::min<double>(worst_box + (raw ? 16 : 32), (double)cap);
     op->lds_per_wave = std::max(256, (need + 15) / 16 * 16);
     op->waves_per_block = std::max(1, std::min(op->ctx->warp_wpb, op->ctx->max_lds_per_block / op->lds_per_wave));
     const int passes = op->ctx->warp_passes;
     const int tiles_x = (max_dw + 31) / 32, tiles_y = (max_dh + 16 * passes - 1) / (16 * passes);
     op->strips = tiles_x * tiles_y;
     op->aux0 = tiles_x;
-    // aux1 bit 0: the shapes allow packed 16-byte stores (whole 8-pixel groups, rows a multiple of 8 pixels wide);
-    // bits 8..: passes of 16 rows per tile
-    bool aligned = op->dst.w % 8 == 0;
-    for (int i = 0; i < op->n && aligned; i++) aligned = (t[i].dst_w % 8 == 0);
-    op->aux1 = (aligned ? 1 : 0) | (passes << 8);
+    op->aux1 = passes << 8;  // passes of 16 rows per tile
     return commit_slot(op, slot);
 }
 

@@ -4,18 +4,25 @@
 // A wavefront owns a destination tile of 32 columns x (16 x passes) rows. The tile's corners are pushed
 // through the affine map to get the source bounding box (every pixel of the tile maps inside it: each
 // step of the coordinate law is monotone in x and in y, also after rounding), which is staged into the
-// wavefront's LDS slice, one dword per pixel, with all loads of the box in flight together; one extra
+// wavefront's LDS slice with all loads of the box in flight together; one extra
 // column and row repeat the ROI's last column / row, so the right and lower neighbours of a tap are always
-// at +1 and +pitch. Each lane then produces 8 adjacent destination pixels of one row per pass, branch-free:
+// at +3 bytes and +pitch. Each lane then produces 8 adjacent destination pixels of one row per pass, branch-free:
 // taps of pixels that fall outside the ROI are read from wherever their (meaningless) address points inside
 // the slice and the result is replaced by 0. When the box does not fit the slice (strong minification) the
 // wavefront gathers from global memory instead.
 //
-// RAW (every source row starts at the same byte phase: row strides multiples of 4): the box travels from global memory
-// straight into LDS as packed bytes (global_load_lds_dwordx4, 16 bytes per lane: no vector register, no unpacking, no LDS
-// store; piece i of the box, rows one after the other, is loaded by lane i & 63 of load instruction i >> 6), three bytes
-// per pixel instead of four, and a tap pair (two packed pixels, 6 bytes at any byte phase) is read as three aligned dwords
-// and realigned with two v_alignbyte. Values and operations from there on are the same.
+// The box travels from global memory straight into LDS as packed bytes (global_load_lds_dwordx4, 16 bytes per lane: no vector
+// register, no unpacking, no LDS store), three bytes per pixel, and a tap pair (two packed pixels, 6 bytes at any byte phase) is
+// read as three aligned dwords and realigned with two v_alignbyte. Two forms:
+//   RAW    every source row starts at the same byte phase (row strides multiples of 4): piece i of the box, rows one after the
+//          other, is loaded by lane i & 63 of load instruction i >> 6;
+//   any    rows at any byte phase (299 pixels are 897 bytes; images packed without padding): a load starts at a dword, so bytes
+//          keep their place within a dword on the way into LDS. The LDS pitch therefore leaves the same remainder mod 4 as the row
+//          stride: a tap's address stays linear in its coordinates, and the only cost in the loop is that the lower row's address
+//          is masked by itself (two instructions per pixel). Against staging through registers with one dword per pixel (111 registers,
+//          13 KB): 64 rotations of 299 x 299, bytes, with the wide stores below, 18.4 -> 15.1 us per batch. Rows at one phase keep RAW:
+//          its loop has the masks' two instructions less, of 58.
+// Bound by the vector pipe: 128 images of 512 x 512 take 63 us, of which the bytes are 36 at the rate of a large copy.
 #include "rmx_device.h"
 #include "rmx_launch.h"
 
@@ -31,8 +38,7 @@ extern __shared__ uint32_t rmx_lds_warp[];
 typedef __attribute__((address_space(3))) uint32_t lds_u32;  // explicit LDS pointers: 32-bit address arithmetic
 
 constexpr int WTW = 32, WTH = 16;  // destination tile: 4 lanes x 8 px wide, 16 rows per pass
-constexpr int WFP = 60;            // fixed LDS pitch (dwords) of boxes that fit it
-constexpr int WRP = kWarpRawPieces;  // RAW: fixed LDS pitch in 16-byte pieces (an odd number spreads the rows over the LDS banks)
+constexpr int WRP = kWarpRawPieces;  // LDS pitch of boxes that fit it, in 16-byte pieces (an odd number spreads the rows over the LDS banks)
 
 RMX_DEV uint32_t load_px_global(const uint8_t *p) {
     return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16);
@@ -57,7 +63,6 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     wave_to_sample(a, wave, s, tile);
     const int tiles_x = a.aux0;
     const int passes = a.aux1 >> 8;
-    const bool packed_ok = (a.aux1 & 1) != 0;
     const int ty = tile / tiles_x, tx = tile - ty * tiles_x;
     // the whole table row in one round trip
     const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_M6>(a, s);
@@ -107,25 +112,39 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     const int bw = bx1 - bx0 + 1, bh = by1 - by0 + 1;
     const bool empty = bw <= 0 || bh <= 0;
     // staged box: bw columns + the repeated last one, bh rows + the repeated last one
-    const int items = (max(bw, 0) + 1 + 3) >> 2;
-    // Boxes of at most WFP - 1 columns (every tile of a map that does not minify) are staged at ONE pitch, known to the
-    // compiler: the address of a tap is two instructions (a 24-bit multiply-add and a shift-add) and the row below is an
-    // offset inside the read instruction. 15 items: an odd number of 16-byte items spreads the rows over the LDS banks.
-    // RAW: a row is ppr 16-byte pieces from the dword that holds pixel bx0 (byte phase ph inside it)
+    // RAW: a row is ppr 16-byte pieces from the dword that holds pixel bx0 (byte phase ph inside it). Boxes of at most WRP pieces
+    // per row (every tile of a map that does not minify) are staged at ONE pitch, known to the compiler: the row below is an
+    // offset inside the read instruction.
     const uint32_t skew = (uint32_t)((uintptr_t)simg & 3u);
     const uint32_t colb = (uint32_t)max(bx0, 0) * 3u + skew;
-    const int ph = (int)(colb & 3u);
-    const int ppr_box = (ph + 3 * (max(bw, 0) + 1) + 15) >> 4;
-    const bool fixed = RAW ? ppr_box <= WRP : items * 4 <= WFP;
+    const int ppr_box = ((int)(colb & 3u) + 3 * (max(bw, 0) + 1) + 15) >> 4;
+    const bool fixed = RAW && ppr_box <= WRP;
     const int ppr = fixed ? WRP : ppr_box;
-    const int pitch = RAW ? ppr * 4 : (fixed ? WFP : items * 4);  // dwords
-    const int total = (bh + 1) * (RAW ? ppr : items);            // 16-byte pieces (RAW) or four-pixel items of the box
+    // Any phase: rows at a pitch that leaves the same remainder mod 4 as the row stride, so that a row's bytes keep their place
+    // within a dword on the way into LDS; at least 16 bytes between two rows' data, so that no piece holds data of both.
+    const int need = 3 * max(bw, 0) + 16;
+    const int pitch_b = RAW ? ppr * 16 : max(WRP * 16, (need + 3) & ~3) + (int)(row_stride & 3u);  // bytes
+    const int ph = (int)((RAW ? colb : colb + (uint32_t)max(by0, 0) * row_stride) & 3u);  // LDS byte of the box's first pixel
+    const int total = RAW ? (bh + 1) * ppr : (int)(((int64_t)ph + (int64_t)(bh - 1) * pitch_b + 3 * bw + 15) >> 4);  // 16-byte pieces
     // (RAW: the three dwords read for the last tap of the last row may reach 8 bytes behind the box)
-    const bool use_lds = !empty && total <= 16 * RMX_WAVE && (size_t)(bh + 1) * pitch * 4 + (RAW ? 16 : 0) <= (size_t)a.lds_bytes;
+    const bool use_lds = !empty && (!RAW || total <= 16 * RMX_WAVE) && (uint64_t)(bh + 1) * (uint32_t)pitch_b + (RAW ? 16 : 32) <= (uint64_t)a.lds_bytes;
 
     const int lr = lane >> 2, g = lane & 3;
-    const int x0 = X0 + g * PX;
+    int x0 = X0 + g * PX;
+    // The short last group of a row moves left until it is whole (its pixels belong to this tile): it recomputes pixels of the group
+    // before it and stores the same values to the same places. Only a tile narrower than 8 pixels keeps a short group.
+    if (x0 < dw) x0 = max(min(x0, dw - PX), X0);
     const int cnt = min(PX, dw - x0);
+    // Whole groups leave as wide stores at the alignment of an element (the same instructions as for aligned rows).
+    auto store = [&](int y, const float (&v)[3][PX]) {
+        if (cnt == PX) {
+            PackedGroup<T> packed;
+            pack_group_dir<T, LAYOUT, false>(v, packed);
+            store_packed<T, LAYOUT, RMX_WARP_NT, true>(dimg, a.dst_h, a.dst_w, y, x0, packed);
+        } else {
+            store_group<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, cnt, v, false);
+        }
+    };
     const float xr0 = (float)x0 - dcx;
 
     if (empty) {
@@ -137,7 +156,7 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             for (int k = 0; k < PX; k++) z[c][k] = 0.0f;
         for (int pass = 0; pass < passes; pass++) {
             const int y = Y0 + pass * WTH + lr;
-            if (y < dh && cnt > 0) store_group<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, cnt, z, false);
+            if (y < dh && cnt > 0) store(y, z);
         }
         return;
     }
@@ -183,16 +202,16 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
                 }
                 v[0][k] = o0; v[1][k] = o1; v[2][k] = o2;
             }
-            store_group<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, cnt, v, false);
+            store(y, v);
         }
         return;
     }
 
+    lds_u8 *ldsb = (lds_u8 *)(lds_ptr_t)rmx_lds_warp + (uint32_t)to_sgpr((int)((uint32_t)wib * (uint32_t)a.lds_bytes));
+    const uint8_t *base4 = simg - skew;
     if constexpr (RAW) {
         // ---- the box straight into LDS: piece idx = (row, piece of the row) in row order lands at byte 16 idx of the slice
-        const uint8_t *base4 = simg - skew;
         const uint32_t col4 = colb & ~3u;
-        lds_u8 *ldsb = (lds_u8 *)(lds_ptr_t)rmx_lds_warp + (uint32_t)to_sgpr((int)((uint32_t)wib * (uint32_t)a.lds_bytes));
         // every piece of the box lies inside the batch buffer (the last rows of the last sample may not)
         const bool safe = simg + ((size_t)min(by1 + 1, yhi) * row_stride + (size_t)bx0 * 3 + 16 * (size_t)ppr) <= buf_end;
         const float inv_ppr = 1.0f / (float)ppr;
@@ -231,75 +250,75 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
         // the column behind the box repeats its last column where that is the ROI's last column (only then is it read)
         if (bx1 == xhi) {
             for (int r = lane; r <= bh; r += RMX_WAVE) {
-                lds_u8 *px = ldsb + r * (pitch * 4) + ph + 3 * (bw - 1);
+                lds_u8 *px = ldsb + r * pitch_b + ph + 3 * (bw - 1);
                 px[3] = px[0];
                 px[4] = px[1];
                 px[5] = px[2];
             }
             wave_sync();
         }
-    } else
-    // ---- stage the box: (row, 4-pixel item) pairs form one flat index space dealt to the lanes; rows beyond
-    // the box repeat the ROI's last row (the clamp does it); all loads go out before the first is consumed
-    {
-        const uint8_t *base4 = simg - skew;
-        const uint32_t col0 = (uint32_t)bx0 * 3u + skew;
-        const float inv_items = 1.0f / (float)items;
-        // the last load of the box stays inside the batch buffer
-        const bool safe = simg + ((size_t)min(by1 + 1, yhi) * row_stride + (size_t)bx0 * 3 + 12 * (size_t)items + 4) <= buf_end;
-        auto stage = [&](auto nsc) {
-            constexpr int NS = decltype(nsc)::value;
-            u32x4_a4 v[NS];
-            uint32_t dst_off[NS], ph[NS];
-#pragma unroll
-            for (int j = 0; j < NS; j++) {
-                const int idx = min(j * RMX_WAVE + lane, total - 1);
-                // idx / items: (idx + 0.5) / items is at least 0.5/items away from an integer, so the truncation is exact
-                const int r = (int)(((float)idx + 0.5f) * inv_items);
-                const int c = idx - __mul24(r, items);
-                const int ysrc = min(by0 + r, yhi);
-                const uint32_t off = (uint32_t)ysrc * row_stride + col0 + 12u * (uint32_t)c;
-                v[j] = *reinterpret_cast<const u32x4_a4 *>(base4 + (off & ~3u));
-                dst_off[j] = (uint32_t)(__mul24(r, pitch) + 4 * c);
-                ph[j] = off & 3u;
-            }
-#pragma unroll
-            for (int j = 0; j < NS; j++) {
-                const uint32_t d[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
-                const uint4 px = expand4(d, ph[j]);
-                if (j * RMX_WAVE + lane < total) *reinterpret_cast<uint4 *>(lds + dst_off[j]) = px;
-            }
-        };
+    } else {
+        // ---- the box straight into LDS, any phase: LDS byte b belongs to row r of the box (r * pitch_b + ph is the row's first
+        // pixel) and holds the source byte at the same distance from that row's first pixel; a piece is the row's that its last
+        // byte lies in (what a piece holds in front of a row is never read). Pitch and stride agree mod 4 and the box's first dword
+        // is a source dword, so every piece is loaded from a dword.
+        const uint32_t first = (uint32_t)by0 * row_stride + colb - (uint32_t)ph;  // source byte (from base4) of LDS byte 0
+        const uint32_t step = row_stride - (uint32_t)pitch_b;
+        const uint64_t left = (uint64_t)(buf_end - base4);
+        // every piece lies inside the batch buffer (the last rows of the last sample may not, nor the first rows of the first one
+        // where a piece starts up to 15 bytes in front of its row)
+        const bool safe = (uint64_t)by1 * row_stride + colb + (uint32_t)pitch_b + 32u <= left && (bh == 1 || first + row_stride >= 16u);
+        const float inv_pitch = 1.0f / (float)pitch_b;
+        // (x + 0.5) / pitch is at least 0.5 / pitch away from an integer, so the truncation is exact
+        auto row_of = [&](int idx) { return min((int)(((float)(16 * idx + 15 - ph) + 0.5f) * inv_pitch), bh - 1); };
         if (safe) {
-            if (total <= 4 * RMX_WAVE) stage(std::integral_constant<int, 4>{});
-            else if (total <= 8 * RMX_WAVE) stage(std::integral_constant<int, 8>{});
-            else stage(std::integral_constant<int, 16>{});
+            for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
+                const int idx = j0 + lane;
+                const uint32_t off = first + 16u * (uint32_t)idx + (uint32_t)row_of(idx) * step;
+                if (idx < total) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
+            }
+            // the compiler does not order LDS reads behind loads into LDS: await them explicitly
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         } else {
-            // the box touches the last bytes of the batch buffer: bounds-checked loads
             for (int idx = lane; idx < total; idx += RMX_WAVE) {
-                const int r = idx / items, c = idx - r * items;
-                const uint8_t *p = simg + (size_t)min(by0 + r, yhi) * row_stride + (size_t)(bx0 + 4 * c) * 3;
-                uint32_t w[3];
-                load_realigned<4>(p, buf_end, w);
-                uint4 px;
-                px.x = w[0];
-                px.y = __builtin_amdgcn_alignbyte(w[1], w[0], 3);
-                px.z = __builtin_amdgcn_alignbyte(w[2], w[1], 2);
-                px.w = w[2] >> 8;
-                *reinterpret_cast<uint4 *>(lds + r * pitch + 4 * c) = px;
+                const int r = row_of(idx);
+                const int64_t off = (int64_t)(uint32_t)(by0 + r) * row_stride + colb - ph + (16 * idx - r * pitch_b);
+                lds_u32 *dst4 = (lds_u32 *)(ldsb + 16 * idx);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    uint32_t v = 0;
+#pragma unroll
+                    for (int b = 0; b < 4; b++) {
+                        const int64_t ob = off + 4 * i + b;
+                        v |= (ob >= 0 && (uint64_t)ob < left ? (uint32_t)base4[ob] : 0u) << (8 * b);
+                    }
+                    dst4[i] = v;
+                }
             }
         }
         wave_sync();
-        // the column behind the box repeats its last column (it is read only when that is the ROI's last column)
-        for (int r = lane; r <= bh; r += RMX_WAVE) lds[r * pitch + bw] = lds[r * pitch + bw - 1];
-        wave_sync();
+        // the column behind the box repeats its last column where that is the ROI's last column, and the row below the box its
+        // last row where that is the ROI's last row (only then are they read)
+        if (bx1 == xhi) {
+            for (int r = lane; r < bh; r += RMX_WAVE) {
+                lds_u8 *px = ldsb + r * pitch_b + ph + 3 * (bw - 1);
+                px[3] = px[0];
+                px[4] = px[1];
+                px[5] = px[2];
+            }
+            wave_sync();
+        }
+        if (!NEAREST && by1 == yhi) {
+            lds_u8 *last = ldsb + (bh - 1) * pitch_b + ph;
+            for (int b = lane; b < 3 * (bw + 1); b += RMX_WAVE) last[pitch_b + b] = last[b];
+            wave_sync();
+        }
     }
 
     // ---- gather and blend, branch-free
-    // LDS byte address of source pixel (0, 0): the slice's base minus the box origin (may lie below the slice)
-    // (RAW: byte address of the first byte of source pixel (0, 0), three bytes per pixel)
-    const int lbase0 = RAW ? (int)(uint32_t)(uintptr_t)(lds_u32 *)lds + ph - (4 * by0 * pitch + 3 * bx0)
-                           : (int)(uint32_t)(uintptr_t)(lds_u32 *)lds - 4 * (by0 * pitch + bx0);
+    // LDS byte address of the first byte of source pixel (0, 0), three bytes per pixel: the slice's base minus the box origin (may
+    // lie below the slice)
+    const int lbase0 = (int)(uint32_t)(uintptr_t)(lds_u32 *)lds + ph - (by0 * pitch_b + 3 * bx0);
     // pixels whose floor lies inside the ROI: xlo <= s < xhi + 1 (and not NaN), tested on the clamped coordinate
     // (upper bounds: the float just below xhi + 1, a positive number, so one step down in its bit pattern)
     const float cx_lo = (float)xlo, cx_hi = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, (float)(xhi + 1)) - 1u);
@@ -321,10 +340,10 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             // on 128 images of 512 x 512.
             typedef uint32_t u32x2_r __attribute__((ext_vector_type(2)));
             struct Taps {
-                u32x2_r top, bot;  // the first two dwords of the upper and of the lower row (RAW), or the two pixels of each row
-                uint32_t t2, b2;   // RAW: the third dword of each row
+                u32x2_r top, bot;   // the first two dwords of the upper and of the lower row
+                uint32_t t2, b2;    // the third dword of each row
                 float sx, sy;
-                uint32_t tph;
+                uint32_t tph, bph;  // addresses of the tap pairs: their two low bits are the phase inside the first dword
                 bool inb;
             };
             // RAW bilinear taps at the fixed pitch: the reads are written out (one address register for both rows, the row
@@ -354,28 +373,16 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
                 t.sx = sx;
                 t.sy = sy;
                 const int ix0 = floor_i32(sx), iy0 = floor_i32(sy);
-                const lds_u32 *t0p, *t1p;
-                t.tph = 0;  // RAW: byte phase of the tap pair inside its first dword
-                if constexpr (RAW) {
-                    uint32_t rowb, adr;
-                    if constexpr (FIXED) asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(rowb) : "v"(iy0), "s"(WRP * 16), "v"(lbase_v));
-                    else rowb = (uint32_t)(__mul24(iy0, pitch * 4) + lbase0);
-                    asm("v_mad_i32_i24 %0, %1, 3, %2" : "=v"(adr) : "v"(ix0), "v"(rowb));
-                    t.tph = adr & 3u;
-                    t0p = (const lds_u32 *)(adr & ~3u);
-                    t1p = FIXED ? t0p + WRP * 4 : t0p + pitch;
-                } else if constexpr (FIXED) {
-                    // byte address: a 24-bit multiply-add of the row onto the (scalar) slice base, a shift-add of the column
-                    // (spelled out: left to itself the compiler makes a shift, a multiply and a three-way add of it)
-                    uint32_t rowb, adr;
-                    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(rowb) : "v"(iy0), "s"(WFP * 4), "v"(lbase_v));
-                    asm("v_lshl_add_u32 %0, %1, 2, %2" : "=v"(adr) : "v"(ix0), "v"(rowb));
-                    t0p = (const lds_u32 *)adr;
-                    t1p = t0p + WFP;
-                } else {
-                    t0p = (const lds_u32 *)(uint32_t)(((uint32_t)(__mul24(iy0, pitch) + ix0) << 2) + (uint32_t)lbase0);
-                    t1p = t0p + pitch;
-                }
+                // byte address: a 24-bit multiply-add of the row onto the slice base, another of the column
+                uint32_t rowb, adr;
+                if constexpr (FIXED) asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(rowb) : "v"(iy0), "s"(WRP * 16), "v"(lbase_v));
+                else asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(rowb) : "v"(iy0), "s"(pitch_b), "v"(lbase_v));
+                asm("v_mad_i32_i24 %0, %1, 3, %2" : "=v"(adr) : "v"(ix0), "v"(rowb));
+                const uint32_t adr1 = adr + (uint32_t)pitch_b;
+                t.tph = adr;
+                t.bph = RAW ? adr : adr1;
+                const lds_u32 *t0p = (const lds_u32 *)(adr & ~3u);
+                const lds_u32 *t1p = FIXED ? t0p + WRP * 4 : (const lds_u32 *)(adr1 & ~3u);
                 if constexpr (BY_HAND) {
                     static_assert(WRP * 4 + 2 < 256, "the row below must be reachable by the 8-bit dword offsets of ds_read2_b32");
                     // (the values are taken apart only behind the wait: nothing may copy a register before its data has arrived)
@@ -385,17 +392,13 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
                                  : "v"((uint32_t)(uintptr_t)t0p), "n"(WRP * 4), "n"(WRP * 4 + 1), "n"(WRP * 16 + 8));
                     return t;
                 }
-                t.top = (u32x2_r){t0p[0], 0u};
+                t.top = (u32x2_r){t0p[0], t0p[1]};
                 t.bot = (u32x2_r){0u, 0u};
                 t.t2 = t.b2 = 0u;
-                if constexpr (RAW) t.top.y = t0p[1];
                 if constexpr (!NEAREST) {
-                    t.top.y = t0p[1];
+                    t.t2 = t0p[2];
                     t.bot = (u32x2_r){t1p[0], t1p[1]};
-                    if constexpr (RAW) {
-                        t.t2 = t0p[2];
-                        t.b2 = t1p[2];
-                    }
+                    t.b2 = t1p[2];
                 }
                 return t;
             };
@@ -406,29 +409,22 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
                     asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(t.top), "+v"(t.t2), "+v"(t.bot), "+v"(t.b2) : "n"(decltype(behind)::value));
             };
             auto blend = [&](int k, const Taps &tp) {
-                struct { uint32_t tl, tr, t2, bl, br, b2; float sx, sy; uint32_t tph; bool inb; } t = {tp.top.x, tp.top.y, tp.t2, tp.bot.x, tp.bot.y, tp.b2, tp.sx, tp.sy, tp.tph, tp.inb};
+                struct { uint32_t tl, tr, t2, bl, br, b2; float sx, sy; uint32_t tph, bph; bool inb; } t = {tp.top.x, tp.top.y, tp.t2, tp.bot.x, tp.bot.y, tp.b2, tp.sx, tp.sy, tp.tph, tp.bph, tp.inb};
                 float o0, o1, o2;
                 if constexpr (NEAREST) {
-                    uint32_t tl = t.tl;
-                    if constexpr (RAW) tl = __builtin_amdgcn_alignbyte(t.tr, tl, t.tph);
+                    const uint32_t tl = __builtin_amdgcn_alignbyte(t.tr, t.tl, t.tph);
                     o0 = ubyte0(tl); o1 = ubyte1(tl); o2 = ubyte2(tl);
                 } else {
                     // s - floor(s): exact for the non-negative coordinates of pixels inside the ROI
                     const float wx = __builtin_amdgcn_fractf(t.sx), wy = __builtin_amdgcn_fractf(t.sy);
                     const float omx = 1.0f - wx, omy = 1.0f - wy;
                     const float w00 = omy * omx, w01 = omy * wx, w10 = wy * omx;
-                    if constexpr (RAW) {
-                        // six bytes from byte tph on: TL in bytes 0..2 of the first realigned dword, TR from its byte 3 on
-                        const uint32_t tlo = __builtin_amdgcn_alignbyte(t.tr, t.tl, t.tph), thi = __builtin_amdgcn_alignbyte(t.t2, t.tr, t.tph);
-                        const uint32_t blo = __builtin_amdgcn_alignbyte(t.br, t.bl, t.tph), bhi = __builtin_amdgcn_alignbyte(t.b2, t.br, t.tph);
-                        o0 = __builtin_fmaf(ubyte0(tlo), w00, __builtin_fmaf(ubyte3(tlo), w01, __builtin_fmaf(ubyte0(blo), w10, ubyte3(blo) * wy * wx)));
-                        o1 = __builtin_fmaf(ubyte1(tlo), w00, __builtin_fmaf(ubyte0(thi), w01, __builtin_fmaf(ubyte1(blo), w10, ubyte0(bhi) * wy * wx)));
-                        o2 = __builtin_fmaf(ubyte2(tlo), w00, __builtin_fmaf(ubyte1(thi), w01, __builtin_fmaf(ubyte2(blo), w10, ubyte1(bhi) * wy * wx)));
-                    } else {
-                        o0 = __builtin_fmaf(ubyte0(t.tl), w00, __builtin_fmaf(ubyte0(t.tr), w01, __builtin_fmaf(ubyte0(t.bl), w10, ubyte0(t.br) * wy * wx)));
-                        o1 = __builtin_fmaf(ubyte1(t.tl), w00, __builtin_fmaf(ubyte1(t.tr), w01, __builtin_fmaf(ubyte1(t.bl), w10, ubyte1(t.br) * wy * wx)));
-                        o2 = __builtin_fmaf(ubyte2(t.tl), w00, __builtin_fmaf(ubyte2(t.tr), w01, __builtin_fmaf(ubyte2(t.bl), w10, ubyte2(t.br) * wy * wx)));
-                    }
+                    // six bytes from byte tph on: TL in bytes 0..2 of the first realigned dword, TR from its byte 3 on
+                    const uint32_t tlo = __builtin_amdgcn_alignbyte(t.tr, t.tl, t.tph), thi = __builtin_amdgcn_alignbyte(t.t2, t.tr, t.tph);
+                    const uint32_t blo = __builtin_amdgcn_alignbyte(t.br, t.bl, t.bph), bhi = __builtin_amdgcn_alignbyte(t.b2, t.br, t.bph);
+                    o0 = __builtin_fmaf(ubyte0(tlo), w00, __builtin_fmaf(ubyte3(tlo), w01, __builtin_fmaf(ubyte0(blo), w10, ubyte3(blo) * wy * wx)));
+                    o1 = __builtin_fmaf(ubyte1(tlo), w00, __builtin_fmaf(ubyte0(thi), w01, __builtin_fmaf(ubyte1(blo), w10, ubyte0(bhi) * wy * wx)));
+                    o2 = __builtin_fmaf(ubyte2(tlo), w00, __builtin_fmaf(ubyte1(thi), w01, __builtin_fmaf(ubyte2(blo), w10, ubyte1(bhi) * wy * wx)));
                 }
                 v[0][k] = t.inb ? o0 : 0.0f;
                 v[1][k] = t.inb ? o1 : 0.0f;
@@ -449,24 +445,18 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
                 blend(k, cur);
                 cur = nxt;
             }
-            // whole group into 16-byte aligned destination rows: packed stores (the host sets the flag when every
-            // written width and the padded width are multiples of 8 and the destination base is 16-byte aligned)
-            if (packed_ok && cnt == PX) {
-                PackedGroup<T> packed;
-                pack_group_dir<T, LAYOUT, false>(v, packed);
-                store_packed<T, LAYOUT, RMX_WARP_NT>(dimg, a.dst_h, a.dst_w, y, x0, packed);
-            } else {
-                store_group<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, cnt, v, false);
-            }
+            store(y, v);
         }
     };
-    if (fixed) {
-        if (all_in) gather(std::false_type{}, std::true_type{});
-        else gather(std::true_type{}, std::true_type{});
-    } else {
-        if (all_in) gather(std::false_type{}, std::false_type{});
-        else gather(std::true_type{}, std::false_type{});
+    if constexpr (RAW) {
+        if (fixed) {
+            if (all_in) gather(std::false_type{}, std::true_type{});
+            else gather(std::true_type{}, std::true_type{});
+            return;
+        }
     }
+    if (all_in) gather(std::false_type{}, std::false_type{});
+    else gather(std::true_type{}, std::false_type{});
 }
 
 template <bool NEAREST, bool RAW>
@@ -485,7 +475,7 @@ static KernelFn pick(int dtype, int layout) {
     }
 }
 
-// raw: the box as packed bytes, loaded straight into LDS (every source row must start at the same byte phase)
+// raw: the form for source rows that all start at the same byte phase
 KernelFn select_warp_kernel(int interp, int dtype, int layout, bool raw, const char **name) {
     *name = raw ? "rmx_warp_kernel(raw)" : "rmx_warp_kernel";
     if (raw) return interp == RMX_INTERP_NEAREST ? pick<true, true>(dtype, layout) : pick<false, true>(dtype, layout);
