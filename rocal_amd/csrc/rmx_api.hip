@@ -280,7 +280,7 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
     op->compact = 0;
     if (!op->ctx->compact || op->extra_per_sample || op->n > RMX_C_WORDS) return false;
     constexpr int W = (int)(sizeof(RmxSample) / 4);
-    enum { SRC = 0, DST = 4, FLAGS = 10, STRIP_ROWS = 11, RX = 12, COLOR = 22, M = 26 };  // dword of a field
+    enum { SRC = 0, DST = 4, PC = 6, FLAGS = 10, STRIP_ROWS = 11, RX = 12, COLOR = 22, M = 26 };  // dword of a field
     // bits in which the rows differ, per dword
     uint32_t diff[W] = {};
     const uint32_t *first = reinterpret_cast<const uint32_t *>(t);
@@ -313,14 +313,21 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
             break;
         }
         case OP_RESIZE: {
-            if (t[0].dst_w <= 0 || t[0].dst_h <= 0) return false;
+            // (a crop behind the resize: one centre crop of resized images of different sizes writes a window of its own per sample)
+            const bool crop = (diff[DST] | diff[DST + 1] | diff[PC] | diff[PC + 1]) != 0;
+            for (int i = 0; i < (crop ? op->n : 1); i++)
+                if (t[i].dst_w <= 0 || t[i].dst_h <= 0) return false;
             const bool tri = op->interp == RMX_INTERP_TRIANGULAR;
             tiles = !tri && (op->fn_mid || op->fn_fast);  // the streaming kernels' x-tiles
             if (!tri && op->fn_mid) diff[STRIP_ROWS] = 0;  // (the general kernel, which reads it, is not reached)
             bool order = false;
             for (int i = 0; i < op->n; i++) order = order || t[i].plan[2] != i;
             if (tiles) window |= diff[COLOR + 1];
-            if (window) {
+            if (crop) {
+                c |= RMX_C_CROP;
+                diff[DST] = diff[DST + 1] = diff[PC] = diff[PC + 1] = 0;
+            }
+            if (window || crop) {
                 c |= RMX_C_WINDOW | RMX_C_RATIO;
                 for (int k = 0; k < 4; k++) diff[RX + k] = 0;
             }
@@ -352,12 +359,12 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
     for (int k = 0; k < W; k++) rest |= diff[k];
     if (rest) return false;
     if (!op->layout.empty()) c |= RMX_C_LAYOUT;
-    uint32_t words = ((c & RMX_C_WINDOW) ? 2u : 0u) + ((c & RMX_C_M4) ? 4u : 0u) + ((c & RMX_C_M6) ? 6u : 0u) + ((c & RMX_C_ORDER) ? 1u : 0u) + ((c & RMX_C_LAYOUT) ? 2u : 0u);
+    uint32_t words = ((c & RMX_C_WINDOW) ? 2u : 0u) + ((c & RMX_C_CROP) ? 2u : 0u) + ((c & RMX_C_M4) ? 4u : 0u) + ((c & RMX_C_M6) ? 6u : 0u) + ((c & RMX_C_ORDER) ? 1u : 0u) + ((c & RMX_C_LAYOUT) ? 2u : 0u);
     for (int k = 0; k < 4; k++) words += (c & (RMX_C_COLOR0 << k)) ? 1u : 0u;
     if ((uint64_t)words * op->n > (uint64_t)RMX_C_WORDS) return false;
     // an x-tile width as its code: 0 the whole row, k: RMX_C_TILE_WHOLE >> k
-    const int whole = std::min(std::max((int)t[0].dst_w, 8), RMX_C_TILE_WHOLE);
-    auto tile_code = [&](int tw) -> uint32_t {
+    auto tile_code = [](int tw, int dst_w) -> uint32_t {
+        const int whole = std::min(std::max(dst_w, 8), RMX_C_TILE_WHOLE);
         if (tw == whole) return 0u;
         for (uint32_t k = 1; k < 8; k++)
             if (tw == RMX_C_TILE_WHOLE >> k) return k;
@@ -369,10 +376,15 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
         if (c & RMX_C_WINDOW) {
             if ((uint32_t)(s.src_x | s.src_y | s.src_w | s.src_h) > 0x3fffu) return false;
             if ((c & RMX_C_RATIO) && (s.src_w <= 0 || s.src_h <= 0)) return false;
-            const uint32_t code = tiles ? tile_code(s.plan[1]) : 0u;
+            const uint32_t code = tiles ? tile_code(s.plan[1], s.dst_w) : 0u;
             if (code > 7) return false;
             *r++ = (uint32_t)s.src_x | (uint32_t)s.src_y << 14 | (s.flags & (RMX_S_HFLIP | RMX_S_VFLIP)) << 28;
             *r++ = (uint32_t)s.src_w | (uint32_t)s.src_h << 14 | code << 28;
+        }
+        if (c & RMX_C_CROP) {
+            if ((uint32_t)(s.pc_x | s.pc_y | s.dst_w | s.dst_h) > 0x3fffu) return false;
+            *r++ = (uint32_t)s.pc_x | (uint32_t)s.pc_y << 14;
+            *r++ = (uint32_t)s.dst_w | (uint32_t)s.dst_h << 14;
         }
         for (int k = 0; k < 4; k++)
             if (c & (RMX_C_COLOR0 << k)) memcpy(r++, &s.color[k], 4);

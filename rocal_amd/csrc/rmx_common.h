@@ -61,6 +61,7 @@ enum : uint32_t {
     RMX_C_M4 = 256u,      // m[0..3]
     RMX_C_M6 = 512u,      // m[0..5]
     RMX_C_ORDER = 1024u,  // the sample this row belongs to (plan[2])
+    RMX_C_CROP = 4096u,   // two dwords behind the window's: a resize whose samples write windows of their own (pc_x, pc_y, dst_w, dst_h)
     RMX_C_LAYOUT = 2048u  // two dwords, of the sample and not of the row: source offset (40 bits) and row stride (24 bits)
 };
 constexpr int RMX_C_WORDS = 768;  // 3 KB: 256 windows with their order, 192 colour twists, 128 matrices

@@ -55,6 +55,14 @@ RMX_DEV RmxSample load_sample(const RmxKArgs &a, int i) {
                 P.dst_h = P.src_h;
             }
             if constexpr (CAN & RMX_C_RATIO) {
+                if (a.compact & RMX_C_CROP) {
+                    const uint32_t c0 = r[0], c1 = r[1];
+                    r += 2;
+                    P.pc_x = (int32_t)(c0 & 0x3fffu);
+                    P.pc_y = (int32_t)(c0 >> 14);
+                    P.dst_w = (int32_t)(c1 & 0x3fffu);
+                    P.dst_h = (int32_t)(c1 >> 14);
+                }
                 const int whole = min(max(P.dst_w, 8), RMX_C_TILE_WHOLE);
                 const uint32_t code = (w1 >> 28) & 7u;
                 P.plan[1] = code ? RMX_C_TILE_WHOLE >> code : whole;

@@ -43,6 +43,26 @@ def _resize(c, rng_seed, n, interp, packed=False, chain=False):
     return op, img
 
 
+def _resize_crops(c, seed, n, interp, packed=False, chain=False):
+    """Resized images of one size of which every sample writes a window of its own size, odd ones and one-pixel ones among them."""
+    rng = np.random.default_rng(seed)
+    h, w, o = 40, 56, 37
+    flags = (ops.F_QUANTIZE_U8 | (ops.F_COLOR_TWIST if chain else 0)) if interp == ops.LINEAR else 0
+    op = ops.Resize(c, ops.desc(n, h, w, ops.NHWC, ops.UINT8), ops.desc(n, o, o, ops.NCHW, ops.FP32), interp, flags=flags)
+    roi, d = _windows(rng, n, h, w, 9), np.full(n, o, np.uint32)
+    scale, bias = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
+    crop, mirror = _windows(rng, n, o, o, 1), rng.integers(0, 2, n).astype(np.uint32)
+    if packed:
+        W, H = np.full(n, w, np.uint32), np.full(n, h, np.uint32)
+        op.set_ragged_source(np.arange(n, dtype=np.uint64) * h * w * 3, W, H, n * h * w * 3)
+    if chain:
+        f = lambda lo, hi: rng.uniform(lo, hi, n).astype(np.float32)  # noqa: E731
+        op.update_color_cmn(roi, d, d, scale, bias, (f(0.7, 1.3), f(-9, 9), f(-30, 30), f(0.5, 1.5)), mirror, crop_roi=crop)
+    else:
+        op.update_cmn(roi, d, d, scale, bias, mirror, crop_roi=crop)
+    return op, rng.integers(0, 256, (n, h, w, 3), dtype=np.uint8)
+
+
 def _crop(c, seed, n):
     rng = np.random.default_rng(seed)
     op = ops.CropMirrorNormalize(c, ops.desc(n, 30, 40, ops.NHWC, ops.UINT8), ops.desc(n, 24, 33, ops.NCHW, ops.FP32))
@@ -94,6 +114,11 @@ MAKERS = {
     "nearest": (lambda c, s, n: _resize(c, s, n, ops.NEAREST), 2),
     "triangular": (lambda c, s, n: _resize(c, s, n, ops.TRIANGULAR), 3),
     "triangular packed": (lambda c, s, n: _resize(c, s, n, ops.TRIANGULAR, packed=True), 5),
+    "resize crops": (lambda c, s, n: _resize_crops(c, s, n, ops.LINEAR), 4),
+    "resize crops packed": (lambda c, s, n: _resize_crops(c, s, n, ops.LINEAR, packed=True), 6),
+    "chain crops": (lambda c, s, n: _resize_crops(c, s, n, ops.LINEAR, chain=True), 8),
+    "nearest crops": (lambda c, s, n: _resize_crops(c, s, n, ops.NEAREST), 4),
+    "triangular crops": (lambda c, s, n: _resize_crops(c, s, n, ops.TRIANGULAR), 5),
     "crop": (_crop, 2),
     "flip": (_flip, 2),
     "twist": (_twist, 4),
