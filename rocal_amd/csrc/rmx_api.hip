@@ -445,12 +445,12 @@ size_t dtype_size(int dtype) { return dtype == RMX_FP32 ? 4 : dtype == RMX_FP16 
 // the whole row and the powers of two below it, of which those whose window fits `cap` bytes (need_of(tw)) compete. Measured on 256
 // images to 299 x 299: tiles of 128 + 128 + 43 pixels 75.5 us, of 144 + 144 + 11 (the whole row halved until it fits) 86.6 us.
 struct TileCost {
-    int of_lanes[65];  // twice the cost of a tile of L lanes per row: a window counts half a pass
-    explicit TileCost(int rows) {
+    int of_lanes[65];  // twice the cost of a tile of L lanes per row: a window counts half a pass, and `seam` what a tile costs besides
+    explicit TileCost(int rows, int seam) {
         of_lanes[0] = 0;
         for (int lanes = 1; lanes <= 64; lanes++) {
             const int per_pass = 64 / lanes;
-            of_lanes[lanes] = 1 + 2 * ((rows + per_pass - 1) / per_pass);
+            of_lanes[lanes] = 1 + seam + 2 * ((rows + per_pass - 1) / per_pass);
         }
     }
 };
@@ -1395,7 +1395,13 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
     // 4 rows and a 10 KB slice measured best on MI355X: smaller caps cut more rows into two tiles, and the kernel's registers
     // allow 16 wavefronts per CU, which 10 KB each still fit
     const int rows = op->ctx->fast_rows, bufcap = op->ctx->dma_lds;
-    const TileCost tile_cost(rows);
+    // Planes of fp32 are bound by their stores: a row written in one piece is worth a pass more than one cut into tiles for fuller lanes
+    // (every seam is a cache line written twice, and tiles of a few columns write short runs). 96 RandomResizedCrops to 299 x 299
+    // 48.3 -> 43.0 us, 64 to 383 wide 48.3 -> 38.0, 384 wide 42.4 -> 36.9, 320 39.6 -> 37.1, up to 256 wide unchanged. With a
+    // colour node in the chain the arithmetic decides (300 wide 28.8 - 31.0 without, 29.7 - 30.2 with), and half-precision planes gain nothing (299 wide, rows
+    // whole at 3 and 2 per window: 31.8 and 34.4 against 32.2).
+    const int seam = (op->dst.dtype == RMX_FP32 && op->dst.layout == RMX_NCHW && !chain) ? 2 : 0;
+    const TileCost tile_cost(rows, seam);
     int need_max = 64;
     for (int i = 0; i < op->n && ok; i++) {
         RmxSample &s = t[i];
