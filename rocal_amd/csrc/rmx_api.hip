@@ -122,7 +122,7 @@ struct rmx_op {
     hipEvent_t uploaded[2] = {};      // per half of the ring: its last upload has completed
     bool half_pending[2] = {};        // ... was recorded and not yet waited for
     int cur = -1;  // slot of the last update that went through the table, -1 before the first
-    bool updated = false;
+    bool updated = false;  // the last update that was committed succeeded
     // the rows of the last update in the form that travels in the kernel's arguments (compact 0: they are in table slot `cur`)
     uint32_t compact = 0, compact_words = 0;
     RmxSample shared{};
@@ -241,8 +241,11 @@ int next_slot(rmx_op *op, RmxSample **row) {
 bool compact_rows(rmx_op *op, const RmxSample *t);
 
 int commit_slot(rmx_op *op, int slot) {
-    op->updated = true;
-    if (compact_rows(op, op->h_table[slot])) return RMX_OK;  // (the slot stays free: nothing on the device reads it)
+    op->updated = false;  // (until the rows are on their way: the plan is the new one already, rows of an earlier update do not go with it)
+    if (compact_rows(op, op->h_table[slot])) {  // (the slot stays free: nothing on the device reads it)
+        op->updated = true;
+        return RMX_OK;
+    }
     HIP_TRY(hipSetDevice(op->ctx->device));
     size_t bytes = sizeof(RmxSample) * (size_t)op->n;
     if (!op->layout.empty()) {
@@ -271,6 +274,7 @@ int commit_slot(rmx_op *op, int slot) {
         op->half_pending[slot / RING_HALF] = true;
     }
     op->cur = slot;
+    op->updated = true;
     return RMX_OK;
 }
 
@@ -668,7 +672,7 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
                         const void *src, const void *src2, void *dst);
 
 static int launch_impl(rmx_op *op, const void *src, const void *src2, void *dst) {
-    if (!op->updated || !op->fn) return fail(RMX_ERR_INVALID, "op launched before its first update");
+    if (!op->updated || !op->fn) return fail(RMX_ERR_INVALID, "op launched before its first update, or behind one that failed");
     if (op->compact) return launch_table(op, nullptr, nullptr, nullptr, (op->compact & RMX_C_LAYOUT) ? op->compact_src_bytes : 0, src, src2, dst);
     const bool ragged = op->slot_ragged[op->cur];
     return launch_table(op, op->d_table[op->cur], ragged ? reinterpret_cast<const RmxSrcLayout *>(op->d_table[op->cur] + op->n) : nullptr,
