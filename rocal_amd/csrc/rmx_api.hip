@@ -756,7 +756,11 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
         HIP_TRY(hipGetLastError());
     }
     void *kargs[1] = {&a};
-    HIP_TRY(hipLaunchKernel(reinterpret_cast<const void *>(fn), dim3((unsigned)blocks), dim3(wpb * RMX_WAVE), kargs, lds, op->ctx->stream));
+    const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void *>(fn), dim3((unsigned)blocks), dim3(wpb * RMX_WAVE), kargs, lds, op->ctx->stream);
+    if (launched != hipSuccess) {
+        (void)hipGetLastError();  // (told here; the thread's next check, here or in the caller's own code, is about its own call)
+        return fail(RMX_ERR_HIP, "launching %s failed: %d (%s)", rmx_op_kernel_name(op), (int)launched, hipGetErrorString(launched));
+    }
     if (!op->captured) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(op->ctx->stream, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusActive) op->captured = true;

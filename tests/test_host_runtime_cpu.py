@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["ring", "failed upload"])
+@pytest.mark.parametrize("what", ["ring", "failed upload", "failed launch"])
 def test_host_side(program, what):
     from rocal_amd import _lib
     r = subprocess.run([program, _lib.LIB_PATH, what], capture_output=True, text=True, timeout=60)
