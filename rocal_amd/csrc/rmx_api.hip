@@ -404,6 +404,11 @@ bool compact_rows(rmx_op *op, const RmxSample *t) {
         }
     }
     op->shared = t[0];
+    if (c & RMX_C_RATIO) {
+        if ((uint32_t)(t[0].rs_w | t[0].rs_h) > 0x3fffu) return false;
+        op->shared.fsx = 1.0f / (float)t[0].rs_w;
+        op->shared.fsy = 1.0f / (float)t[0].rs_h;
+    }
     if (c & RMX_C_WINDOW) op->shared.flags &= ~(uint32_t)(RMX_S_HFLIP | RMX_S_VFLIP);
     op->compact = c;
     op->compact_words = words;

@@ -16,7 +16,7 @@ struct __attribute__((aligned(16))) RmxSample {
     int32_t rs_w, rs_h;                  // virtual resized size (== dst when there is no post-crop)
     uint32_t flags;                      // RMX_S_*
     int32_t strip_rows;                  // output rows per wave strip for this sample
-    float rx, ry;                        // src_len / rs_len (IEEE division done on the host)
+    float rx, ry;                        // src_len / rs_len, the IEEE quotient
     float fsx, fsy;                      // triangular: ratio > 1 ? 1/ratio : 1
     float scale[3], bias[3];             // normalisation: out = v*scale + bias
     union {
@@ -49,8 +49,9 @@ enum : uint32_t {
 // A batch whose rows differ in little (crop windows and mirror flags, colour factors, a matrix) travels in the kernel's
 // arguments: one row of what all samples share and a few dwords per sample, from which load_sample() (rmx_device.h) makes the
 // row again. A table in device memory costs a launch of its own in front of every batch's kernel (the upload, 3 - 4 us on the
-// GPU and, with the event that guards its slot, 8 us of the host), the arguments 0.3 us and 1 us: measured for 2 KB of them
-// read by 14 336 wavefronts. Whole batches, one update and launch after the other: 256 RandomResizedCrop windows to 224 x 224 fp16
+// GPU and, with the event that guards its slot, 8 us of the host), the arguments 1 us of the host. A kernel launched again and again on
+// the rows of one update is 0.1 - 0.8 us longer with them than with a table that stays in the caches (256 windows 40.5 -> 40.8 us, bytes
+// 21.9 -> 22.3, 128 windows with antialiasing 41.2 -> 41.9). Whole batches, one update and launch after the other: 256 RandomResizedCrop windows to 224 x 224 fp16
 // 37.4 -> 31.5 us, 128 crops of 224 x 224 to fp32 planes 22.2 -> 16.8 us, 14 small crops 16.9 -> 11.0 us. What a sample's dwords hold, in this order:
 enum : uint32_t {
     RMX_C_ON = 1u,        // the rows are in the arguments
@@ -65,6 +66,7 @@ enum : uint32_t {
     RMX_C_LAYOUT = 2048u  // two dwords, of the sample and not of the row: source offset (40 bits) and row stride (24 bits)
 };
 constexpr int RMX_C_WORDS = 768;  // 3 KB: 256 windows with their order, 192 colour twists, 128 matrices
+constexpr int RMX_C_PAD = 4;      // (load_sample reads this many dwords from a record's start, however many it has)
 constexpr int RMX_C_TILE_WHOLE = 512;  // code k of an x-tile width: 0 the whole row (up to this many pixels), else this >> k
 
 struct RmxKArgs {
@@ -89,9 +91,17 @@ struct RmxKArgs {
     uint32_t compact;            // RMX_C_*: 0 when the rows are in `table`
     uint32_t compact_words;      // dwords per sample in `rec`
     RmxSample shared;            // what every sample's row holds
-    uint32_t rec[RMX_C_WORDS];
+    uint32_t rec[RMX_C_WORDS + RMX_C_PAD];
 };
 static_assert(sizeof(RmxKArgs) <= 4096, "kernel arguments are limited to 4 KB");
+
+// a / b, correctly rounded, for whole numbers a and b of up to 14 bits and recip = 1 / b correctly rounded: the product with the
+// reciprocal is off by an ulp at most, its remainder is exact, and one correction of the quotient by it rounds as the
+// division does (Markstein, IBM J. Res. Dev. 34, 1990; every pair is checked by tests/test_quotients_cpu.py).
+__host__ __device__ inline float ratio_of(float a, float b, float recip) {
+    const float q = a * recip;
+    return __builtin_fmaf(__builtin_fmaf(-b, q, a), recip, q);
+}
 
 #define RMX_WAVE 64
 #define RMX_MOMENT_PARTS 8  // workgroups per sample of the moments pass (Normalize): 6 x 8 shares, one per lane of a streaming wavefront

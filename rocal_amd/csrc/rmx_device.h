@@ -29,21 +29,55 @@ RMX_DEV float round_u8(float v) {
 // The compact records of the kernel's arguments, read where the hardware put them (indexed as a member of the by-value struct,
 // they would be copied to scratch memory first).
 typedef const __attribute__((address_space(4))) uint32_t *karg_u32;
+// A wave-uniform read of memory that nothing writes while a kernel runs (rows, layout entries), through scalar loads. (Behind an asm
+// statement the compiler takes plain loads for vector ones.)
+template <typename T>
+RMX_DEV T load_constant(const T *p) {
+    const karg_u32 q = (karg_u32)(uintptr_t)p;
+    uint32_t w[sizeof(T) / 4];
+#pragma unroll
+    for (unsigned k = 0; k < sizeof(T) / 4; k++) w[k] = q[k];
+    return __builtin_bit_cast(T, w);
+}
+
 RMX_DEV karg_u32 compact_record(const RmxKArgs &a, int i) {
     return (karg_u32)((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(RmxKArgs, rec)) +
            (uint32_t)i * a.compact_words;
 }
 
+// Asks for the arguments that every wavefront reads, all of them in front of the first branch: loads behind a branch are a round
+// trip to memory of their own (fields in the order of their use were four in front of the first source load).
+RMX_DEV void fetch_header(const RmxKArgs &a) {
+    asm volatile("" : : "s"(a.src), "s"(a.dst), "s"(a.table), "s"(a.src_bytes), "s"(a.layout), "s"(a.n), "s"(a.src_h), "s"(a.src_w), "s"(a.dst_h), "s"(a.dst_w),
+                 "s"(a.strips), "s"(a.lds_bytes), "s"(a.aux0), "s"(a.aux1), "s"(a.wpb), "s"(a.nblocks), "s"(a.inv_strips), "s"(a.per_xcd), "s"(a.inv_per_xcd),
+                 "s"(a.compact), "s"(a.compact_words));
+}
+
 // Row i of the batch's parameter table: from device memory, or made again from the kernel's arguments (RMX_C_*). CAN: what a
-// record of this kernel's ops can hold. Everything is wave-uniform. The quotients are the host's (both IEEE divisions).
-template <uint32_t CAN>
+// record of this kernel's ops can hold. Everything is wave-uniform. The ratios are the host's quotients, as two multiply-adds
+// behind its reciprocals: divisions, run by every wavefront in front of its first load, were a quarter of what the records cost a
+// launch (256 windows to 224 x 224 fp16: 41.1 -> 40.9 us).
+// AHEAD: the record's first dwords are asked for together with the shared row, before any branch, whether the record holds
+// them or not (RMX_C_PAD keeps those behind the last record inside the arguments): one round trip in the place of three (the
+// same launch 40.9 -> 40.6 us; bytes 22.4 -> 22.2 us). Only the resize kernels that are not bound by their arithmetic take it: with a
+// colour twist in the chain they are slower for it (320 wide to fp32 planes 34.9 -> 36.4 us), and so is the triangular one.
+template <uint32_t CAN, bool AHEAD = false>
 RMX_DEV RmxSample load_sample(const RmxKArgs &a, int i) {
-    if (!(a.compact & RMX_C_ON)) return a.table[i];
+    if (!(a.compact & RMX_C_ON)) {
+        if constexpr (AHEAD) return load_constant(a.table + i);
+        else return a.table[i];
+    }
     RmxSample P = a.shared;
     karg_u32 r = compact_record(a, i);
+    uint32_t ahead[4] = {};
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) ahead[k] = r[k];
+        asm volatile("" : : "s"(ahead[0]), "s"(ahead[1]), "s"(ahead[2]), "s"(ahead[3]));
+    }
     if constexpr (CAN & RMX_C_WINDOW) {
         if (a.compact & RMX_C_WINDOW) {
-            const uint32_t w0 = r[0], w1 = r[1];
+            const uint32_t w0 = AHEAD ? ahead[0] : r[0], w1 = AHEAD ? ahead[1] : r[1];
             r += 2;
             P.src_x = (int32_t)(w0 & 0x3fffu);
             P.src_y = (int32_t)((w0 >> 14) & 0x3fffu);
@@ -56,7 +90,7 @@ RMX_DEV RmxSample load_sample(const RmxKArgs &a, int i) {
             }
             if constexpr (CAN & RMX_C_RATIO) {
                 if (a.compact & RMX_C_CROP) {
-                    const uint32_t c0 = r[0], c1 = r[1];
+                    const uint32_t c0 = AHEAD ? ahead[2] : r[0], c1 = AHEAD ? ahead[3] : r[1];
                     r += 2;
                     P.pc_x = (int32_t)(c0 & 0x3fffu);
                     P.pc_y = (int32_t)(c0 >> 14);
@@ -66,8 +100,9 @@ RMX_DEV RmxSample load_sample(const RmxKArgs &a, int i) {
                 const int whole = min(max(P.dst_w, 8), RMX_C_TILE_WHOLE);
                 const uint32_t code = (w1 >> 28) & 7u;
                 P.plan[1] = code ? RMX_C_TILE_WHOLE >> code : whole;
-                P.rx = (float)P.src_w / (float)P.rs_w;
-                P.ry = (float)P.src_h / (float)P.rs_h;
+                // (the shared row's fsx and fsy hold the reciprocals of rs_w and rs_h)
+                P.rx = ratio_of((float)P.src_w, (float)P.rs_w, P.fsx);
+                P.ry = ratio_of((float)P.src_h, (float)P.rs_h, P.fsy);
                 P.fsx = P.rx > 1.0f ? 1.0f / P.rx : 1.0f;
                 P.fsy = P.ry > 1.0f ? 1.0f / P.ry : 1.0f;
             }
@@ -101,7 +136,7 @@ RMX_DEV const uint8_t *sample_base(const RmxKArgs &a, int s, uint32_t &row_strid
         return a.src + (((uint64_t)(hi >> 24) << 32) | lo);
     }
     if (a.layout) {
-        const RmxSrcLayout L = a.layout[s];
+        const RmxSrcLayout L = load_constant(a.layout + s);
         row_stride = L.row_stride;
         return a.src + L.offset;
     }

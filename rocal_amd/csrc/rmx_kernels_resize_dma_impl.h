@@ -90,17 +90,19 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     // Interleaved fp32 (96 bytes per lane): the lanes of a row exchange their runs through LDS before storing (57.1 -> 48.4 us on
     // the RandomResizedCrop batch); the slab is the tail of the wavefront's slice, the host adds its size.
     constexpr bool COALESCE = sizeof(T) == 4 && LAYOUT == RMX_NHWC;
+    constexpr bool AHEAD = CHAIN != CHAIN_TWIST;  // (see load_sample)
     static_assert(!(ALIGNED && COALESCE), "interleaved fp32 has one form");
     __shared__ __attribute__((aligned(16))) float chain_tables[CHAIN == CHAIN_TWIST ? sizeof(ColorTables) / 4 : 4];
     const int lane = threadIdx.x & (RMX_WAVE - 1);
     const int wib = threadIdx.x / RMX_WAVE;
+    if constexpr (AHEAD) fetch_header(a);
     const uint32_t nwaves = (uint32_t)a.n * (uint32_t)a.strips;
     uint32_t wave = xcd_swizzle(blockIdx.x, a.nblocks) * (uint32_t)a.wpb + wib;
     wave = __builtin_amdgcn_readfirstlane(wave);
     if (wave >= nwaves) return;
     int s, grp;
     wave_to_sample(a, wave, s, grp);
-    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | (CHAIN == CHAIN_NONE ? 0u : RMX_C_M4)>(a, s);
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | (CHAIN == CHAIN_NONE ? 0u : RMX_C_M4), AHEAD>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.pc_x), "s"(P.flags), "s"(P.rx), "s"(P.scale[0]), "s"(P.bias[2]), "s"(P.plan[1]));
 
     const int dw = P.dst_w, dh = P.dst_h;
@@ -147,7 +149,7 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     const uint32_t lim = left > 0xffffffffull ? 0xffffffffu : (uint32_t)left;
 
     const int tile_w = max(P.plan[1], PX);  // never 0: it is the step of the tile loop
-    const int ntx = (dw + tile_w - 1) / tile_w;
+    const int ntx = tile_w >= dw ? 1 : (dw + tile_w - 1) >> (31 - __builtin_clz(tile_w));  // (a tile is the whole row or a power of two wide)
 
     // ---- geometry of an x-tile and of a window of it (all wave-uniform)
     // nearest: the index of the pixel whose centre is closest, clamped into the window
