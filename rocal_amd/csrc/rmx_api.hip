@@ -154,6 +154,7 @@ struct rmx_op {
     // (224 pixels are 28 groups of 8: two rows per step keep 56 lanes busy; 299 pixels keep 38). 0: the images' own rows.
     int flat_h = 0;
     bool own_moments = false;          // Normalize: the mean or the deviation of the last update is computed on the device
+    int moment_parts = 1, moment_threads = RMX_WAVE;  // ... by so many workgroups per sample of so many threads
     unsigned long long *moments = nullptr;  // ... from these shares (device workspace of the op, written in front of every streaming pass)
     rmx::KernelFn lds_fn[3] = {};  // kernels whose static LDS size has been asked of the runtime ([0] general, [1] fast, [2] mid)
     int lds_static[3] = {};
@@ -634,24 +635,24 @@ int rmx_op_destroy(rmx_op *op) {
 uint64_t rmx_op_algorithmic_bytes(const rmx_op *op) { return op ? op->algo_bytes : 0; }
 
 const char *rmx_op_plan(const rmx_op *op) {
-    static thread_local char buf[256];
+    static thread_local char buf[320];
     if (!op) return "";
-    if (op->flat_h) {  // whole frames as rows of 512 pixels
-        snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=%d flat_rows=%d",
-                 (long long)op->n * op->strips, op->strips, op->aux0, 0, op->waves_per_block, op->fn_fast ? 1 : 0, op->flat_h);
-        return buf;
-    }
-    if (op->fn_fast)
-        snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=1 group=%d",
-                 (long long)op->n * op->fast_strips, op->fast_strips, op->fast_rows, op->fast_lds, op->fast_wpb, std::max(1, op->fast_aux1));
+    int len;
+    if (op->flat_h)  // whole frames as rows of 512 pixels
+        len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=%d flat_rows=%d",
+                       (long long)op->n * op->strips, op->strips, op->aux0, 0, op->waves_per_block, op->fn_fast ? 1 : 0, op->flat_h);
+    else if (op->fn_fast)
+        len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=1 group=%d",
+                       (long long)op->n * op->fast_strips, op->fast_strips, op->fast_rows, op->fast_lds, op->fast_wpb, std::max(1, op->fast_aux1));
     else if (op->fn_mid)
-        snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=0 any_width=1 group=%d",
-                 (long long)op->n * op->mid_strips, op->mid_strips, op->mid_rows, op->mid_lds, op->mid_wpb, std::max(1, op->mid_aux1));
+        len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=0 any_width=1 group=%d",
+                       (long long)op->n * op->mid_strips, op->mid_strips, op->mid_rows, op->mid_lds, op->mid_wpb, std::max(1, op->mid_aux1));
     else {
-        int len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d tile_w=%d lds_per_wave=%d waves_per_block=%d fast=0",
-                           (long long)op->n * op->strips, op->strips, op->strip_rows, op->tile_w, op->lds_per_wave, op->waves_per_block);
-        if (op->tri_rows_in_flight && len > 0 && len < (int)sizeof(buf)) snprintf(buf + len, sizeof(buf) - len, " rows_in_flight=%d", op->tri_rows_in_flight);
+        len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d tile_w=%d lds_per_wave=%d waves_per_block=%d fast=0",
+                       (long long)op->n * op->strips, op->strips, op->strip_rows, op->tile_w, op->lds_per_wave, op->waves_per_block);
+        if (op->tri_rows_in_flight) len += snprintf(buf + len, sizeof(buf) - len, " rows_in_flight=%d", op->tri_rows_in_flight);
     }
+    if (op->own_moments) len += snprintf(buf + len, sizeof(buf) - len, " moments=%dx%d", op->moment_parts, op->moment_threads);
     return buf;
 }
 const char *rmx_op_kernel_name(const rmx_op *op) { return op ? (op->fn_fast ? op->fast_name : (op->fn_mid ? op->mid_name : op->kernel_name)) : ""; }
@@ -757,7 +758,7 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
     }
     if (op->own_moments) {  // shares of every sample's moments, which the streaming pass makes its constants from
         a.extra = reinterpret_cast<const uint8_t *>(op->moments);
-        rmx::launch_moments(op->ctx->stream, a, op->moments);
+        rmx::launch_moments(op->ctx->stream, a, op->moments, __builtin_ctz(op->moment_parts), op->moment_threads);
         HIP_TRY(hipGetLastError());
     }
     void *kargs[1] = {&a};
@@ -951,11 +952,19 @@ int rmx_update_to_tensor(rmx_op *op, const float *multiplier, const float *offse
 
 /* ------------------------------------------------------------------ Normalize */
 
+// Workgroups per sample of the moments pass at most: eight, and with fewer than 64 samples so many that the batch still makes 512
+// of them, two for every CU (one image of 2160 x 3840: 97 us with eight, 37 with 64; four: 151 and 97).
+static int moment_parts_max(int n) {
+    int p = 8;
+    while (p < RMX_MOMENT_PARTS && (long)n * p * 2 <= 512) p *= 2;
+    return p;
+}
+
 int rmx_create_normalize(rmx_ctx *ctx, const rmx_tensor_desc *src, const rmx_tensor_desc *dst, int roi_type, rmx_op **out) {
     int rc = make_op(ctx, OP_NORMALIZE, src, dst, roi_type, out);
     if (rc) return rc;
     (*out)->norm = true;
-    hipError_t e = hipMalloc((void **)&(*out)->moments, (size_t)src->n * 6 * RMX_MOMENT_PARTS * sizeof(unsigned long long));
+    hipError_t e = hipMalloc((void **)&(*out)->moments, (size_t)src->n * 6 * moment_parts_max((*out)->n) * sizeof(unsigned long long));
     if (e != hipSuccess) {
         rmx_op_destroy(*out);
         *out = nullptr;
@@ -979,6 +988,15 @@ int rmx_update_normalize(rmx_op *op, const uint32_t *src_roi, uint32_t axis_mask
     if (rc) return rc;
     // given statistics, or neutral ones; with both given the constants are made here and the streaming pass runs alone
     op->own_moments = !mean || !stddev;
+    // The moments pass in workgroups that keep their lanes busy: four groups of 8 pixels per lane, so a wavefront per 256 groups, up to
+    // eight of them, then several workgroups. (1024 images of 32 x 32, whole batches: a fixed eight workgroups of eight wavefronts,
+    // of which 16 lanes had work, 31.6 us; now 9.0. 64 of 300 x 400 have eight of eight either way.)
+    long groups = 1;
+    for (int i = 0; i < op->n; i++) groups = std::max(groups, (long)((op->h_table[slot][i].dst_w + 7) / 8) * op->h_table[slot][i].dst_h);
+    const int parts_max = moment_parts_max(op->n);
+    op->moment_threads = (int)std::min<long>(8, (groups + 255) / 256) * RMX_WAVE;
+    op->moment_parts = 1;
+    while (op->moment_parts < parts_max && (long)op->moment_parts * 2048 < groups) op->moment_parts *= 2;
     for (int i = 0; i < op->n; i++) {
         RmxSample &s = op->h_table[slot][i];
         for (int c = 0; c < 3; c++) {
@@ -989,6 +1007,7 @@ int rmx_update_normalize(rmx_op *op, const uint32_t *src_roi, uint32_t axis_mask
         }
         s.color[0] = scale;
         s.color[1] = shift;
+        s.strip_rows = __builtin_ctz(op->moment_parts);
         s.flags |= (mean ? 0u : RMX_S_OWN_MEAN) | (stddev ? 0u : RMX_S_OWN_STD) | (axis_mask == 3u ? RMX_S_PER_CHANNEL : 0u);
     }
     const int knorm = op->own_moments ? 2 : 1;

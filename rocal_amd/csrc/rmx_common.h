@@ -15,7 +15,7 @@ struct __attribute__((aligned(16))) RmxSample {
     int32_t pc_x, pc_y;                  // offset of the written window inside the virtual resized image
     int32_t rs_w, rs_h;                  // virtual resized size (== dst when there is no post-crop)
     uint32_t flags;                      // RMX_S_*
-    int32_t strip_rows;                  // output rows per wave strip for this sample
+    int32_t strip_rows;                  // output rows per wave strip for this sample; Normalize: shares of its moments (log2)
     float rx, ry;                        // src_len / rs_len, the IEEE quotient
     float fsx, fsy;                      // triangular: ratio > 1 ? 1/ratio : 1
     float scale[3], bias[3];             // normalisation: out = v*scale + bias
@@ -104,7 +104,7 @@ __host__ __device__ inline float ratio_of(float a, float b, float recip) {
 }
 
 #define RMX_WAVE 64
-#define RMX_MOMENT_PARTS 8  // workgroups per sample of the moments pass (Normalize): 6 x 8 shares, one per lane of a streaming wavefront
+#define RMX_MOMENT_PARTS 64  // workgroups per sample of the moments pass (Normalize) at most
 
 // Hue shift of a sample in sextants (ColorTwist, Hue, Saturation). A pixel's hue before it is brought back into [0, 6] lies in
 // [shift - 1.0000002, shift + 5.0000002]; below RMX_HUE_SHIFT_LOW it can never reach 6, from RMX_HUE_SHIFT_HIGH on never fall

@@ -31,19 +31,22 @@ namespace rmx {
 enum { CMN_GENERAL = 0, CMN_FAST = 1, CMN_FAST_ANY = 2, CMN_FLAT = 3, CMN_FLAT_ANY = 4 };
 enum { NORM_NONE = 0, NORM_ROW = 1, NORM_OWN = 2 };
 
-// FMA constants of a Normalize sample from the shares of its moments (rmx_kernels_stats.hip): lane 8 k + p holds share p of moment
-// k (three sums, three sums of squares), eight lanes add up, lane c makes channel c's constants. The double arithmetic runs
-// once per wavefront, in three lanes.
+// FMA constants of a Normalize sample from the shares of its moments (rmx_kernels_stats.hip): lane 8 k + p adds up shares p, p + 8, ...
+// of moment k (three sums, three sums of squares), eight lanes add up, lane c makes channel c's constants. The double arithmetic
+// runs once per wavefront, in three lanes.
 struct OwnStats {
     uint32_t flags;
+    int log2_parts;
     float w, h, mean0, mean1, mean2, std0, std1, std2, scale, shift;
 };
 RMX_DEV void own_constants(const OwnStats o, const uint8_t *shares, int s, int lane, float (&sc)[3], float (&bi)[3]) {
-    static_assert(RMX_MOMENT_PARTS == 8, "eight lanes per moment");
-    const unsigned long long *mine = reinterpret_cast<const unsigned long long *>(shares) + (size_t)s * 6 * RMX_MOMENT_PARTS;
-    unsigned long long v = lane < 6 * RMX_MOMENT_PARTS ? mine[lane] : 0ull;
+    const unsigned long long *all = reinterpret_cast<const unsigned long long *>(shares) + (((size_t)s * 6) << o.log2_parts);
+    const int p = lane & 7, nparts = 1 << o.log2_parts;
+    const uint32_t mine = ((uint32_t)(lane >> 3) << o.log2_parts) + (uint32_t)p;
+    unsigned long long v = lane < 48 && p < nparts ? all[mine] : 0ull;
+    for (int more = 8; more < nparts; more += 8) v += lane < 48 ? all[mine + more] : 0ull;
 #pragma unroll
-    for (int off = 1; off < RMX_MOMENT_PARTS; off <<= 1) v += __shfl_xor(v, off, RMX_WAVE);
+    for (int off = 1; off < 8; off <<= 1) v += __shfl_xor(v, off, RMX_WAVE);
     const bool per_channel = (o.flags & RMX_S_PER_CHANNEL) != 0;
     const int c = min(lane, 2);
     double cnt = (double)o.w * (double)o.h;
@@ -121,7 +124,7 @@ __global__ void __launch_bounds__(256) rmx_cmn_kernel(RmxKArgs a) {
     }
     // (made behind the start of the first pixel loads where there is a pipeline, so that the two round trips and the double
     // arithmetic run while those are on their way)
-    const OwnStats stats = {P.flags, (float)P.dst_w, (float)P.dst_h, P.m[0], P.m[1], P.m[2], P.m[3], P.m[4], P.m[5], P.color[0], P.color[1]};
+    const OwnStats stats = {P.flags, P.strip_rows, (float)P.dst_w, (float)P.dst_h, P.m[0], P.m[1], P.m[2], P.m[3], P.m[4], P.m[5], P.color[0], P.color[1]};
     auto own = [&](int xt) {
         if constexpr (NORM == NORM_OWN) {
             if (xt == 0) own_constants(stats, a.extra, s, lane, sc, bi);

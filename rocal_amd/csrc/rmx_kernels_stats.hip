@@ -1,5 +1,5 @@
 // Normalize (mean / standard deviation over the image axes of each sample): the pass in front of the streaming one.
-//   rmx_moments_kernel  RMX_MOMENT_PARTS workgroups per sample, each a share of the window's rows: per-channel sum and sum of
+//   rmx_moments_kernel  1 to RMX_MOMENT_PARTS workgroups per sample, each a share of the window's rows: per-channel sum and sum of
 //                       squares as exact integers (bytes: no rounding, so the order of the additions does not matter), six
 //                       64-bit numbers per workgroup, written to a workspace of the op.
 // The streaming pass is the CropMirrorNormalize kernel in its form NORM_OWN: every wavefront adds its sample's shares up, makes
@@ -15,7 +15,7 @@
 
 namespace rmx {
 
-constexpr int MOM_THREADS = 512;
+constexpr int MOM_THREADS = 512;  // at most
 constexpr int MOM_WAVES = MOM_THREADS / RMX_WAVE;
 
 // sum over the wavefront, in lane 63 (row shifts inside rows of 16 lanes, then the broadcasts of their last lanes)
@@ -29,12 +29,12 @@ RMX_DEV uint32_t wave_sum_lane63(uint32_t v) {
     return v;
 }
 
-__global__ void __launch_bounds__(MOM_THREADS) rmx_moments_kernel(RmxKArgs a, unsigned long long *parts) {
+__global__ void __launch_bounds__(MOM_THREADS) rmx_moments_kernel(RmxKArgs a, unsigned long long *parts, int log2_parts) {
     __shared__ unsigned long long wave_sums[MOM_WAVES][6];
-    const int s = blockIdx.x / RMX_MOMENT_PARTS, part = blockIdx.x % RMX_MOMENT_PARTS;
+    const int s = (int)(blockIdx.x >> log2_parts), part = (int)(blockIdx.x & ((1u << log2_parts) - 1u)), threads = blockDim.x;
     const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_DST>(a, s);
     const int w = max(P.dst_w, 0), h = max(P.dst_h, 0);
-    const int r0 = (int)((long long)h * part / RMX_MOMENT_PARTS), r1 = (int)((long long)h * (part + 1) / RMX_MOMENT_PARTS);
+    const int r0 = (int)(((long long)h * part) >> log2_parts), r1 = (int)(((long long)h * (part + 1)) >> log2_parts);
     uint32_t row_stride;
     const uint8_t *simg = sample_base(a, s, row_stride);
     const uint8_t *first = simg + (size_t)P.src_y * row_stride + (size_t)P.src_x * 3;
@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(MOM_THREADS) rmx_moments_kernel(RmxKArgs a, un
 
     // groups of 8 pixels, row after row, dealt to the threads
     const int groups = (w + PX - 1) / PX;
-    const int dr = groups ? MOM_THREADS / groups : 0, dg = MOM_THREADS - dr * groups;
+    const int dr = groups ? threads / groups : 0, dg = threads - dr * groups;
     int r = r0 + (groups ? (int)threadIdx.x / groups : 0), g = groups ? (int)threadIdx.x % groups : 0;
     if (groups == 0) r = r1;
     unsigned long long total[6] = {};
@@ -111,13 +111,13 @@ __global__ void __launch_bounds__(MOM_THREADS) rmx_moments_kernel(RmxKArgs a, un
     if (threadIdx.x < 6) {
         unsigned long long t = 0;
 #pragma unroll
-        for (int v = 0; v < MOM_WAVES; v++) t += wave_sums[v][threadIdx.x];
-        parts[((size_t)s * 6 + threadIdx.x) * RMX_MOMENT_PARTS + part] = t;
+        for (int v = 0; v < MOM_WAVES; v++) t += v * RMX_WAVE < threads ? wave_sums[v][threadIdx.x] : 0ull;
+        parts[(((size_t)s * 6 + threadIdx.x) << log2_parts) + part] = t;
     }
 }
 
-void launch_moments(hipStream_t stream, const RmxKArgs &a, unsigned long long *parts) {
-    hipLaunchKernelGGL(rmx_moments_kernel, dim3((unsigned)a.n * RMX_MOMENT_PARTS), dim3(MOM_THREADS), 0, stream, a, parts);
+void launch_moments(hipStream_t stream, const RmxKArgs &a, unsigned long long *parts, int log2_parts, int threads) {
+    hipLaunchKernelGGL(rmx_moments_kernel, dim3((unsigned)a.n << log2_parts), dim3(threads), 0, stream, a, parts, log2_parts);
 }
 
 }  // namespace rmx

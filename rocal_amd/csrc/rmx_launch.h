@@ -25,8 +25,9 @@ KernelFn select_warp_kernel(int interp, int dtype, int layout, bool raw, const c
 #define RMX_WARP_RAW_PIECES 11
 #endif
 constexpr int kWarpRawPieces = RMX_WARP_RAW_PIECES;
-// Normalize: integer moments of every sample's window, RMX_MOMENT_PARTS shares of six 64-bit numbers per sample
-void launch_moments(hipStream_t stream, const RmxKArgs &a, unsigned long long *parts);
+// Normalize: integer moments of every sample's window, 1 << log2_parts shares of six 64-bit numbers per sample, each made by a workgroup
+// of `threads` (whole wavefronts, at most 512)
+void launch_moments(hipStream_t stream, const RmxKArgs &a, unsigned long long *parts, int log2_parts, int threads);
 void launch_copy(hipStream_t stream, const void *src, void *dst, size_t nbytes, int num_cus);
 // mode 0 copy, 1 read only, 2 write only; groups_per_cu 0 = the default (16)
 void launch_stream(hipStream_t stream, int mode, const void *src, void *dst, size_t nbytes, int num_cus, int groups_per_cu);

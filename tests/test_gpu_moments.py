@@ -35,3 +35,24 @@ def test_moments(ctx, h, w, mask, given):
         for i in range(n):
             x = (slice(None), slice(0, roi[i, 3]), slice(0, roi[i, 2]))
             assert np.array_equal(got[i][x].view(np.uint32), exp[i][x].view(np.uint32)), (i, ragged)
+
+
+@pytest.mark.parametrize("n,h,w,shares", [
+    (1, 1, 8, "1x64"), (3, 32, 64, "1x64"), (1, 257, 8, "1x128"), (2, 2048, 7, "1x512"), (1, 2049, 8, "2x512"),  # wavefronts of 256 groups
+    (1, 3, 32800, "8x512"), (1, 1030, 1024, "64x512"), (9, 1030, 1024, "32x512"), (65, 150, 1000, "8x512"), (200, 32, 32, "1x64")])
+def test_moment_shares(ctx, n, h, w, shares):
+    """Shares of a sample's moments: as many workgroups and wavefronts as its groups of 8 pixels keep busy, more of them in small
+    batches; also more shares than rows."""
+    import torch
+    rng = np.random.default_rng(h + w)
+    img = rng.integers(0, 256, (n, h, w, 3), dtype=np.uint8)
+    img[0] |= 0xc0  # (large sums)
+    roi = np.tile(np.array([0, 0, w, h], np.uint32), (n, 1))
+    op = ops.Normalize(ctx, ops.desc(n, h, w, ops.NHWC, ops.UINT8), ops.desc(n, h, w, ops.NHWC, ops.FP16))
+    op.update(roi, axis_mask=3, scale=1.5, shift=0.25)
+    assert op.plan.endswith("moments=" + shares), op.plan
+    out = op.alloc_output()
+    op.launch(torch.from_numpy(img).cuda(), out)
+    ctx.sync()
+    exp = orc.normalize(img, roi, axis_mask=3, scale=1.5, shift=0.25, layout=ops.NHWC, dtype=ops.FP16)
+    assert np.array_equal(out.cpu().numpy().view(np.uint16), exp.view(np.uint16))
