@@ -1475,10 +1475,9 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         op->fn_mid = rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, false, &op->mid_name);
         if (widths8) op->fn_fast = rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &op->fast_name);
     } else if (op->ctx->dma) {
-        op->fn_mid = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, &op->mid_name);
+        op->fn_mid = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, false, &op->mid_name);
     }
-    // (also interleaved fp32 of whole groups)
-    if (widths8 && !op->fn_fast) op->fn_fast = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, &op->fast_name);
+    if (widths8 && !op->fn_fast) op->fn_fast = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &op->fast_name);
     return RMX_OK;
 }
 

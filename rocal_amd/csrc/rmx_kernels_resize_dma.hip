@@ -18,8 +18,8 @@ static KernelFn pick3(bool norm, bool quant, int chain) {
     return (KernelFn)rmx_resize_dma_kernel<T, LAYOUT, false, false, CHAIN_NONE, ALIGNED>;
 }
 
-// aligned: the form for whole groups and 16-byte aligned rows; null for interleaved fp32, which leaves through the coalescing
-// stores of its one form (rmx_resize_fast_kernel for whole groups).
+// aligned: the form for whole groups and 16-byte aligned rows; null for interleaved fp32, which is bound by its stores and has
+// one such form for rows at any phase (rmx_resize_runs_kernel).
 KernelFn select_resize_dma_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool aligned, const char **name) {
     *name = "rmx_resize_dma_kernel";
     if (!aligned) {

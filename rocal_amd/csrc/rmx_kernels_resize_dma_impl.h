@@ -91,7 +91,6 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     // the RandomResizedCrop batch); the slab is the tail of the wavefront's slice, the host adds its size.
     constexpr bool COALESCE = sizeof(T) == 4 && LAYOUT == RMX_NHWC;
     constexpr bool AHEAD = CHAIN != CHAIN_TWIST;  // (see load_sample)
-    static_assert(!(ALIGNED && COALESCE), "interleaved fp32 has one form");
     __shared__ __attribute__((aligned(16))) float chain_tables[CHAIN == CHAIN_TWIST ? sizeof(ColorTables) / 4 : 4];
     const int lane = threadIdx.x & (RMX_WAVE - 1);
     const int wib = threadIdx.x / RMX_WAVE;
@@ -412,7 +411,8 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
                 else if constexpr (COALESCE) {
                     // (a row's lanes hold its runs left to right, or right to left under a mirror: a run goes to its own place in the slab)
                     const int L = (g.tw + PX - 1) / PX, l = lane - lr * L, xs = hf ? dw - g.xt - g.tw : g.xt;
-                    store_packed_coalesced_any<T, LAYOUT, RMX_DMA_NT>(slab, lane - l, l, L, xs, g.tw, dimg, a.dst_h, a.dst_w, r, x0, packed);
+                    if constexpr (ALIGNED) store_packed_coalesced<T, LAYOUT, RMX_DMA_NT>(slab, lane - l, hf ? L - 1 - l : l, L, dimg, a.dst_h, a.dst_w, r, x0, packed);
+                    else store_packed_coalesced_any<T, LAYOUT, RMX_DMA_NT>(slab, lane - l, l, L, xs, g.tw, dimg, a.dst_h, a.dst_w, r, x0, packed);
                 } else store_packed<T, LAYOUT, RMX_DMA_NT, !ALIGNED>(dimg, a.dst_h, a.dst_w, r, x0, packed);
             }
         }

@@ -9,7 +9,7 @@ typedef void (*KernelFn)(RmxKArgs);
 // norm: 0 plain values, 1 the row's scale and bias, 2 constants from the sample's own moments (Normalize)
 KernelFn select_cmn_kernel(int dtype, int layout, int norm, int mode, const char **name);
 KernelFn select_resize_linear_kernel(int dtype, int layout, bool norm, bool quant, int chain, const char **name);
-KernelFn select_resize_fast_kernel(int dtype, int layout, bool norm, bool quant, int chain, const char **name);
+KernelFn select_resize_fast_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool aligned, const char **name);
 KernelFn select_resize_dma_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool aligned, const char **name);
 KernelFn select_resize_near_kernel(int dtype, int layout, bool norm, const char **name);
 KernelFn select_resize_nearest_kernel(int dtype, int layout, bool norm, bool quant, const char **name);

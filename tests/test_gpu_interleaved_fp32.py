@@ -1,0 +1,47 @@
+"""Bilinear resizes to interleaved fp32 of whole groups, whose rows leave as 16-byte pieces through LDS, bit for bit against the
+oracle: one lane a row, one row a wavefront, several x-tiles, mirrored and not, source rows at one phase and packed at any,
+normalised and plain, and the same op on a destination that is not 16-byte aligned."""
+import numpy as np
+import pytest
+
+from oracle import orc
+from rocal_amd import ops, workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("OW,OH", [(8, 1), (8, 70), (16, 5), (72, 3), (264, 9), (512, 4), (520, 5), (1032, 6)])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("norm", [False, True])
+def test_whole_groups(ctx, ctx_dma_small, OW, OH, packed, norm):
+    import torch
+    rng = np.random.default_rng(OW * 10 + OH)
+    n, H, W = 6, 40, 101 if packed else 100
+    img = rng.integers(0, 256, (n, H, W, 3), dtype=np.uint8)
+    roi = np.array([(0, 0, W, H), (0, 0, W, H), (3, 5, 1, 1), (W - 30, H - 20, 30, 20), (7, 1, 60, 30), (0, 0, 9, 9)], np.uint32)
+    dw, dh = np.full(n, OW, np.uint32), np.full(n, OH, np.uint32)
+    dw[4] = max(8, OW // 16 * 8)
+    mirror = np.array([0, 1, 0, 1, 1, 0], np.uint32)
+    scale, bias = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
+    kw = dict(scale=scale, bias=bias, flags=orc.F_QUANTIZE_U8) if norm else {}
+    exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.LINEAR, mirror=mirror, layout=ops.NHWC, dtype=ops.FP32, **kw)
+    src = torch.from_numpy(img).cuda()
+    for c in (ctx, ctx_dma_small):
+        op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, ops.NHWC, ops.FP32), ops.LINEAR, flags=ops.F_QUANTIZE_U8 if norm else 0)
+        if packed:
+            op.set_ragged_source(np.arange(n, dtype=np.uint64) * H * W * 3, np.full(n, W), np.full(n, H), src.numel())
+        if norm:
+            op.update_cmn(roi, dw, dh, scale, bias, mirror)
+        else:
+            op.update(roi, dw, dh, mirror)
+        assert op.kernel_name == "rmx_resize_fast_kernel" or c is ctx_dma_small, op.plan
+        for shift in (0, 1):  # (1: the destination starts 4 bytes behind an aligned address and takes the form for any)
+            whole = torch.full((n * OH * OW * 3 + 1,), 5.0, dtype=torch.float32, device="cuda")
+            out = whole[shift:shift + n * OH * OW * 3].view(n, OH, OW, 3)
+            op.launch(src, out)
+            c.sync()
+            got = out.cpu().numpy()
+            for i in range(n):
+                assert np.array_equal(got[i, :, :dw[i]].view(np.uint32), exp[i, :, :dw[i]].view(np.uint32)), (i, shift, op.plan)
+                assert (got[i, :, dw[i]:] == 5.0).all(), (i, shift)
+            assert float(whole[-1 if shift == 0 else 0]) == 5.0

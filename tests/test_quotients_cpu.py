@@ -22,7 +22,7 @@ def test_ratio_is_the_quotient(tmp_path):
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
 @pytest.mark.parametrize("src,name", [("rmx_kernels_resize_dma.hip", "rmx_resize_dma_kernel"), ("rmx_kernels_resize_fast.hip", "rmx_resize_fast_kernel"),
-                                      ("rmx_kernels_resize_near.hip", "rmx_resize_near_kernel")])
+                                      ("rmx_kernels_resize_fast.hip", "rmx_resize_runs_kernel"), ("rmx_kernels_resize_near.hip", "rmx_resize_near_kernel")])
 def test_no_division_in_front_of_the_first_load(src, name):
     """Every wavefront runs its kernel's beginning in front of its first source load: no division there."""
     found = 0
@@ -32,4 +32,4 @@ def test_no_division_in_front_of_the_first_load(src, name):
             continue
         found += 1
         assert "v_div_" not in f.split("s_endpgm")[0].split("global_load_lds")[0], m.group(1)
-    assert found >= 12
+    assert found >= 5
