@@ -128,8 +128,9 @@ struct rmx_op {
     RmxSample shared{};
     uint32_t rec[RMX_C_WORDS];
     uint64_t compact_src_bytes = 0;   // extent of the ragged source the records name
-    // A launch of this op was recorded into a HIP graph: the graph's kernel node holds the address of the table slot of the
-    // last update, which the ring would hand out again four updates later. Such an op keeps its parameters: updates are refused.
+    // A launch of this op was recorded into a HIP graph: the graph's kernel node holds the rows of the last update, or the address
+    // of their table slot, which the ring would hand out again up to eight updates later. Such an op keeps its parameters: updates
+    // are refused.
     bool captured = false;
 
     // launch plan of the last update
@@ -652,6 +653,9 @@ const char *rmx_op_plan(const rmx_op *op) {
                        (long long)op->n * op->strips, op->strips, op->strip_rows, op->tile_w, op->lds_per_wave, op->waves_per_block);
         if (op->tri_rows_in_flight) len += snprintf(buf + len, sizeof(buf) - len, " rows_in_flight=%d", op->tri_rows_in_flight);
     }
+    // (how the rows of the last update reach the kernel: dwords per sample in its arguments, or a table)
+    if (op->updated && op->compact) len += snprintf(buf + len, sizeof(buf) - len, " rows=arguments words=%u", op->compact_words);
+    else if (op->updated) len += snprintf(buf + len, sizeof(buf) - len, " rows=table");
     if (op->own_moments) len += snprintf(buf + len, sizeof(buf) - len, " moments=%dx%d", op->moment_parts, op->moment_threads);
     return buf;
 }

@@ -43,10 +43,10 @@ def _resize(c, rng_seed, n, interp, packed=False, chain=False):
     return op, img
 
 
-def _resize_crops(c, seed, n, interp, packed=False, chain=False):
+def _resize_crops(c, seed, n, interp, packed=False, chain=False, o=37):
     """Resized images of one size of which every sample writes a window of its own size, odd ones and one-pixel ones among them."""
     rng = np.random.default_rng(seed)
-    h, w, o = 40, 56, 37
+    h, w = 40, 56
     flags = (ops.F_QUANTIZE_U8 | (ops.F_COLOR_TWIST if chain else 0)) if interp == ops.LINEAR else 0
     op = ops.Resize(c, ops.desc(n, h, w, ops.NHWC, ops.UINT8), ops.desc(n, o, o, ops.NCHW, ops.FP32), interp, flags=flags)
     roi, d = _windows(rng, n, h, w, 9), np.full(n, o, np.uint32)
@@ -118,7 +118,8 @@ MAKERS = {
     "resize crops packed": (lambda c, s, n: _resize_crops(c, s, n, ops.LINEAR, packed=True), 6),
     "chain crops": (lambda c, s, n: _resize_crops(c, s, n, ops.LINEAR, chain=True), 8),
     "nearest crops": (lambda c, s, n: _resize_crops(c, s, n, ops.NEAREST), 4),
-    "triangular crops": (lambda c, s, n: _resize_crops(c, s, n, ops.TRIANGULAR), 5),
+    "triangular crops": (lambda c, s, n: _resize_crops(c, s, n, ops.TRIANGULAR), 4),  # (in batch order)
+    "triangular crops sorted": (lambda c, s, n: _resize_crops(c, s, n, ops.TRIANGULAR, o=24), 5),
     "crop": (_crop, 2),
     "flip": (_flip, 2),
     "twist": (_twist, 4),
@@ -138,6 +139,8 @@ def test_records_and_table_agree(ctx, ctx_table, what, size):
     got = []
     for c in (ctx, ctx_table):
         op, img = make(c, 17 + n, n)
+        route = "rows=table" if c is ctx_table or size == "over" else "rows=arguments" if size in ("one", "few") else "rows=arguments words=%d" % words
+        assert route in op.plan, op.plan
         out = op.alloc_output(fill=3)
         src = torch.from_numpy(img).cuda()
         op.launch(src, out)
@@ -180,6 +183,7 @@ def test_coordinates_beyond_a_record(ctx):
     d = np.array([48, 48], np.uint32), np.array([4, 4], np.uint32)
     op = ops.Resize(ctx, ops.desc(2, 4, 16600, ops.NHWC, ops.UINT8), ops.desc(2, 4, 48, ops.NHWC, ops.UINT8), ops.LINEAR)
     op.update(roi, *d)
+    assert "rows=table" in op.plan, op.plan
     out = op.alloc_output()
     op.launch(torch.from_numpy(img).cuda(), out)
     ctx.sync()
