@@ -147,7 +147,6 @@ struct rmx_op {
     rmx::KernelFn fn_mid = nullptr;
     const char *mid_name = "";
     int mid_lds = 0, mid_strips = 1, mid_rows = 4, mid_wpb = 1, mid_aux1 = 1;
-    bool fast_needs_src16 = false;                                   // fn_fast also wants a 16-byte aligned source base
     uint64_t algo_bytes = 0;
     int tri_rows_in_flight = 0;  // streaming triangular kernel: accumulator sets (2 or 4), 0 for every other kernel
     // Point operations on whole frames (every sample's window is the whole padded image, source and destination of one
@@ -718,8 +717,8 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
     a.aux0 = op->aux0;
     a.aux1 = op->aux1;
     if ((((uintptr_t)src) | ((uintptr_t)src2)) & 3u) return fail(RMX_ERR_INVALID, "the source batch must start at a 4-byte aligned address");
-    // the fast specialisation wants 16-byte aligned batch bases (rows of both sides are then aligned too)
-    const bool fast = op->fn_fast && (((uintptr_t)dst) & 15u) == 0 && (!op->fast_needs_src16 || (((uintptr_t)src) & 15u) == 0);
+    // the fast specialisation wants a 16-byte aligned destination base (its rows are then aligned too)
+    const bool fast = op->fn_fast && (((uintptr_t)dst) & 15u) == 0;
     const bool mid = !fast && op->fn_mid;
     int wpb = op->waves_per_block;
     if (fast) {
@@ -893,7 +892,6 @@ static int update_k1(rmx_op *op, const uint32_t *roi, const float *scale, const 
         op->fast_lds = 0;
         op->fast_rows = op->aux0;
         op->fast_wpb = op->waves_per_block;
-        op->fast_needs_src16 = false;
     }
     // the same pipeline for rows of any width from 8 pixels on and a destination at any element (also what an aligned plan
     // falls back to when the destination base it is launched on is not 16-byte aligned)
@@ -1470,7 +1468,6 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
     // (default 1: a workgroup's LDS is released only when its last wavefront ends, one-wave groups keep the CU full)
     op->mid_wpb = op->fast_wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, slice)));
     op->mid_aux1 = op->fast_aux1 = group;
-    op->fast_needs_src16 = false;
     if (nearest) {
         op->fn_mid = rmx::select_resize_near_kernel(op->dst.dtype, op->dst.layout, op->norm, &op->mid_name);
         return RMX_OK;
@@ -1662,7 +1659,6 @@ static int update_color(rmx_op *op, const uint32_t *roi, const float *p0, const 
         op->fast_lds = 0;
         op->fast_rows = op->aux0;
         op->fast_wpb = op->waves_per_block;
-        op->fast_needs_src16 = false;
     }
     // the same pipeline for rows of any width from 8 pixels on and a destination at any element
     bool wide8 = true;
@@ -1815,7 +1811,6 @@ static int update_point(rmx_op *op, const uint32_t *roi, const float *p0, const 
         op->fast_lds = 0;
         op->fast_rows = op->aux0;
         op->fast_wpb = op->waves_per_block;
-        op->fast_needs_src16 = false;
     }
     // the same pipeline for rows of any width from 8 pixels on and a destination at any element
     bool wide8 = true;

@@ -65,7 +65,7 @@ enum : uint32_t {
     RMX_C_CROP = 4096u,   // two dwords behind the window's: a resize whose samples write windows of their own (pc_x, pc_y, dst_w, dst_h)
     RMX_C_LAYOUT = 2048u  // two dwords, of the sample and not of the row: source offset (40 bits) and row stride (24 bits)
 };
-constexpr int RMX_C_WORDS = 768;  // 3 KB: 256 windows with their order, 192 colour twists, 128 matrices
+constexpr int RMX_C_WORDS = 768;  // 3 KB of the 4 KB that arguments may take: 384 windows, 256 with their order, 192 colour twists, 128 matrices
 constexpr int RMX_C_PAD = 4;      // (load_sample reads this many dwords from a record's start, however many it has)
 constexpr int RMX_C_TILE_WHOLE = 512;  // code k of an x-tile width: 0 the whole row (up to this many pixels), else this >> k
 

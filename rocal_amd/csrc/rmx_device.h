@@ -239,21 +239,6 @@ RMX_DEV void load_realigned(const uint8_t *p, const uint8_t *buf_end, uint32_t (
     for (int i = 0; i < ND - 1; i++) out[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], phase);
 }
 
-// Split form of load_realigned<4> for software pipelining: issue the 128-bit load now, realign
-// later (so that several loads can be in flight before the first use).
-RMX_DEV uint32_t load_raw4(const uint8_t *p, const uint8_t *buf_end, uint32_t (&d)[4]) {
-    const uint32_t phase = (uint32_t)((uintptr_t)p & 3u);
-    const uint32_t *q = reinterpret_cast<const uint32_t *>(p - phase);
-    if ((const uint8_t *)(q + 4) <= buf_end) {
-        u32x4_a4 t = *reinterpret_cast<const u32x4_a4 *>(q);
-        d[0] = t.x; d[1] = t.y; d[2] = t.z; d[3] = t.w;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) d[i] = ((const uint8_t *)(q + i) < buf_end) ? q[i] : 0u;
-    }
-    return phase;
-}
-
 // A whole frame as rows of FLAT_ROW pixels, for operations that do not know the image's own rows: every lane of a wavefront takes
 // 8 pixels whatever the image is wide (a 299-pixel row fills 38 lanes), and a wavefront's loads and stores are contiguous
 // kilobytes. Frames are contiguous in source and destination (no crop, no padding); the last row takes what is left, and where

@@ -11,8 +11,8 @@
 //            masks out of the loop.
 //   NEAREST  one source row per destination row, so only rows that are read are loaded.
 //
-// One wavefront = a strip of destination rows of one sample, one x-tile at a time, as in the staged kernel
-// (rmx_kernels_resize_fast.hip), but the source window travels from global memory straight into LDS
+// One wavefront = a strip of destination rows of one sample, one x-tile at a time. It loads the whole source window of the strip's
+// rows, with all loads in flight together, and the window travels from global memory straight into LDS
 // (global_load_lds_dwordx4: 16 bytes per lane, no vector register, no unpacking, no LDS store instruction):
 //   1. LDS holds the raw packed-RGB rows. A row is a sequence of 16-byte pieces: piece 0 is a margin for the left
 //      edge replica, pieces 1.. are the row's bytes from the dword that holds the window's first pixel. One load
@@ -24,10 +24,10 @@
 //      operation for operation (bit-identical results);
 //   3. the stores of a window's last pass wait in registers until the next window's loads have been started, so that
 //      the wait for those loads (operations of a wavefront complete in issue order) never waits for a store.
-// Against the staged kernel this trades about 25 staging instructions per 4 source pixels for 4 realignments per
-// destination pixel, frees the registers the staged loads occupy and needs a quarter less LDS (3 bytes per pixel
-// instead of 4). Measured on the RandomResizedCrop batch (256 images to 224 x 224 fp16) with every launch reading and
-// writing buffers that were not touched for a gigabyte: 32.1 us against 36.4 us; replayed on one cache-resident pair
+// Staging the window through registers instead (16-byte loads, realignment to one dword per pixel, LDS stores) costs about 25
+// instructions per 4 source pixels where this costs 4 realignments per destination pixel, the registers of the loads in flight and a
+// third more LDS (4 bytes per pixel). Measured on the RandomResizedCrop batch (256 images to 224 x 224 fp16) with every launch reading and
+// writing buffers that were not touched for a gigabyte: 32.1 us against 36.4 us staged; replayed on one cache-resident pair
 // 26.3 against 29.4 us. Tried and measured slower: two LDS windows per wavefront with the next window's loads in flight
 // during the blend (38-41 us: 12 KB of LDS per wavefront leaves 13 wavefronts per CU), all LDS reads of a pass issued
 // before its arithmetic (129 registers, 3 wavefronts per SIMD), register budgets of 96 and 80 (spills), several windows

@@ -40,8 +40,8 @@ def _ctx_with_env(**env):
 
 @pytest.fixture(scope="session")
 def ctx_staged():
-    """A context whose bilinear fast path always stages its windows through registers (the kernel that otherwise serves
-    row strides that are not a multiple of 4 and interleaved fp32 only)."""
+    """A context without the forms that need source rows at one byte phase: bilinear batches of whole groups take the form for any
+    phase, all others the general kernel; triangular ones stage their rows through registers; warps take the form for any phase."""
     c = _ctx_with_env(RMX_TUNE_DMA=0)
     yield c
     c.sync()

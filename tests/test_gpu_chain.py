@@ -72,7 +72,7 @@ def test_resize_colour_cmn_chain(ctx, ctx_staged, kind, aligned):
     mirror = rng.integers(0, 2, n).astype(np.uint32)
     scale, bias = _scale_bias(n)
     flag, arrays, colour_fn = _colour_params(kind, rng, n)
-    # aligned: the streaming kernel (planar fp16; the source rows are 360 bytes) or the staged one (interleaved fp32).
+    # aligned: the streaming kernel (planar fp16; the source rows are 360 bytes) or its form for any phase (interleaved fp32).
     # Any other width: the streaming kernel's any-width form, and the general kernel on a context without streaming.
     streaming = {True: lambda dtype: "rmx_resize_dma_kernel" if dtype == ops.FP16 else "rmx_resize_fast_kernel",
                  False: lambda dtype: "rmx_resize_dma_kernel"}[aligned]

@@ -1,5 +1,5 @@
-"""The two aligned bilinear kernels against each other and against the oracle, bit for bit: the streaming kernel (source rows
-straight into LDS) and the staged kernel (windows through registers). Covers what is specific to the streaming kernel: the
+"""The streaming bilinear kernel (source rows straight into LDS) in its two forms, for source rows at one byte phase and at any, against
+each other and against the oracle, bit for bit. (Both forms are one body: the oracle is the independent check.) Covers what is specific to the streaming kernel: the
 byte phases of packed pixels inside LDS rows, both edge replicas, rows cut into several x-tiles, strips of one to eight rows,
 the window that ends on the last byte of the batch buffer, ragged sources and every destination format it serves."""
 import numpy as np
@@ -159,7 +159,7 @@ def test_strip_heights(rows):
 
 def test_ragged_source_with_dword_row_strides(ctx):
     """Tightly packed images whose widths are multiples of 4 (row strides multiples of 4 bytes, bases at any dword): the streaming
-    kernel; one odd width sends the batch to the staged kernel. Same results."""
+    kernel for rows at one phase; one odd width sends the batch to the form for any. Same results."""
     rng = np.random.default_rng(5)
     n = 6
     widths = np.array([64, 100, 36, 128, 88, 12], np.uint32)

@@ -320,7 +320,7 @@ def test_color_twist_all_rgb_values(ctx, hue):
 
 @pytest.mark.parametrize("interp", [ops.LINEAR, ops.NEAREST])
 def test_warp_affine_config3_small(ctx, ctx_staged, interp):
-    """(both forms of the kernel: boxes straight into LDS as packed bytes, and staged through registers)"""
+    """(both forms of the kernel: source rows at one byte phase, and at any)"""
     n = 6
     c = wl.config3(n=n, size=160)
     dw = np.full(n, 160, np.uint32)
