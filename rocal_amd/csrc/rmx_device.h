@@ -29,7 +29,7 @@ RMX_DEV float round_u8(float v) {
 // The compact records of the kernel's arguments, read where the hardware put them (indexed as a member of the by-value struct,
 // they would be copied to scratch memory first).
 typedef const __attribute__((address_space(4))) uint32_t *karg_u32;
-// A wave-uniform read of memory that nothing writes while a kernel runs (rows, layout entries), through scalar loads. (Behind an asm
+// A wave-uniform read of memory that nothing writes while a kernel runs (rows), through scalar loads. (Behind an asm
 // statement the compiler takes plain loads for vector ones.)
 template <typename T>
 RMX_DEV T load_constant(const T *p) {
@@ -136,7 +136,7 @@ RMX_DEV const uint8_t *sample_base(const RmxKArgs &a, int s, uint32_t &row_strid
         return a.src + (((uint64_t)(hi >> 24) << 32) | lo);
     }
     if (a.layout) {
-        const RmxSrcLayout L = load_constant(a.layout + s);
+        const RmxSrcLayout L = a.layout[s];
         row_stride = L.row_stride;
         return a.src + L.offset;
     }
