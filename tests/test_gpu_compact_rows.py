@@ -188,3 +188,27 @@ def test_coordinates_beyond_a_record(ctx):
     op.launch(torch.from_numpy(img).cuda(), out)
     ctx.sync()
     assert np.array_equal(out.cpu().numpy(), orc.resize(img, roi, *d, 4, 48, interp=orc.LINEAR))
+
+
+@pytest.mark.parametrize("width", [16383, 16384])
+@pytest.mark.parametrize("interp", [ops.LINEAR, ops.NEAREST, ops.TRIANGULAR])
+def test_widest_resized_image_of_a_record(ctx, width, interp):
+    """Ratios are made from the sizes up to 14 bits of either; a wider resized image takes the table."""
+    import torch
+    rng = np.random.default_rng(6)
+    n, h, w, o = 3, 5, 16390, 40
+    img = rng.integers(0, 256, (n, h, w, 3), dtype=np.uint8)
+    roi = np.array([[0, 0, 16383, 5], [7, 1, 16001, 3], [5000, 0, 9000, 5]], np.uint32)
+    dw, dh = np.full(n, width, np.uint32), np.full(n, 4, np.uint32)
+    crop = np.array([[0, 0, o, 4], [16300, 1, o, 3], [8001, 0, o - 3, 4]], np.uint32)
+    scale, bias = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
+    op = ops.Resize(ctx, ops.desc(n, h, w, ops.NHWC, ops.UINT8), ops.desc(n, 4, o, ops.NCHW, ops.FP32), interp)
+    op.update_cmn(roi, dw, dh, scale, bias, crop_roi=crop)
+    assert ("rows=arguments" if width == 16383 else "rows=table") in op.plan, op.plan
+    out = op.alloc_output()
+    op.launch(torch.from_numpy(img).cuda(), out)
+    ctx.sync()
+    got = out.cpu().numpy()
+    exp = orc.resize(img, roi, dw, dh, 4, width, interp=interp, scale=scale, bias=bias, layout=ops.NCHW, dtype=ops.FP32)
+    for i, (x, y, cw, ch) in enumerate(crop.astype(int)):
+        assert np.array_equal(got[i, :, :ch, :cw].view(np.uint32), exp[i, :, y:y + ch, x:x + cw].view(np.uint32)), i
