@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256) rmx_resize_tri_kernel(RmxKArgs a) {
     wave_to_sample(a, wave, s, part);
     const int tiles_x = a.aux1;
     const int strip = part / tiles_x, tx = part - strip * tiles_x;
-    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | RMX_C_ORDER>(a, s);
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | RMX_C_ORDER, false, true>(a, s);
     s = P.plan[2];  // (the host may have put the rows in another order: the row names its sample)
 
     const int dw = P.dst_w, dh = P.dst_h;
@@ -311,7 +311,7 @@ __global__ void __launch_bounds__(256, RMX_TRI_DOWN_WAVES(NPX)) rmx_resize_tri_d
     const int tiles_x = a.aux1;
     const int strip = part / tiles_x, tx = part - strip * tiles_x;
     // the whole table row in one round trip
-    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | RMX_C_ORDER>(a, s);
+    const RmxSample P = load_sample<RMX_C_WINDOW | RMX_C_RATIO | RMX_C_ORDER, false, true>(a, s);
     asm volatile("" : : "s"(P.src_x), "s"(P.dst_w), "s"(P.pc_x), "s"(P.flags), "s"(P.rx), "s"(P.scale[0]), "s"(P.bias[2]), "s"(P.fsx));
     s = P.plan[2];  // (the host may have put the rows in another order: the row names its sample)
 
