@@ -21,7 +21,7 @@ struct __attribute__((aligned(16))) RmxSample {
     float scale[3], bias[3];             // normalisation: out = v*scale + bias
     union {
         float color[4];                  // colour twist: alpha, beta, hue shift in sextants [0,6], saturation
-        int32_t plan[4];                 // [1] x-tile width of the streaming resize kernels, [2] the row's sample (triangular)
+        int32_t plan[4];                 // [1] x-tile width of the streaming resize kernels; triangular: RMX_TRI_FOUR / RMX_TRI_EIGHT, [2] the row's sample
     };
     float m[6];                          // warp: destination -> source affine about the centres
 };
@@ -68,6 +68,9 @@ enum : uint32_t {
 constexpr int RMX_C_WORDS = 768;  // 3 KB of the 4 KB that arguments may take: 384 windows, 256 with their order, 192 colour twists, 128 matrices
 constexpr int RMX_C_PAD = 4;      // (load_sample reads this many dwords from a record's start, however many it has)
 constexpr int RMX_C_TILE_WHOLE = 512;  // code k of an x-tile width: 0 the whole row (up to this many pixels), else this >> k
+// Output rows that a source row of the sample may enter, in the streaming triangular kernel with eight accumulator sets (as x-tile
+// widths, so that a record holds them as it holds those).
+constexpr int RMX_TRI_FOUR = RMX_C_TILE_WHOLE >> 1, RMX_TRI_EIGHT = RMX_C_TILE_WHOLE >> 2;
 
 struct RmxKArgs {
     const uint8_t *src;      // batch base, u8 NHWC

@@ -154,10 +154,10 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
     const int pcx = P.pc_x, pcy = P.pc_y;
     const TriAxis ax = tri_axis(P.rx, P.fsx), ay = tri_axis(P.ry, P.fsy);
     const int kx = to_sgpr(ax.ksize), ky = to_sgpr(ay.ksize);
-    // Accumulator sets this sample uses: output row r lives in set (r - r0) & smask. A sample that shrinks vertically never has
-    // more than four rows in flight (the host has established that for every sample with a vertical ratio of 1 and more), so
-    // in the kernel with eight sets it leaves the upper four alone: half the vertical FMAs per source row.
-    const int smask = SLOTS == 8 ? to_sgpr(P.ry >= 1.0f ? 3 : 7) : SLOTS - 1;
+    // Accumulator sets this sample uses: output row r lives in set (r - r0) & smask. In the kernel with eight sets a sample for
+    // which the host has established that four suffice (every one with a vertical ratio of 1 and more, most with 1/2 and
+    // more) leaves the upper four alone: half the vertical FMAs per source row.
+    const int smask = SLOTS == 8 && P.plan[1] != RMX_TRI_FOUR ? 7 : SLOTS == 8 ? 3 : SLOTS - 1;
 
     // (a sample is smaller than 4 GiB: the host checks it, so offsets inside a sample are 32-bit)
     uint32_t row_stride_v;
