@@ -99,10 +99,34 @@ RMX_DEV void store_elem(const T *row, uint32_t voff, uint32_t bits) {
     else asm volatile("global_store_byte %0, %1, %2 offset:%3" ::"v"(voff), "v"(bits), "s"(row), "n"(OFF) : "memory");
 }
 
-// acc += h * c and acc = 0 on the accumulator's own register. (Written as plain expressions, the accumulators of the rows
+// acc += h * c on the accumulator's own register. (Written as plain expressions, the accumulators of the rows
 // in flight are renamed at every join of the row loop's paths and copied back: two dozen moves per source row.)
 RMX_DEV void fmac_inplace(float &acc, float h, float c) { asm("v_fmac_f32 %0, %1, %2" : "+v"(acc) : "v"(h), "v"(c)); }
-RMX_DEV void zero_inplace(float &acc) { asm("v_mov_b32 %0, 0" : "+v"(acc)); }
+
+// Six accumulators back to zero when idx == M, the branch inside the statement: as a branch of the program's own, every other
+// accumulator would be copied at the place where its paths meet again (24 - 36 moves per output row).
+template <int M>
+RMX_DEV void zero_if(int idx, float (&acc)[3][2]) {
+    asm("s_cmp_lg_u32 %6, %7\n\ts_cbranch_scc1 .Lkeep%=\n\tv_mov_b32 %0, 0\n\tv_mov_b32 %1, 0\n\tv_mov_b32 %2, 0\n\tv_mov_b32 %3, 0\n\tv_mov_b32 %4, 0\n\tv_mov_b32 %5, 0\n.Lkeep%=:"
+        : "+v"(acc[0][0]), "+v"(acc[0][1]), "+v"(acc[1][0]), "+v"(acc[1][1]), "+v"(acc[2][0]), "+v"(acc[2][1])
+        : "s"(idx), "n"(M)
+        : "scc");
+}
+template <int LIVE, int SLOTS, int M = 0>
+RMX_DEV void zero_set(int idx, float (&acc)[SLOTS][3][2]) {
+    if constexpr (M < LIVE) {
+        zero_if<M>(idx, acc[M]);
+        zero_set<LIVE, SLOTS, M + 1>(idx, acc);
+    }
+}
+
+// 1 / b correctly rounded, for the products of coefficient sums (b far from the ends of the exponent range): the hardware's
+// reciprocal and one correction by its remainder (Markstein, IBM J. Res. Dev. 34, 1990). Equal to the division for every
+// significand at every exponent from -40 to 40 (run through on the device): three instructions where the division is ten.
+RMX_DEV float recip(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
 
 template <typename T>
 RMX_DEV uint32_t elem_bits(float v) {
@@ -410,34 +434,34 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
         wave_sync();
     };
 
-    // An output row whose last tap row has been added: normalise, epilogue, store; its slot starts again at zero. orow walks
+    // An output row whose last tap row has been added: normalise, epilogue, store (its slot starts again at zero). orow walks
     // down the output rows (planar: the row of channel 0; the other planes lie `plane` elements on).
     T *orow = dimg + (size_t)r0 * a.dst_w * (LAYOUT == RMX_NCHW ? 1 : 3);
     const size_t plane = (size_t)a.dst_h * a.dst_w;
     const int orow_step = a.dst_w * (LAYOUT == RMX_NCHW ? 1 : 3);
     int rsum_idx = 0;
-    // 1 / (row sum x column sum) is kept from one output row to the next: rows of an integer ratio all have the same sum,
-    // and the division is a dozen instructions per column
+    // 1 / (row sum x column sum) is kept from one output row to the next: rows of an integer ratio all have the same sum
     int rsum_bits_prev = 0;  // (no row sum is +0: a zero sum is replaced by 1)
     float inv_c[TPX];
 #pragma unroll
     for (int i = 0; i < TPX; i++) inv_c[i] = 0.0f;
-    auto emit = [&](auto slot) {
-        constexpr int M = decltype(slot)::value;
+    auto row_sums = [&]() {
         const int rsum_bits = __builtin_amdgcn_readlane(__builtin_bit_cast(int, rsum_v), rsum_idx);
         if (rsum_bits != rsum_bits_prev) {
             rsum_bits_prev = rsum_bits;
             const float rsum = __builtin_bit_cast(float, rsum_bits);
 #pragma unroll
-            for (int i = 0; i < TPX; i++) inv_c[i] = 1 / (rsum * colsum[i]);
+            for (int i = 0; i < TPX; i++) inv_c[i] = recip(rsum * colsum[i]);
         }
+    };
+    auto emit = [&](auto slot) {
+        constexpr int M = decltype(slot)::value;
 #pragma unroll
         for (int i = 0; i < TPX; i++) {
             const float inv = inv_c[i];
 #pragma unroll
             for (int ch = 0; ch < 3; ch++) {
                 float t = acc[M][ch][i] * inv;
-                zero_inplace(acc[M][ch][i]);
                 if constexpr (QUANT) t = round_u8(t);
                 if constexpr (NORM) t = __builtin_fmaf(t, sc[ch], bi[ch]);
                 // wave-uniform row pointer + the lane's column offset
@@ -542,6 +566,7 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
         }
         // ---- rows whose last tap was this source row
         while (qlast <= yy) {
+            row_sums();
             if constexpr (TS_SLOTS == 2) {
                 if (rsum_idx & 1) emit(std::integral_constant<int, 1>{});
                 else emit(std::integral_constant<int, 0>{});
@@ -564,6 +589,7 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
                     default: emit(std::integral_constant<int, 3>{}); break;
                 }
             }
+            zero_set<LIVE>(rsum_idx & (LIVE - 1), acc);
             rq++;
             rsum_idx++;
             orow += orow_step;
