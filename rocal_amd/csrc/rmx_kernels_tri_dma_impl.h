@@ -64,6 +64,12 @@ constexpr int TS_NCH = 2;    // load instructions per row at most (64 pieces of 
 constexpr int TS_TAB = 64;   // source rows of the table of vertical coefficients
 constexpr int TS_EDGE = 16;  // passes of an edge row at most (= vertical taps the host admits)
 
+template <int COLS, int DWORDS, typename CV>
+struct RowDwords {
+    uint32_t w[COLS][DWORDS];
+    CV cv;
+};
+
 template <int B>
 RMX_DEV float ubyte_at(uint32_t v) {
     if constexpr (B == 0) return ubyte0(v);
@@ -473,11 +479,25 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
         }
     };
 
+    // A source row's part of a lane: the dwords that hold the taps of its two columns, and the row's vertical coefficients.
+    auto fetch_row = [&](auto nt, auto pair, const lds_u8 *srow) {
+        constexpr int NT = decltype(nt)::value, PR = decltype(pair)::value;
+        RowDwords<(PR > 0 ? 1 : TPX), (3 * (NT + PR) + 3) / 4 + 1, slotv> f;
+        f.cv = slots_read<SLOTS>(cv_next++);
+#pragma unroll
+        for (int i = 0; i < (PR > 0 ? 1 : TPX); i++) {
+            const lds_u32 *p0 = (const lds_u32 *)(srow + tap_w[i]);
+#pragma unroll
+            for (int j = 0; j < (3 * (NT + PR) + 3) / 4 + 1; j++) f.w[i][j] = p0[j];
+        }
+        return f;
+    };
+
     // The row in ring slot `slot` is source row yy: filter it and add it to the output rows in flight. NT = taps of the
     // unrolled horizontal pass (4, 5, 6 or 8 >= the taps that are run): taps beyond those carry coefficient 0 (fma(p, 0, a) == a
     // for the finite p an unpacked byte always is), so no bound test is needed inside. A column's 3 NT bytes start at byte
     // tap_ph of dword tap_w: NE + 1 dwords are read and realigned into NE.
-    auto process_row = [&](auto nt, auto lower_only, auto pair, const lds_u8 *srow, int yy) {
+    auto process_row = [&](auto nt, auto lower_only, auto pair, const auto &f, int yy) {
         constexpr int NT = decltype(nt)::value;
         constexpr int PR = decltype(pair)::value;  // the lane's two columns are neighbours whose first taps lie PR pixels apart; 0: not
         // LIVE: the accumulator sets this instance of the row loop adds to and stores from (the lower four of eight for a sample
@@ -488,7 +508,8 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
         // A row inside the window is one tap of every output row that reads it: one pass, coefficients from the table. The
         // first / last row of the window is also read by every tap index that leaves the window: one pass per such tap, in
         // tap order, coefficients computed here by lane p for pass p (rare: twice per image column of strips at most).
-        const lds_slotv *cvp = cv_next++;
+        const lds_slotv *cvp = nullptr;
+        slotv cv4 = f.cv;
         int npass = 1;
         if ((uint32_t)(yy - ylo - 1) >= (uint32_t)(yhi - ylo - 1)) {  // yy == ylo or yy == yhi (rows lie inside the window)
             float ec[TS_SLOTS];
@@ -514,38 +535,26 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
             if (lane < TS_EDGE) slots_write<SLOTS>((lds_slotv *)(etab + TS_SLOTS * lane), ecv);
             wave_sync();
             cvp = (const lds_slotv *)etab;
-            npass = max(npass, 1);
+            cv4 = slots_read<SLOTS>(cvp);
         }
-        slotv cv4 = slots_read<SLOTS>(cvp);
         float h[3][TPX];
         if constexpr (PR > 0) {
             // one read of the union of both columns' taps: NT + PR pixels from the first column's first tap
             constexpr int NEP = (3 * (NT + PR) + 3) / 4;
-            uint32_t w[NEP + 1];
-            const lds_u32 *p0 = (const lds_u32 *)(srow + tap_w[0]);
-#pragma unroll
-            for (int j = 0; j <= NEP; j++) w[j] = p0[j];
             uint32_t e[NEP];
 #pragma unroll
-            for (int j = 0; j < NEP; j++) e[j] = __builtin_amdgcn_alignbyte(w[j + 1], w[j], tap_ph[0]);
+            for (int j = 0; j < NEP; j++) e[j] = __builtin_amdgcn_alignbyte(f.w[0][j + 1], f.w[0][j], tap_ph[0]);
             float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
             tri_taps<NT, NEP, 0>(e, creg[0], a0, a1, a2);
             tri_taps<NT, NEP, PR>(e, creg[1], b0, b1, b2);
             h[0][0] = a0; h[1][0] = a1; h[2][0] = a2;
             h[0][1] = b0; h[1][1] = b1; h[2][1] = b2;
         } else {
-            uint32_t w[TPX][NE + 1];
-#pragma unroll
-            for (int i = 0; i < TPX; i++) {
-                const lds_u32 *p0 = (const lds_u32 *)(srow + tap_w[i]);
-#pragma unroll
-                for (int j = 0; j <= NE; j++) w[i][j] = p0[j];
-            }
 #pragma unroll
             for (int i = 0; i < TPX; i++) {
                 uint32_t e[NE];
 #pragma unroll
-                for (int j = 0; j < NE; j++) e[j] = __builtin_amdgcn_alignbyte(w[i][j + 1], w[i][j], tap_ph[i]);
+                for (int j = 0; j < NE; j++) e[j] = __builtin_amdgcn_alignbyte(f.w[i][j + 1], f.w[i][j], tap_ph[i]);
                 float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
                 tri_taps<NT, NE>(e, creg[i], a0, a1, a2);
                 h[0][i] = a0;
@@ -554,15 +563,18 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
             }
         }
         // ---- vertical pass: every pass adds the filtered row to all four slots with that pass's coefficients (0: none)
-        for (int p = 0;;) {
+        auto add_row = [&]() {
 #pragma unroll
             for (int m = 0; m < LIVE; m++)
 #pragma unroll
                 for (int ch = 0; ch < 3; ch++)
 #pragma unroll
                     for (int i = 0; i < TPX; i++) fmac_inplace(acc[m][ch][i], h[ch][i], cv4[m]);
-            if (++p >= npass) break;
+        };
+        add_row();
+        for (int p = 1; p < npass; p++) {
             cv4 = slots_read<SLOTS>(cvp + p);
+            add_row();
         }
         // ---- rows whose last tap was this source row
         while (qlast <= yy) {
@@ -623,7 +635,18 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
             emitted = 0;
             by_lanes = (y + TS_RPS <= y_last) ? issue(half_nxt) : false;
             replicate(half_cur, nr);
-            for (int q = 0; q < nr; q++) process_row(nt, lower_only, pair, half_cur + q * pitch, y + q);
+            // Both rows' reads are started before the first row is filtered (the second row's slot holds a row also where the
+            // window ends with the first one) by the wavefronts that use four sets of eight: the others have no registers left for it.
+            constexpr bool AHEAD = decltype(lower_only)::value;
+            auto row = fetch_row(nt, pair, half_cur);
+            auto second = row;
+            if constexpr (AHEAD) second = fetch_row(nt, pair, half_cur + pitch);
+            for (int q = 0;;) {
+                process_row(nt, lower_only, pair, row, y + q);
+                if (++q >= nr) break;
+                if constexpr (!AHEAD) second = fetch_row(nt, pair, half_cur + pitch);
+                row = second;
+            }
             wave_sync();  // the slots are reused two steps on
             lds_u8 *t = half_cur;
             half_cur = half_nxt;
