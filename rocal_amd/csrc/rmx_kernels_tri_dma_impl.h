@@ -338,30 +338,43 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
     }
     const int pair_lane = min(lane, (tw >> 1) - 1);
     uint32_t xoff[TPX], tap_w[TPX], tap_ph[TPX];
-    float colsum[TPX], creg[TPX][8];
+    float colsum[TPX] = {}, creg[TPX][8] = {};
     int locx[TPX];
     float w0x[TPX];
-    bool lead = false;  // some column's first tap has a coefficient other than 0
 #pragma unroll
     for (int i = 0; i < TPX; i++) {
         const int col = pair_r ? xt + 2 * pair_lane + i : xt + lane + RMX_WAVE * i;
         const int colc = min(col, dw - 1);
         xoff[i] = (uint32_t)(hf ? (dw - 1 - colc) : colc) * (uint32_t)(LAYOUT == RMX_NCHW ? sizeof(T) : 3 * sizeof(T));
         tri_loc(ax, pcx + colc, (float)xlo, locx[i], w0x[i]);
-        float sum = 0.0f;
-        for (int k = 0; k < kx; k++) sum += tri_coeff(w0x[i], ax.radius, k, ax.fscale);
-        colsum[i] = (sum == 0.0f) ? 1.0f : sum;
-        lead = lead || !(tri_coeff(w0x[i], ax.radius, 0, ax.fscale) == 0.0f);
     }
+    // (the host admits at most eight taps; a wavefront-wide branch per tap, so that only those there are cost anything)
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        if (k < kx) {
+#pragma unroll
+            for (int i = 0; i < TPX; i++) {
+                creg[i][k] = tri_coeff(w0x[i], ax.radius, k, ax.fscale);
+                colsum[i] += creg[i][k];
+            }
+        }
+    }
+    const bool lead = !(creg[0][0] == 0.0f) || !(creg[1][0] == 0.0f);  // some column's first tap has a coefficient other than 0
+#pragma unroll
+    for (int i = 0; i < TPX; i++) colsum[i] = (colsum[i] == 0.0f) ? 1.0f : colsum[i];
     // When the first tap of every column of the tile has coefficient 0 (ratios 1 and 3, the odd whole numbers: the first tap then
     // lies a whole radius from the centre), the horizontal pass starts one pixel on with one tap less: fma(p, 0, 0) is the 0
     // the accumulation starts from anyway. Wave-uniform.
     const int skip = (kx > 1 && __builtin_amdgcn_ballot_w64(lead) == 0) ? 1 : 0;
     const int kx_run = kx - skip;
+    if (skip) {
+#pragma unroll
+        for (int i = 0; i < TPX; i++)
+#pragma unroll
+            for (int k = 0; k < 8; k++) creg[i][k] = k < 7 ? creg[i][k + 1] : 0.0f;
+    }
 #pragma unroll
     for (int i = 0; i < TPX; i++) {
-#pragma unroll
-        for (int k = 0; k < 8; k++) creg[i][k] = (k < kx_run) ? tri_coeff(w0x[i], ax.radius, k + skip, ax.fscale) : 0.0f;
         // the first tap's byte inside an LDS row (a tap left of the window reads a replica in or behind the margin)
         const uint32_t tb = (uint32_t)(lm + ph + 3 * (locx[i] + skip - cs));
         tap_w[i] = tb & ~3u;
@@ -399,44 +412,35 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
     // ---- output rows in flight: row r accumulates in slot (r - r0) & 3 until its last tap row has been added. rq is the
     // oldest row in flight, qlast its last tap row (wave-uniform state).
     float acc[TS_SLOTS][3][TPX];
-#pragma unroll
-    for (int m = 0; m < TS_SLOTS; m++)
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-            for (int i = 0; i < TPX; i++) acc[m][c][i] = 0.0f;
     int rq = r0;
     int qlast = last_tap_row(r0);
     int emitted = 0;  // output rows stored since the loads of the rows in work were started
 
-    // ---- vertical coefficients by source row, a table of 64 rows x 4 slots in the tail of the LDS slice: entry (l, k) is
-    // the coefficient with which source row ytab + l enters the output row of slot k (0: none; fma(h, 0, acc) == acc for
-    // the finite h a filtered row is, so all four slots take every row and no branch is needed). Lane l writes row l; the
-    // filter loop reads a row's entry with one broadcast read. Rebuilt every 64 source rows. The first and the last row
-    // of the window serve several taps of a row each (clamped tap indices) and take their own path below.
+    // ---- vertical coefficients by source row, a table of 64 rows x the sets in the tail of the LDS slice: entry (l, k) is
+    // the coefficient with which source row ytab + l enters the output row of set k (0: none; fma(h, 0, acc) == acc for
+    // the finite h a filtered row is, so all sets take every row and no branch is needed). Lane r writes the taps of output row
+    // r0 + r, which no other row of its set shares a source row with; the filter loop reads a source row's entry with one
+    // broadcast read. Rebuilt every 64 source rows. The first and the last row of the window serve several taps of a row
+    // each (clamped tap indices) and take their own path below.
+    // (Written by source rows instead, lane l going through all the strip's output rows for row l's coefficients, the table
+    // and the coefficients of the columns, made twice, were a third of the instructions in front of the row loop: 256 RandomResizedCrop windows to
+    // 224 x 224 fp16 47.8 -> 45.3 us.)
     lds_f32 *cftab = (lds_f32 *)(bufb + tab_off);
     const lds_slotv *cv_next = (const lds_slotv *)cftab;  // the table entry of the next source row
     int ytab = y_first;
     auto build_table = [&]() {
-        const int y = ytab + lane;
-        float cf[TS_SLOTS];
-#pragma unroll
-        for (int k = 0; k < TS_SLOTS; k++) cf[k] = 0.0f;
-        for (int rb = r0; rb < r1; rb += smask + 1) {
-#pragma unroll
-            for (int k = 0; k < TS_SLOTS; k++) {
-                const int r = rb + k;
-                if (k <= smask && r < r1) {
-                    const int j = y - row_loc(r);
-                    const float c = tri_coeff(row_w0(r), ay.radius, j, ay.fscale);
-                    if ((uint32_t)j < (uint32_t)ky) cf[k] = c;
-                }
-            }
+        slots_write<SLOTS>((lds_slotv *)(cftab + TS_SLOTS * lane), slotv{});
+        wave_sync();
+        int loc = oloc_v, row = lane;
+        float w0 = ow0_v;
+        asm volatile("" : "+v"(loc), "+v"(w0), "+v"(row));  // (or the taps' coefficients and places would be kept in registers from one table to the next)
+        const int l0 = loc - ytab;
+        lds_f32 *mine = cftab + TS_SLOTS * l0 + (row & smask);
+#pragma unroll 1
+        for (int j = 0; j < ky; j++) {
+            const float c = tri_coeff(w0, ay.radius, j, ay.fscale);
+            if (row < r1 - r0 && (uint32_t)(l0 + j) < (uint32_t)TS_TAB) mine[TS_SLOTS * j] = c;
         }
-        slotv cfv;
-#pragma unroll
-        for (int k = 0; k < TS_SLOTS; k++) cfv[k] = cf[k];
-        slots_write<SLOTS>((lds_slotv *)(cftab + TS_SLOTS * lane), cfv);
         wave_sync();
     };
 
@@ -619,6 +623,12 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
     auto run = [&](auto nt, auto lower_only, auto pair) {
         lds_u8 *half_cur = bufb, *half_nxt = bufb + TS_RPS * pitch;
         bool by_lanes = first_by_lanes;
+#pragma unroll
+        for (int m = 0; m < (TS_SLOTS == 8 && decltype(lower_only)::value ? 4 : TS_SLOTS); m++)
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+#pragma unroll
+                for (int i = 0; i < TPX; i++) acc[m][c][i] = 0.0f;
         build_table();  // (under the round trip of the first loads)
         for (int y = y_first; y <= y_last; y += TS_RPS) {
             const int nr = min(TS_RPS, y_last - y + 1);

@@ -30,7 +30,7 @@ RMX_DEV void tri_loc(const TriAxis &t, int d, float lo, int &loc, float &w0) {
 
 RMX_DEV float tri_coeff(float w0, float radius, int k, float fscale) {
     float c = 1 - fabsf((w0 - radius + (float)k) * fscale);
-    return c < 0 ? 0 : c;
+    return __builtin_fmaxf(c, 0.0f);  // (c < 0 ? 0 : c, for a c that is a number: ratios are finite)
 }
 
 }  // namespace rmx
