@@ -230,26 +230,18 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
                 }
             }
         } else {
-            // the window touches the last bytes of the batch buffer: bounds-checked byte loads, stored by the lanes
+            // the window touches the last bytes of the batch buffer: the pieces that leave it are stored by their lanes
             const int tp = nrows * g.ppr;
-            for (int idx = lane; idx < tp; idx += RMX_WAVE) {
+            for (int j0 = 0; j0 < tp; j0 += RMX_WAVE) {
+                const int idx = j0 + lane;
                 const int r = idx / g.ppr;
-                const int c = idx - r * g.ppr;
-                const int piece = max(min(c - 1, g.nd - 1), 0);
-                const uint32_t off = row_off(g, row_of(a_v + r)) + 16u * (uint32_t)piece;
-                uint32_t w[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    uint32_t v = 0;
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        const uint32_t ob = off + 4u * i + b;
-                        v |= (ob < lim ? (uint32_t)base4[ob] : 0u) << (8 * b);
-                    }
-                    w[i] = v;
+                const uint32_t off = row_off(g, row_of(a_v + r)) + 16u * (uint32_t)max(min(idx - r * g.ppr - 1, g.nd - 1), 0);
+                if (idx < tp && (uint64_t)off + 16 <= lim) {
+                    __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(bufb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
+                } else if (idx < tp) {
+                    const uint4 v = load_piece_bounded<uint32_t>(base4, off, lim);
+                    *(lds_u32x4 *)(bufb + 16 * idx) = (u32x4_a4){v.x, v.y, v.z, v.w};
                 }
-                lds_u32 *dst4 = (lds_u32 *)(bufb + 16 * idx);
-                dst4[0] = w[0]; dst4[1] = w[1]; dst4[2] = w[2]; dst4[3] = w[3];
             }
         }
         return a_v;

@@ -288,18 +288,8 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
             } else {
                 by_lanes = true;
                 for (int c = lane; c < ppr; c += RMX_WAVE) {
-                    const uint32_t off = roff + 16u * (uint32_t)max(min(c - (lm >> 4), nd - 1), 0);
-                    lds_u32 *dst4 = (lds_u32 *)(slot + 16 * c);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        uint32_t v = 0;
-#pragma unroll
-                        for (int b = 0; b < 4; b++) {
-                            const uint32_t ob = off + 4u * i + b;
-                            v |= (ob < lim ? (uint32_t)base4[ob] : 0u) << (8 * b);
-                        }
-                        dst4[i] = v;
-                    }
+                    const uint4 v = load_piece_bounded<uint32_t>(base4, roff + 16u * (uint32_t)max(min(c - (lm >> 4), nd - 1), 0), lim);
+                    *(lds_u32x4 *)(slot + 16 * c) = (u32x4_a4){v.x, v.y, v.z, v.w};
                 }
             }
             if (y_next < y_last) {

@@ -227,24 +227,19 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             // the compiler does not order LDS reads behind loads into LDS: await them explicitly
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         } else {
-            // the box touches the last bytes of the batch buffer: bounds-checked byte loads, stored by the lanes
-            const uint64_t left = (uint64_t)(buf_end - base4);
-            const uint32_t lim = left > 0xffffffffull ? 0xffffffffu : (uint32_t)left;
-            for (int idx = lane; idx < total; idx += RMX_WAVE) {
+            // the box touches the last bytes of the batch buffer: the pieces that leave it are stored by their lanes
+            const uint64_t lim = (uint64_t)(buf_end - base4);
+            for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
+                const int idx = j0 + lane;
                 const int r = idx / ppr, c = idx - r * ppr;
-                const uint32_t off = (uint32_t)min(by0 + r, yhi) * row_stride + col4 + 16u * (uint32_t)c;
-                lds_u32 *dst4 = (lds_u32 *)(ldsb + 16 * idx);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    uint32_t v = 0;
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        const uint32_t ob = off + 4u * i + b;
-                        v |= (ob < lim ? (uint32_t)base4[ob] : 0u) << (8 * b);
-                    }
-                    dst4[i] = v;
+                const uint64_t off = (uint64_t)((uint32_t)min(by0 + r, yhi) * row_stride + col4 + 16u * (uint32_t)c);
+                if (idx < total && off + 16 <= lim) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
+                else if (idx < total) {
+                    const uint4 v = load_piece_bounded<int64_t>(base4, (int64_t)off, (int64_t)lim);
+                    *(lds_u32x4 *)(ldsb + 16 * idx) = (u32x4_a4){v.x, v.y, v.z, v.w};
                 }
             }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         wave_sync();
         // the column behind the box repeats its last column where that is the ROI's last column (only then is it read)
@@ -280,21 +275,16 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             // the compiler does not order LDS reads behind loads into LDS: await them explicitly
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         } else {
-            for (int idx = lane; idx < total; idx += RMX_WAVE) {
-                const int r = row_of(idx);
+            for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
+                const int idx = j0 + lane, r = row_of(idx);
                 const int64_t off = (int64_t)(uint32_t)(by0 + r) * row_stride + colb - ph + (16 * idx - r * pitch_b);
-                lds_u32 *dst4 = (lds_u32 *)(ldsb + 16 * idx);
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    uint32_t v = 0;
-#pragma unroll
-                    for (int b = 0; b < 4; b++) {
-                        const int64_t ob = off + 4 * i + b;
-                        v |= (ob >= 0 && (uint64_t)ob < left ? (uint32_t)base4[ob] : 0u) << (8 * b);
-                    }
-                    dst4[i] = v;
+                if (idx < total && off >= 0 && off + 16 <= (int64_t)left) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
+                else if (idx < total) {
+                    const uint4 v = load_piece_bounded<int64_t>(base4, off, (int64_t)left);
+                    *(lds_u32x4 *)(ldsb + 16 * idx) = (u32x4_a4){v.x, v.y, v.z, v.w};
                 }
             }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         wave_sync();
         // the column behind the box repeats its last column where that is the ROI's last column, and the row below the box its
