@@ -69,7 +69,13 @@ RMX_DEV void twist_px(float &r, float &g, float &b, const float *rcp, const Sect
     s = s * satf;
     s = __builtin_fminf(__builtin_fmaxf(s, 0.0f), 1.0f);
     // sector and fraction; hh lies in [0, 6], where hh - floor(hh) is exact and equals hh - trunc(hh)
-    const SectorRow row = sect[(int)hh];
+    // (a row as a 16- and an 8-byte vector: read as a structure, its first access waited for all of a resize kernel's memory operations)
+    typedef float row_lo __attribute__((ext_vector_type(4)));
+    typedef float row_hi __attribute__((ext_vector_type(2)));
+    const lds_u8 *at = (const lds_u8 *)sect + sizeof(SectorRow) * (uint32_t)(int)hh;
+    const row_lo lo = *(const __attribute__((address_space(3))) row_lo *)at;
+    const row_hi hi = *(const __attribute__((address_space(3))) row_hi *)(at + 16);
+    const SectorRow row = {{lo.x, lo.y, lo.z}, lo.w, hi.x, hi.y, 0.0f, 0.0f};
     const float hf = __builtin_amdgcn_fractf(hh);
     const float vsat = cmax * s;
     const float vsatf = vsat * hf;
@@ -96,15 +102,15 @@ constexpr ColorTables make_color_tables() {
 }
 static __device__ const ColorTables rmx_color_tables_rom = make_color_tables();
 
-// Copies the tables into LDS from one wavefront: 80 pieces of 16 bytes, one per lane and 16 more. Every wavefront of a
-// workgroup writes the same values, so none has to wait for another: each reads only what it has written itself.
-RMX_DEV void color_tables_fill(ColorTables *t, int lane) {
+// Starts the copy of the tables into LDS, straight from memory, by one wavefront: 80 pieces of 16 bytes, one per lane and 16 more.
+// They have arrived when the wavefront has waited for its vector memory operations. Every wavefront of a workgroup writes the
+// same values, so none has to wait for another: each reads only what it has written itself.
+RMX_DEV void color_tables_fetch(ColorTables *t, int lane) {
     static_assert(sizeof(ColorTables) == 80 * 16, "layout of the colour tables");
-    const uint4 *src = reinterpret_cast<const uint4 *>(&rmx_color_tables_rom);
-    uint4 *dst = reinterpret_cast<uint4 *>(t);
-    dst[lane] = src[lane];
-    if (lane < 16) dst[RMX_WAVE + lane] = src[RMX_WAVE + lane];
-    wave_sync();
+    const uint8_t *src = reinterpret_cast<const uint8_t *>(&rmx_color_tables_rom) + 16 * lane;
+    lds_u8 *dst = (lds_u8 *)t;
+    __builtin_amdgcn_global_load_lds((glb_ptr_t)src, (lds_ptr_t)dst, 16, 0, 0);
+    if (lane < 16) __builtin_amdgcn_global_load_lds((glb_ptr_t)(src + 16 * RMX_WAVE), (lds_ptr_t)(dst + 16 * RMX_WAVE), 16, 0, 0);
 }
 
 // Colour node in the middle of a fused chain resize(u8) -> colour(u8) -> CropMirrorNormalize: the values come in as the rounded

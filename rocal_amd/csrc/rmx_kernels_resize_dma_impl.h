@@ -133,7 +133,7 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     const float cp[4] = {P.m[0], P.m[1], P.m[2], P.m[3]};
     const float sh2 = cp[2] + 2.0f, sh4 = cp[2] + 4.0f;
     const ColorTables *ctab = reinterpret_cast<const ColorTables *>(chain_tables);
-    if constexpr (CHAIN == CHAIN_TWIST) color_tables_fill(reinterpret_cast<ColorTables *>(chain_tables), lane);
+    if constexpr (CHAIN == CHAIN_TWIST) color_tables_fetch(reinterpret_cast<ColorTables *>(chain_tables), lane);  // (awaited with the first window)
     uint32_t *slab = nullptr;
     if constexpr (COALESCE) slab = rmx_lds_dma + (slice_off >> 2) + (a.lds_bytes >> 2) - RMX_WAVE * coalesce_slab_dwords<T, LAYOUT>();
 

@@ -145,7 +145,11 @@ __global__ void __launch_bounds__(256) rmx_resize_kernel(RmxKArgs a) {
     const float cp[4] = {P.m[0], P.m[1], P.m[2], P.m[3]};
     const float sh2 = cp[2] + 2.0f, sh4 = cp[2] + 4.0f;
     const ColorTables *ctab = reinterpret_cast<const ColorTables *>(chain_tables);
-    if constexpr (CHAIN == CHAIN_TWIST) color_tables_fill(reinterpret_cast<ColorTables *>(chain_tables), lane);
+    if constexpr (CHAIN == CHAIN_TWIST) {
+        color_tables_fetch(reinterpret_cast<ColorTables *>(chain_tables), lane);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        wave_sync();
+    }
 
     StageCtx S;
     {
