@@ -50,7 +50,6 @@
 #endif
 
 namespace rmx {
-
 extern __shared__ uint32_t rmx_lds_dma[];
 
 // (measurement builds: every word of a group that is not stored still has to be computed)
@@ -87,9 +86,13 @@ template <typename T, int LAYOUT, bool NORM, bool QUANT, int CHAIN, bool ALIGNED
 RMX_DEV void resize_stream(const RmxKArgs &a) {
     static_assert(CHAIN == CHAIN_NONE || QUANT, "a colour node in the chain reads the u8 output of the resize node");
     static_assert(CHAIN == CHAIN_NONE || !NEAREST, "a colour node in the chain follows a bilinear resize node");
-    // Interleaved fp32 (96 bytes per lane): the lanes of a row exchange their runs through LDS before storing (57.1 -> 48.4 us on
-    // the RandomResizedCrop batch); the slab is the tail of the wavefront's slice, the host adds its size.
-    constexpr bool COALESCE = sizeof(T) == 4 && LAYOUT == RMX_NHWC;
+    // fp32 runs are longer than one store: the lanes of a row exchange them through LDS before storing, so that every store
+    // instruction writes whole pieces one behind the other, as streaming stores. (The slab is the tail of the wavefront's slice,
+    // the host adds its size.) Interleaved rows always; planes of whole groups (128 RandomResizedCrops to 224 x 224 33.5 -> 24.3
+    // us, 144 x 144 9.4 -> 8.3), and under a colour chain those of other widths that are multiples of 4 (64 images to
+    // 300 x 300 36.8 -> 33.8). Without the chain planes of such widths gain nothing (300 wide 33.2 -> 34.1, 708 wide 47.0 -> 47.8).
+    constexpr bool QUADS = !ALIGNED && LAYOUT == RMX_NCHW && CHAIN == CHAIN_TWIST;
+    constexpr bool COALESCE = sizeof(T) == 4 && (LAYOUT == RMX_NHWC || ALIGNED || QUADS);
     constexpr bool AHEAD = CHAIN != CHAIN_TWIST;  // (see load_sample)
     __shared__ __attribute__((aligned(16))) float chain_tables[CHAIN == CHAIN_TWIST ? sizeof(ColorTables) / 4 : 4];
     const int lane = threadIdx.x & (RMX_WAVE - 1);
@@ -135,6 +138,8 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     const ColorTables *ctab = reinterpret_cast<const ColorTables *>(chain_tables);
     if constexpr (CHAIN == CHAIN_TWIST) color_tables_fetch(reinterpret_cast<ColorTables *>(chain_tables), lane);  // (awaited with the first window)
     uint32_t *slab = nullptr;
+    // (planes whose rows all start and end at 16-byte pieces; the host has made room for the slab whenever the padded width allows it)
+    const bool quads = QUADS && ((dw | a.dst_w) & 3) == 0 && ((uintptr_t)a.dst & 15u) == 0;
     if constexpr (COALESCE) slab = rmx_lds_dma + (slice_off >> 2) + (a.lds_bytes >> 2) - RMX_WAVE * coalesce_slab_dwords<T, LAYOUT>();
 
     uint32_t row_stride_v;
@@ -403,8 +408,12 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
                 else if constexpr (COALESCE) {
                     // (a row's lanes hold its runs left to right, or right to left under a mirror: a run goes to its own place in the slab)
                     const int L = (g.tw + PX - 1) / PX, l = lane - lr * L, xs = hf ? dw - g.xt - g.tw : g.xt;
-                    if constexpr (ALIGNED) store_packed_coalesced<T, LAYOUT, RMX_DMA_NT>(slab, lane - l, hf ? L - 1 - l : l, L, dimg, a.dst_h, a.dst_w, r, x0, packed);
-                    else store_packed_coalesced_any<T, LAYOUT, RMX_DMA_NT>(slab, lane - l, l, L, xs, g.tw, dimg, a.dst_h, a.dst_w, r, x0, packed);
+                    if constexpr (ALIGNED) store_packed_coalesced<T, LAYOUT, true>(slab, lane - l, hf ? L - 1 - l : l, L, dimg, a.dst_h, a.dst_w, r, x0, packed);
+                    else if constexpr (QUADS) {
+                        if (quads) store_packed_quads<T, true>(slab, lane - l, l, L, xs, g.tw, dimg, a.dst_h, a.dst_w, r, x0, packed);
+                        else store_packed<T, LAYOUT, RMX_DMA_NT, true>(dimg, a.dst_h, a.dst_w, r, x0, packed);
+                    }
+                    else store_packed_coalesced_any<T, LAYOUT, true>(slab, lane - l, l, L, xs, g.tw, dimg, a.dst_h, a.dst_w, r, x0, packed);
                 } else store_packed<T, LAYOUT, RMX_DMA_NT, !ALIGNED>(dimg, a.dst_h, a.dst_w, r, x0, packed);
             }
         }
