@@ -1911,18 +1911,18 @@ static int update_warp(rmx_op *op, const uint32_t *roi, const float *affine, con
         bytes += (uint64_t)s.src_w * s.src_h * 3 + (uint64_t)s.dst_w * s.dst_h * 3 * dtype_size(op->dst.dtype);
         max_dw = std::max(max_dw, (int)s.dst_w);
         max_dh = std::max(max_dh, (int)s.dst_h);
-        // LDS need of a destination tile (32 x 16*passes): bounding box of its image under M, margins, and the
-        // repeated column and row
-        const double th = 16.0 * op->ctx->warp_passes;
-        double bw = 32.0 * std::fabs(s.m[0]) + th * std::fabs(s.m[1]) + 6.0;
-        double bh = 32.0 * std::fabs(s.m[3]) + th * std::fabs(s.m[4]) + 6.0;
+        // LDS need of a destination tile (32 x 16*passes): bounding box of its pixels' images under M (an extent e touches at most
+        // ceil(e) + 1 pixels; 1/32 for the coordinates' rounding) with the right and lower neighbours
+        const double last = 16.0 * op->ctx->warp_passes - 1.0;
+        double bw = std::ceil(31.0 * std::fabs(s.m[0]) + last * std::fabs(s.m[1]) + 0.03125) + 2.0;
+        double bh = std::ceil(31.0 * std::fabs(s.m[3]) + last * std::fabs(s.m[4]) + 0.03125) + 2.0;
         if (std::isfinite(bw) && std::isfinite(bh)) {
             bw = std::min(bw, (double)s.src_w + 1);
             bh = std::min(bh, (double)s.src_h + 1);
             // (packed bytes: rows of whole 16-byte pieces from the dword that holds the box's first pixel, at least kWarpRawPieces
             // of them; the form for any phase leaves 16 bytes between rows and up to 3 for the stride's remainder)
-            const double pieces = std::max<double>(std::ceil(((raw ? 3.0 : 22.0) + 3.0 * (bw + 1.0)) / 16.0), rmx::kWarpRawPieces);
-            worst_box = std::max(worst_box, (pieces * 16.0 + (raw ? 0.0 : 3.0)) * bh);
+            const double pitch = raw ? std::ceil((3.0 + 3.0 * (bw + 1.0)) / 16.0) * 16.0 : std::ceil((3.0 * bw + 16.0) / 4.0) * 4.0;
+            worst_box = std::max(worst_box, (std::max(pitch, 16.0 * rmx::kWarpRawPieces) + (raw ? 0.0 : 3.0)) * bh);
         }
     }
     op->algo_bytes = bytes;

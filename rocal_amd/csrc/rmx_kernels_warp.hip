@@ -22,7 +22,13 @@
 //          is masked by itself (two instructions per pixel). Against staging through registers with one dword per pixel (111 registers,
 //          13 KB): 64 rotations of 299 x 299, bytes, with the wide stores below, 18.4 -> 15.1 us per batch. Rows at one phase keep RAW:
 //          its loop has the masks' two instructions less, of 58.
-// Bound by the vector pipe: 128 images of 512 x 512 take 63 us, of which the bytes are 36 at the rate of a large copy.
+// Bound by how many wavefronts are there to compute while others wait for their box: 128 images of 512 x 512 take 61 - 63 us; without the
+// box's loads 47, without the stores 52, without both 42, with taps that meet no bank conflict the same; the bytes are 36 at the rate of
+// a large copy. The LDS slice therefore holds the box and nothing besides: no pixel of margin (the corners bound it exactly), the
+// repeated row only where it is read, rows of 10 pieces where they fit instead of 11 (a batch turned by up to 30 degrees and scaled by a
+// tenth: 9.4 -> 7.9 KB a wavefront, 20 of them per CU instead of 16; 500 pieces to load instead of 583): 63.2 -> 60.9 us, and
+// 62.6 where one image of the batch needs more than 8 000 bytes. Fewer instructions alone (taps widened inside
+// v_fma_mix_f32: a fifth fewer) measured the same beside it.
 #include "rmx_device.h"
 #include "rmx_launch.h"
 
@@ -38,7 +44,7 @@ extern __shared__ uint32_t rmx_lds_warp[];
 typedef __attribute__((address_space(3))) uint32_t lds_u32;  // explicit LDS pointers: 32-bit address arithmetic
 
 constexpr int WTW = 32, WTH = 16;  // destination tile: 4 lanes x 8 px wide, 16 rows per pass
-constexpr int WRP = kWarpRawPieces;  // LDS pitch of boxes that fit it, in 16-byte pieces (an odd number spreads the rows over the LDS banks)
+constexpr int WRP = kWarpRawPieces;  // LDS pitch of boxes that fit it, in 16-byte pieces
 
 RMX_DEV uint32_t load_px_global(const uint8_t *p) {
     return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16);
@@ -83,7 +89,7 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     T *dimg = reinterpret_cast<T *>(a.dst) + (size_t)s * 3 * a.dst_h * a.dst_w;
     uint32_t *lds = rmx_lds_warp + (size_t)wib * (a.lds_bytes >> 2);
 
-    // source bounding box of the tile (wave-uniform), one pixel of margin, clipped to the ROI
+    // source bounding box of the tile (wave-uniform) with the right and lower neighbours, clipped to the ROI
     const int X1 = min(X0 + WTW, dw) - 1, Y1 = min(Y0 + WTH * passes, dh) - 1;
     float bxmin = 3.0e38f, bxmax = -3.0e38f, bymin = 3.0e38f, bymax = -3.0e38f;
     bool corners_ok = true;
@@ -107,27 +113,28 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     // keep the float->int conversions in range for degenerate matrices
     bxmin = __builtin_fmaxf(bxmin, -1.0e6f); bxmax = __builtin_fminf(bxmax, 1.0e6f);
     bymin = __builtin_fmaxf(bymin, -1.0e6f); bymax = __builtin_fminf(bymax, 1.0e6f);
-    const int bx0 = max((int)floorf(bxmin) - 1, xlo), bx1 = min((int)floorf(bxmax) + 2, xhi);
-    const int by0 = max((int)floorf(bymin) - 1, ylo), by1 = min((int)floorf(bymax) + 2, yhi);
+    const int bx0 = max((int)floorf(bxmin), xlo), bx1 = min((int)floorf(bxmax) + 1, xhi);
+    const int by0 = max((int)floorf(bymin), ylo), by1 = min((int)floorf(bymax) + 1, yhi);
     const int bw = bx1 - bx0 + 1, bh = by1 - by0 + 1;
     const bool empty = bw <= 0 || bh <= 0;
-    // staged box: bw columns + the repeated last one, bh rows + the repeated last one
+    // staged box: bw columns + the repeated last one, bh rows + one more where a tap can lie in the box's last row: in the ROI's last
+    // row, or (a tile above the ROI, whose pixels are clamped to it and replaced) in its first one
+    const int nr = bh + (int)(bymax >= (float)yhi || bymax < (float)ylo);
     // RAW: a row is ppr 16-byte pieces from the dword that holds pixel bx0 (byte phase ph inside it). Boxes of at most WRP pieces
-    // per row (every tile of a map that does not minify) are staged at ONE pitch, known to the compiler: the row below is an
-    // offset inside the read instruction.
+    // per row (every tile of a map that minifies by less than a tenth or so) and those of one piece more are staged at a pitch known to
+    // the compiler: the row below is an offset inside the read instruction.
     const uint32_t skew = (uint32_t)((uintptr_t)simg & 3u);
     const uint32_t colb = (uint32_t)max(bx0, 0) * 3u + skew;
     const int ppr_box = ((int)(colb & 3u) + 3 * (max(bw, 0) + 1) + 15) >> 4;
-    const bool fixed = RAW && ppr_box <= WRP;
-    const int ppr = fixed ? WRP : ppr_box;
+    const int ppr = max(ppr_box, WRP);
     // Any phase: rows at a pitch that leaves the same remainder mod 4 as the row stride, so that a row's bytes keep their place
     // within a dword on the way into LDS; at least 16 bytes between two rows' data, so that no piece holds data of both.
     const int need = 3 * max(bw, 0) + 16;
     const int pitch_b = RAW ? ppr * 16 : max(WRP * 16, (need + 3) & ~3) + (int)(row_stride & 3u);  // bytes
     const int ph = (int)((RAW ? colb : colb + (uint32_t)max(by0, 0) * row_stride) & 3u);  // LDS byte of the box's first pixel
-    const int total = RAW ? (bh + 1) * ppr : (int)(((int64_t)ph + (int64_t)(bh - 1) * pitch_b + 3 * bw + 15) >> 4);  // 16-byte pieces
+    const int total = RAW ? nr * ppr : (int)(((int64_t)ph + (int64_t)(bh - 1) * pitch_b + 3 * bw + 15) >> 4);  // 16-byte pieces
     // (RAW: the three dwords read for the last tap of the last row may reach 8 bytes behind the box)
-    const bool use_lds = !empty && (!RAW || total <= 16 * RMX_WAVE) && (uint64_t)(bh + 1) * (uint32_t)pitch_b + (RAW ? 16 : 32) <= (uint64_t)a.lds_bytes;
+    const bool use_lds = !empty && (!RAW || total <= 16 * RMX_WAVE) && (uint64_t)nr * (uint32_t)pitch_b + (RAW ? 16 : 32) <= (uint64_t)a.lds_bytes;
 
     const int lr = lane >> 2, g = lane & 3;
     int x0 = X0 + g * PX;
@@ -213,13 +220,13 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
         // ---- the box straight into LDS: piece idx = (row, piece of the row) in row order lands at byte 16 idx of the slice
         const uint32_t col4 = colb & ~3u;
         // every piece of the box lies inside the batch buffer (the last rows of the last sample may not)
-        const bool safe = simg + ((size_t)min(by1 + 1, yhi) * row_stride + (size_t)bx0 * 3 + 16 * (size_t)ppr) <= buf_end;
+        const bool safe = simg + ((size_t)by1 * row_stride + (size_t)bx0 * 3 + 16 * (size_t)ppr) <= buf_end;
         const float inv_ppr = 1.0f / (float)ppr;
         if (safe) {
             for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
                 const int idx = j0 + lane;
                 // idx / ppr: (idx + 0.5) / ppr is at least 0.5/ppr away from an integer, so the truncation is exact
-                const int r = fixed ? idx / WRP : (int)(((float)idx + 0.5f) * inv_ppr);
+                const int r = (int)(((float)idx + 0.5f) * inv_ppr);
                 const int c = idx - __mul24(r, ppr);
                 const uint32_t off = (uint32_t)min(by0 + r, yhi) * row_stride + col4 + 16u * (uint32_t)c;
                 if (idx < total) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
@@ -244,7 +251,7 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
         wave_sync();
         // the column behind the box repeats its last column where that is the ROI's last column (only then is it read)
         if (bx1 == xhi) {
-            for (int r = lane; r <= bh; r += RMX_WAVE) {
+            for (int r = lane; r < nr; r += RMX_WAVE) {
                 lds_u8 *px = ldsb + r * pitch_b + ph + 3 * (bw - 1);
                 px[3] = px[0];
                 px[4] = px[1];
@@ -298,7 +305,7 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             }
             wave_sync();
         }
-        if (!NEAREST && by1 == yhi) {
+        if (!NEAREST && nr > bh) {
             lds_u8 *last = ldsb + (bh - 1) * pitch_b + ph;
             for (int b = lane; b < 3 * (bw + 1); b += RMX_WAVE) last[pitch_b + b] = last[b];
             wave_sync();
@@ -317,7 +324,8 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     asm volatile("" : "+v"(lbase_v));
     auto gather = [&](auto chk, auto fix) {
         constexpr bool CHECK = decltype(chk)::value;
-        constexpr bool FIXED = decltype(fix)::value;
+        constexpr int PITCH = decltype(fix)::value;  // 16-byte pieces, 0: not known before
+        constexpr bool FIXED = PITCH != 0;
         for (int pass = 0; pass < passes; pass++) {
             const int y = Y0 + pass * WTH + lr;
             if (y >= dh || cnt <= 0) continue;
@@ -365,21 +373,21 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
                 const int ix0 = floor_i32(sx), iy0 = floor_i32(sy);
                 // byte address: a 24-bit multiply-add of the row onto the slice base, another of the column
                 uint32_t rowb, adr;
-                if constexpr (FIXED) asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(rowb) : "v"(iy0), "s"(WRP * 16), "v"(lbase_v));
+                if constexpr (FIXED) asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(rowb) : "v"(iy0), "s"(PITCH * 16), "v"(lbase_v));
                 else asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(rowb) : "v"(iy0), "s"(pitch_b), "v"(lbase_v));
                 asm("v_mad_i32_i24 %0, %1, 3, %2" : "=v"(adr) : "v"(ix0), "v"(rowb));
                 const uint32_t adr1 = adr + (uint32_t)pitch_b;
                 t.tph = adr;
                 t.bph = RAW ? adr : adr1;
                 const lds_u32 *t0p = (const lds_u32 *)(adr & ~3u);
-                const lds_u32 *t1p = FIXED ? t0p + WRP * 4 : (const lds_u32 *)(adr1 & ~3u);
+                const lds_u32 *t1p = FIXED ? t0p + PITCH * 4 : (const lds_u32 *)(adr1 & ~3u);
                 if constexpr (BY_HAND) {
-                    static_assert(WRP * 4 + 2 < 256, "the row below must be reachable by the 8-bit dword offsets of ds_read2_b32");
+                    static_assert(PITCH * 4 + 2 < 256, "the row below must be reachable by the 8-bit dword offsets of ds_read2_b32");
                     // (the values are taken apart only behind the wait: nothing may copy a register before its data has arrived)
                     asm volatile("ds_read2_b32 %0, %4 offset1:1\n\tds_read_b32 %1, %4 offset:8\n\t"
                                  "ds_read2_b32 %2, %4 offset0:%5 offset1:%6\n\tds_read_b32 %3, %4 offset:%7"
                                  : "=&v"(t.top), "=&v"(t.t2), "=&v"(t.bot), "=&v"(t.b2)
-                                 : "v"((uint32_t)(uintptr_t)t0p), "n"(WRP * 4), "n"(WRP * 4 + 1), "n"(WRP * 16 + 8));
+                                 : "v"((uint32_t)(uintptr_t)t0p), "n"(PITCH * 4), "n"(PITCH * 4 + 1), "n"(PITCH * 16 + 8));
                     return t;
                 }
                 t.top = (u32x2_r){t0p[0], t0p[1]};
@@ -438,15 +446,15 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             store(y, v);
         }
     };
+    auto run = [&](auto fix) {
+        if (all_in) gather(std::false_type{}, fix);
+        else gather(std::true_type{}, fix);
+    };
     if constexpr (RAW) {
-        if (fixed) {
-            if (all_in) gather(std::false_type{}, std::true_type{});
-            else gather(std::true_type{}, std::true_type{});
-            return;
-        }
+        if (ppr == WRP) return run(std::integral_constant<int, WRP>{});
+        if (ppr == WRP + 1) return run(std::integral_constant<int, WRP + 1>{});
     }
-    if (all_in) gather(std::false_type{}, std::false_type{});
-    else gather(std::true_type{}, std::false_type{});
+    run(std::integral_constant<int, 0>{});
 }
 
 template <bool NEAREST, bool RAW>
