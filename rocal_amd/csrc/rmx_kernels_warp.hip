@@ -26,9 +26,8 @@
 // box's loads 47, without the stores 52, without both 42, with taps that meet no bank conflict the same; the bytes are 36 at the rate of
 // a large copy. The LDS slice therefore holds the box and nothing besides: no pixel of margin (the corners bound it exactly), the
 // repeated row only where it is read, rows of 10 pieces where they fit instead of 11 (a batch turned by up to 30 degrees and scaled by a
-// tenth: 9.4 -> 7.9 KB a wavefront, 20 of them per CU instead of 16; 500 pieces to load instead of 583): 63.2 -> 60.9 us, and
-// 62.6 where one image of the batch needs more than 8 000 bytes. Fewer instructions alone (taps widened inside
-// v_fma_mix_f32: a fifth fewer) measured the same beside it.
+// tenth: 9.4 -> 7.7 KB a wavefront, 20 of them per CU instead of 16; a seventh fewer pieces to load): 63.2 - 64.0 -> 60.9 - 63.1 us on
+// several inputs, in turn. Fewer instructions alone (taps widened inside v_fma_mix_f32: a fifth fewer) measured the same beside it.
 #include "rmx_device.h"
 #include "rmx_launch.h"
 
