@@ -15,6 +15,7 @@
 
 #include "rmx_common.h"
 #include "rmx_launch.h"
+#include "rmx_warp_box.h"
 
 namespace {
 

@@ -30,6 +30,7 @@
 // several inputs, in turn. Fewer instructions alone (taps widened inside v_fma_mix_f32: a fifth fewer) measured the same beside it.
 #include "rmx_device.h"
 #include "rmx_launch.h"
+#include "rmx_warp_box.h"
 
 #include <type_traits>
 
@@ -42,8 +43,7 @@ namespace rmx {
 extern __shared__ uint32_t rmx_lds_warp[];
 typedef __attribute__((address_space(3))) uint32_t lds_u32;  // explicit LDS pointers: 32-bit address arithmetic
 
-constexpr int WTW = 32, WTH = 16;  // destination tile: 4 lanes x 8 px wide, 16 rows per pass
-constexpr int WRP = kWarpRawPieces;  // LDS pitch of boxes that fit it, in 16-byte pieces
+constexpr int WRP = kWarpRawPieces;
 
 RMX_DEV uint32_t load_px_global(const uint8_t *p) {
     return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16);
@@ -76,11 +76,9 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     const int X0 = tx * WTW, Y0 = ty * (WTH * passes);
     if (X0 >= dw || Y0 >= dh) return;
 
-    const int xlo = P.src_x, ylo = P.src_y;
-    const int xhi = xlo + P.src_w - 1, yhi = ylo + P.src_h - 1;
     const float m0 = P.m[0], m1 = P.m[1], m2 = P.m[2], m3 = P.m[3], m4 = P.m[4], m5 = P.m[5];
     const float dcx = (float)(dw >> 1), dcy = (float)(dh >> 1);
-    const float scx = (float)(xlo + (P.src_w >> 1)), scy = (float)(ylo + (P.src_h >> 1));
+    const float scx = (float)(P.src_x + (P.src_w >> 1)), scy = (float)(P.src_y + (P.src_h >> 1));
 
     uint32_t row_stride;
     const uint8_t *simg = sample_base(a, s, row_stride);
@@ -88,52 +86,13 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     T *dimg = reinterpret_cast<T *>(a.dst) + (size_t)s * 3 * a.dst_h * a.dst_w;
     uint32_t *lds = rmx_lds_warp + (size_t)wib * (a.lds_bytes >> 2);
 
-    // source bounding box of the tile (wave-uniform) with the right and lower neighbours, clipped to the ROI
-    const int X1 = min(X0 + WTW, dw) - 1, Y1 = min(Y0 + WTH * passes, dh) - 1;
-    float bxmin = 3.0e38f, bxmax = -3.0e38f, bymin = 3.0e38f, bymax = -3.0e38f;
-    bool corners_ok = true;
-#pragma unroll
-    for (int cy = 0; cy < 2; cy++)
-#pragma unroll
-        for (int cx = 0; cx < 2; cx++) {
-            float xr = (float)(cx ? X1 : X0) - dcx, yr = (float)(cy ? Y1 : Y0) - dcy;
-            float sx = __builtin_fmaf(xr, m0, __builtin_fmaf(yr, m1, m2)) + scx;
-            float sy = __builtin_fmaf(xr, m3, __builtin_fmaf(yr, m4, m5)) + scy;
-            if constexpr (NEAREST) {
-                sx += 0.5f;
-                sy += 0.5f;
-            }
-            bxmin = __builtin_fminf(bxmin, sx); bxmax = __builtin_fmaxf(bxmax, sx);
-            bymin = __builtin_fminf(bymin, sy); bymax = __builtin_fmaxf(bymax, sy);
-            corners_ok = corners_ok && sx == sx && sy == sy;
-        }
-    // every pixel of the tile maps between the corner extremes: when those lie inside the ROI no pixel needs a test
-    const bool all_in = corners_ok && bxmin >= (float)xlo && bymin >= (float)ylo && bxmax < (float)(xhi + 1) && bymax < (float)(yhi + 1);
-    // keep the float->int conversions in range for degenerate matrices
-    bxmin = __builtin_fmaxf(bxmin, -1.0e6f); bxmax = __builtin_fminf(bxmax, 1.0e6f);
-    bymin = __builtin_fmaxf(bymin, -1.0e6f); bymax = __builtin_fminf(bymax, 1.0e6f);
-    const int bx0 = max((int)floorf(bxmin), xlo), bx1 = min((int)floorf(bxmax) + 1, xhi);
-    const int by0 = max((int)floorf(bymin), ylo), by1 = min((int)floorf(bymax) + 1, yhi);
-    const int bw = bx1 - bx0 + 1, bh = by1 - by0 + 1;
-    const bool empty = bw <= 0 || bh <= 0;
-    // staged box: bw columns + the repeated last one, bh rows + one more where a tap can lie in the box's last row: in the ROI's last
-    // row, or (a tile above the ROI, whose pixels are clamped to it and replaced) in its first one
-    const int nr = bh + (int)(bymax >= (float)yhi || bymax < (float)ylo);
-    // RAW: a row is ppr 16-byte pieces from the dword that holds pixel bx0 (byte phase ph inside it). Boxes of at most WRP pieces
-    // per row (every tile of a map that minifies by less than a tenth or so) and those of one piece more are staged at a pitch known to
-    // the compiler: the row below is an offset inside the read instruction.
+    // source bounding box of the tile (wave-uniform)
     const uint32_t skew = (uint32_t)((uintptr_t)simg & 3u);
-    const uint32_t colb = (uint32_t)max(bx0, 0) * 3u + skew;
-    const int ppr_box = ((int)(colb & 3u) + 3 * (max(bw, 0) + 1) + 15) >> 4;
-    const int ppr = max(ppr_box, WRP);
-    // Any phase: rows at a pitch that leaves the same remainder mod 4 as the row stride, so that a row's bytes keep their place
-    // within a dword on the way into LDS; at least 16 bytes between two rows' data, so that no piece holds data of both.
-    const int need = 3 * max(bw, 0) + 16;
-    const int pitch_b = RAW ? ppr * 16 : max(WRP * 16, (need + 3) & ~3) + (int)(row_stride & 3u);  // bytes
-    const int ph = (int)((RAW ? colb : colb + (uint32_t)max(by0, 0) * row_stride) & 3u);  // LDS byte of the box's first pixel
-    const int total = RAW ? nr * ppr : (int)(((int64_t)ph + (int64_t)(bh - 1) * pitch_b + 3 * bw + 15) >> 4);  // 16-byte pieces
-    // (RAW: the three dwords read for the last tap of the last row may reach 8 bytes behind the box)
-    const bool use_lds = !empty && (!RAW || total <= 16 * RMX_WAVE) && (uint64_t)nr * (uint32_t)pitch_b + (RAW ? 16 : 32) <= (uint64_t)a.lds_bytes;
+    const WarpBox box = warp_box<NEAREST, RAW>(P.src_x, P.src_y, P.src_w, P.src_h, dw, dh, m0, m1, m2, m3, m4, m5, X0, Y0, passes, skew, row_stride, a.lds_bytes);
+    const int xlo = box.xlo, ylo = box.ylo, xhi = box.xhi, yhi = box.yhi;
+    const int bx0 = box.bx0, by0 = box.by0, bw = box.bw, bh = box.bh, nr = box.nr;
+    const int ppr = box.ppr, pitch_b = box.pitch_b, ph = box.ph, total = box.total;
+    const bool empty = box.empty, all_in = box.all_in;
 
     const int lr = lane >> 2, g = lane & 3;
     int x0 = X0 + g * PX;
@@ -166,7 +125,7 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
         }
         return;
     }
-    if (!use_lds) {
+    if (!box.use_lds) {
         // a box too large for the slice: per-pixel gathers from global memory
         for (int pass = 0; pass < passes; pass++) {
             const int y = Y0 + pass * WTH + lr;
@@ -215,100 +174,45 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
 
     lds_u8 *ldsb = (lds_u8 *)(lds_ptr_t)rmx_lds_warp + (uint32_t)to_sgpr((int)((uint32_t)wib * (uint32_t)a.lds_bytes));
     const uint8_t *base4 = simg - skew;
-    if constexpr (RAW) {
-        // ---- the box straight into LDS: piece idx = (row, piece of the row) in row order lands at byte 16 idx of the slice
-        const uint32_t col4 = colb & ~3u;
-        // every piece of the box lies inside the batch buffer (the last rows of the last sample may not)
-        const bool safe = simg + ((size_t)by1 * row_stride + (size_t)bx0 * 3 + 16 * (size_t)ppr) <= buf_end;
-        const float inv_ppr = 1.0f / (float)ppr;
-        if (safe) {
-            for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
-                const int idx = j0 + lane;
-                // idx / ppr: (idx + 0.5) / ppr is at least 0.5/ppr away from an integer, so the truncation is exact
-                const int r = (int)(((float)idx + 0.5f) * inv_ppr);
-                const int c = idx - __mul24(r, ppr);
-                const uint32_t off = (uint32_t)min(by0 + r, yhi) * row_stride + col4 + 16u * (uint32_t)c;
-                if (idx < total) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
-            }
-            // the compiler does not order LDS reads behind loads into LDS: await them explicitly
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        } else {
-            // the box touches the last bytes of the batch buffer: the pieces that leave it are stored by their lanes
-            const uint64_t lim = (uint64_t)(buf_end - base4);
-            for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
-                const int idx = j0 + lane;
-                const int r = idx / ppr, c = idx - r * ppr;
-                const uint64_t off = (uint64_t)((uint32_t)min(by0 + r, yhi) * row_stride + col4 + 16u * (uint32_t)c);
-                if (idx < total && off + 16 <= lim) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
-                else if (idx < total) {
-                    const uint4 v = load_piece_bounded<int64_t>(base4, (int64_t)off, (int64_t)lim);
-                    *(lds_u32x4 *)(ldsb + 16 * idx) = (u32x4_a4){v.x, v.y, v.z, v.w};
-                }
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        }
-        wave_sync();
-        // the column behind the box repeats its last column where that is the ROI's last column (only then is it read)
-        if (bx1 == xhi) {
-            for (int r = lane; r < nr; r += RMX_WAVE) {
-                lds_u8 *px = ldsb + r * pitch_b + ph + 3 * (bw - 1);
-                px[3] = px[0];
-                px[4] = px[1];
-                px[5] = px[2];
-            }
-            wave_sync();
+    // ---- the box straight into LDS: piece idx lands at byte 16 idx of the slice
+    const uint64_t left = (uint64_t)(buf_end - base4);
+    const float inv = 1.0f / (float)(RAW ? ppr : pitch_b);
+    if (warp_box_inside<RAW>(box, row_stride, left)) {
+        for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
+            const int idx = j0 + lane;
+            const uint32_t off = (uint32_t)warp_piece<RAW>(box, row_stride, idx, inv);
+            if (idx < total) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
         }
     } else {
-        // ---- the box straight into LDS, any phase: LDS byte b belongs to row r of the box (r * pitch_b + ph is the row's first
-        // pixel) and holds the source byte at the same distance from that row's first pixel; a piece is the row's that its last
-        // byte lies in (what a piece holds in front of a row is never read). Pitch and stride agree mod 4 and the box's first dword
-        // is a source dword, so every piece is loaded from a dword.
-        const uint32_t first = (uint32_t)by0 * row_stride + colb - (uint32_t)ph;  // source byte (from base4) of LDS byte 0
-        const uint32_t step = row_stride - (uint32_t)pitch_b;
-        const uint64_t left = (uint64_t)(buf_end - base4);
-        // every piece lies inside the batch buffer (the last rows of the last sample may not, nor the first rows of the first one
-        // where a piece starts up to 15 bytes in front of its row)
-        const bool safe = (uint64_t)by1 * row_stride + colb + (uint32_t)pitch_b + 32u <= left && (bh == 1 || first + row_stride >= 16u);
-        const float inv_pitch = 1.0f / (float)pitch_b;
-        // (x + 0.5) / pitch is at least 0.5 / pitch away from an integer, so the truncation is exact
-        auto row_of = [&](int idx) { return min((int)(((float)(16 * idx + 15 - ph) + 0.5f) * inv_pitch), bh - 1); };
-        if (safe) {
-            for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
-                const int idx = j0 + lane;
-                const uint32_t off = first + 16u * (uint32_t)idx + (uint32_t)row_of(idx) * step;
-                if (idx < total) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
+        // the box touches the ends of the batch buffer: the pieces that leave it are stored by their lanes
+        for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
+            const int idx = j0 + lane;
+            const int64_t off = warp_piece<RAW>(box, row_stride, idx, inv);
+            if (idx < total && off >= 0 && off + 16 <= (int64_t)left) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
+            else if (idx < total) {
+                const uint4 v = load_piece_bounded<int64_t>(base4, off, (int64_t)left);
+                *(lds_u32x4 *)(ldsb + 16 * idx) = (u32x4_a4){v.x, v.y, v.z, v.w};
             }
-            // the compiler does not order LDS reads behind loads into LDS: await them explicitly
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        } else {
-            for (int j0 = 0; j0 < total; j0 += RMX_WAVE) {
-                const int idx = j0 + lane, r = row_of(idx);
-                const int64_t off = (int64_t)(uint32_t)(by0 + r) * row_stride + colb - ph + (16 * idx - r * pitch_b);
-                if (idx < total && off >= 0 && off + 16 <= (int64_t)left) __builtin_amdgcn_global_load_lds((glb_ptr_t)(base4 + off), (lds_ptr_t)(ldsb + 16 * j0), 16, 0, RMX_LDS_LOAD_AUX);
-                else if (idx < total) {
-                    const uint4 v = load_piece_bounded<int64_t>(base4, off, (int64_t)left);
-                    *(lds_u32x4 *)(ldsb + 16 * idx) = (u32x4_a4){v.x, v.y, v.z, v.w};
-                }
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+    }
+    // the compiler does not order LDS reads behind loads into LDS: await them explicitly
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wave_sync();
+    // the column behind the box repeats its last column where that is the ROI's last column, and (rows at any phase) the row below
+    // the box its last row where a tap can lie in that (only then are they read; RAW has loaded that row)
+    if (box.bx1 == xhi) {
+        for (int r = lane; r < (RAW ? nr : bh); r += RMX_WAVE) {
+            lds_u8 *px = ldsb + r * pitch_b + ph + 3 * (bw - 1);
+            px[3] = px[0];
+            px[4] = px[1];
+            px[5] = px[2];
         }
         wave_sync();
-        // the column behind the box repeats its last column where that is the ROI's last column, and the row below the box its
-        // last row where that is the ROI's last row (only then are they read)
-        if (bx1 == xhi) {
-            for (int r = lane; r < bh; r += RMX_WAVE) {
-                lds_u8 *px = ldsb + r * pitch_b + ph + 3 * (bw - 1);
-                px[3] = px[0];
-                px[4] = px[1];
-                px[5] = px[2];
-            }
-            wave_sync();
-        }
-        if (!NEAREST && nr > bh) {
-            lds_u8 *last = ldsb + (bh - 1) * pitch_b + ph;
-            for (int b = lane; b < 3 * (bw + 1); b += RMX_WAVE) last[pitch_b + b] = last[b];
-            wave_sync();
-        }
+    }
+    if (!RAW && !NEAREST && nr > bh) {
+        lds_u8 *last = ldsb + (bh - 1) * pitch_b + ph;
+        for (int b = lane; b < 3 * (bw + 1); b += RMX_WAVE) last[pitch_b + b] = last[b];
+        wave_sync();
     }
 
     // ---- gather and blend, branch-free

@@ -20,8 +20,6 @@ KernelFn select_color_kernel(int kind, int dtype, int layout, int mode, const ch
 KernelFn select_point_kernel(int kind, int dtype, int layout, int mode, const char **name);
 KernelFn select_transpose_kernel(int dtype, int layout, const char **name);
 KernelFn select_warp_kernel(int interp, int dtype, int layout, bool raw, const char **name);
-// LDS pitch, in 16-byte pieces, at which the warp kernel stages every box that fits it
-constexpr int kWarpRawPieces = 10;
 // Normalize: integer moments of every sample's window, 1 << log2_parts shares of six 64-bit numbers per sample, each made by a workgroup
 // of `threads` (whole wavefronts, at most 512)
 void launch_moments(hipStream_t stream, const RmxKArgs &a, unsigned long long *parts, int log2_parts, int threads);

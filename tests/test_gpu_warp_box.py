@@ -38,3 +38,30 @@ def test_boxes(ctx, shrink, interp, width):
     want = orc.warp_affine(img, roi, np.stack([orc.affine_from_rocal(a) for a in affine]), dw, dh, H, width, interp=interp)
     got = got.cpu().numpy()
     assert np.array_equal(got, want), [(i, int((got[i] != want[i]).sum())) for i in range(n) if not np.array_equal(got[i], want[i])]
+
+
+@pytest.mark.parametrize("width", [200, 201])
+@pytest.mark.parametrize("interp", [ops.LINEAR, ops.NEAREST])
+@pytest.mark.parametrize("rows", [1, 2, 3])
+def test_windows_of_few_rows_at_the_buffers_end(ctx, rows, interp, width):
+    """Maps that leave tiles less than a row above such a window, beside it and below it."""
+    import torch
+    H, dh = 60, 64
+    rng = np.random.default_rng(width + rows)
+    affine = np.array([(1, 0, 0, 1, 0, s) for s in (0, -0.5, 0.25, 1, -1, 25, -25.5, 31.5, -31.75)] +
+                      [(0.98, 0.2, -0.2, 0.98, x, s) for x, s in ((0, 0.5), (60, 9), (-60, -9.5))], np.float32)
+    n = len(affine)
+    for height in (H, rows):  # the last rows of images, images of these rows
+        img = rng.integers(0, 256, (n, height, width, 3), dtype=np.uint8)
+        roi = np.tile(np.array([0, height - rows, width, rows], np.uint32), (n, 1))
+        dw, dhs = np.full(n, width, np.uint32), np.full(n, dh, np.uint32)
+        op = ops.WarpAffine(ctx, ops.desc(n, height, width, ops.NHWC, ops.UINT8), ops.desc(n, dh, width, ops.NHWC, ops.UINT8), interp)
+        for first in range(n):  # (every map at the end of the buffer once)
+            a = np.roll(affine, first, axis=0)
+            op.update(roi, a, dw, dhs)
+            got = op.alloc_output(fill=3)
+            op.launch(torch.from_numpy(img).cuda(), got)
+            ctx.sync()
+            want = orc.warp_affine(img, roi, np.stack([orc.affine_from_rocal(v) for v in a]), dw, dhs, dh, width, interp=interp)
+            got = got.cpu().numpy()
+            assert np.array_equal(got, want), [(i, int((got[i] != want[i]).sum())) for i in range(n) if not np.array_equal(got[i], want[i])]
