@@ -1466,22 +1466,25 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         need_max = std::max<int>(need_max, (int)need);
     }
     // fp32 output: room for the slab through which the lanes of a row exchange their runs before storing (the dwords of one lane's run
-    // for each of 64; the kernel takes it from the tail of the slice): interleaved rows, planes of whole groups, and planes of other
-    // whole 16-byte pieces behind a colour twist.
-    const bool planes = op->dst.layout == RMX_NCHW;
-    const int slab = op->dst.dtype == RMX_FP32 ? 64 * 4 * (planes ? 8 : 24) : 0;
-    const int slice = (need_max + 15) / 16 * 16, slice_mid = slice + (!planes || (chain == 2 && op->dst.w % 4 == 0) ? slab : 0);
-    if (!ok || slice + slab > op->ctx->max_lds_per_block - kStaticLdsMax) return RMX_OK;
+    // for each of 64; the kernel takes it from the tail of the slice), where the kernel has one: interleaved rows, planes of whole
+    // groups from source rows at one phase, and behind a colour twist planes of any whole 16-byte pieces.
+    const bool planes = op->dst.layout == RMX_NCHW, fp32 = op->dst.dtype == RMX_FP32;
+    const int slab = fp32 ? 64 * 4 * (planes ? 8 : 24) : 0;
+    const int slice = (need_max + 15) / 16 * 16;
+    const int slice_fast = slice + (rmx::resize_exchanges(fp32, planes, one_phase, chain == 2) ? slab : 0);
+    const int slice_mid = slice + (rmx::resize_exchanges(fp32, planes, false, chain == 2 && op->dst.w % 4 == 0) ? slab : 0);
+    const int widest = std::max(slice_fast, slice_mid);
+    if (!ok || widest > op->ctx->max_lds_per_block - kStaticLdsMax) return RMX_OK;
     // A wavefront works through `group` windows (of `rows` destination rows) below each other per x-tile, so that the
     // tile's x taps are computed once for all of them (1 measured best: more leave too few wavefronts to fill the chip evenly).
     const long windows = (long)op->n * ((max_dh + rows - 1) / rows);
     const int group = op->ctx->dma_group ? op->ctx->dma_group : (int)std::max<long>(1, std::min<long>(8, windows / 4096));
-    op->fast_lds = slice + slab;
+    op->fast_lds = slice_fast;
     op->mid_lds = slice_mid;
     op->mid_rows = op->fast_rows = rows;
     op->mid_strips = op->fast_strips = std::max(1, (max_dh + rows * group - 1) / (rows * group));
     // (default 1: a workgroup's LDS is released only when its last wavefront ends, one-wave groups keep the CU full)
-    op->mid_wpb = op->fast_wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, slice + slab)));
+    op->mid_wpb = op->fast_wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, widest)));
     op->mid_aux1 = op->fast_aux1 = group;
     if (nearest) {
         op->fn_mid = rmx::select_resize_near_kernel(op->dst.dtype, op->dst.layout, op->norm, &op->mid_name);

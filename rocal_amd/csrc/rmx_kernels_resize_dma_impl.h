@@ -92,7 +92,7 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     // us, 144 x 144 9.4 -> 8.3), and under a colour chain those of other widths that are multiples of 4 (64 images to
     // 300 x 300 36.8 -> 33.8). Without the chain planes of such widths gain nothing (300 wide 33.2 -> 34.1, 708 wide 47.0 -> 47.8).
     constexpr bool QUADS = !ALIGNED && LAYOUT == RMX_NCHW && CHAIN == CHAIN_TWIST;
-    constexpr bool COALESCE = sizeof(T) == 4 && (LAYOUT == RMX_NHWC || ALIGNED || QUADS);
+    constexpr bool COALESCE = resize_exchanges(sizeof(T) == 4, LAYOUT == RMX_NCHW, ALIGNED, CHAIN == CHAIN_TWIST);
     constexpr bool AHEAD = CHAIN != CHAIN_TWIST;  // (see load_sample)
     __shared__ __attribute__((aligned(16))) float chain_tables[CHAIN == CHAIN_TWIST ? sizeof(ColorTables) / 4 : 4];
     const int lane = threadIdx.x & (RMX_WAVE - 1);

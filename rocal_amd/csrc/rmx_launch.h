@@ -11,6 +11,12 @@ KernelFn select_cmn_kernel(int dtype, int layout, int norm, int mode, const char
 KernelFn select_resize_linear_kernel(int dtype, int layout, bool norm, bool quant, int chain, const char **name);
 KernelFn select_resize_fast_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool aligned, const char **name);
 KernelFn select_resize_dma_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool aligned, const char **name);
+// Whether a streaming resize kernel's lanes exchange their fp32 runs through LDS before storing (and how it is built: rmx_kernels_resize_dma_impl.h).
+// The plan makes room for the exchange where this says so and nowhere else: 2 KB more than a full slice of 10 are three of sixteen
+// wavefronts per CU. fp32 planes from rows at any phase, without room / with room that their kernel does not use: 96 windows to 160 x 160
+// 16.0 / 18.4 us, 64 to 224 x 224 14.0 / 14.9, 100 to 200 x 200 15.9 / 16.5; 128 to 224 x 224, whose stores fewer wavefronts in
+// flight disturb less, 32.5 / 31.3.
+constexpr bool resize_exchanges(bool fp32, bool planes, bool aligned, bool twist) { return fp32 && (!planes || aligned || twist); }
 KernelFn select_resize_near_kernel(int dtype, int layout, bool norm, const char **name);
 KernelFn select_resize_nearest_kernel(int dtype, int layout, bool norm, bool quant, const char **name);
 KernelFn select_resize_tri_kernel(int dtype, int layout, bool norm, bool quant, const char **name);

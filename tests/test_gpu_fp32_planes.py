@@ -46,3 +46,27 @@ def test_planes_of_every_kind(ctx, width, source_width, twist):
         for i in range(n):
             view[i, :, :rh[i], :rw[i]] = exp[i, :, :rh[i], :rw[i]]
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), "shift %d (%s): %d values differ" % (shift, op.plan, int((got != want).sum()))
+
+
+@pytest.mark.parametrize("twist", [False, True])
+@pytest.mark.parametrize("layout", [ops.NCHW, ops.NHWC])
+@pytest.mark.parametrize("source_width", [96, 97])
+@pytest.mark.parametrize("width", [64, 72, 100, 101])
+def test_room_for_the_exchange_where_there_is_one(ctx, width, source_width, layout, twist):
+    """The LDS slice of an fp32 plan against the half-precision one's: as large but for the slab of kernels that exchange their runs."""
+    n, H, oh = 3, 40, 20
+    roi = np.tile(np.array([0, 0, source_width, H], np.uint32), (n, 1))
+    rw, rh = np.full(n, width, np.uint32), np.full(n, oh, np.uint32)
+    scale, bias = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
+    lds = {}
+    for dtype in (ops.FP32, ops.FP16):
+        op = ops.Resize(ctx, ops.desc(n, H, source_width, ops.NHWC, ops.UINT8), ops.desc(n, oh, width, layout, dtype), ops.LINEAR,
+                        flags=ops.F_QUANTIZE_U8 | (ops.F_COLOR_TWIST if twist else 0))
+        if twist:
+            op.update_color_cmn(roi, rw, rh, scale, bias, [np.full(n, v, np.float32) for v in (1.1, 2.0, 30.0, 0.9)], None)
+        else:
+            op.update_cmn(roi, rw, rh, scale, bias, None)
+        lds[dtype] = int(dict(p.split("=") for p in op.plan.split())["lds_per_wave"])
+    whole, one_phase = width % 8 == 0, source_width % 4 == 0
+    exchange = layout == ops.NHWC or (whole and one_phase) or (twist and width % 4 == 0)
+    assert lds[ops.FP32] - lds[ops.FP16] == (0 if not exchange else 2048 if layout == ops.NCHW else 6144), (lds, op.plan)
