@@ -71,5 +71,13 @@ def build(verbose=False, incremental=False):
     return LIB
 
 
+def build_checks():
+    """The kernel of tests/test_gpu_reciprocals.py, beside the library and with its flags."""
+    out = os.path.join(HERE, "lib", "libreciprocals_check.so")
+    src = os.path.join(HERE, "..", "tests", "cpp", "reciprocals.hip")
+    subprocess.run([HIPCC] + FLAGS + ["-I" + CSRC, "-shared", src, "-o", out], check=True, stderr=subprocess.DEVNULL)
+    return out
+
+
 if __name__ == "__main__":
     print(build(verbose=True, incremental="--incremental" in sys.argv))

@@ -126,14 +126,6 @@ RMX_DEV void zero_set(int idx, float (&acc)[SLOTS][3][2]) {
     }
 }
 
-// 1 / b correctly rounded, for the products of coefficient sums (b far from the ends of the exponent range): the hardware's
-// reciprocal and one correction by its remainder (Markstein, IBM J. Res. Dev. 34, 1990). Equal to the division for every
-// significand at every exponent from -40 to 40 (run through on the device): three instructions where the division is ten.
-RMX_DEV float recip(float b) {
-    const float y = __builtin_amdgcn_rcpf(b);
-    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
-}
-
 template <typename T>
 RMX_DEV uint32_t elem_bits(float v) {
     const T o = OutCvt<T>::cvt(v);
