@@ -149,7 +149,7 @@ struct rmx_op {
     const char *mid_name = "";
     int mid_lds = 0, mid_strips = 1, mid_rows = 4, mid_wpb = 1, mid_aux1 = 1;
     uint64_t algo_bytes = 0;
-    int tri_rows_in_flight = 0;  // streaming triangular kernel: accumulator sets (2 or 4), 0 for every other kernel
+    int tri_rows_in_flight = 0;  // streaming triangular kernel: accumulator sets (2, 4 or 8), 0 for every other kernel
     // Point operations on whole frames (every sample's window is the whole padded image, source and destination of one
     // shape): the kernel walks a frame as flat_h rows of 512 pixels, so that all 64 lanes work whatever the image width is
     // (224 pixels are 28 groups of 8: two rows per step keep 56 lanes busy; 299 pixels keep 38). 0: the images' own rows.

@@ -88,9 +88,10 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     static_assert(CHAIN == CHAIN_NONE || !NEAREST, "a colour node in the chain follows a bilinear resize node");
     // fp32 runs are longer than one store: the lanes of a row exchange them through LDS before storing, so that every store
     // instruction writes whole pieces one behind the other, as streaming stores. (The slab is the tail of the wavefront's slice,
-    // the host adds its size.) Interleaved rows always; planes of whole groups (128 RandomResizedCrops to 224 x 224 33.5 -> 24.3
-    // us, 144 x 144 9.4 -> 8.3), and under a colour chain those of other widths that are multiples of 4 (64 images to
-    // 300 x 300 36.8 -> 33.8). Without the chain planes of such widths gain nothing (300 wide 33.2 -> 34.1, 708 wide 47.0 -> 47.8).
+    // the host adds its size.) Interleaved rows always; planes of whole groups from rows at one phase (128 RandomResizedCrops to
+    // 224 x 224 33.5 -> 24.3 us, 144 x 144 9.4 -> 8.3), and under a colour chain those of other widths that are multiples of 4
+    // (launches of 64 images to 300 x 300 36.8 -> 33.8; a pipeline's whole batches of them wait for the host). Without the chain planes of
+    // such widths gain nothing (300 wide 33.2 -> 34.1, 708 wide 47.0 -> 47.8).
     constexpr bool QUADS = !ALIGNED && LAYOUT == RMX_NCHW && CHAIN == CHAIN_TWIST;
     constexpr bool COALESCE = resize_exchanges(sizeof(T) == 4, LAYOUT == RMX_NCHW, ALIGNED, CHAIN == CHAIN_TWIST);
     constexpr bool AHEAD = CHAIN != CHAIN_TWIST;  // (see load_sample)

@@ -1,7 +1,7 @@
 // K2t streaming path: triangular (antialiased) downscaling for batches in which every source row starts at the same byte
 // phase (row stride a multiple of 4). Same arithmetic as rmx_resize_tri_down_kernel (rmx_kernels_tri.hip), operation for
 // operation: a wavefront owns 128 output columns (two per lane) and a strip of output rows, filters its source rows
-// horizontally in ascending order and adds each filtered row, from registers, to the output rows in flight (four slots).
+// horizontally in ascending order and adds each filtered row, from registers, to the output rows in flight (two, four or eight accumulator sets).
 // What differs is how the source rows reach the horizontal pass:
 //   * rows travel from global memory straight into LDS (global_load_lds_dwordx4: 16 bytes per lane, no vector register, no
 //     unpacking, no LDS store instruction). An LDS row holds the raw packed-RGB bytes: a margin for the left edge replicas,
@@ -135,11 +135,11 @@ RMX_DEV uint32_t elem_bits(float v) {
 }
 
 // SLOTS: output rows in flight. Four cover every downscale (rows four apart never share a source row); eight cover samples
-// that grow vertically by up to about 3.8 (two taps, several output rows per source row; 113 registers, four wavefronts per
+// that grow vertically by up to about 3.8 (two taps, several output rows per source row; 119 registers, four wavefronts per
 // SIMD), so that a batch of RandomResizedCrop windows, some of which shrink and some of which grow, stays in this kernel
-// (measured on 256 such windows to 224 x 224: 160 us through the ring kernel; in that kernel a sample that shrinks runs a row
-// loop of its own that adds to the lower four sets only, and windows with two or three horizontal taps have their own
-// unrolled passes: 70.2 -> 67.2 us on those windows). Two are enough when
+// (measured on 256 such windows to 224 x 224: 160 us through the ring kernel; a sample for which the host has shown that four sets suffice,
+// every one that shrinks and most that grow by less than two, runs a row loop of its own that adds to the lower four only, and
+// windows with two or three horizontal taps have their own unrolled passes). Two are enough when
 // rows two apart never do, which the host establishes for ratios that are whole or half numbers (1080 -> 360 rows, any
 // decimation by 2, 3, 4 or 1.5): every source row then enters two accumulator sets instead of four.
 template <typename T, int LAYOUT, bool NORM, bool QUANT, int SLOTS>
@@ -391,7 +391,7 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
         }
     };
 
-    // ---- output rows in flight: row r accumulates in slot (r - r0) & 3 until its last tap row has been added. rq is the
+    // ---- output rows in flight: row r accumulates in set (r - r0) & smask until its last tap row has been added. rq is the
     // oldest row in flight, qlast its last tap row (wave-uniform state).
     float acc[TS_SLOTS][3][TPX];
     int rq = r0;
@@ -487,7 +487,7 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
         constexpr int NT = decltype(nt)::value;
         constexpr int PR = decltype(pair)::value;  // the lane's two columns are neighbours whose first taps lie PR pixels apart; 0: not
         // LIVE: the accumulator sets this instance of the row loop adds to and stores from (the lower four of eight for a sample
-        // that shrinks: a loop of its own rather than a branch around the upper sets' FMAs, at whose join the accumulators
+        // that needs no more: a loop of its own rather than a branch around the upper sets' FMAs, at whose join the accumulators
         // would be copied)
         constexpr int LIVE = (TS_SLOTS == 8 && decltype(lower_only)::value) ? 4 : TS_SLOTS;
         constexpr int NE = (3 * NT + 3) / 4;
@@ -548,7 +548,7 @@ __global__ void __launch_bounds__(256, SLOTS == 8 ? 4 : RMX_TDMA_WAVES) rmx_resi
                 h[2][i] = a2;
             }
         }
-        // ---- vertical pass: every pass adds the filtered row to all four slots with that pass's coefficients (0: none)
+        // ---- vertical pass: every pass adds the filtered row to all LIVE sets with that pass's coefficients (0: none)
         auto add_row = [&]() {
 #pragma unroll
             for (int m = 0; m < LIVE; m++)
