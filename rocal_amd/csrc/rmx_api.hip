@@ -91,7 +91,7 @@ struct rmx_ctx {
     // Launch-plan tunables (rows per wavefront strip, LDS budget of the resize fast path). Defaults are the
     // values measured best on MI355X; RMX_TUNE_* environment variables, read once when the context is
     // created and clamped to safe ranges, override them for sweeps. They change plans, never results.
-    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, warp_passes = 2, warp_wpb = 4;
+    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, tri_adj = 1, warp_passes = 2, warp_wpb = 4;
 };
 
 static int tune_env(const char *name, int def, int lo, int hi) {
@@ -149,6 +149,7 @@ struct rmx_op {
     const char *mid_name = "";
     int mid_lds = 0, mid_strips = 1, mid_rows = 4, mid_wpb = 1, mid_aux1 = 1;
     uint64_t algo_bytes = 0;
+    bool tri_adjacent = false;   // streaming triangular kernel whose lanes own neighbouring columns
     int tri_rows_in_flight = 0;  // streaming triangular kernel: accumulator sets (2, 4 or 8), 0 for every other kernel
     // Point operations on whole frames (every sample's window is the whole padded image, source and destination of one
     // shape): the kernel walks a frame as flat_h rows of 512 pixels, so that all 64 lanes work whatever the image width is
@@ -577,6 +578,7 @@ int rmx_ctx_create(int device, void *stream, int own_stream, rmx_ctx **out) {
         ctx->tri_slots = tune_env("RMX_TUNE_TRI_SLOTS", ctx->tri_slots, 0, 4);  // 4: the streaming triangular kernel always keeps four rows in flight (batches that need eight go to the ring kernel)
         ctx->deal_xcd = tune_env("RMX_TUNE_DEAL_XCD", ctx->deal_xcd, 0, 1);  // samples dealt round-robin to the XCDs (0: eight runs in batch order)
         ctx->tri_sort = tune_env("RMX_TUNE_TRI_SORT", ctx->tri_sort, 0, 1);  // rows of batches of uneven cost go largest window first
+        ctx->tri_adj = tune_env("RMX_TUNE_TRI_ADJ", ctx->tri_adj, 0, 1);     // 0: no streaming triangular kernel whose lanes own neighbouring columns
         ctx->tri_per_cu = tune_env("RMX_TUNE_TRI_PER_CU", ctx->tri_per_cu, 0, 32);  // wavefronts per CU the strip planner counts on (0: by registers and LDS)
     }
     *out = ctx;
@@ -651,7 +653,7 @@ const char *rmx_op_plan(const rmx_op *op) {
     else {
         len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d tile_w=%d lds_per_wave=%d waves_per_block=%d fast=0",
                        (long long)op->n * op->strips, op->strips, op->strip_rows, op->tile_w, op->lds_per_wave, op->waves_per_block);
-        if (op->tri_rows_in_flight) len += snprintf(buf + len, sizeof(buf) - len, " rows_in_flight=%d", op->tri_rows_in_flight);
+        if (op->tri_rows_in_flight) len += snprintf(buf + len, sizeof(buf) - len, " rows_in_flight=%d%s", op->tri_rows_in_flight, op->tri_adjacent ? " adjacent=1" : "");
     }
     // (how the rows of the last update reach the kernel: dwords per sample in its arguments, or a table)
     if (op->updated && op->compact) len += snprintf(buf + len, sizeof(buf) - len, " rows=arguments words=%u", op->compact_words);
@@ -1159,7 +1161,8 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         // A sample that grows vertically (two taps, several output rows per source row) needs eight rows in flight, which
         // the streaming form has for ratios from about 0.26 on: first row of r+8 strictly below the last row of r.
         bool down = kx_cap <= 8 && !op->ctx->tri_ring;
-        int flight = 4;  // rows in flight the batch needs
+        bool far = false;  // some sample grows by more than eight rows in flight allow
+        int flight = 4;    // rows in flight the batch needs
         for (int i = 0; i < op->n; i++) t[i].plan[1] = RMX_TRI_EIGHT;
         for (int i = 0; i < op->n && down; i++) {
             RmxSample &s = t[i];
@@ -1195,16 +1198,19 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
             }
             const int apart = s.ry >= 1.0f ? 4 : 8;
             if (s.dst_h <= apart) continue;
-            if (far_apart(apart)) {
-                down = ends_apart(apart);
-                continue;
+            bool fits = true;
+            if (far_apart(apart)) fits = ends_apart(apart);
+            else
+                for (int r = 0; r + apart < s.dst_h && fits; r++) {  // ratios just above 1 or just above 1/4: walk the rows
+                    const int last = std::max(std::min(loc_of(r) + ksz - 1, yhi), ylo);
+                    const int first = std::max(std::min(loc_of(r + apart), yhi), ylo);
+                    fits = first > last;
+                }
+            if (apart == 8) far = far || !fits;
+            else {
+                down = fits;
+                if (fits) s.plan[1] = RMX_TRI_FOUR;
             }
-            for (int r = 0; r + apart < s.dst_h && down; r++) {  // ratios just above 1 or just above 1/4: walk the rows
-                const int last = std::max(std::min(loc_of(r) + ksz - 1, yhi), ylo);
-                const int first = std::max(std::min(loc_of(r + apart), yhi), ylo);
-                down = first > last;
-            }
-            if (down && apart == 4) s.plan[1] = RMX_TRI_FOUR;
         }
         int rows = op->ctx->tri_rows > 0 ? op->ctx->tri_rows : 12;
         bool sort_rows = false;
@@ -1212,18 +1218,26 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         // at the same byte phase (row stride a multiple of 4), and four LDS rows of the widest tile plus the table of vertical
         // coefficients must leave room for ten wavefronts per CU at least.
         op->tri_rows_in_flight = 0;
+        // Two kernels of this form. rmx_resize_tri_dma_kernel (columns 64 apart): rows that all start at the same byte phase (row strides
+        // multiples of 4), ratios for which two, four or eight rows in flight do. rmx_resize_tri_adj_kernel (neighbouring columns per
+        // lane): rows at any phase, any ratio; not rows of one pixel, of which no lane has two. Where both could, two rows in flight
+        // stay with the first and everything else goes to the second (figures there).
         bool tdma = down && op->ctx->dma && op->ctx->tri_tpx == 2 && ky <= 16;
-        if (flight > 4 && (!tdma || op->ctx->tri_slots == 4)) down = tdma = false;  // (only the streaming form has eight)
-        if (tdma) {
-            if (op->layout.empty()) tdma = (op->src.w * 3u) % 4u == 0;
-            else
-                for (int i = 0; i < op->n && tdma; i++) tdma = op->layout[i].row_stride % 4u == 0;
-        }
-        if (tdma) {
+        bool adj = tdma && op->ctx->tri_adj && op->ctx->tri_slots != 4 && (uint64_t)op->dst.h * op->dst.w * 3 * dtype_size(op->dst.dtype) < (1ull << 32);
+        for (int i = 0; i < op->n && adj; i++) adj = t[i].dst_w != 1;
+        bool one_phase = true;
+        if (op->layout.empty()) one_phase = (op->src.w * 3u) % 4u == 0;
+        else
+            for (int i = 0; i < op->n; i++) {
+                one_phase = one_phase && op->layout[i].row_stride % 4u == 0;
+                adj = adj && (uint64_t)op->layout[i].row_stride * op->layout[i].rows < (1ull << 32);
+            }
+        tdma = tdma && one_phase && !far && !(flight > 4 && op->ctx->tri_slots == 4);
+        if (tdma || adj) {
             // The widest LDS row over all tiles, by the kernel's own fp32 law for a tile's first and last tap (its byte phase
             // inside a dword is taken at its worst, 3).
             size_t pitch_max = 64;
-            for (int i = 0; i < op->n && tdma; i++) {
+            for (int i = 0; i < op->n && (tdma || adj); i++) {
                 const RmxSample &s = t[i];
                 if (s.dst_w <= 0 || s.dst_h <= 0) continue;
                 const float radius = s.rx > 1.0f ? s.rx : 1.0f;
@@ -1245,14 +1259,15 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
                     const int lm = ((3 * nrep_l + 15) >> 4) << 4;
                     const int body = std::max(3 + 3 * (ll + 8 - cs) + 8, 16 * nd);
                     const int pitch = lm + (((body + 15) >> 4) << 4);
-                    if (pitch > 128 * 16 || 3 * (nrep_l + nrep_r) > 64) tdma = false;
+                    if (pitch > 128 * 16 || 3 * (nrep_l + nrep_r) > 64) tdma = adj = false;
                     pitch_max = std::max(pitch_max, (size_t)pitch);
                 }
             }
             // ring of four source rows (six were measured: 18 instead of 20 wavefronts per CU, a fifth slower) + vertical
-            // coefficients: 64 source rows and 16 passes x 4 slots
-            const size_t lds = 4 * pitch_max + (64 + 16) * (size_t)flight * 4;
-            if (lds > 16 * 1024) tdma = false;
+            // coefficients: 64 source rows and 16 passes x the sets
+            if (4 * pitch_max + (64 + 16) * (size_t)flight * 4 > 16 * 1024) tdma = false;
+            if (4 * pitch_max + (64 + 16) * (size_t)2 * 4 > 16 * 1024) adj = false;
+            bool two = false;
             if (tdma) {
                 // Two output rows in flight instead of four when rows two apart never read the same source row. That holds
                 // for a vertical ratio that is a whole or a half number: every product and sum of the kernel's coordinate
@@ -1260,7 +1275,7 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
                 // 2 x ratio = taps rows apart, and only the clamp at the window's ends could fold two such rows onto one
                 // source row: when row 2 starts at or above the first source row, or the taps of the last row but two
                 // reach the last one.
-                bool two = op->ctx->tri_slots != 4 && flight == 4;
+                two = op->ctx->tri_slots != 4 && flight == 4;
                 for (int i = 0; i < op->n && two; i++) {
                     const RmxSample &s = t[i];
                     if (s.dst_w <= 0 || s.dst_h <= 2) continue;
@@ -1281,12 +1296,21 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
                     };
                     two = loc_of(2) > ylo && loc_of((int)s.dst_h - 3) + ksz - 1 < yhi;
                 }
-                op->tri_rows_in_flight = two ? 2 : flight;
-                op->fn = rmx::select_resize_tri_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, op->tri_rows_in_flight, &op->kernel_name);
-                op->lds_per_wave = (int)lds;
+                op->fn = rmx::select_resize_tri_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, two ? 2 : flight, &op->kernel_name);
+                op->lds_per_wave = (int)(4 * pitch_max + (64 + 16) * (size_t)flight * 4);
             }
+            adj = adj && !two;
+            if (adj) {
+                op->fn = rmx::select_resize_tri_adj_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, !one_phase);
+                // (such batches keep the name of the kernel that takes them without this form, which the plan tells apart)
+                op->kernel_name = tdma ? "rmx_resize_tri_dma_kernel" : flight == 4 ? "rmx_resize_tri_down_kernel" : "rmx_resize_tri_kernel";
+                op->lds_per_wave = (int)(4 * pitch_max + (64 + 16) * (size_t)2 * 4);
+            }
+            op->tri_rows_in_flight = !tdma && !adj ? 0 : two ? 2 : flight;
         }
-        if (!tdma && flight > 4) down = false;  // (the kernel that stages through registers keeps four rows in flight)
+        op->tri_adjacent = adj;
+        tdma = tdma || adj;
+        if (!tdma && (flight > 4 || far)) down = false;  // (the kernel that stages through registers keeps four rows in flight)
         if (down && !tdma) {
             tile_w = 64 * op->ctx->tri_tpx;
             op->fn = rmx::select_resize_tri_down_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, op->ctx->tri_tpx, &op->kernel_name);
@@ -1323,7 +1347,7 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
             if (op->ctx->tri_rows == 0) {
                 // (wavefronts per CU: 16 by the registers of the kernel that stages through registers, 20 by those of the streaming
                 // one, 24 when it keeps two rows in flight)
-                const int by_regs = tdma ? (op->tri_rows_in_flight == 2 ? 24 : (op->tri_rows_in_flight == 8 ? 16 : 20)) : 16;
+                const int by_regs = tdma ? (op->tri_rows_in_flight == 2 ? 24 : (op->tri_rows_in_flight == 8 && !adj ? 16 : 20)) : 16;
                 const int per_cu = op->ctx->tri_per_cu > 0 ? op->ctx->tri_per_cu : std::max(1, std::min(by_regs, (160 * 1024) / op->lds_per_wave));
                 const long slots = (long)op->ctx->num_cus * per_cu;
                 // Such a batch is only spread evenly over the device when there are several strips per wavefront slot for the

@@ -1,0 +1,6 @@
+// K2t streaming path, lanes that own neighbouring columns, source rows at any byte phase (see rmx_kernels_tri_adj_impl.h).
+#include "rmx_kernels_tri_adj_impl.h"
+
+namespace rmx {
+RMX_TADJ_UNIT(RMX_NCHW, true, tadj_unit_nchw_any)
+}  // namespace rmx

@@ -1,0 +1,6 @@
+// K2t streaming path, lanes that own neighbouring columns, source rows that start at one byte phase (see rmx_kernels_tri_adj_impl.h).
+#include "rmx_kernels_tri_adj_impl.h"
+
+namespace rmx {
+RMX_TADJ_UNIT(RMX_NHWC, false, tadj_unit_nhwc)
+}  // namespace rmx

@@ -21,4 +21,16 @@ KernelFn select_resize_tri_dma_kernel(int dtype, int layout, bool norm, bool qua
     return planar ? tdma_unit_4_nchw(dtype, norm, quant) : tdma_unit_4_nhwc(dtype, norm, quant);
 }
 
+KernelFn tadj_unit_nchw(int dtype, bool norm, bool quant);
+KernelFn tadj_unit_nhwc(int dtype, bool norm, bool quant);
+KernelFn tadj_unit_nchw_any(int dtype, bool norm, bool quant);
+KernelFn tadj_unit_nhwc_any(int dtype, bool norm, bool quant);
+
+// The instances of rmx_resize_tri_adj_kernel (rmx_kernels_tri_adj_impl.h); any_phase: source rows that do not all start at one byte phase
+KernelFn select_resize_tri_adj_kernel(int dtype, int layout, bool norm, bool quant, bool any_phase) {
+    const bool planar = layout == RMX_NCHW;
+    if (any_phase) return planar ? tadj_unit_nchw_any(dtype, norm, quant) : tadj_unit_nhwc_any(dtype, norm, quant);
+    return planar ? tadj_unit_nchw(dtype, norm, quant) : tadj_unit_nhwc(dtype, norm, quant);
+}
+
 }  // namespace rmx
