@@ -91,7 +91,7 @@ struct rmx_ctx {
     // Launch-plan tunables (rows per wavefront strip, LDS budget of the resize fast path). Defaults are the
     // values measured best on MI355X; RMX_TUNE_* environment variables, read once when the context is
     // created and clamped to safe ranges, override them for sweeps. They change plans, never results.
-    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, tri_adj = 1, warp_passes = 2, warp_wpb = 4;
+    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, dma_split = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, tri_adj = 1, warp_passes = 2, warp_wpb = 4;
 };
 
 static int tune_env(const char *name, int def, int lo, int hi) {
@@ -568,6 +568,7 @@ int rmx_ctx_create(int device, void *stream, int own_stream, rmx_ctx **out) {
         ctx->upload_kernel = tune_env("RMX_TUNE_UPLOAD_KERNEL", ctx->upload_kernel, 0, 1);
         ctx->dma = tune_env("RMX_TUNE_DMA", ctx->dma, 0, 1);  // 0: resizes of whole groups use the form for any byte phase, all others the general kernel; the triangular kernel stages through registers, the warp kernel uses its form for any byte phase
         ctx->dma_lds = tune_env("RMX_TUNE_DMA_LDS", ctx->dma_lds, 2048, 32 * 1024) & ~15;  // LDS window of a wavefront
+        ctx->dma_split = tune_env("RMX_TUNE_DMA_SPLIT", ctx->dma_split, 0, 1);  // 0: a wavefront always works through all x-tiles of its window
         ctx->dma_group = tune_env("RMX_TUNE_DMA_GROUP", ctx->dma_group, 0, 16);  // windows per wavefront, 0: chosen per batch
         ctx->flat_frames = tune_env("RMX_TUNE_FLAT_FRAMES", ctx->flat_frames, 0, 1);  // 0: point operations always walk the images' own rows
         ctx->tri_wpb = tune_env("RMX_TUNE_TRI_WPB", ctx->tri_wpb, 1, 4);
@@ -646,10 +647,10 @@ const char *rmx_op_plan(const rmx_op *op) {
                        (long long)op->n * op->strips, op->strips, op->aux0, 0, op->waves_per_block, op->fn_fast ? 1 : 0, op->flat_h);
     else if (op->fn_fast)
         len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=1 group=%d",
-                       (long long)op->n * op->fast_strips, op->fast_strips, op->fast_rows, op->fast_lds, op->fast_wpb, std::max(1, op->fast_aux1));
+                       (long long)op->n * op->fast_strips, op->fast_strips, op->fast_rows, op->fast_lds, op->fast_wpb, std::max(1, op->fast_aux1 & 0xffff));
     else if (op->fn_mid)
         len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d lds_per_wave=%d waves_per_block=%d fast=0 any_width=1 group=%d",
-                       (long long)op->n * op->mid_strips, op->mid_strips, op->mid_rows, op->mid_lds, op->mid_wpb, std::max(1, op->mid_aux1));
+                       (long long)op->n * op->mid_strips, op->mid_strips, op->mid_rows, op->mid_lds, op->mid_wpb, std::max(1, op->mid_aux1 & 0xffff));
     else {
         len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d tile_w=%d lds_per_wave=%d waves_per_block=%d fast=0",
                        (long long)op->n * op->strips, op->strips, op->strip_rows, op->tile_w, op->lds_per_wave, op->waves_per_block);
@@ -1472,7 +1473,7 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
     // whole at 3 and 2 per window: 31.8 and 34.4 against 32.2).
     const int seam = (op->dst.dtype == RMX_FP32 && op->dst.layout == RMX_NCHW && !chain) ? 2 : 0;
     const TileCost tile_cost(rows, seam);
-    int need_max = 64;
+    int need_max = 64, most_tiles = 1, all_tiles = 0;
     for (int i = 0; i < op->n && ok; i++) {
         RmxSample &s = t[i];
         s.plan[1] = 8;
@@ -1487,6 +1488,11 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         }, &need);
         if (tw == 0) ok = false;
         s.plan[1] = tw;
+        if (tw > 0) {
+            const int tiles = ((int)s.dst_w + tw - 1) / tw;
+            most_tiles = std::max(most_tiles, tiles);
+            all_tiles += tiles;
+        }
         need_max = std::max<int>(need_max, (int)need);
     }
     // fp32 output: room for the slab through which the lanes of a row exchange their runs before storing (the dwords of one lane's run
@@ -1506,21 +1512,33 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
     op->fast_lds = slice_fast;
     op->mid_lds = slice_mid;
     op->mid_rows = op->fast_rows = rows;
-    op->mid_strips = op->fast_strips = std::max(1, (max_dh + rows * group - 1) / (rows * group));
+    const int ystrips = std::max(1, (max_dh + rows * group - 1) / (rows * group));
+    // A wavefront that works through the x-tiles of a window waits for every tile's source pixels anew. A batch whose windows leave
+    // wavefront slots of the chip idle gives the tiles to 2^split wavefronts, as long as all of them are there at once (16 per CU); one
+    // that shrinks much, whose windows are cut into many narrow tiles, up to four times as many. Whole batches, one wavefront per window / split:
+    // 2 frames to 390 x 235 interleaved fp32 22.7 -> 8.5 us, 7 to 396 x 339 planes 13.4 -> 8.5, 8 to 1000 x 600 fp16 19.5 -> 15.7; beyond 16 per
+    // CU 20 frames to 960 x 540 (15 tiles) 42.0 -> 37.5, but 40 RandomResizedCrops to 299 x 299 (3 tiles) 12.7 -> 13.7.
+    const long most_waves = (all_tiles >= 6 * op->n ? 64L : 16L) * op->ctx->num_cus;
+    int split = 0;
+    while (op->ctx->dma_split && (1 << split) < most_tiles && ((long)op->n * ystrips << (split + 1)) <= most_waves) split++;
+    op->mid_strips = op->fast_strips = ystrips << split;
     // (default 1: a workgroup's LDS is released only when its last wavefront ends, one-wave groups keep the CU full)
     op->mid_wpb = op->fast_wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, widest)));
-    op->mid_aux1 = op->fast_aux1 = group;
+    op->mid_aux1 = op->fast_aux1 = group | split << 16;
     if (nearest) {
         op->fn_mid = rmx::select_resize_near_kernel(op->dst.dtype, op->dst.layout, op->norm, &op->mid_name);
-        return RMX_OK;
-    }
-    if (one_phase) {
+    } else if (one_phase) {
         op->fn_mid = rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, false, &op->mid_name);
         if (widths8) op->fn_fast = rmx::select_resize_dma_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &op->fast_name);
     } else if (op->ctx->dma) {
         op->fn_mid = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, false, &op->mid_name);
     }
-    if (widths8 && !op->fn_fast) op->fn_fast = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &op->fast_name);
+    if (!nearest && widths8 && !op->fn_fast) op->fn_fast = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &op->fast_name);
+    if (split) {  // (they keep the names of the kernels whose form they are)
+        const rmx::KernelFn shared = rmx::select_resize_split_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, nearest);
+        if (op->fn_mid) op->fn_mid = shared;
+        if (op->fn_fast) op->fn_fast = shared;
+    }
     return RMX_OK;
 }
 

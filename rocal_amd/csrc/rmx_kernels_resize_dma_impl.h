@@ -10,6 +10,7 @@
 //            dword, which is two instructions more per pixel. The kernel for rows at one phase (rmx_resize_dma_kernel) keeps the
 //            masks out of the loop.
 //   NEAREST  one source row per destination row, so only rows that are read are loaded.
+//   SPLIT    several wavefronts share the x-tiles of a window (rmx_kernels_resize_split.hip).
 //
 // One wavefront = a strip of destination rows of one sample, one x-tile at a time. It loads the whole source window of the strip's
 // rows, with all loads in flight together, and the window travels from global memory straight into LDS
@@ -82,7 +83,7 @@ struct DmaTile {
 // ALIGNED: every written width is a multiple of 8 and the destination base is 16-byte aligned (whole groups, packed 16-byte
 // stores, stores held back); otherwise any width and any base: groups are stored at the alignment of an element, and only a
 // tile narrower than 8 pixels has a partial group, stored element by element.
-template <typename T, int LAYOUT, bool NORM, bool QUANT, int CHAIN, bool ALIGNED, bool PHASED, bool NEAREST>
+template <typename T, int LAYOUT, bool NORM, bool QUANT, int CHAIN, bool ALIGNED, bool PHASED, bool NEAREST, bool SPLIT = false>
 RMX_DEV void resize_stream(const RmxKArgs &a) {
     static_assert(CHAIN == CHAIN_NONE || QUANT, "a colour node in the chain reads the u8 output of the resize node");
     static_assert(CHAIN == CHAIN_NONE || !NEAREST, "a colour node in the chain follows a bilinear resize node");
@@ -110,9 +111,11 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
 
     const int dw = P.dst_w, dh = P.dst_h;
     const int wrows = a.aux0;                        // destination rows of one window
-    const int r_begin = grp * wrows * max(a.aux1, 1);  // this wavefront: max(aux1, 1) windows below each other
+    // This wavefront: `group` windows below each other, of them (SPLIT) every 2^split-th x-tile from `part` on
+    const int group = max(SPLIT ? a.aux1 & 0xffff : a.aux1, 1), split = SPLIT ? a.aux1 >> 16 : 0, part = SPLIT ? grp & ((1 << split) - 1) : 0;
+    const int r_begin = (SPLIT ? grp >> split : grp) * wrows * group;
     if (r_begin >= dh || dw <= 0) return;
-    const int r_end = min(r_begin + wrows * max(a.aux1, 1), dh);
+    const int r_end = min(r_begin + wrows * group, dh);
     const bool hf = (P.flags & RMX_S_HFLIP) != 0;
 
     const int xlo = P.src_x, ylo = P.src_y;
@@ -155,6 +158,7 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
 
     const int tile_w = max(P.plan[1], PX);  // never 0: it is the step of the tile loop
     const int ntx = tile_w >= dw ? 1 : (dw + tile_w - 1) >> (31 - __builtin_clz(tile_w));  // (a tile is the whole row or a power of two wide)
+    if (SPLIT && part >= ntx) return;
 
     // ---- geometry of an x-tile and of a window of it (all wave-uniform)
     // nearest: the index of the pixel whose centre is closest, clamped into the window
@@ -298,8 +302,8 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
     // wait): three planes are three instructions; an interleaved run is contiguous and the compiler merges its stores up to
     // 16 bytes each: 48 bytes of fp16 are three, 24 bytes of u8 two. tests/test_dma_waitcnt_cpu.py checks the generated code.
     constexpr int DEFERRED = (LAYOUT == RMX_NHWC && sizeof(T) == 1) ? 2 : 3;
-    int tile = 0, r0 = r_begin;
-    DmaTile g = tile_geom(0);
+    int tile = part, r0 = r_begin;
+    DmaTile g = tile_geom(tile);
     int a_v = issue(g, r0, min(r0 + wrows, r_end));
     taps(g);  // while the loads are in flight
     bool held = false;
@@ -423,7 +427,7 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
         int nr0 = r0 + wrows, ntile = tile;
         if (nr0 >= r_end) {
             nr0 = r_begin;
-            ntile = tile + 1;
+            ntile = tile + (1 << split);
         }
         const bool more = ntile < ntx;
         DmaTile ng = g;

@@ -18,6 +18,7 @@ KernelFn select_resize_dma_kernel(int dtype, int layout, bool norm, bool quant, 
 // flight disturb less, 32.5 / 31.3.
 constexpr bool resize_exchanges(bool fp32, bool planes, bool aligned, bool twist) { return fp32 && (!planes || aligned || twist); }
 KernelFn select_resize_near_kernel(int dtype, int layout, bool norm, const char **name);
+KernelFn select_resize_split_kernel(int dtype, int layout, bool norm, bool quant, int chain, bool nearest);
 KernelFn select_resize_nearest_kernel(int dtype, int layout, bool norm, bool quant, const char **name);
 KernelFn select_resize_tri_kernel(int dtype, int layout, bool norm, bool quant, const char **name);
 KernelFn select_resize_tri_down_kernel(int dtype, int layout, bool norm, bool quant, int columns_per_lane, const char **name);

@@ -1,0 +1,47 @@
+"""Resizes whose x-tiles are dealt to several wavefronts (small batches): the same bits as with one wavefront per window, and as the oracle.
+Widths at the edges of tiles and of groups, samples of one tile beside samples of many (whose other wavefronts have nothing to do),
+mirrors, windows up to the last byte of the buffer."""
+import numpy as np
+import pytest
+
+from oracle import orc
+from rocal_amd import ops, workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("layout,dtype", [(ops.NCHW, ops.FP16), (ops.NHWC, ops.FP16), (ops.NCHW, ops.FP32), (ops.NHWC, ops.FP32), (ops.NHWC, ops.UINT8)])
+@pytest.mark.parametrize("W,OW,interp", [(700, 256, ops.LINEAR), (701, 299, ops.LINEAR), (700, 263, ops.LINEAR), (501, 131, ops.LINEAR), (701, 513, ops.NEAREST)])
+def test_tiles_of_a_window_in_several_wavefronts(layout, dtype, W, OW, interp):
+    import torch
+    from conftest import _ctx_with_env
+    rng = np.random.default_rng(W + OW + dtype)
+    n, H, OH = 3, 90, 23
+    img = wl.smooth_noise(rng, n, H, W, sigma=1.0)
+    roi = np.array([[0, 0, W, H], [3, 1, W - 3, H - 1], [W - 60, H - 30, 60, 30]], np.uint32)
+    dw, dh = np.array([OW, OW - 8, 40], np.uint32), np.array([OH, OH - 1, 9], np.uint32)
+    mirror = np.array([0, 1, 1], np.uint32)
+    norm = dtype != ops.UINT8
+    s, b = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
+    kw = dict(scale=s if norm else None, bias=b if norm else None)
+    exp = orc.resize(img, roi, dw, dh, OH, OW, interp=interp, mirror=mirror, layout=layout, dtype=dtype, **kw)
+    src = torch.from_numpy(img.reshape(-1).copy()).cuda().view(n, H, W, 3)
+    got = []
+    for split in (0, 1):
+        c = _ctx_with_env(RMX_TUNE_DMA_SPLIT=split)
+        op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, layout, dtype), interp)
+        if norm:
+            op.update_cmn(roi, dw, dh, s, b, mirror)
+        else:
+            op.update(roi, dw, dh, mirror)
+        waves = int(op.plan.split("waves=")[1].split()[0])
+        assert waves == n * 6 if not split else waves > n * 6, op.plan
+        out = op.alloc_output(fill=3)
+        op.launch(src, out)
+        c.sync()
+        got.append(out.cpu().numpy())
+        c.close()
+    assert np.array_equal(got[0].view(np.uint8), got[1].view(np.uint8))
+    for i in range(n):
+        g, e = (got[1][i][:, :dh[i], :dw[i]], exp[i][:, :dh[i], :dw[i]]) if layout == ops.NCHW else (got[1][i][:dh[i], :dw[i]], exp[i][:dh[i], :dw[i]])
+        assert np.array_equal(np.ascontiguousarray(g).view(np.uint8), np.ascontiguousarray(e).view(np.uint8)), (i, op.plan)
