@@ -91,7 +91,7 @@ struct rmx_ctx {
     // Launch-plan tunables (rows per wavefront strip, LDS budget of the resize fast path). Defaults are the
     // values measured best on MI355X; RMX_TUNE_* environment variables, read once when the context is
     // created and clamped to safe ranges, override them for sweeps. They change plans, never results.
-    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, dma_split = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, tri_adj = 1, warp_passes = 2, warp_wpb = 4;
+    int k1_rows = 4, k1_flat_rows = 0, k3_rows = 8, k3_flat_rows = 0, tri_rows = 0, gen_rows = 8, fast_rows = 4, fast_wpb = 1, dma = 1, dma_lds = 10 * 1024, dma_group = 1, dma_split = 1, flat_frames = 1, deal_xcd = 1, tri_wpb = 1, tri_ring = 0, tri_tpx = 2, tri_slots = 0, tri_per_cu = 0, tri_sort = 1, tri_adj = 1, warp_passes = 2, warp_wpb = 4, warp_together = 1;
 };
 
 static int tune_env(const char *name, int def, int lo, int hi) {
@@ -147,6 +147,8 @@ struct rmx_op {
     // a destination base off 16-byte alignment), before the general kernel
     rmx::KernelFn fn_mid = nullptr;
     const char *mid_name = "";
+    int warp_rows = 0;      // warps: how rows leave (RMX_WARP_*), where the destination's address allows it
+    bool warp_raw = false;  // warps: the form for source rows at one byte phase
     int mid_lds = 0, mid_strips = 1, mid_rows = 4, mid_wpb = 1, mid_aux1 = 1;
     uint64_t algo_bytes = 0;
     bool tri_adjacent = false;   // streaming triangular kernel whose lanes own neighbouring columns
@@ -573,6 +575,7 @@ int rmx_ctx_create(int device, void *stream, int own_stream, rmx_ctx **out) {
         ctx->flat_frames = tune_env("RMX_TUNE_FLAT_FRAMES", ctx->flat_frames, 0, 1);  // 0: point operations always walk the images' own rows
         ctx->tri_wpb = tune_env("RMX_TUNE_TRI_WPB", ctx->tri_wpb, 1, 4);
         ctx->warp_passes = tune_env("RMX_TUNE_WARP_PASSES", ctx->warp_passes, 1, 8);
+        ctx->warp_together = tune_env("RMX_TUNE_WARP_TOGETHER", ctx->warp_together, 0, 2);  // 0: the lanes of a warp store their own groups; 2: rows leave together in bilinear batches of any size
         ctx->warp_wpb = tune_env("RMX_TUNE_WARP_WPB", ctx->warp_wpb, 1, 4);
         ctx->tri_ring = tune_env("RMX_TUNE_TRI_RING", ctx->tri_ring, 0, 1);  // 1: always the ring kernel
         ctx->tri_tpx = tune_env("RMX_TUNE_TRI_TPX", ctx->tri_tpx, 1, 2);     // output columns per lane of the downscaling kernel
@@ -745,6 +748,13 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
     const int static_lds = static_lds_of(op, fn);
     if (static_lds < 0) return RMX_ERR_HIP;
     while (wpb > 1 && (size_t)a.lds_bytes * wpb + (size_t)static_lds > (size_t)op->ctx->max_lds_per_block) wpb--;
+    // Warps whose rows leave together: by teams where these write whole cache lines, else by tiles, else as the lanes have them
+    if (op->warp_rows) {
+        int how = op->warp_rows;
+        if (how == rmx::RMX_WARP_TEAMS && (wpb != rmx::kWarpTeam || (((uintptr_t)dst) & 127u))) how = rmx::RMX_WARP_TILES;
+        if (how == rmx::RMX_WARP_TILES && op->interp != RMX_INTERP_NEAREST && (((uintptr_t)dst) & 15u)) how = rmx::RMX_WARP_LANES;
+        if (how != rmx::RMX_WARP_LANES) fn = rmx::select_warp_rows_kernel(op->interp, op->warp_raw, how);
+    }
     const size_t lds = (size_t)a.lds_bytes * wpb;
     if (lds + (size_t)static_lds > (size_t)op->ctx->max_lds_per_block)
         return fail(RMX_ERR_INVALID, "plan needs %zu + %d bytes of LDS per workgroup (limit %d)", lds, static_lds, op->ctx->max_lds_per_block);
@@ -1981,6 +1991,19 @@ static int update_warp(rmx_op *op, const uint32_t *roi, const float *affine, con
     op->strips = tiles_x * tiles_y;
     op->aux0 = tiles_x;
     op->aux1 = passes << 8;  // passes of 16 rows per tile
+    // Interleaved bytes: rows leave by tiles, or by teams of four where every row is whole cache lines. Bilinear rows at other than 16-byte
+    // places keep the lanes' own stores: pieces across such places cost what they gain (226 turned images 410 wide 72.4 -> 72.0 us, 64 of 299
+    // 15.1 -> 15.4, but the nearest pixel of 249 images 426 wide 70.2 -> 63.2), and so do bilinear batches of less than two rounds of wavefronts,
+    // whose last stores come later for it (40 images of 200 x 240 8.3 -> 8.7; 200 of 377 x 400 61.6 -> 60.4, 128 of 512 x 512 62.0 -> 59.8).
+    op->warp_raw = raw;
+    op->warp_rows = rmx::RMX_WARP_LANES;
+    if (op->ctx->warp_together && op->dst.dtype == RMX_UINT8 && op->dst.layout == RMX_NHWC && passes == 2 && op->lds_per_wave >= rmx::kWarpTileBytes) {
+        const bool nearest = op->interp == RMX_INTERP_NEAREST;
+        const bool rounds = op->ctx->warp_together == 2 || (long)op->n * op->strips >= 2L * 20 * op->ctx->num_cus;  // (20 wavefronts per CU)
+        if (!nearest && !rounds) op->warp_rows = rmx::RMX_WARP_LANES;
+        else if (op->dst.w % 128 == 0 && tiles_x % rmx::kWarpTeam == 0) op->warp_rows = rmx::RMX_WARP_TEAMS;
+        else if (nearest || op->dst.w % 16 == 0) op->warp_rows = rmx::RMX_WARP_TILES;
+    }
     return commit_slot(op, slot);
 }
 

@@ -22,6 +22,11 @@
 //          is masked by itself (two instructions per pixel). Against staging through registers with one dword per pixel (111 registers,
 //          13 KB): 64 rotations of 299 x 299, bytes, with the wide stores below, 18.4 -> 15.1 us per batch. Rows at one phase keep RAW:
 //          its loop has the masks' two instructions less, of 58.
+// Interleaved bytes leave by whole rows of a tile, or of four tiles side by side (ROWS): stored by each lane as they
+// came, 24 bytes in two pieces, every cache line was written by up to six instructions with part of it each, and that, not the bytes, made loads
+// and stores wait for one another (nearest pixel, 128 images of 512 x 512, in a trace: 60 us, without stores 38, without loads 36). 128 images
+// of 512 x 512, whole batches: nearest pixel 57.3 -> 48.6 us by tiles -> 44.5 by four tiles as streaming stores (these cost the stores of
+// single lanes 8 us: part of a line at a time, they go to memory before their neighbours come); bilinear 61.2 - 64.3 -> 58.5 - 61.6.
 // Bound by how many wavefronts are there to compute while others wait for their box: 128 images of 512 x 512 take 61 - 63 us; without the
 // box's loads 47, without the stores 52, without both 42, with taps that meet no bank conflict the same; the bytes are 36 at the rate of
 // a large copy. The LDS slice therefore holds the box and nothing besides: no pixel of margin (the corners bound it exactly), the
@@ -43,7 +48,17 @@ namespace rmx {
 extern __shared__ uint32_t rmx_lds_warp[];
 typedef __attribute__((address_space(3))) uint32_t lds_u32;  // explicit LDS pointers: 32-bit address arithmetic
 
+typedef uint32_t u32x2_l __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_l __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));  // (global memory takes any address)
+typedef __attribute__((address_space(3))) u32x2_l lds_u32x2;
+typedef __attribute__((address_space(3))) u32x4_l lds_u32x4_l;
+
 constexpr int WRP = kWarpRawPieces;
+constexpr int WTEAM = kWarpTeam;                 // tiles side by side whose wavefronts store their rows together
+constexpr int WROW = WTW * 3;                    // bytes of a tile's row, u8
+constexpr int WTILE_BYTES = 2 * WTH * WROW;      // of a tile of two passes
+static_assert(WTILE_BYTES == kWarpTileBytes, "the host gives a slice room for a tile");
 
 RMX_DEV uint32_t load_px_global(const uint8_t *p) {
     return (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16);
@@ -56,8 +71,8 @@ RMX_DEV int floor_i32(float x) {
     return r;
 }
 
-template <typename T, int LAYOUT, bool NEAREST, bool RAW>
-__global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
+template <typename T, int LAYOUT, bool NEAREST, bool RAW, int ROWS>
+RMX_DEV void warp_body(const RmxKArgs &a) {
     const int lane = threadIdx.x & (RMX_WAVE - 1);
     const int wib = threadIdx.x / RMX_WAVE;
     const uint32_t nwaves = (uint32_t)a.n * (uint32_t)a.strips;
@@ -94,6 +109,13 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     const int ppr = box.ppr, pitch_b = box.pitch_b, ph = box.ph, total = box.total;
     const bool empty = box.empty, all_in = box.all_in;
 
+    // ROWS: a tile's groups wait in registers until both its passes are done, change places through the slice, and rows leave as 16-byte
+    // pieces that lie one behind the other in memory (a tile of fewer than 32 columns keeps the lanes' own stores); RMX_WARP_TEAMS: the
+    // rows of the workgroup's four tiles side by side, 128 pixels, whole cache lines, as streaming stores.
+    const bool together = ROWS != RMX_WARP_LANES && dw - X0 >= WTW;
+    // (the same in all wavefronts of the workgroup: none of them leaves early then, and all reach the barrier)
+    const bool team = ROWS == RMX_WARP_TEAMS && dw - (X0 - wib * WTW) >= WTEAM * WTW;
+    [[maybe_unused]] PackedGroup<T> upper, lower;
     const int lr = lane >> 2, g = lane & 3;
     int x0 = X0 + g * PX;
     // The short last group of a row moves left until it is whole (its pixels belong to this tile): it recomputes pixels of the group
@@ -102,7 +124,12 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
     const int cnt = min(PX, dw - x0);
     // Whole groups leave as wide stores at the alignment of an element (the same instructions as for aligned rows).
     auto store = [&](int y, const float (&v)[3][PX]) {
-        if (cnt == PX) {
+        if (ROWS != RMX_WARP_LANES && together) {
+            PackedGroup<T> packed;
+            pack_group_dir<T, LAYOUT, false>(v, packed);
+            if (y < Y0 + WTH) upper = packed;
+            else lower = packed;
+        } else if (cnt == PX) {
             PackedGroup<T> packed;
             pack_group_dir<T, LAYOUT, false>(v, packed);
             store_packed<T, LAYOUT, RMX_WARP_NT, true>(dimg, a.dst_h, a.dst_w, y, x0, packed);
@@ -111,6 +138,39 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
         }
     };
     const float xr0 = (float)x0 - dcx;
+    lds_u8 *ldsb = (lds_u8 *)(lds_ptr_t)rmx_lds_warp + (uint32_t)to_sgpr((int)((uint32_t)wib * (uint32_t)a.lds_bytes));
+    auto leave = [&]() {
+        if constexpr (ROWS != RMX_WARP_LANES) {
+            if (!together) return;
+            wave_sync();  // (the box has been read for the last time)
+            lds_u8 *mine = ldsb + lr * WROW + g * (PX * 3);
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                *(lds_u32x2 *)(mine + 8 * k) = (u32x2_l){upper.w[2 * k], upper.w[2 * k + 1]};
+                *(lds_u32x2 *)(mine + WTH * WROW + 8 * k) = (u32x2_l){lower.w[2 * k], lower.w[2 * k + 1]};
+            }
+            uint8_t *out = reinterpret_cast<uint8_t *>(dimg) + ((size_t)Y0 * a.dst_w + X0) * 3;
+            constexpr int NK = WTILE_BYTES / 16 / RMX_WAVE, PCS = WROW / 16;  // pieces of a lane, of a tile's row
+            if (ROWS == RMX_WARP_TEAMS && team) {
+                __syncthreads();
+                out -= wib * WROW;
+#pragma unroll
+                for (int k = 0; k < NK; k++) {
+                    const int idx = (wib * NK + k) * RMX_WAVE + lane, row = idx / (WTEAM * PCS), c = idx - row * (WTEAM * PCS), t = c / PCS;
+                    const u32x4_l v = *(lds_u32x4_l *)((lds_u8 *)(lds_ptr_t)rmx_lds_warp + t * a.lds_bytes + row * WROW + (c - t * PCS) * 16);
+                    if (Y0 + row < dh) __builtin_nontemporal_store(u32x4_b(v), reinterpret_cast<u32x4_b *>(out + (uint32_t)(row * a.dst_w * 3 + c * 16)));
+                }
+                return;
+            }
+            wave_sync();
+#pragma unroll
+            for (int k = 0; k < NK; k++) {
+                const int idx = k * RMX_WAVE + lane, row = idx / PCS;
+                const u32x4_l v = *(lds_u32x4_l *)(ldsb + 16 * idx);
+                if (Y0 + row < dh) *reinterpret_cast<u32x4_b *>(out + (uint32_t)(row * a.dst_w * 3 + (idx - row * PCS) * 16)) = v;
+            }
+        }
+    };
 
     if (empty) {
         // every pixel of the tile maps outside the ROI: the fill value
@@ -123,7 +183,7 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             const int y = Y0 + pass * WTH + lr;
             if (y < dh && cnt > 0) store(y, z);
         }
-        return;
+        return leave();
     }
     if (!box.use_lds) {
         // a box too large for the slice: per-pixel gathers from global memory
@@ -169,10 +229,9 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
             }
             store(y, v);
         }
-        return;
+        return leave();
     }
 
-    lds_u8 *ldsb = (lds_u8 *)(lds_ptr_t)rmx_lds_warp + (uint32_t)to_sgpr((int)((uint32_t)wib * (uint32_t)a.lds_bytes));
     const uint8_t *base4 = simg - skew;
     // ---- the box straight into LDS: piece idx lands at byte 16 idx of the slice
     const uint64_t left = (uint64_t)(buf_end - base4);
@@ -353,11 +412,20 @@ __global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
         if (all_in) gather(std::false_type{}, fix);
         else gather(std::true_type{}, fix);
     };
-    if constexpr (RAW) {
-        if (ppr == WRP) return run(std::integral_constant<int, WRP>{});
-        if (ppr == WRP + 1) return run(std::integral_constant<int, WRP + 1>{});
-    }
-    run(std::integral_constant<int, 0>{});
+    if (RAW && ppr == WRP) run(std::integral_constant<int, RAW ? WRP : 0>{});
+    else if (RAW && ppr == WRP + 1) run(std::integral_constant<int, RAW ? WRP + 1 : 0>{});
+    else run(std::integral_constant<int, 0>{});
+    leave();
+}
+
+template <typename T, int LAYOUT, bool NEAREST, bool RAW>
+__global__ void __launch_bounds__(256) rmx_warp_kernel(RmxKArgs a) {
+    warp_body<T, LAYOUT, NEAREST, RAW, RMX_WARP_LANES>(a);
+}
+
+template <bool NEAREST, bool RAW, int ROWS>
+__global__ void __launch_bounds__(256) rmx_warp_rows_kernel(RmxKArgs a) {
+    warp_body<uint8_t, RMX_NHWC, NEAREST, RAW, ROWS>(a);
 }
 
 template <bool NEAREST, bool RAW>
@@ -381,6 +449,16 @@ KernelFn select_warp_kernel(int interp, int dtype, int layout, bool raw, const c
     *name = raw ? "rmx_warp_kernel(raw)" : "rmx_warp_kernel";
     if (raw) return interp == RMX_INTERP_NEAREST ? pick<true, true>(dtype, layout) : pick<false, true>(dtype, layout);
     return interp == RMX_INTERP_NEAREST ? pick<true, false>(dtype, layout) : pick<false, false>(dtype, layout);
+}
+
+template <bool NEAREST, bool RAW>
+static KernelFn pick_rows(int rows) {
+    return rows == RMX_WARP_TEAMS ? (KernelFn)rmx_warp_rows_kernel<NEAREST, RAW, RMX_WARP_TEAMS> : (KernelFn)rmx_warp_rows_kernel<NEAREST, RAW, RMX_WARP_TILES>;
+}
+
+KernelFn select_warp_rows_kernel(int interp, bool raw, int rows) {
+    if (raw) return interp == RMX_INTERP_NEAREST ? pick_rows<true, true>(rows) : pick_rows<false, true>(rows);
+    return interp == RMX_INTERP_NEAREST ? pick_rows<true, false>(rows) : pick_rows<false, false>(rows);
 }
 
 }  // namespace rmx

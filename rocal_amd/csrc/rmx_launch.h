@@ -28,6 +28,10 @@ KernelFn select_color_kernel(int kind, int dtype, int layout, int mode, const ch
 KernelFn select_point_kernel(int kind, int dtype, int layout, int mode, const char **name);
 KernelFn select_transpose_kernel(int dtype, int layout, const char **name);
 KernelFn select_warp_kernel(int interp, int dtype, int layout, bool raw, const char **name);
+// Warps to interleaved bytes: how rows leave (see warp_body, rmx_kernels_warp.hip)
+enum { RMX_WARP_LANES = 0, RMX_WARP_TILES = 1, RMX_WARP_TEAMS = 2 };
+constexpr int kWarpTeam = 4, kWarpTileBytes = 32 * 32 * 3;  // tiles of a team; bytes of a tile's rows, of which a wavefront's slice must have room
+KernelFn select_warp_rows_kernel(int interp, bool raw, int rows);
 // Normalize: integer moments of every sample's window, 1 << log2_parts shares of six 64-bit numbers per sample, each made by a workgroup
 // of `threads` (whole wavefronts, at most 512)
 void launch_moments(hipStream_t stream, const RmxKArgs &a, unsigned long long *parts, int log2_parts, int threads);
