@@ -575,7 +575,7 @@ int rmx_ctx_create(int device, void *stream, int own_stream, rmx_ctx **out) {
         ctx->flat_frames = tune_env("RMX_TUNE_FLAT_FRAMES", ctx->flat_frames, 0, 1);  // 0: point operations always walk the images' own rows
         ctx->tri_wpb = tune_env("RMX_TUNE_TRI_WPB", ctx->tri_wpb, 1, 4);
         ctx->warp_passes = tune_env("RMX_TUNE_WARP_PASSES", ctx->warp_passes, 1, 8);
-        ctx->warp_together = tune_env("RMX_TUNE_WARP_TOGETHER", ctx->warp_together, 0, 2);  // 0: the lanes of a warp store their own groups; 2: rows leave together in bilinear batches of any size
+        ctx->warp_together = tune_env("RMX_TUNE_WARP_TOGETHER", ctx->warp_together, 0, 2);  // 0: the lanes of a warp store their own groups; 2: rows leave together in batches of any size
         ctx->warp_wpb = tune_env("RMX_TUNE_WARP_WPB", ctx->warp_wpb, 1, 4);
         ctx->tri_ring = tune_env("RMX_TUNE_TRI_RING", ctx->tri_ring, 0, 1);  // 1: always the ring kernel
         ctx->tri_tpx = tune_env("RMX_TUNE_TRI_TPX", ctx->tri_tpx, 1, 2);     // output columns per lane of the downscaling kernel
@@ -1524,11 +1524,13 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
     op->mid_rows = op->fast_rows = rows;
     const int ystrips = std::max(1, (max_dh + rows * group - 1) / (rows * group));
     // A wavefront that works through the x-tiles of a window waits for every tile's source pixels anew. A batch whose windows leave
-    // wavefront slots of the chip idle gives the tiles to 2^split wavefronts, as long as all of them are there at once (16 per CU); one
+    // wavefront slots of the chip idle gives the tiles to 2^split wavefronts, as long as all of them are there at once (16 per CU by registers); one
     // that shrinks much, whose windows are cut into many narrow tiles, up to four times as many. Whole batches, one wavefront per window / split:
     // 2 frames to 390 x 235 interleaved fp32 22.7 -> 8.5 us, 7 to 396 x 339 planes 13.4 -> 8.5, 8 to 1000 x 600 fp16 19.5 -> 15.7; beyond 16 per
     // CU 20 frames to 960 x 540 (15 tiles) 42.0 -> 37.5, but 40 RandomResizedCrops to 299 x 299 (3 tiles) 12.7 -> 13.7.
-    const long most_waves = (all_tiles >= 6 * op->n ? 64L : 16L) * op->ctx->num_cus;
+    // Kernels with an exchange are bound by their stores sooner, and tiles cut rows into shorter runs: half as many (interleaved fp32 at
+    // 299 x 299, 13 windows split in two 11.4 -> 11.3, 21 windows 13.6 -> 15.8).
+    const long most_waves = (slice_mid > slice ? 8L : 16L) * (all_tiles >= 6 * op->n ? 4 : 1) * op->ctx->num_cus;
     int split = 0;
     while (op->ctx->dma_split && (1 << split) < most_tiles && ((long)op->n * ystrips << (split + 1)) <= most_waves) split++;
     op->mid_strips = op->fast_strips = ystrips << split;
@@ -1993,16 +1995,15 @@ static int update_warp(rmx_op *op, const uint32_t *roi, const float *affine, con
     op->aux1 = passes << 8;  // passes of 16 rows per tile
     // Interleaved bytes: rows leave by tiles, or by teams of four where every row is whole cache lines. Bilinear rows at other than 16-byte
     // places keep the lanes' own stores: pieces across such places cost what they gain (226 turned images 410 wide 72.4 -> 72.0 us, 64 of 299
-    // 15.1 -> 15.4, but the nearest pixel of 249 images 426 wide 70.2 -> 63.2), and so do bilinear batches of less than two rounds of wavefronts,
-    // whose last stores come later for it (40 images of 200 x 240 8.3 -> 8.7; 200 of 377 x 400 61.6 -> 60.4, 128 of 512 x 512 62.0 -> 59.8).
+    // 15.1 -> 15.4, but the nearest pixel of 249 images 426 wide 70.2 -> 63.2), and so do batches of less than two rounds of wavefronts, whose last
+    // stores come later for it (bilinear, 40 images of 200 x 240 8.3 -> 8.7; nearest, 112 of 483 x 109 11.8 -> 12.5; but 200 of 377 x 400 61.6 -> 60.4).
     op->warp_raw = raw;
     op->warp_rows = rmx::RMX_WARP_LANES;
     if (op->ctx->warp_together && op->dst.dtype == RMX_UINT8 && op->dst.layout == RMX_NHWC && passes == 2 && op->lds_per_wave >= rmx::kWarpTileBytes) {
-        const bool nearest = op->interp == RMX_INTERP_NEAREST;
         const bool rounds = op->ctx->warp_together == 2 || (long)op->n * op->strips >= 2L * 20 * op->ctx->num_cus;  // (20 wavefronts per CU)
-        if (!nearest && !rounds) op->warp_rows = rmx::RMX_WARP_LANES;
+        if (!rounds) op->warp_rows = rmx::RMX_WARP_LANES;
         else if (op->dst.w % 128 == 0 && tiles_x % rmx::kWarpTeam == 0) op->warp_rows = rmx::RMX_WARP_TEAMS;
-        else if (nearest || op->dst.w % 16 == 0) op->warp_rows = rmx::RMX_WARP_TILES;
+        else if (op->interp == RMX_INTERP_NEAREST || op->dst.w % 16 == 0) op->warp_rows = rmx::RMX_WARP_TILES;
     }
     return commit_slot(op, slot);
 }

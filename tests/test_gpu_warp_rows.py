@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(scope="module")
 def ctx_together():
-    """(bilinear rows leave together in large batches only, unless told)"""
+    """(rows leave together in large batches only, unless told)"""
     from conftest import _ctx_with_env
     c = _ctx_with_env(RMX_TUNE_WARP_TOGETHER=2)
     yield c
