@@ -256,6 +256,9 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
         }
         return a_v;
     };
+    // Nearest bytes to interleaved bytes: nothing is computed, a pixel's three bytes go from the dword they are read into to their places in
+    // the run. The taps of a mirrored row are made in the order of the destination.
+    constexpr bool BYTES = NEAREST && !NORM && sizeof(T) == 1 && LAYOUT == RMX_NHWC;
     // A lane's x taps in a tile: byte offset of the left neighbour inside an LDS row (dword part and byte phase; PHASED: the whole
     // offset, less the row's phase), weights
     uint32_t bo4[PX], bsh[PX];
@@ -280,7 +283,8 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
 #pragma unroll
         for (int k = 0; k < PX; k++) {
             // (pixels behind a partial group repeat the tile's last column: their taps stay inside the window, they are not stored)
-            const int col = ALIGNED ? t0 + k : min(t0 + k, last);
+            const int kk = BYTES && hf ? PX - 1 - k : k;
+            const int col = ALIGNED ? t0 + kk : min(t0 + kk, last);
             const float sx = src_coord_d(pcx + col, rx, offx, fxlo);
             const float fx = floorf(sx);
             wx[k] = sx - fx;
@@ -343,18 +347,31 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
                 float v[3][PX];
                 if constexpr (NEAREST) {
                     // (a pixel is three bytes at any phase: two dwords)
+                    [[maybe_unused]] uint32_t bytes[PX];
                     const uint32_t rowb = (uint32_t)(uintptr_t)(bufb + (r - a_v) * pitch_b) + (PHASED ? row_phase(g, near_of(src_coord_d(pcy + r, ry, offy, fylo), ylo, yhi)) : 0u);
 #pragma unroll
                     for (int k = 0; k < PX; k++) {
                         const uint32_t adr = rowb + bo4[k];
                         const lds_u32 *q = (const lds_u32 *)(PHASED ? adr & ~3u : adr);
                         const uint32_t px = __builtin_amdgcn_alignbyte(q[1], q[0], PHASED ? adr : bsh[k]);
+                        if constexpr (BYTES) {
+                            bytes[k] = px;
+                            continue;
+                        }
                         v[0][k] = ubyte0(px);
                         v[1][k] = ubyte1(px);
                         v[2][k] = ubyte2(px);
                         if constexpr (NORM) {
 #pragma unroll
                             for (int c = 0; c < 3; c++) v[c][k] = __builtin_fmaf(v[c][k], sc[c], bi[c]);
+                        }
+                    }
+                    if constexpr (BYTES) {
+#pragma unroll
+                        for (int j = 0; j < PX / 4; j++) {
+                            packed.w[3 * j] = __builtin_amdgcn_perm(bytes[4 * j + 1], bytes[4 * j], 0x04020100u);
+                            packed.w[3 * j + 1] = __builtin_amdgcn_perm(bytes[4 * j + 2], bytes[4 * j + 1], 0x05040201u);
+                            packed.w[3 * j + 2] = __builtin_amdgcn_perm(bytes[4 * j + 3], bytes[4 * j + 2], 0x06050402u);
                         }
                     }
                 } else {
@@ -399,7 +416,7 @@ RMX_DEV void resize_stream(const RmxKArgs &a) {
                         v[0][k] = o0; v[1][k] = o1; v[2][k] = o2;
                     }
                 }
-                pack_group<T, LAYOUT>(v, hf, packed);
+                if constexpr (!BYTES) pack_group<T, LAYOUT>(v, hf, packed);
                 if constexpr (!ALIGNED) {  // (a destination narrower than 8 pixels: element by element, at once)
                     full = cnt == PX;
                     if (!full) store_packed_part<T, LAYOUT>(dimg, a.dst_h, a.dst_w, r, x0, hf ? PX - cnt : 0, cnt, packed);
