@@ -27,6 +27,7 @@
 // and stores wait for one another (nearest pixel, 128 images of 512 x 512, in a trace: 60 us, without stores 38, without loads 36). 128 images
 // of 512 x 512, whole batches: nearest pixel 57.3 -> 48.6 us by tiles -> 44.5 by four tiles as streaming stores (these cost the stores of
 // single lanes 8 us: part of a line at a time, they go to memory before their neighbours come); bilinear 61.2 - 64.3 -> 58.5 - 61.6.
+// The nearest pixel's bytes are moved, not converted to float and back (BYTES): 43.8 -> 43.1, 86 turned images of 151 x 447 10.7 -> 10.2.
 // Bound by how many wavefronts are there to compute while others wait for their box: 128 images of 512 x 512 take 61 - 63 us; without the
 // box's loads 47, without the stores 52, without both 42, with taps that meet no bank conflict the same; the bytes are 36 at the rate of
 // a large copy. The LDS slice therefore holds the box and nothing besides: no pixel of margin (the corners bound it exactly), the
@@ -123,19 +124,37 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
     if (x0 < dw) x0 = max(min(x0, dw - PX), X0);
     const int cnt = min(PX, dw - x0);
     // Whole groups leave as wide stores at the alignment of an element (the same instructions as for aligned rows).
-    auto store = [&](int y, const float (&v)[3][PX]) {
+    auto store_run = [&](int y, const PackedGroup<T> &packed) {
         if (ROWS != RMX_WARP_LANES && together) {
-            PackedGroup<T> packed;
-            pack_group_dir<T, LAYOUT, false>(v, packed);
             if (y < Y0 + WTH) upper = packed;
             else lower = packed;
-        } else if (cnt == PX) {
+        } else {
+            store_packed<T, LAYOUT, RMX_WARP_NT, true>(dimg, a.dst_h, a.dst_w, y, x0, packed);
+        }
+    };
+    auto store = [&](int y, const float (&v)[3][PX]) {
+        if ((ROWS != RMX_WARP_LANES && together) || cnt == PX) {
             PackedGroup<T> packed;
             pack_group_dir<T, LAYOUT, false>(v, packed);
-            store_packed<T, LAYOUT, RMX_WARP_NT, true>(dimg, a.dst_h, a.dst_w, y, x0, packed);
+            store_run(y, packed);
         } else {
             store_group<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, cnt, v, false);
         }
+    };
+    // Nearest bytes to interleaved bytes are moved, not converted: a pixel in the low three bytes of each dword
+    constexpr bool BYTES = NEAREST && sizeof(T) == 1 && LAYOUT == RMX_NHWC;
+    auto store_bytes = [&](int y, const uint32_t (&px)[PX]) {
+        PackedGroup<T> packed;
+        if constexpr (BYTES) {
+#pragma unroll
+            for (int k = 0; k < PX / 4; k++) {
+                packed.w[3 * k] = __builtin_amdgcn_perm(px[4 * k + 1], px[4 * k], 0x04020100u);
+                packed.w[3 * k + 1] = __builtin_amdgcn_perm(px[4 * k + 2], px[4 * k + 1], 0x05040201u);
+                packed.w[3 * k + 2] = __builtin_amdgcn_perm(px[4 * k + 3], px[4 * k + 2], 0x06050402u);
+            }
+        }
+        if (cnt == PX) store_run(y, packed);
+        else store_packed_part<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, 0, cnt, packed);
     };
     const float xr0 = (float)x0 - dcx;
     lds_u8 *ldsb = (lds_u8 *)(lds_ptr_t)rmx_lds_warp + (uint32_t)to_sgpr((int)((uint32_t)wib * (uint32_t)a.lds_bytes));
@@ -294,6 +313,7 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
             const float yr = (float)y - dcy;
             const float cxy = __builtin_fmaf(yr, m1, m2), cyy = __builtin_fmaf(yr, m4, m5);
             float v[3][PX];
+            [[maybe_unused]] uint32_t bytes[PX];
             // A pixel in two steps: fetch (coordinates, tap address, the LDS reads of its taps) and blend. The reads of pixel
             // k + 1 are issued before pixel k is blended, so that a wavefront waits for LDS once per row instead of once per
             // pixel (left to the compiler's order, every pixel's reads were followed at once by the wait for them): 65.6 -> 64.1 us
@@ -373,6 +393,10 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
                 float o0, o1, o2;
                 if constexpr (NEAREST) {
                     const uint32_t tl = __builtin_amdgcn_alignbyte(t.tr, t.tl, t.tph);
+                    if constexpr (BYTES) {
+                        bytes[k] = t.inb ? tl : 0u;
+                        return;
+                    }
                     o0 = ubyte0(tl); o1 = ubyte1(tl); o2 = ubyte2(tl);
                 } else {
                     // s - floor(s): exact for the non-negative coordinates of pixels inside the ROI
@@ -405,7 +429,8 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
                 blend(k, cur);
                 cur = nxt;
             }
-            store(y, v);
+            if constexpr (BYTES) store_bytes(y, bytes);
+            else store(y, v);
         }
     };
     auto run = [&](auto fix) {
