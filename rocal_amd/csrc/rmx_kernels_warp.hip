@@ -25,9 +25,9 @@
 // Interleaved bytes leave by whole rows of a tile, or of four tiles side by side (ROWS): stored by each lane as they
 // came, 24 bytes in two pieces, every cache line was written by up to six instructions with part of it each, and that, not the bytes, made loads
 // and stores wait for one another (nearest pixel, 128 images of 512 x 512, in a trace: 60 us, without stores 38, without loads 36). 128 images
-// of 512 x 512, whole batches: nearest pixel 57.3 -> 48.6 us by tiles -> 44.5 by four tiles as streaming stores (these cost the stores of
-// single lanes 8 us: part of a line at a time, they go to memory before their neighbours come); bilinear 61.2 - 64.3 -> 58.5 - 61.6.
-// The nearest pixel's bytes are moved, not converted to float and back (BYTES): 43.8 -> 43.1, 86 turned images of 151 x 447 10.7 -> 10.2.
+// of 512 x 512, whole batches: nearest pixel 57.3 -> 48.6 us by tiles -> 43.4 by four tiles as streaming stores (these cost the stores of
+// single lanes 8 us: part of a line at a time, they go to memory before their neighbours come); bilinear 63.4 -> 61.0.
+// The nearest pixel's bytes are moved, not converted to float and back (BYTES): 43.4 -> 42.7, 86 turned images of 151 x 447 10.7 -> 10.2.
 // Bound by how many wavefronts are there to compute while others wait for their box: 128 images of 512 x 512 take 61 - 63 us; without the
 // box's loads 47, without the stores 52, without both 42, with taps that meet no bank conflict the same; the bytes are 36 at the rate of
 // a large copy. The LDS slice therefore holds the box and nothing besides: no pixel of margin (the corners bound it exactly), the
@@ -124,26 +124,26 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
     if (x0 < dw) x0 = max(min(x0, dw - PX), X0);
     const int cnt = min(PX, dw - x0);
     // Whole groups leave as wide stores at the alignment of an element (the same instructions as for aligned rows).
-    auto store_run = [&](int y, const PackedGroup<T> &packed) {
+    auto store_run = [&](int pass, int y, const PackedGroup<T> &packed) {
         if (ROWS != RMX_WARP_LANES && together) {
-            if (y < Y0 + WTH) upper = packed;
+            if (pass == 0) upper = packed;
             else lower = packed;
         } else {
             store_packed<T, LAYOUT, RMX_WARP_NT, true>(dimg, a.dst_h, a.dst_w, y, x0, packed);
         }
     };
-    auto store = [&](int y, const float (&v)[3][PX]) {
+    auto store = [&](int pass, int y, const float (&v)[3][PX]) {
         if ((ROWS != RMX_WARP_LANES && together) || cnt == PX) {
             PackedGroup<T> packed;
             pack_group_dir<T, LAYOUT, false>(v, packed);
-            store_run(y, packed);
+            store_run(pass, y, packed);
         } else {
             store_group<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, cnt, v, false);
         }
     };
     // Nearest bytes to interleaved bytes are moved, not converted: a pixel in the low three bytes of each dword
     constexpr bool BYTES = NEAREST && sizeof(T) == 1 && LAYOUT == RMX_NHWC;
-    auto store_bytes = [&](int y, const uint32_t (&px)[PX]) {
+    auto store_bytes = [&](int pass, int y, const uint32_t (&px)[PX]) {
         PackedGroup<T> packed;
         if constexpr (BYTES) {
 #pragma unroll
@@ -153,7 +153,7 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
                 packed.w[3 * k + 2] = __builtin_amdgcn_perm(px[4 * k + 3], px[4 * k + 2], 0x06050402u);
             }
         }
-        if (cnt == PX) store_run(y, packed);
+        if (cnt == PX) store_run(pass, y, packed);
         else store_packed_part<T, LAYOUT>(dimg, a.dst_h, a.dst_w, y, x0, 0, cnt, packed);
     };
     const float xr0 = (float)x0 - dcx;
@@ -168,25 +168,33 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
                 *(lds_u32x2 *)(mine + 8 * k) = (u32x2_l){upper.w[2 * k], upper.w[2 * k + 1]};
                 *(lds_u32x2 *)(mine + WTH * WROW + 8 * k) = (u32x2_l){lower.w[2 * k], lower.w[2 * k + 1]};
             }
+            // (A team's lanes store the same piece of every second row, 48 of them, so that their places are made once: 62.4 -> 61.1 us; a
+            // tile's ten rows at a time, 60 lanes, gain nothing, 62.6 -> 63.3)
             uint8_t *out = reinterpret_cast<uint8_t *>(dimg) + ((size_t)Y0 * a.dst_w + X0) * 3;
-            constexpr int NK = WTILE_BYTES / 16 / RMX_WAVE, PCS = WROW / 16;  // pieces of a lane, of a tile's row
+            constexpr int PCS = WROW / 16;  // pieces of a tile's row
+            const uint32_t pitch = (uint32_t)a.dst_w * 3u;
             if (ROWS == RMX_WARP_TEAMS && team) {
                 __syncthreads();
+                constexpr int PCT = WTEAM * PCS, AT_ONCE = 2, PART = 2 * WTH / WTEAM;  // (a wavefront stores a quarter of the rows)
+                const int rr = lane >= PCT ? 1 : 0, c = lane - rr * PCT, t = c / PCS, row = wib * PART + rr;
+                const lds_u8 *from = (lds_u8 *)(lds_ptr_t)rmx_lds_warp + t * a.lds_bytes + row * WROW + (c - t * PCS) * 16;
+                const uint32_t to = (uint32_t)row * pitch + (uint32_t)c * 16u;
                 out -= wib * WROW;
+                if (lane < AT_ONCE * PCT) {
 #pragma unroll
-                for (int k = 0; k < NK; k++) {
-                    const int idx = (wib * NK + k) * RMX_WAVE + lane, row = idx / (WTEAM * PCS), c = idx - row * (WTEAM * PCS), t = c / PCS;
-                    const u32x4_l v = *(lds_u32x4_l *)((lds_u8 *)(lds_ptr_t)rmx_lds_warp + t * a.lds_bytes + row * WROW + (c - t * PCS) * 16);
-                    if (Y0 + row < dh) __builtin_nontemporal_store(u32x4_b(v), reinterpret_cast<u32x4_b *>(out + (uint32_t)(row * a.dst_w * 3 + c * 16)));
+                    for (int k = 0; k < PART / AT_ONCE; k++) {
+                        const u32x4_l v = *(const lds_u32x4_l *)(from + k * AT_ONCE * WROW);
+                        if (Y0 + row + k * AT_ONCE < dh) __builtin_nontemporal_store(u32x4_b(v), reinterpret_cast<u32x4_b *>(out + (size_t)(k * AT_ONCE) * pitch + to));
+                    }
                 }
                 return;
             }
             wave_sync();
 #pragma unroll
-            for (int k = 0; k < NK; k++) {
+            for (int k = 0; k < WTILE_BYTES / 16 / RMX_WAVE; k++) {
                 const int idx = k * RMX_WAVE + lane, row = idx / PCS;
-                const u32x4_l v = *(lds_u32x4_l *)(ldsb + 16 * idx);
-                if (Y0 + row < dh) *reinterpret_cast<u32x4_b *>(out + (uint32_t)(row * a.dst_w * 3 + (idx - row * PCS) * 16)) = v;
+                const u32x4_l v = *(const lds_u32x4_l *)(ldsb + 16 * idx);
+                if (Y0 + row < dh) *reinterpret_cast<u32x4_b *>(out + ((uint32_t)row * pitch + (uint32_t)(idx - row * PCS) * 16u)) = v;
             }
         }
     };
@@ -200,7 +208,7 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
             for (int k = 0; k < PX; k++) z[c][k] = 0.0f;
         for (int pass = 0; pass < passes; pass++) {
             const int y = Y0 + pass * WTH + lr;
-            if (y < dh && cnt > 0) store(y, z);
+            if (y < dh && cnt > 0) store(pass, y, z);
         }
         return leave();
     }
@@ -246,7 +254,7 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
                 }
                 v[0][k] = o0; v[1][k] = o1; v[2][k] = o2;
             }
-            store(y, v);
+            store(pass, y, v);
         }
         return leave();
     }
@@ -429,8 +437,8 @@ RMX_DEV void warp_body(const RmxKArgs &a) {
                 blend(k, cur);
                 cur = nxt;
             }
-            if constexpr (BYTES) store_bytes(y, bytes);
-            else store(y, v);
+            if constexpr (BYTES) store_bytes(pass, y, bytes);
+            else store(pass, y, v);
         }
     };
     auto run = [&](auto fix) {
