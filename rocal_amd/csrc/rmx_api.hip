@@ -1236,6 +1236,8 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         bool tdma = down && op->ctx->dma && op->ctx->tri_tpx == 2 && ky <= 16;
         bool adj = tdma && op->ctx->tri_adj && op->ctx->tri_slots != 4 && (uint64_t)op->dst.h * op->dst.w * 3 * dtype_size(op->dst.dtype) < (1ull << 32);
         for (int i = 0; i < op->n && adj; i++) adj = t[i].dst_w != 1;
+        // (two accumulator sets for every ratio rely on coordinates that are exact to half a row: fp32 is, below 2^20 rows)
+        adj = adj && op->src.h < (1u << 20);
         bool one_phase = true;
         if (op->layout.empty()) one_phase = (op->src.w * 3u) % 4u == 0;
         else

@@ -29,6 +29,16 @@ typedef __attribute__((address_space(3))) f32x2 lds_f32x2;
 
 constexpr int TS_GROW = 4;  // output rows made behind one another without going back, from two rows of a sample that grows
 
+// Six accumulators to h * c (c 0: to 0) when idx == M, the branch inside the statement as in zero_if. h is a sum of products that are not
+// negative: with c 0 this is +0.
+template <int M>
+RMX_DEV void start_over_if(int idx, float (&acc)[3][2], const float (&h)[3][2], float c) {
+    asm("s_cmp_lg_u32 %6, %7\n\ts_cbranch_scc1 .Lkeep%=\n\tv_mul_f32 %0, %8, %9\n\tv_mul_f32 %1, %8, %10\n\tv_mul_f32 %2, %8, %11\n\tv_mul_f32 %3, %8, %12\n\tv_mul_f32 %4, %8, %13\n\tv_mul_f32 %5, %8, %14\n.Lkeep%=:"
+        : "+&v"(acc[0][0]), "+&v"(acc[0][1]), "+&v"(acc[1][0]), "+&v"(acc[1][1]), "+&v"(acc[2][0]), "+&v"(acc[2][1])
+        : "s"(idx), "n"(M), "s"(c), "v"(h[0][0]), "v"(h[0][1]), "v"(h[1][0]), "v"(h[1][1]), "v"(h[2][0]), "v"(h[2][1])
+        : "scc");
+}
+
 template <int DWORDS>
 struct PairDwords {
     uint32_t w[2][DWORDS];
@@ -281,23 +291,23 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
     // coefficient other than 0. Whoever needs a row's entry fetches it from the lane that holds it.
     float rsum_v = 0.0f;
     int ylast_v = max(min(oloc_v + ky - 1, yhi), ylo);
-    bool twice = false;  // a source row enters more than two output rows of this strip
+    // Output row r + 2 takes the set of row r when that has been stored. Its source rows lie behind row r's, but for one that both may have:
+    // rounding can leave its first tap and row r's last one a coefficient other than 0 in one source row. Row r's is then in the
+    // table, and the other one, kept here by row r's lane, starts the set that row r leaves (see `run`).
+    float late_v = 0.0f;
     if (ky == 2) {
         rsum_v = rsum_v + tri_coeff(ow0_v, ay.radius, 0, ay.fscale) + tri_coeff(ow0_v, ay.radius, 1, ay.fscale);
     } else {
-        int ja = ky - 1, jb = 0;
+        int jb = 0;
         for (int j = 0; j < ky; j++) {
             const float c = tri_coeff(ow0_v, ay.radius, j, ay.fscale);
             rsum_v += c;
-            if (c > 0.0f) {
-                ja = min(ja, j);
-                jb = j;
-            }
+            if (c > 0.0f) jb = j;
         }
         ylast_v = max(min(oloc_v + jb, yhi), ylo);
-        const int yfirst_v = max(min(oloc_v + ja, yhi), ylo);
-        const int below = __builtin_amdgcn_ds_bpermute(4 * (lane + 2), yfirst_v);  // (of the output row two below)
-        twice = to_sgpr((int)(__builtin_amdgcn_ballot_w64(lane + 2 < r1 - r0 && below <= ylast_v) != 0)) != 0;
+        const int below = __builtin_amdgcn_ds_bpermute(4 * (lane + 2), oloc_v);  // (of the output row two below)
+        const float below_w0 = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (lane + 2), __builtin_bit_cast(int, ow0_v)));
+        if (lane + 2 < r1 - r0 && below <= ylast_v) late_v = tri_coeff(below_w0, ay.radius, 0, ay.fscale);
     }
     rsum_v = (rsum_v == 0.0f) ? 1.0f : rsum_v;
     auto last_tap_row = [&](int r) { return __builtin_amdgcn_readlane(ylast_v, r - r0); };
@@ -331,8 +341,8 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
     // ---- vertical coefficients by source row, a table of 64 rows x the two sets in the tail of the LDS slice: entry (l, k) is
     // the coefficient with which source row ytab + l enters the output row of set k (0: none; fma(h, 0, acc) == acc for
     // the finite h a filtered row is, so both sets take every row and no branch is needed). Lane r writes the taps of output row
-    // r0 + r, which no other row of its set shares a source row with; the filter loop reads a source row's entry with one
-    // broadcast read. Rebuilt every 64 source rows. The first and the last row of the window serve several taps of a row
+    // r0 + r, in their order: where a first tap's source row is the last one of the output row two above (late_v), that one stays; the
+    // filter loop reads a source row's entry with one broadcast read. Rebuilt every 64 source rows. The first and the last row of the window serve several taps of a row
     // each (clamped tap indices) and take their own path below.
     // (Written by source rows instead, lane l going through all the strip's output rows for row l's coefficients, the table
     // and the coefficients of the columns, made twice, were a third of the instructions in front of the row loop: 256 RandomResizedCrop windows to
@@ -340,7 +350,6 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
     lds_f32 *cftab = (lds_f32 *)(bufb + tab_off);
     const lds_f32x2 *cv_next = (const lds_f32x2 *)cftab;  // the table entry of the next source row
     int ytab = y_first;
-    int pairs = 0;  // `twice`: which pairs of output rows are in work, the even or the odd ones
     auto build_table = [&]() TS_INLINE {
         *(lds_f32x2 *)(cftab + 2 * lane) = f32x2{};
         wave_sync();
@@ -349,7 +358,7 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
         asm volatile("" : "+v"(loc), "+v"(w0), "+v"(row));  // (or the taps' coefficients and places would be kept in registers from one table to the next)
         const int l0 = loc - ytab;
         lds_f32 *mine = cftab + 2 * l0 + (row & 1);
-        const bool on = row < r1 - r0 && (!twice || ((row >> 1) & 1) == pairs);
+        const bool on = row < r1 - r0;
 #pragma unroll 1
         for (int j = 0; j < ky; j++) {
             const float c = tri_coeff(w0, ay.radius, j, ay.fscale);
@@ -392,13 +401,10 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
             }
         store_pair<T, LAYOUT>(reinterpret_cast<uint8_t *>(dimg), plane * sizeof(T), xoff + out_row, v);
     };
-    // From output row rq to the next one of those in work: all of the strip, or (`twice`) every second pair of them.
-    auto to_next = [&]() { return twice && (rsum_idx & 1) ? 3 : 1; };
     auto next_output_row = [&]() TS_INLINE {
-        const int d = to_next();
-        rq += d;
-        rsum_idx += d;
-        out_row += d * out_step;
+        rq++;
+        rsum_idx++;
+        out_row += out_step;
         emitted++;
         qlast = rq < r1 ? last_tap_row(rq) : 0x7fffffff;  // (behind the last row: no source row completes anything)
     };
@@ -467,9 +473,13 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
     };
 
     // ---- samples that shrink vertically. A source row has a coefficient other than 0 in two output rows, so two accumulator sets do:
-    // output row r accumulates in set (r - r0) & 1 until its last such row has been added. Where rounding gives a third output row a
-    // last or first coefficient that is not quite 0 (one strip in 400 of random ratios), the strip is done in two goes, the even pairs of
-    // its output rows and then the odd ones: rows four apart share no source row whatever their coefficients, the host has shown.
+    // output row r accumulates in set (r - r0) & 1 until its last such row has been added. Rounding can give that row to output row r + 2
+    // as well (late_v): the set then starts over from it instead of from 0. The rows two apart lie two radii apart, so no other row can be in both,
+    // and that one is neither the window's first nor its last (tests/test_tri_rows_cpu.py; the host keeps windows whose coordinates
+    // are no longer exact to half a row from this kernel). How many output rows are so is the ratio's doing: one strip in 400 of random
+    // ones, but half of them at 11 / 7. (Such strips done in two goes, the even pairs of their output rows and then the odd ones: 96 images
+    // of 550 x 550 to 350 x 350 fp16 69.2 us instead of 43.2, 192 of 476 x 476 to
+    // 140 x 140 94.8 instead of 55.5; with four accumulator sets 48.9 and 56.7.)
     auto run = [&](auto nt) TS_INLINE {
         float acc[2][3][TPX];
         // The row in work is source row yy: filter it and add it to the output rows in flight.
@@ -485,7 +495,7 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
                 int npass = 0;
 #pragma unroll
                 for (int m = 0; m < 2; m++) {
-                    const int r = (rsum_idx & 1) == m ? rq : rq + to_next();  // the row in flight that lives in set m
+                    const int r = (rsum_idx & 1) == m ? rq : rq + 1;  // the row in flight that lives in set m
                     ec[m] = 0.0f;
                     if (r < r1) {
                         const int loc = row_loc(r);
@@ -525,8 +535,9 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
                 row_sums();
                 if (rsum_idx & 1) emit(acc[1]);
                 else emit(acc[0]);
-                zero_if<0>(rsum_idx & 1, acc[0]);
-                zero_if<1>(rsum_idx & 1, acc[1]);
+                const float late = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, late_v), rsum_idx));
+                start_over_if<0>(rsum_idx & 1, acc[0], h, late);
+                start_over_if<1>(rsum_idx & 1, acc[1], h, late);
                 next_output_row();
             }
         };
@@ -536,41 +547,27 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
             for (int c = 0; c < 3; c++)
 #pragma unroll
                 for (int i = 0; i < TPX; i++) acc[m][c][i] = 0.0f;
-        for (;;) {
-            build_table();  // (under the round trip of the first loads)
-            for (int y = y_first; y <= y_last; y += TS_RPS) {
-                const int nr = min(TS_RPS, y_last - y + 1);
-                if (y + nr - ytab > RMX_WAVE) {
-                    ytab = y;
-                    cv_next = (const lds_f32x2 *)cftab;
-                    build_table();
-                }
-                step_in(y, nr);
-                auto row = fetch_row(nt, std::true_type{}, half_cur, rb_cur);
-                // Both rows' reads are started before the first row is filtered (the second row's slot holds a row also where
-                // the window ends with the first one) where the registers allow it.
-                constexpr bool AHEAD = decltype(nt)::value <= 4;
-                auto second = row;
-                if constexpr (AHEAD) second = fetch_row(nt, std::true_type{}, half_cur + pitch, rb_cur + row_stride);
-                process_row(row, y);
-                if (nr > 1) {
-                    if constexpr (!AHEAD) second = fetch_row(nt, std::true_type{}, half_cur + pitch, rb_cur + row_stride);
-                    process_row(second, y + 1);
-                }
-                step_out();
+        build_table();  // (under the round trip of the first loads)
+        for (int y = y_first; y <= y_last; y += TS_RPS) {
+            const int nr = min(TS_RPS, y_last - y + 1);
+            if (y + nr - ytab > RMX_WAVE) {
+                ytab = y;
+                cv_next = (const lds_f32x2 *)cftab;
+                build_table();
             }
-            if (!twice || pairs == 1 || r0 + 2 >= r1) break;
-            // once more for the odd pairs
-            pairs = 1;
-            ytab = y_next = y_first;
-            rb_next = rb_cur = (uint32_t)y_first * row_stride + colb;
-            cv_next = (const lds_f32x2 *)cftab;
-            out_row = (uint32_t)(r0 + 2) * out_step;
-            rq = r0 + 2;
-            rsum_idx = 2;
-            qlast = last_tap_row(rq);
-            emitted = 0;
-            by_lanes = issue(half_cur);
+            step_in(y, nr);
+            auto row = fetch_row(nt, std::true_type{}, half_cur, rb_cur);
+            // Both rows' reads are started before the first row is filtered (the second row's slot holds a row also where
+            // the window ends with the first one) where the registers allow it.
+            constexpr bool AHEAD = decltype(nt)::value <= 4;
+            auto second = row;
+            if constexpr (AHEAD) second = fetch_row(nt, std::true_type{}, half_cur + pitch, rb_cur + row_stride);
+            process_row(row, y);
+            if (nr > 1) {
+                if constexpr (!AHEAD) second = fetch_row(nt, std::true_type{}, half_cur + pitch, rb_cur + row_stride);
+                process_row(second, y + 1);
+            }
+            step_out();
         }
     };
 

@@ -1,7 +1,7 @@
 """The streaming triangular kernel whose lanes own neighbouring columns, bit for bit against the oracle, where it can go wrong: rows at every
 byte phase (padded and packed images), windows that grow by any ratio and those that shrink in one batch, clamped taps at all four
 edges, rows of two and three pixels, a last tile of one column, mirrors, crops behind the resize, strips of every length, and windows
-whose rounding gives a source row to three output rows (the strip is then done in two goes)."""
+whose rounding gives a source row to three output rows (the third starts its accumulators from it)."""
 import numpy as np
 import pytest
 
@@ -133,5 +133,29 @@ def test_source_rows_of_three_output_rows(rows):
     try:
         _check(c, img, roi, dw, dh, int(dh.max()), 55, ops.NCHW, ops.FP32, np.array([0, 1, 0, 1, 0], np.uint32))
         _check(c, img, roi, dw, dh, int(dh.max()), 55, ops.NHWC, ops.UINT8, np.array([1, 0, 0, 1, 0], np.uint32))
+    finally:
+        c.close()
+
+
+# ratios at which that happens every few rows: 11/7, 3.4
+OFTEN = [(550, 350, 0), (476, 140, 7), (352, 224, 200), (330, 210, 61), (352, 224, 0)]
+
+
+@pytest.mark.parametrize("rows", [0, 7, 64])
+@pytest.mark.parametrize("W,layout,dtype", [(140, ops.NCHW, ops.FP16), (141, ops.NCHW, ops.FP16), (141, ops.NHWC, ops.FP32), (140, ops.NHWC, ops.UINT8)])
+def test_ratios_whose_rows_meet_again_and_again(rows, W, layout, dtype):
+    """Strips in which many output rows start their accumulators from a source row that they share: 12 to 64 output rows of 2 to 4 source
+    rows each (the table of coefficients is made again on the way, also right at such rows), horizontal taps of every number."""
+    assert all(_third_rows(*t) > 2 for t in OFTEN)
+    from conftest import _ctx_with_env
+    c = _ctx_with_env(RMX_TUNE_TRI_ROWS=rows)
+    rng = np.random.default_rng(W + rows)
+    n, H = len(OFTEN), 560
+    img = rng.integers(0, 256, (n, H, W, 3), dtype=np.uint8)
+    roi = np.array([[i, y0, W - 3 - i, sh] for i, (sh, _, y0) in enumerate(OFTEN)], np.uint32)
+    dh = np.array([d for _, d, _ in OFTEN], np.uint32)
+    dw = np.array([130, 100, 70, 46, 36], np.uint32)
+    try:
+        _check(c, img, roi, dw, dh, int(dh.max()), 130, layout, dtype, np.array([0, 1, 0, 1, 0], np.uint32))
     finally:
         c.close()
