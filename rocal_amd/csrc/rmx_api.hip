@@ -1532,9 +1532,17 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
     // CU 20 frames to 960 x 540 (15 tiles) 42.0 -> 37.5, but 40 RandomResizedCrops to 299 x 299 (3 tiles) 12.7 -> 13.7.
     // Kernels with an exchange are bound by their stores sooner, and tiles cut rows into shorter runs: half as many (interleaved fp32 at
     // 299 x 299, 13 windows split in two 11.4 -> 11.3, 21 windows 13.6 -> 15.8).
-    const long most_waves = (slice_mid > slice ? 8L : 16L) * (all_tiles >= 6 * op->n ? 4 : 1) * op->ctx->num_cus;
+    // Wavefronts without a tile of their own have their price too: a batch whose windows have less than 1.5 x 2^(split-1) tiles on average splits up
+    // to 6 per CU only (27 windows of 1.4 tiles to 266 x 249 fp16, 3 618 wavefronts, 8.8 us unsplit, 10.7 split; 9 to 375 x 408 bytes, 1 692,
+    // 9.2 and 10.6; 5 to 339 x 519 interleaved fp32 15.2, 12.9 in two and 16.7 in four; but 17 to 98 x 103, 850, 7.2 and 4.9).
+    const long per_cu = slice_mid > slice ? 8 : 16;
     int split = 0;
-    while (op->ctx->dma_split && (1 << split) < most_tiles && ((long)op->n * ystrips << (split + 1)) <= most_waves) split++;
+    while (op->ctx->dma_split && (1 << split) < most_tiles) {
+        const bool ragged = 2L * all_tiles < (3L * op->n) << split;
+        const long most_waves = (ragged ? std::min(per_cu, 6L) : per_cu) * (all_tiles >= 6 * op->n ? 4 : 1) * op->ctx->num_cus;
+        if (((long)op->n * ystrips << (split + 1)) > most_waves) break;
+        split++;
+    }
     op->mid_strips = op->fast_strips = ystrips << split;
     // (default 1: a workgroup's LDS is released only when its last wavefront ends, one-wave groups keep the CU full)
     op->mid_wpb = op->fast_wpb = std::max(1, std::min(op->ctx->fast_wpb, (op->ctx->max_lds_per_block - kStaticLdsMax) / std::max(1, widest)));

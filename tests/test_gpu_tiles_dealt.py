@@ -45,3 +45,25 @@ def test_tiles_of_a_window_in_several_wavefronts(layout, dtype, W, OW, interp):
     for i in range(n):
         g, e = (got[1][i][:, :dh[i], :dw[i]], exp[i][:, :dh[i], :dw[i]]) if layout == ops.NCHW else (got[1][i][:dh[i], :dw[i]], exp[i][:dh[i], :dw[i]])
         assert np.array_equal(np.ascontiguousarray(g).view(np.uint8), np.ascontiguousarray(e).view(np.uint8)), (i, op.plan)
+
+
+@pytest.mark.parametrize("n,tiles,parts", [(27, 1, 1), (27, 2, 2), (5, 1, 2), (5, 2, 2)])
+def test_batches_of_mostly_one_tile(ctx, n, tiles, parts):
+    """Windows of one tile beside one window of two: dealt in small batches only, where their idle wavefronts cost less than the wait for the
+    second tile; whole batches of two tiles in larger ones too."""
+    import torch
+    rng = np.random.default_rng(n)
+    H, W, OH, OW = 300, 700, 266, 249
+    img = rng.integers(0, 256, (n, H, W, 3), dtype=np.uint8)
+    roi = np.tile(np.array([[0, 0, 200 if tiles == 1 else W, 200]], np.uint32), (n, 1))
+    roi[n - 1, 2] = W
+    dw, dh = np.full(n, OW, np.uint32), np.full(n, OH, np.uint32)
+    s, b = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
+    op = ops.Resize(ctx, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, ops.NCHW, ops.FP16), ops.LINEAR, flags=ops.F_QUANTIZE_U8)
+    op.update_cmn(roi, dw, dh, s, b, None)
+    assert int(op.plan.split("waves=")[1].split()[0]) == n * 67 * parts, op.plan
+    out = op.alloc_output()
+    op.launch(torch.from_numpy(img).cuda(), out)
+    ctx.sync()
+    exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.LINEAR, scale=s, bias=b, layout=orc.NCHW, dtype=orc.FP16, flags=orc.F_QUANTIZE_U8)
+    assert np.array_equal(out.cpu().numpy().view(np.uint8), exp.view(np.uint8)), op.plan
