@@ -104,7 +104,8 @@ RMX_API int rmx_op_set_ragged_source_strided(rmx_op *op, const uint64_t *offsets
 RMX_API uint64_t rmx_op_algorithmic_bytes(const rmx_op *op);
 /* Launch plan of the last update as text (waves, strips, LDS per wave ...), for logs and benchmarks. */
 RMX_API const char *rmx_op_plan(const rmx_op *op);
-/* Name of the kernel the op launches (as it appears in a rocprofv3 kernel trace). */
+/* Name of the kernel the op launches (as it appears in a rocprofv3 kernel trace) to a destination at a multiple of 128 bytes; some ops
+ * launch another one to other addresses. */
 RMX_API const char *rmx_op_kernel_name(const rmx_op *op);
 
 /* ---- CropMirrorNormalize: replaces vxExtRppCropMirrorNormalize

@@ -149,10 +149,11 @@ struct rmx_op {
     const char *mid_name = "";
     int warp_rows = 0;      // warps: how rows leave (RMX_WARP_*), where the destination's address allows it
     bool warp_raw = false;  // warps: the form for source rows at one byte phase
+    const char *warp_name = "";  // ... and the kernel whose lanes store their own groups
     int mid_lds = 0, mid_strips = 1, mid_rows = 4, mid_wpb = 1, mid_aux1 = 1;
     uint64_t algo_bytes = 0;
     bool tri_adjacent = false;   // streaming triangular kernel whose lanes own neighbouring columns
-    int tri_rows_in_flight = 0;  // streaming triangular kernel: accumulator sets (2, 4 or 8), 0 for every other kernel
+    int tri_rows_in_flight = 0;  // streaming triangular kernel whose columns lie 64 apart: accumulator sets (2, 4 or 8), 0 for every other kernel
     // Point operations on whole frames (every sample's window is the whole padded image, source and destination of one
     // shape): the kernel walks a frame as flat_h rows of 512 pixels, so that all 64 lanes work whatever the image width is
     // (224 pixels are 28 groups of 8: two rows per step keep 56 lanes busy; 299 pixels keep 38). 0: the images' own rows.
@@ -657,8 +658,13 @@ const char *rmx_op_plan(const rmx_op *op) {
     else {
         len = snprintf(buf, sizeof(buf), "waves=%lld strips=%d strip_rows=%d tile_w=%d lds_per_wave=%d waves_per_block=%d fast=0",
                        (long long)op->n * op->strips, op->strips, op->strip_rows, op->tile_w, op->lds_per_wave, op->waves_per_block);
-        if (op->tri_rows_in_flight) len += snprintf(buf + len, sizeof(buf) - len, " rows_in_flight=%d%s", op->tri_rows_in_flight, op->tri_adjacent ? " adjacent=1" : "");
+        if (op->tri_rows_in_flight) len += snprintf(buf + len, sizeof(buf) - len, " rows_in_flight=%d", op->tri_rows_in_flight);
+        if (op->tri_adjacent) len += snprintf(buf + len, sizeof(buf) - len, " adjacent=1");
+        if (op->kind == OP_WARP_AFFINE || op->kind == OP_ROTATE)  // (at a destination at a multiple of 128 bytes)
+            len += snprintf(buf + len, sizeof(buf) - len, " leave=%s", op->warp_rows == rmx::RMX_WARP_TEAMS ? "teams" : op->warp_rows == rmx::RMX_WARP_TILES ? "tiles" : "lanes");
     }
+    if (op->fn_mid || op->fn_fast)  // (wavefronts that share the x-tiles of a window)
+        if (const int split = (op->fn_fast ? op->fast_aux1 : op->mid_aux1) >> 16) len += snprintf(buf + len, sizeof(buf) - len, " split=%d", 1 << split);
     // (how the rows of the last update reach the kernel: dwords per sample in its arguments, or a table)
     if (op->updated && op->compact) len += snprintf(buf + len, sizeof(buf) - len, " rows=arguments words=%u", op->compact_words);
     else if (op->updated) len += snprintf(buf + len, sizeof(buf) - len, " rows=table");
@@ -743,6 +749,7 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
     }
     HIP_TRY(hipSetDevice(op->ctx->device));
     rmx::KernelFn fn = fast ? op->fn_fast : (mid ? op->fn_mid : op->fn);
+    const char *name = fast ? op->fast_name : (mid ? op->mid_name : op->kernel_name);
     // a workgroup's LDS = the wavefronts' dynamic slices + what the kernel declares statically (coalescing slabs, colour
     // tables): fewer wavefronts per workgroup when the sum would not fit
     const int static_lds = static_lds_of(op, fn);
@@ -754,6 +761,7 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
         if (how == rmx::RMX_WARP_TEAMS && (wpb != rmx::kWarpTeam || (((uintptr_t)dst) & 127u))) how = rmx::RMX_WARP_TILES;
         if (how == rmx::RMX_WARP_TILES && op->interp != RMX_INTERP_NEAREST && (((uintptr_t)dst) & 15u)) how = rmx::RMX_WARP_LANES;
         if (how != rmx::RMX_WARP_LANES) fn = rmx::select_warp_rows_kernel(op->interp, op->warp_raw, how);
+        else name = op->warp_name;
     }
     const size_t lds = (size_t)a.lds_bytes * wpb;
     if (lds + (size_t)static_lds > (size_t)op->ctx->max_lds_per_block)
@@ -782,7 +790,7 @@ static int launch_table(rmx_op *op, const RmxSample *table, const RmxSrcLayout *
     const hipError_t launched = hipLaunchKernel(reinterpret_cast<const void *>(fn), dim3((unsigned)blocks), dim3(wpb * RMX_WAVE), kargs, lds, op->ctx->stream);
     if (launched != hipSuccess) {
         (void)hipGetLastError();  // (told here; the thread's next check, here or in the caller's own code, is about its own call)
-        return fail(RMX_ERR_HIP, "launching %s failed: %d (%s)", rmx_op_kernel_name(op), (int)launched, hipGetErrorString(launched));
+        return fail(RMX_ERR_HIP, "launching %s failed: %d (%s)", name, (int)launched, hipGetErrorString(launched));
     }
     if (!op->captured) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -1315,11 +1323,10 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
             adj = adj && !two;
             if (adj) {
                 op->fn = rmx::select_resize_tri_adj_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, !one_phase);
-                // (such batches keep the name of the kernel that takes them without this form, which the plan tells apart)
-                op->kernel_name = tdma ? "rmx_resize_tri_dma_kernel" : flight == 4 ? "rmx_resize_tri_down_kernel" : "rmx_resize_tri_kernel";
+                op->kernel_name = "rmx_resize_tri_adj_kernel";
                 op->lds_per_wave = (int)(4 * pitch_max + (64 + 16) * (size_t)2 * 4);
             }
-            op->tri_rows_in_flight = !tdma && !adj ? 0 : two ? 2 : flight;
+            op->tri_rows_in_flight = !tdma || adj ? 0 : two ? 2 : flight;
         }
         op->tri_adjacent = adj;
         tdma = tdma || adj;
@@ -1360,7 +1367,7 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
             if (op->ctx->tri_rows == 0) {
                 // (wavefronts per CU: 16 by the registers of the kernel that stages through registers, 20 by those of the streaming
                 // one, 24 when it keeps two rows in flight)
-                const int by_regs = tdma ? (op->tri_rows_in_flight == 2 ? 24 : (op->tri_rows_in_flight == 8 && !adj ? 16 : 20)) : 16;
+                const int by_regs = tdma ? (op->tri_rows_in_flight == 2 ? 24 : (op->tri_rows_in_flight == 8 ? 16 : 20)) : 16;
                 const int per_cu = op->ctx->tri_per_cu > 0 ? op->ctx->tri_per_cu : std::max(1, std::min(by_regs, (160 * 1024) / op->lds_per_wave));
                 const long slots = (long)op->ctx->num_cus * per_cu;
                 // Such a batch is only spread evenly over the device when there are several strips per wavefront slot for the
@@ -1556,10 +1563,11 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         op->fn_mid = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, false, &op->mid_name);
     }
     if (!nearest && widths8 && !op->fn_fast) op->fn_fast = rmx::select_resize_fast_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, true, &op->fast_name);
-    if (split) {  // (they keep the names of the kernels whose form they are)
+    if (split) {
         const rmx::KernelFn shared = rmx::select_resize_split_kernel(op->dst.dtype, op->dst.layout, op->norm, op->quant, chain, nearest);
         if (op->fn_mid) op->fn_mid = shared;
         if (op->fn_fast) op->fn_fast = shared;
+        op->mid_name = op->fast_name = "rmx_resize_split_kernel";
     }
     return RMX_OK;
 }
@@ -1956,7 +1964,7 @@ static int update_warp(rmx_op *op, const uint32_t *roi, const float *affine, con
         else
             for (int i = 0; i < op->n && raw; i++) raw = op->layout[i].row_stride % 4u == 0;
     }
-    op->fn = rmx::select_warp_kernel(op->interp, op->dst.dtype, op->dst.layout, raw, &op->kernel_name);
+    op->fn = rmx::select_warp_kernel(op->interp, op->dst.dtype, op->dst.layout, raw, &op->warp_name);
     for (int i = 0; i < op->n; i++) {
         RmxSample &s = t[i];
         int rc = read_roi(op, roi, i, &s.src_x, &s.src_y, &s.src_w, &s.src_h);
@@ -2015,6 +2023,7 @@ static int update_warp(rmx_op *op, const uint32_t *roi, const float *affine, con
         else if (op->dst.w % 128 == 0 && tiles_x % rmx::kWarpTeam == 0) op->warp_rows = rmx::RMX_WARP_TEAMS;
         else if (op->interp == RMX_INTERP_NEAREST || op->dst.w % 16 == 0) op->warp_rows = rmx::RMX_WARP_TILES;
     }
+    op->kernel_name = op->warp_rows == rmx::RMX_WARP_LANES ? op->warp_name : raw ? "rmx_warp_rows_kernel(raw)" : "rmx_warp_rows_kernel";
     return commit_slot(op, slot);
 }
 

@@ -49,7 +49,23 @@ def ctx_staged():
 
 @pytest.fixture(scope="session")
 def ctx_dma_small():
-    """The streaming bilinear kernel with small LDS windows (rows are cut into several x-tiles)."""
+    """The streaming bilinear kernel with small LDS windows (rows are cut into several x-tiles, through which one wavefront works)."""
+    c = _ctx_with_env(RMX_TUNE_DMA_LDS=2560, RMX_TUNE_DMA_SPLIT=0)
+    yield c
+    c.sync()
+
+
+@pytest.fixture(scope="session")
+def ctx_dma_split():
+    """The same windows, their x-tiles dealt to several wavefronts where the batch is small."""
     c = _ctx_with_env(RMX_TUNE_DMA_LDS=2560)
+    yield c
+    c.sync()
+
+
+@pytest.fixture(scope="session")
+def ctx_undealt():
+    """Windows of the default size whose x-tiles one wavefront works through, in batches of any size."""
+    c = _ctx_with_env(RMX_TUNE_DMA_SPLIT=0)
     yield c
     c.sync()

@@ -15,7 +15,7 @@ COMBOS = [(ops.NCHW, ops.FP16), (ops.NCHW, ops.FP32), (ops.NCHW, ops.UINT8), (op
 @pytest.mark.parametrize("interp", [ops.LINEAR, ops.NEAREST])
 @pytest.mark.parametrize("W", [149, 150, 151, 152])
 @pytest.mark.parametrize("packed", [False, True])
-def test_rows_at_every_phase(ctx, ctx_dma_small, layout, dtype, interp, W, packed):
+def test_rows_at_every_phase(ctx, ctx_undealt, ctx_dma_small, ctx_dma_split, layout, dtype, interp, W, packed):
     import torch
     rng = np.random.default_rng(W * 100 + 10 * layout + dtype + (7 if packed else 0))
     n, H, OH, OW = 12, 90, 70, 140
@@ -47,7 +47,7 @@ def test_rows_at_every_phase(ctx, ctx_dma_small, layout, dtype, interp, W, packe
         offsets = np.cumsum(sizes) - sizes
         flat = torch.from_numpy(np.concatenate([img[i, :heights[i], :widths[i]].reshape(-1) for i in range(n)])).cuda()
     src = flat if packed else torch.from_numpy(img).cuda()
-    for c in (ctx, ctx_dma_small):
+    for c in (ctx, ctx_undealt, ctx_dma_small, ctx_dma_split):
         op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, layout, dtype), interp, flags=ops.F_QUANTIZE_U8 if quant else 0)
         if packed:
             op.set_ragged_source(offsets.astype(np.uint64), widths, heights, flat.numel())
@@ -56,7 +56,10 @@ def test_rows_at_every_phase(ctx, ctx_dma_small, layout, dtype, interp, W, packe
         else:
             op.update(roi, dw, dh, mirror)
         want = {ops.NEAREST: "rmx_resize_near_kernel", ops.LINEAR: "rmx_resize_fast_kernel" if packed or W % 4 else "rmx_resize_dma_kernel"}[interp]
-        assert op.kernel_name == want or c is ctx_dma_small, op.plan  # (a window too tall for the small budget takes the general kernel)
+        dealt = "split=" in op.plan
+        assert not dealt or c in (ctx, ctx_dma_split), op.plan
+        # (a window too tall for the small budget takes the general kernel)
+        assert op.kernel_name == ("rmx_resize_split_kernel" if dealt else want) or c in (ctx_dma_small, ctx_dma_split), op.plan
         out = op.alloc_output(fill=5)
         op.launch(src, out)
         c.sync()

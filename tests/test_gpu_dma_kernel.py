@@ -30,7 +30,7 @@ def _scale_bias(n):
 
 
 @pytest.mark.parametrize("layout,dtype", [(ops.NCHW, ops.FP16), (ops.NCHW, ops.FP32), (ops.NCHW, ops.UINT8), (ops.NHWC, ops.FP16), (ops.NHWC, ops.UINT8)])
-def test_streaming_and_staged_kernels_agree_with_the_oracle(ctx, ctx_staged, ctx_dma_small, layout, dtype):
+def test_streaming_and_staged_kernels_agree_with_the_oracle(ctx, ctx_staged, ctx_dma_small, ctx_dma_split, layout, dtype):
     rng = np.random.default_rng(4400 + 7 * layout + dtype)
     n, H, W = 10, 150, 200  # 600-byte rows: every row starts at the same byte phase
     img = rng.integers(0, 256, (n, H, W, 3), dtype=np.uint8)
@@ -62,7 +62,7 @@ def test_streaming_and_staged_kernels_agree_with_the_oracle(ctx, ctx_staged, ctx
             op.update(roi, dw, dh, mirror)
     dimg = _gpu(img)
     names = []
-    for c in (ctx, ctx_staged, ctx_dma_small):
+    for c in (ctx, ctx_staged, ctx_dma_small, ctx_dma_split):
         got, name, plan = _run(c, sd, dd, flags, update, dimg)
         names.append(name)
         # written windows only: the rest of the padded destination keeps the fill value on both sides
@@ -70,12 +70,12 @@ def test_streaming_and_staged_kernels_agree_with_the_oracle(ctx, ctx_staged, ctx
             g = got[i, :, :dh[i], :dw[i]] if layout == ops.NCHW else got[i, :dh[i], :dw[i]]
             e = exp[i, :, :dh[i], :dw[i]] if layout == ops.NCHW else exp[i, :dh[i], :dw[i]]
             assert np.array_equal(g.view(np.uint8), e.view(np.uint8)), "sample %d differs (%s, %s)" % (i, name, plan)
-    assert names == ["rmx_resize_dma_kernel", "rmx_resize_fast_kernel", "rmx_resize_dma_kernel"]
+    assert names == ["rmx_resize_dma_kernel", "rmx_resize_fast_kernel", "rmx_resize_dma_kernel", "rmx_resize_split_kernel"]
 
 
 @pytest.mark.parametrize("layout,dtype", [(ops.NCHW, ops.FP16), (ops.NCHW, ops.FP32), (ops.NCHW, ops.UINT8), (ops.NHWC, ops.FP16),
                                           (ops.NHWC, ops.FP32), (ops.NHWC, ops.UINT8)])
-def test_streaming_kernel_any_width_and_any_destination_base(ctx, ctx_dma_small, layout, dtype):
+def test_streaming_kernel_any_width_and_any_destination_base(ctx, ctx_dma_small, ctx_dma_split, layout, dtype):
     """Destination widths that are not multiples of 8 (225, 37, 1 ...) and a destination whose first byte is not 16-byte
     aligned: the streaming kernel's any-width form stores element by element. Every format, interleaved fp32 included; short
     last groups of every length 1..7; mirrored and unmirrored; tiles cut by the small LDS setting; the padding around each
@@ -109,13 +109,13 @@ def test_streaming_kernel_any_width_and_any_destination_base(ctx, ctx_dma_small,
     sd, dd = ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, layout, dtype)
     dimg = _gpu(img)
     esz = exp.dtype.itemsize
-    for c in (ctx, ctx_dma_small):
+    for c in (ctx, ctx_dma_small, ctx_dma_split):
         op = ops.Resize(c, sd, dd, ops.LINEAR, flags=flags)
         if norm:
             op.update_cmn(roi, dw, dh, scale, bias, mirror)
         else:
             op.update(roi, dw, dh, mirror)
-        assert op.kernel_name == "rmx_resize_dma_kernel" and "any_width=1" in op.plan, op.plan
+        assert op.kernel_name == ("rmx_resize_split_kernel" if c is ctx_dma_split else "rmx_resize_dma_kernel") and "any_width=1" in op.plan, op.plan
         for shift in (0, 1, 3):  # elements between a 256-byte boundary and the destination's first byte
             raw = torch.full((exp.size * esz + 256,), 0x5A, dtype=torch.uint8, device="cuda")
             out = raw[shift * esz: shift * esz + exp.size * esz].view(ops.torch_dtype(dtype)).view(exp.shape)
@@ -134,11 +134,12 @@ def test_streaming_kernel_any_width_and_any_destination_base(ctx, ctx_dma_small,
             assert (r[:shift * esz] == 0x5A).all() and (r[shift * esz + exp.size * esz:] == 0x5A).all()
 
 
+@pytest.mark.parametrize("split", [0, 1])
 @pytest.mark.parametrize("rows", [1, 3, 4, 8])
-def test_strip_heights(rows):
+def test_strip_heights(rows, split):
     """Strips of one to eight rows, with destination heights that leave a short last strip."""
     from conftest import _ctx_with_env
-    c = _ctx_with_env(RMX_TUNE_FAST_ROWS=rows)
+    c = _ctx_with_env(RMX_TUNE_FAST_ROWS=rows, RMX_TUNE_DMA_SPLIT=split)
     rng = np.random.default_rng(99)
     n, H, W = 6, 96, 128
     img = wl.smooth_noise(rng, n, H, W, sigma=1.0)
@@ -151,7 +152,7 @@ def test_strip_heights(rows):
                      flags=orc.F_QUANTIZE_U8)
     got, name, plan = _run(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, 96, 128, ops.NCHW, ops.FP16), ops.F_QUANTIZE_U8,
                            lambda op: op.update_cmn(roi, dw, dh, scale, bias, mirror), _gpu(img))
-    assert name == "rmx_resize_dma_kernel" and ("strip_rows=%d " % rows) in plan, plan
+    assert name == ("rmx_resize_split_kernel" if split and rows > 1 else "rmx_resize_dma_kernel") and ("strip_rows=%d " % rows) in plan, plan
     for i in range(n):
         assert np.array_equal(got[i, :, :dh[i], :dw[i]].view(np.uint16), exp[i, :, :dh[i], :dw[i]].view(np.uint16)), "sample %d (%s)" % (i, plan)
     c.close()

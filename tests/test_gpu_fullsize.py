@@ -126,16 +126,19 @@ def test_degenerate_samples(ctx):
     assert np.array_equal(got[0, :8, :8], exp[0, :8, :8]) and np.array_equal(got[2, :8, :16], exp[2, :8, :16])
 
 
+@pytest.mark.parametrize("adjacent", [0, 1])
 @pytest.mark.parametrize("streaming", [False, True])
 @pytest.mark.parametrize("rx,ry", [(1.3, 1.0), (1.9, 2.4), (3.0, 3.0), (3.7, 3.7), (2.5, 1.2)])
-def test_triangular_downscale_tap_and_row_length_classes(ctx, rx, ry, streaming):
+def test_triangular_downscale_tap_and_row_length_classes(rx, ry, streaming, adjacent):
     """The downscaling triangular kernels: 4/6/8-tap specialisations, 1/2/3 load slots per source row, partial
     last tile, per-sample windows (edge replicas on both sides, windows away from the origin at every byte phase), mirror,
     and an exact-size source whose last rows take the bounds-checked loader. (rx, ry) are the ratios of the first sample;
     the others shrink a little more or less. streaming: a source width that is a multiple of 4 (every row starts at the
     same byte phase), which the kernel that loads rows straight into LDS takes; otherwise the one that stages through
-    registers."""
+    registers. adjacent: the one whose lanes own neighbouring columns takes both."""
     import torch
+    from conftest import _ctx_with_env
+    ctx = _ctx_with_env(RMX_TUNE_TRI_ADJ=adjacent)
     rng = np.random.default_rng(int(rx * 100 + ry * 10))
     n, dw0, dh0 = 3, 200, 37
     W, H = int(round(dw0 * rx)) + 9, int(round(dh0 * ry)) + 5
@@ -156,7 +159,7 @@ def test_triangular_downscale_tap_and_row_length_classes(ctx, rx, ry, streaming)
         else:
             op.update_cmn(roi, dw, dh, scale, bias, mirror)
             exp = orc.resize(img, roi, dw, dh, dh0, dw0, interp=orc.TRIANGULAR, mirror=mirror, scale=scale, bias=bias, layout=layout, dtype=dtype)
-        assert op.kernel_name == ("rmx_resize_tri_dma_kernel" if streaming else "rmx_resize_tri_down_kernel")
+        assert op.kernel_name == ("rmx_resize_tri_adj_kernel" if adjacent else "rmx_resize_tri_dma_kernel" if streaming else "rmx_resize_tri_down_kernel")
         out = op.alloc_output()
         op.launch(src.view(n, H, W, 3), out)
         ctx.sync()
@@ -166,7 +169,7 @@ def test_triangular_downscale_tap_and_row_length_classes(ctx, rx, ry, streaming)
 
 def test_triangular_ring_and_downscale_kernels_agree(ctx, monkeypatch):
     """The same downscaling batch through the ring kernel (forced), the kernel that stages rows through registers (forced)
-    and the one that loads them straight into LDS."""
+    and the two that load them straight into LDS."""
     import torch
     rng = np.random.default_rng(77)
     n, H, W = 2, 150, 260
@@ -174,8 +177,10 @@ def test_triangular_ring_and_downscale_kernels_agree(ctx, monkeypatch):
     roi = np.array([[0, 0, W, H], [10, 6, 240, 140]], np.uint32)
     dw, dh = np.array([96, 88], np.uint32), np.array([64, 50], np.uint32)
     outs = []
-    for ring, dma, name in (("1", "1", "rmx_resize_tri_kernel"), ("0", "0", "rmx_resize_tri_down_kernel"), ("0", "1", "rmx_resize_tri_dma_kernel")):
+    for ring, dma, adj, name in (("1", "1", "1", "rmx_resize_tri_kernel"), ("0", "0", "1", "rmx_resize_tri_down_kernel"), ("0", "1", "0", "rmx_resize_tri_dma_kernel"),
+                                 ("0", "1", "1", "rmx_resize_tri_adj_kernel")):
         monkeypatch.setenv("RMX_TUNE_TRI_RING", ring)
+        monkeypatch.setenv("RMX_TUNE_TRI_ADJ", adj)
         monkeypatch.setenv("RMX_TUNE_DMA", dma)
         c2 = ops.Context()
         op = ops.Resize(c2, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, 64, 96, ops.NCHW, ops.FP32), ops.TRIANGULAR)
@@ -185,7 +190,7 @@ def test_triangular_ring_and_downscale_kernels_agree(ctx, monkeypatch):
         op.launch(torch.from_numpy(img).cuda(), out)
         c2.sync()
         outs.append(out.cpu().numpy())
-    assert np.array_equal(_bits(outs[0]), _bits(outs[1])) and np.array_equal(_bits(outs[0]), _bits(outs[2]))
+    assert all(np.array_equal(_bits(outs[0]), _bits(o)) for o in outs[1:])
 
 
 @pytest.mark.parametrize("W", [83, 84])

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("OW,OH", [(8, 1), (8, 70), (16, 5), (72, 3), (264, 9), (512, 4), (520, 5), (1032, 6)])
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("norm", [False, True])
-def test_whole_groups(ctx, ctx_dma_small, OW, OH, packed, norm):
+def test_whole_groups(ctx, ctx_undealt, ctx_dma_small, ctx_dma_split, OW, OH, packed, norm):
     import torch
     rng = np.random.default_rng(OW * 10 + OH)
     n, H, W = 6, 40, 101 if packed else 100
@@ -26,7 +26,7 @@ def test_whole_groups(ctx, ctx_dma_small, OW, OH, packed, norm):
     kw = dict(scale=scale, bias=bias, flags=orc.F_QUANTIZE_U8) if norm else {}
     exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.LINEAR, mirror=mirror, layout=ops.NHWC, dtype=ops.FP32, **kw)
     src = torch.from_numpy(img).cuda()
-    for c in (ctx, ctx_dma_small):
+    for c in (ctx, ctx_undealt, ctx_dma_small, ctx_dma_split):
         op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, ops.NHWC, ops.FP32), ops.LINEAR, flags=ops.F_QUANTIZE_U8 if norm else 0)
         if packed:
             op.set_ragged_source(np.arange(n, dtype=np.uint64) * H * W * 3, np.full(n, W), np.full(n, H), src.numel())
@@ -34,7 +34,9 @@ def test_whole_groups(ctx, ctx_dma_small, OW, OH, packed, norm):
             op.update_cmn(roi, dw, dh, scale, bias, mirror)
         else:
             op.update(roi, dw, dh, mirror)
-        assert op.kernel_name == "rmx_resize_fast_kernel" or c is ctx_dma_small, op.plan
+        dealt = "split=" in op.plan
+        assert not dealt or c in (ctx, ctx_dma_split), op.plan
+        assert op.kernel_name == ("rmx_resize_split_kernel" if dealt else "rmx_resize_fast_kernel") or c in (ctx_dma_small, ctx_dma_split), op.plan
         for shift in (0, 1):  # (1: the destination starts 4 bytes behind an aligned address and takes the form for any)
             whole = torch.full((n * OH * OW * 3 + 1,), 5.0, dtype=torch.float32, device="cuda")
             out = whole[shift:shift + n * OH * OW * 3].view(n, OH, OW, 3)

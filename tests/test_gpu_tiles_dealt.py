@@ -34,6 +34,7 @@ def test_tiles_of_a_window_in_several_wavefronts(layout, dtype, W, OW, interp):
             op.update_cmn(roi, dw, dh, s, b, mirror)
         else:
             op.update(roi, dw, dh, mirror)
+        assert (op.kernel_name == "rmx_resize_split_kernel") == bool(split) == ("split=" in op.plan), (op.kernel_name, op.plan)
         waves = int(op.plan.split("waves=")[1].split()[0])
         assert waves == n * 6 if not split else waves > n * 6, op.plan
         out = op.alloc_output(fill=3)
@@ -67,3 +68,44 @@ def test_batches_of_mostly_one_tile(ctx, n, tiles, parts):
     ctx.sync()
     exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.LINEAR, scale=s, bias=b, layout=orc.NCHW, dtype=orc.FP16, flags=orc.F_QUANTIZE_U8)
     assert np.array_equal(out.cpu().numpy().view(np.uint8), exp.view(np.uint8)), op.plan
+
+
+@pytest.mark.parametrize("layout,dtype", [(ops.NCHW, ops.FP16), (ops.NHWC, ops.FP16), (ops.NCHW, ops.FP32), (ops.NHWC, ops.FP32)])
+@pytest.mark.parametrize("chain", ["none", "linear", "twist"])
+@pytest.mark.parametrize("OW", [264, 261])
+def test_quantised_chains_in_several_wavefronts(layout, dtype, chain, OW):
+    """Resize, colour node, normalisation in one launch (each wavefront of a window has the colour tables of its own): the same bits as with one
+    wavefront per window, which the chain's own tests hold against the nodes one by one."""
+    import torch
+    from conftest import _ctx_with_env
+    rng = np.random.default_rng(OW + dtype + layout)
+    n, H, W, OH = 3, 90, 701, 22
+    img = wl.smooth_noise(rng, n, H, W, sigma=1.0)
+    roi = np.array([[0, 0, W, H], [3, 1, W - 3, H - 1], [W - 60, H - 30, 60, 30]], np.uint32)
+    dw, dh = np.array([OW, OW - 8, 40], np.uint32), np.array([OH, OH - 1, 9], np.uint32)
+    mirror = np.array([0, 1, 1], np.uint32)
+    s, b = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
+    flag = {"none": 0, "linear": ops.F_COLOR_LINEAR, "twist": ops.F_COLOR_TWIST}[chain]
+    u = lambda lo, hi: rng.uniform(lo, hi, n).astype(np.float32)  # noqa: E731
+    colour = {"none": None, "linear": (u(0.6, 1.4), u(-20, 20), u(100, 150)), "twist": (u(0.6, 1.4), u(-20, 20), u(-18, 200), u(0.6, 1.4))}[chain]
+    src = torch.from_numpy(img).cuda()
+    got = []
+    for split in (0, 1):
+        c = _ctx_with_env(RMX_TUNE_DMA_SPLIT=split)
+        op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, layout, dtype), ops.LINEAR, flags=ops.F_QUANTIZE_U8 | flag)
+        if colour is None:
+            op.update_cmn(roi, dw, dh, s, b, mirror)
+        else:
+            op.update_color_cmn(roi, dw, dh, s, b, colour, mirror)
+        assert (op.kernel_name == "rmx_resize_split_kernel") == bool(split), (op.kernel_name, op.plan)
+        out = op.alloc_output(fill=3)
+        op.launch(src, out)
+        c.sync()
+        got.append(out.cpu().numpy())
+        c.close()
+    assert np.array_equal(got[0].view(np.uint8), got[1].view(np.uint8))
+    if colour is None:
+        exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.LINEAR, mirror=mirror, layout=layout, dtype=dtype, scale=s, bias=b, flags=orc.F_QUANTIZE_U8)
+        for i in range(n):
+            x = (i, slice(None), slice(0, dh[i]), slice(0, dw[i])) if layout == ops.NCHW else (i, slice(0, dh[i]), slice(0, dw[i]))
+            assert np.array_equal(np.ascontiguousarray(got[1][x]).view(np.uint8), np.ascontiguousarray(exp[x]).view(np.uint8)), i

@@ -13,12 +13,12 @@ pytestmark = pytest.mark.gpu
 FORMATS = [(ops.NCHW, ops.FP16), (ops.NCHW, ops.FP32), (ops.NCHW, ops.UINT8), (ops.NHWC, ops.FP16), (ops.NHWC, ops.FP32), (ops.NHWC, ops.UINT8)]
 
 
-def _check(c, img, roi, dw, dh, OH, OW, layout, dtype, mirror, packed=None, name=None):
+def _check(c, img, roi, dw, dh, OH, OW, layout, dtype, mirror, packed=None, quant=False, kernel="rmx_resize_tri_adj_kernel"):
     import torch
     n, H, W = img.shape[:3]
     norm = dtype != ops.UINT8
     s, b = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
-    op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, layout, dtype), ops.TRIANGULAR)
+    op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, layout, dtype), ops.TRIANGULAR, flags=ops.F_QUANTIZE_U8 if quant else 0)
     src = img
     if packed is not None:
         src, offsets, strides, widths, heights = packed
@@ -27,12 +27,13 @@ def _check(c, img, roi, dw, dh, OH, OW, layout, dtype, mirror, packed=None, name
         op.update_cmn(roi, dw, dh, s, b, mirror)
     else:
         op.update(roi, dw, dh, mirror)
-    assert "adjacent=1" in op.plan and (name is None or op.kernel_name == name), (op.kernel_name, op.plan)
+    assert op.kernel_name == kernel and ("adjacent=1" in op.plan) == (kernel == "rmx_resize_tri_adj_kernel"), (op.kernel_name, op.plan)
     out = op.alloc_output(fill=6)
     op.launch(torch.from_numpy(np.ascontiguousarray(src)).cuda(), out)
     c.sync()
     got = out.cpu().numpy()
-    exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.TRIANGULAR, mirror=mirror, scale=s if norm else None, bias=b if norm else None, layout=layout, dtype=dtype)
+    exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.TRIANGULAR, mirror=mirror, scale=s if norm else None, bias=b if norm else None, layout=layout, dtype=dtype,
+                     flags=orc.F_QUANTIZE_U8 if quant else 0)
     want = np.full_like(exp, 6)
     for i in range(n):
         if layout == ops.NCHW:
@@ -63,8 +64,27 @@ def _batch(seed, W):
 @pytest.mark.parametrize("W", [132, 133, 134, 135])
 def test_rows_at_every_phase_ratios_and_widths(ctx, layout, dtype, W):
     img, roi, dw, dh, OH, OW, mirror = _batch(W, W)
-    # (windows that grow by more than eight rows in flight allow: the kernel is named after the one that takes them otherwise)
-    _check(ctx, img, roi, dw, dh, OH, OW, layout, dtype, mirror, name="rmx_resize_tri_kernel")
+    _check(ctx, img, roi, dw, dh, OH, OW, layout, dtype, mirror)
+
+
+@pytest.mark.parametrize("layout,dtype", [f for f in FORMATS if f[1] != ops.UINT8])
+@pytest.mark.parametrize("W", [132, 133])
+def test_quantised(ctx, layout, dtype, W):
+    """As a resize node that has taken in the normalisation behind it asks for: rounded to bytes, then normalised."""
+    img, roi, dw, dh, OH, OW, mirror = _batch(W + 7, W)
+    _check(ctx, img, roi, dw, dh, OH, OW, layout, dtype, mirror, quant=True)
+
+
+@pytest.mark.parametrize("W,grow,kernel", [(132, 90, "rmx_resize_tri_dma_kernel"), (133, 90, "rmx_resize_tri_kernel"), (132, 20, "rmx_resize_tri_kernel")])
+def test_a_sample_of_one_pixel_rows_sends_its_batch_to_another_kernel(ctx, W, grow, kernel):
+    """No lane has two columns there: eight accumulator sets where rows start at one phase and no window grows by more than they allow."""
+    rng = np.random.default_rng(W + grow)
+    n, H, OH, OW = 4, 150, 120, 64
+    img = rng.integers(0, 256, (n, H, W, 3), dtype=np.uint8)
+    roi = np.array([[0, 0, W, H], [5, 7, 60, grow], [9, 1, 4, 100], [0, 0, 3, H]], np.uint32)
+    dw, dh = np.array([64, 33, 1, 1], np.uint32), np.array([120, 120, 90, 120], np.uint32)
+    for layout, dtype in ((ops.NCHW, ops.FP16), (ops.NHWC, ops.FP32)):
+        _check(ctx, img, roi, dw, dh, OH, OW, layout, dtype, np.array([0, 1, 1, 0], np.uint32), kernel=kernel)
 
 
 @pytest.mark.parametrize("rows", [4, 5, 23, 64])

@@ -1,8 +1,10 @@
-"""The streaming triangular kernel (source rows straight into LDS as packed bytes) against the oracle, bit for bit, on what is
+"""The streaming triangular kernels (source rows straight into LDS as packed bytes) against the oracle, bit for bit, on what is
 specific to it: windows that start at every byte phase of a dword, edge replicas on both sides, every output format, strips
 whose source rows outnumber the table of vertical coefficients, many vertical taps, mirror, packed (ragged) sources whose
 rows start at multiples of 4 bytes (image bases at every byte phase), and the kernel that stages through registers on the same
 batches; the same packed sources through the raw form of the warp kernel."""
+import os
+
 import numpy as np
 import pytest
 
@@ -10,6 +12,33 @@ from oracle import orc
 from rocal_amd import ops, workloads as wl
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", params=[0, 1], ids=["apart", "adjacent"], autouse=True)
+def adjacent(request):
+    """Every test with both streaming kernels: lanes that own columns 64 apart, or neighbouring ones where a batch is not left to two accumulator
+    sets (contexts take it from the environment)."""
+    old = os.environ.get("RMX_TUNE_TRI_ADJ")
+    os.environ["RMX_TUNE_TRI_ADJ"] = str(request.param)
+    yield request.param
+    if old is None:
+        del os.environ["RMX_TUNE_TRI_ADJ"]
+    else:
+        os.environ["RMX_TUNE_TRI_ADJ"] = old
+
+
+@pytest.fixture(scope="module")
+def ctx(adjacent):
+    c = ops.Context(0)
+    yield c
+    c.close()
+
+
+def _streams(op, sets=None):
+    """Whether the op runs the streaming kernel of this run, with so many accumulator sets where its columns lie 64 apart."""
+    if os.environ["RMX_TUNE_TRI_ADJ"] == "1" and sets != 2:
+        return op.kernel_name == "rmx_resize_tri_adj_kernel" and "adjacent=1" in op.plan and "rows_in_flight" not in op.plan
+    return op.kernel_name == "rmx_resize_tri_dma_kernel" and "adjacent" not in op.plan and (sets is None or "rows_in_flight=%d" % sets in op.plan)
 
 
 def _gpu(a):
@@ -55,17 +84,17 @@ def test_formats_phases_and_edges(ctx, ctx_staged, layout, dtype):
     norm = dtype != ops.UINT8
     exp = orc.resize(img, roi, dw, dh, OH, OW, interp=orc.TRIANGULAR, mirror=mirror, scale=scale if norm else None, bias=bias if norm else None,
                      layout=layout, dtype=dtype)
-    for c, name in ((ctx, "rmx_resize_tri_dma_kernel"), (ctx_staged, "rmx_resize_tri_down_kernel")):
+    for c, name in ((ctx, None), (ctx_staged, "rmx_resize_tri_down_kernel")):
         op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, layout, dtype), ops.TRIANGULAR)
         if norm:
             op.update_cmn(roi, dw, dh, scale, bias, mirror)
         else:
             op.update(roi, dw, dh, mirror)
-        assert op.kernel_name == name, op.plan
+        assert op.kernel_name == name if name else _streams(op), (op.kernel_name, op.plan)
         out = op.alloc_output(fill=7)
         op.launch(_gpu(img), out)
         c.sync()
-        _check_windows(out.cpu().numpy(), exp, dw, dh, layout, 7, name)
+        _check_windows(out.cpu().numpy(), exp, dw, dh, layout, 7, op.kernel_name)
 
 
 @pytest.mark.parametrize("ry,rows", [(7.4, 0), (5.1, 20), (2.0, 64), (1.0, 7)])
@@ -86,7 +115,7 @@ def test_many_vertical_taps_and_long_strips(ctx, ry, rows):
     exp = orc.resize(img, roi, dw, dh, dh0, dw0, interp=orc.TRIANGULAR, mirror=mirror, scale=scale, bias=bias, layout=ops.NCHW, dtype=ops.FP16)
     op = ops.Resize(c, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, dh0, dw0, ops.NCHW, ops.FP16), ops.TRIANGULAR)
     op.update_cmn(roi, dw, dh, scale, bias, mirror)
-    assert op.kernel_name == "rmx_resize_tri_dma_kernel", op.plan
+    assert _streams(op), (op.kernel_name, op.plan)
     out = op.alloc_output(fill=3)
     op.launch(_gpu(img), out)
     c.sync()
@@ -128,7 +157,7 @@ def test_whole_and_half_ratios_keep_two_rows_in_flight(ctx, ctx_four_rows, ry, r
     src = _gpu(img)
     op = ops.Resize(c, sd, dd, ops.TRIANGULAR)
     op.update_cmn(roi, dw, dh, scale, bias, mirror)
-    assert op.kernel_name == "rmx_resize_tri_dma_kernel" and "rows_in_flight=2" in op.plan, op.plan
+    assert _streams(op, 2), (op.kernel_name, op.plan)
     out = op.alloc_output(fill=3)
     op.launch(src, out)
     c.sync()
@@ -145,7 +174,7 @@ def test_whole_and_half_ratios_keep_two_rows_in_flight(ctx, ctx_four_rows, ry, r
     roi2[4, 3] = sh[4] + 3
     exp2 = orc.resize(img, roi2, dw, dh2, OH, OW, interp=orc.TRIANGULAR, mirror=mirror, scale=scale, bias=bias, layout=ops.NCHW, dtype=ops.FP16)
     op.update_cmn(roi2, dw, dh2, scale, bias, mirror)
-    assert "rows_in_flight=4" in op.plan, op.plan
+    assert _streams(op, 4), (op.kernel_name, op.plan)
     out2 = op.alloc_output(fill=3)
     op.launch(src, out2)
     c.sync()
@@ -182,7 +211,7 @@ def test_random_whole_and_half_ratios_with_a_crop_behind_the_resize(ctx, seed):
     exp = orc.crop_mirror_normalize(mid, crop, scale, bias, mirror, OH, OW, ops.NCHW, ops.FP32)
     op = ops.Resize(ctx, ops.desc(n, H, W, ops.NHWC, ops.UINT8), ops.desc(n, OH, OW, ops.NCHW, ops.FP32), ops.TRIANGULAR, flags=ops.F_QUANTIZE_U8)
     op.update_cmn(roi, dw, dh, scale, bias, mirror, crop_roi=crop)
-    assert op.kernel_name == "rmx_resize_tri_dma_kernel" and "rows_in_flight=2" in op.plan, op.plan
+    assert _streams(op, 2), (op.kernel_name, op.plan)
     out = op.alloc_output(fill=5)
     op.launch(_gpu(img), out)
     ctx.sync()
@@ -229,7 +258,7 @@ def test_whole_horizontal_ratios(ctx, ctx_staged, rx, layout, dtype):
 
 @pytest.mark.parametrize("layout,dtype", [(ops.NCHW, ops.FP16), (ops.NHWC, ops.UINT8), (ops.NCHW, ops.FP32)])
 @pytest.mark.parametrize("rows", [0, 7])
-def test_windows_that_grow_keep_eight_rows_in_flight(ctx, ctx_four_rows, layout, dtype, rows):
+def test_windows_that_grow_keep_eight_rows_in_flight(ctx, ctx_four_rows, adjacent, layout, dtype, rows):
     """A batch of windows some of which shrink and some of which grow (vertical ratios 0.28 .. 2.6, as RandomResizedCrop makes
     them): the streaming kernel keeps eight output rows in flight. Windows at the top and at the bottom of the source (the
     clamp), mirrored, growing in one direction and shrinking in the other; against the oracle and, bit for bit, against the
@@ -262,15 +291,16 @@ def test_windows_that_grow_keep_eight_rows_in_flight(ctx, ctx_four_rows, layout,
         return op, out.cpu().numpy()
 
     op, got = run(c, roi, dh)
-    assert op.kernel_name == "rmx_resize_tri_dma_kernel" and "rows_in_flight=8" in op.plan, op.plan
-    _check_windows(got, exp, dw, dh, layout, 4, "eight rows (%s)" % op.plan)
+    assert _streams(op, 8), (op.kernel_name, op.plan)
+    _check_windows(got, exp, dw, dh, layout, 4, "windows that grow (%s)" % op.plan)
     op4, got4 = run(ctx_four_rows, roi, dh)
     assert op4.kernel_name == "rmx_resize_tri_kernel", op4.plan
     assert np.array_equal(_bits(got), _bits(got4))
     roi2 = roi.copy()
     roi2[1, 3] = 12                                            # 12 rows to 64: ratio 0.19
     op2, got2 = run(c, roi2, dh)
-    assert op2.kernel_name == "rmx_resize_tri_kernel", op2.plan
+    # (kept rows make output rows at any ratio, eight sets do not)
+    assert op2.kernel_name == ("rmx_resize_tri_adj_kernel" if adjacent else "rmx_resize_tri_kernel"), op2.plan
     _check_windows(got2, orc.resize(img, roi2, dw, dh, OH, OW, **kw), dw, dh, layout, 4, "ring kernel")
     if rows:
         c.close()
@@ -337,7 +367,7 @@ def test_packed_source_with_rows_at_multiples_of_four(ctx, heights_out):
     op = ops.Resize(ctx, ops.desc(n, 150, 400, ops.NHWC, ops.UINT8), ops.desc(n, 60, 180, ops.NCHW, ops.FP16), ops.TRIANGULAR)
     op.set_ragged_source(offsets, widths, heights, packed.size, row_strides=strides)
     op.update_cmn(roi, dw, dh, scale, bias, mirror)
-    assert op.kernel_name == "rmx_resize_tri_dma_kernel", op.plan
+    assert _streams(op), (op.kernel_name, op.plan)
     # (torch places the buffer at a 256-byte boundary; the kernels require a 4-byte aligned buffer, not aligned images)
     out = op.alloc_output(fill=1)
     op.launch(_gpu(packed), out)
@@ -392,7 +422,7 @@ def test_rows_in_another_order_with_an_empty_sample(ctx):
         dh = np.array([32, 32, 32, 32, 30], np.uint32)
         mirror = np.array([1, 0, 0, 1, 0], np.uint32)
         op.update_cmn(roi, dw, dh, scale, bias, mirror)
-        assert op.kernel_name == "rmx_resize_tri_dma_kernel" and "rows_in_flight=8" in op.plan, op.plan
+        assert _streams(op, 8), (op.kernel_name, op.plan)
         out = op.alloc_output(fill=5)
         op.launch(src, out)
         ctx.sync()

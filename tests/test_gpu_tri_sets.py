@@ -1,5 +1,5 @@
-"""The streaming triangular kernel with eight accumulator sets, at the vertical ratios where a sample changes from all eight sets to
-the lower four (1/2), at the windows' ends, and with so few output rows that every row has a set of its own; rows in the kernel's
+"""The streaming triangular kernels, that with eight accumulator sets (columns 64 apart) at the vertical ratios where a sample changes from all
+eight sets to the lower four (1/2), at the windows' ends, and with so few output rows that every row has a set of its own; rows in the kernel's
 arguments and in a table, in strips of every length. Bit for bit against the oracle and the ring kernel."""
 import numpy as np
 import pytest
@@ -24,7 +24,8 @@ def _run(c, img, roi, rs, crop, out_hw, layout, dtype, mirror):
 
 @pytest.mark.parametrize("layout,dtype", [(ops.NCHW, ops.FP16), (ops.NHWC, ops.FP32)])
 @pytest.mark.parametrize("rows,compact", [(0, 1), (4, 1), (9, 1), (23, 0)])
-def test_ratios_around_one_half_and_short_windows(layout, dtype, rows, compact):
+@pytest.mark.parametrize("adjacent", [0, 1])
+def test_ratios_around_one_half_and_short_windows(layout, dtype, rows, compact, adjacent):
     from conftest import _ctx_with_env
     rng = np.random.default_rng(70 + rows)
     OH, OW = 96, 64
@@ -41,13 +42,14 @@ def test_ratios_around_one_half_and_short_windows(layout, dtype, rows, compact):
     mirror = (np.arange(n) % 3 == 0).astype(np.uint32)
     # the whole resized image, and a crop of it (its first and last written rows are not the window's)
     crop = np.stack([np.full(n, 2), rs[:, 1] // 5, rs[:, 0] - 7, rs[:, 1] - rs[:, 1] // 5 - rs[:, 1] // 6], 1).astype(np.uint32)
-    c = _ctx_with_env(RMX_TUNE_TRI_ROWS=rows, RMX_TUNE_COMPACT=compact)
+    c = _ctx_with_env(RMX_TUNE_TRI_ROWS=rows, RMX_TUNE_COMPACT=compact, RMX_TUNE_TRI_ADJ=adjacent)
     ring = _ctx_with_env(RMX_TUNE_TRI_RING=1)
     s, b = orc.cmn_scale_bias(wl.MEAN, wl.STD, n)
     try:
         for cr in (None, crop):
             op, got = _run(c, img, roi, rs, cr, (OH, OW), layout, dtype, mirror)
-            assert op.kernel_name == "rmx_resize_tri_dma_kernel" and "rows_in_flight=8" in op.plan and ("rows=arguments" if compact else "rows=table") in op.plan, op.plan
+            kernel, form = ("rmx_resize_tri_adj_kernel", "adjacent=1") if adjacent else ("rmx_resize_tri_dma_kernel", "rows_in_flight=8")
+            assert op.kernel_name == kernel and form in op.plan and ("rows=arguments" if compact else "rows=table") in op.plan, op.plan
             _, other = _run(ring, img, roi, rs, cr, (OH, OW), layout, dtype, mirror)
             assert np.array_equal(got.view(np.uint8), other.view(np.uint8)), op.plan
             if cr is None:
