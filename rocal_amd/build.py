@@ -30,7 +30,8 @@ def _newest_header():
 # Sources whose generated code the CPU tests read (explicit wait counts that rely on how many instructions the compiler makes):
 # their device assembly is kept next to the object, so that the tests need not compile them a second time.
 KEEP_ASSEMBLY = ("rmx_kernels_resize_dma.hip", "rmx_kernels_resize_fast.hip", "rmx_kernels_resize_near.hip", "rmx_kernels_tri_dma_2.hip", "rmx_kernels_tri_dma_4.hip", "rmx_kernels_tri_dma_8_nchw.hip",
-                 "rmx_kernels_tri_dma_8_nhwc.hip", "rmx_kernels_warp.hip")
+                 "rmx_kernels_tri_dma_8_nhwc.hip", "rmx_kernels_tri_adj_nchw.hip", "rmx_kernels_tri_adj_nhwc.hip", "rmx_kernels_tri_adj_nchw_any.hip",
+                 "rmx_kernels_tri_adj_nhwc_any.hip", "rmx_kernels_resize_split.hip", "rmx_kernels_warp.hip")
 
 
 def assembly_path(src_name):

@@ -105,13 +105,14 @@ def test_warp_kernel_hand_written_lds_reads_are_awaited_before_use():
         m = re.match(r"v(\d+)$", tok)
         return {int(m.group(1))} if m else set()
 
-    funcs = re.split(r"\n(?=_ZN3rmx15rmx_warp_kernel[^\n]*:\s)", text)
-    loops = 0
+    # (the form whose rows leave together has the same loops)
+    funcs = re.split(r"\n(?=_ZN3rmx\d+rmx_warp(?:_rows)?_kernel[^\n]*:\s)", text)
+    loops = rows_loops = 0
     for f in funcs:
-        m = re.match(r"(_ZN3rmx15rmx_warp_kernel\S*):", f)
+        m = re.match(r"(_ZN3rmx\d+rmx_warp(?:_rows)?_kernel\S*):", f)
         if not m:
             continue
-        body = f.split("s_endpgm")[0]
+        body = f.split(".Lfunc_end")[0]
         blocks = re.split(r"\n(?=\.LBB\d+_\d+:)", body)
         for blk in blocks:
             if not re.search(r"ds_read2_b32 [^\n]* offset0:4[0-9] offset1:4[0-9]", blk):
@@ -142,4 +143,6 @@ def test_warp_kernel_hand_written_lds_reads_are_awaited_before_use():
                         nxt |= regs(ins[n].split()[1].rstrip(","))
                     assert not (nxt & filled), m.group(1)
             loops += 1
-    assert loops >= 12  # two loops (with and without the ROI test) in each of the six formats
+            rows_loops += "rmx_warp_rows_kernel" in m.group(1)
+    assert rows_loops == 8  # with and without the ROI test, at either pitch, by tiles and by teams
+    assert loops - rows_loops >= 12  # two loops (with and without the ROI test) in each of the six formats

@@ -1,4 +1,4 @@
-"""Generated code of the resize kernels for rows at any byte phase and of the nearest-pixel kernel: as for the streaming bilinear
+"""Generated code of the resize kernels for rows at any byte phase, of the nearest-pixel kernel and of the one whose tiles are dealt: as for the streaming bilinear
 kernel, a wait for a window's loads that leaves N operations outstanding needs N stores in the held-back group behind them."""
 import os
 import re
@@ -9,7 +9,8 @@ from test_dma_waitcnt_cpu import HIPCC, _device_assembly
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
-@pytest.mark.parametrize("src,name,instances", [("rmx_kernels_resize_fast.hip", "rmx_resize_fast_kernel", 30), ("rmx_kernels_resize_near.hip", "rmx_resize_near_kernel", 12)])
+@pytest.mark.parametrize("src,name,instances", [("rmx_kernels_resize_fast.hip", "rmx_resize_fast_kernel", 30), ("rmx_kernels_resize_near.hip", "rmx_resize_near_kernel", 12),
+                                                ("rmx_kernels_resize_split.hip", "rmx_resize_split_kernel", 42)])
 def test_held_back_stores_cover_the_wait_count(src, name, instances):
     text = _device_assembly(src)
     checked = 0

@@ -50,3 +50,33 @@ def test_tables_of_vertical_coefficients_wait_for_no_load(unit):
         names += 1
         assert not _idle_waits(f.split(".Lfunc_end")[0]), m.group(1)
     assert names
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
+@pytest.mark.parametrize("unit", ["nchw", "nhwc", "nchw_any", "nhwc_any"])
+def test_kernel_of_neighbouring_columns_counts_its_stores(unit):
+    """rmx_resize_tri_adj_kernel waits for its loads into LDS with s_waitcnt vmcnt(0 | NS | 2 NS | 4 NS), NS the fewest store instructions that an
+    output row can become: three planes, or one interleaved run. The compiler makes the stores, so every place that stores a row must
+    hold as many, nothing may spill to scratch memory, and the numbered waits are the source's own. Its tables of vertical
+    coefficients wait for no load; one idle wait stands on the path of rows that the lanes store at the buffer's end."""
+    text = _device_assembly("rmx_kernels_tri_adj_%s.hip" % unit)
+    ns = 3 if unit.startswith("nchw") else 1
+    checked = 0
+    for f in re.split(r"\n(?=_ZN3rmx25rmx_resize_tri_adj_kernel[^\n]*:\s)", text):
+        m = re.match(r"(_ZN3rmx25rmx_resize_tri_adj_kernel\S*):", f)
+        if not m:
+            continue
+        body = f.split(".Lfunc_end")[0]
+        assert not re.search(r"^\s*(scratch_|buffer_|flat_)", body, re.M), m.group(1)
+        own = [int(x) for part in re.findall(r"#ASMSTART(.*?)#ASMEND", body, re.S) for x in re.findall(r"s_waitcnt vmcnt\((\d+)\)", part)]
+        assert set(own) == {0, ns, 2 * ns, 4 * ns}, "%s: waits %s" % (m.group(1), sorted(set(own)))
+        places = 0
+        for block in re.split(r"\n(?=\.LBB\d+_\d+:|; %bb\.\d+:)", body):
+            stores = re.findall(r"^\s*global_store_\w+", block, re.M)
+            assert not stores or len(stores) >= ns, "%s: a row in %d stores" % (m.group(1), len(stores))
+            places += bool(stores)
+        assert places >= 6 * 2  # six numbers of taps, samples that shrink and that grow
+        assert "global_load_lds_dwordx4" in body
+        assert len(_idle_waits(body)) <= 1, m.group(1)
+        checked += 1
+    assert checked == 9
