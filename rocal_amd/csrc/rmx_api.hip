@@ -1233,14 +1233,14 @@ static int plan_resize(rmx_op *op, RmxSample *t, bool norm) {
         }
         int rows = op->ctx->tri_rows > 0 ? op->ctx->tri_rows : 12;
         bool sort_rows = false;
-        // Streaming form of the downscaling variant (source rows straight into LDS as raw bytes): every source row must start
-        // at the same byte phase (row stride a multiple of 4), and four LDS rows of the widest tile plus the table of vertical
+        // Streaming form (source rows straight into LDS as raw bytes): four LDS rows of the widest tile plus the table of vertical
         // coefficients must leave room for ten wavefronts per CU at least.
         op->tri_rows_in_flight = 0;
         // Two kernels of this form. rmx_resize_tri_dma_kernel (columns 64 apart): rows that all start at the same byte phase (row strides
         // multiples of 4), ratios for which two, four or eight rows in flight do. rmx_resize_tri_adj_kernel (neighbouring columns per
-        // lane): rows at any phase, any ratio; not rows of one pixel, of which no lane has two. Where both could, two rows in flight
-        // stay with the first and everything else goes to the second (figures there).
+        // lane): rows at any phase, any ratio; not rows of one pixel, of which no lane has two. Where both could, batches for which two rows
+        // in flight do stay with the first (32 frames of 1080 x 1920 to 360 x 640 fp16 57.6 us, by the second 58.4) and everything else
+        // goes to the second (256 RandomResizedCrop windows to 224 x 224 fp16 45.1 -> 42.6; more figures there).
         bool tdma = down && op->ctx->dma && op->ctx->tri_tpx == 2 && ky <= 16;
         bool adj = tdma && op->ctx->tri_adj && op->ctx->tri_slots != 4 && (uint64_t)op->dst.h * op->dst.w * 3 * dtype_size(op->dst.dtype) < (1ull << 32);
         for (int i = 0; i < op->n && adj; i++) adj = t[i].dst_w != 1;

@@ -82,7 +82,7 @@ RMX_DEV void store_pair(uint8_t *d, size_t plane_bytes, uint32_t at, const float
 
 template <typename T, int LAYOUT, bool NORM, bool QUANT, bool ANY>
 __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) {
-    constexpr int TPX = 2;               // columns per lane: lane and lane + 64
+    constexpr int TPX = 2;               // columns per lane, side by side
     constexpr int TTW = RMX_WAVE * TPX;  // output columns per wave tile
     const int lane = threadIdx.x & (RMX_WAVE - 1);
     const int wib = threadIdx.x / RMX_WAVE;
@@ -242,16 +242,15 @@ __global__ void __launch_bounds__(256, 5) rmx_resize_tri_adj_kernel(RmxKArgs a) 
     const bool first_by_lanes = issue(bufb);
 
     // ---- per-lane columns: taps, coefficients (registers), column sums, destination column (mirrored if asked)
-    // (a lane whose column lies beyond the row takes the last column again and stores the same value to the same place:
-    // every store instruction is then issued by every wavefront, which the count in the wait below relies on)
+    // (a lane whose columns lie beyond the row takes the last two again and stores the same values to the same places: every
+    // wavefront issues every store instruction, which the count in the wait below relies on)
     uint32_t xoff = 0, tap[TPX];
     float colsum[TPX] = {}, creg[TPX][8] = {};
     int locx[TPX];
     float w0x[TPX];
 #pragma unroll
     for (int i = 0; i < TPX; i++) {
-        // (in the order of the destination; a row's last lane moves left until it has two columns, and stores the same values to the
-        // same places as its neighbour)
+        // (in the order of the destination; at an odd width the last of them moves left by one column)
         const int colc = xt + min(2 * lane, tw - 2) + (hf ? 1 - i : i);
         if (i == 0) xoff = (uint32_t)(hf ? (dw - 1 - colc) : colc) * (uint32_t)(LAYOUT == RMX_NCHW ? sizeof(T) : 3 * sizeof(T));
         tri_loc(ax, pcx + colc, (float)xlo, locx[i], w0x[i]);

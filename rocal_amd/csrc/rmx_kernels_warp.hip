@@ -28,9 +28,9 @@
 // of 512 x 512, whole batches: nearest pixel 57.3 -> 48.6 us by tiles -> 43.4 by four tiles as streaming stores (these cost the stores of
 // single lanes 8 us: part of a line at a time, they go to memory before their neighbours come); bilinear 63.4 -> 61.0.
 // The nearest pixel's bytes are moved, not converted to float and back (BYTES): 43.4 -> 42.7, 86 turned images of 151 x 447 10.7 -> 10.2.
-// Bound by how many wavefronts are there to compute while others wait for their box: 128 images of 512 x 512 take 61 - 63 us; without the
-// box's loads 47, without the stores 52, without both 42, with taps that meet no bank conflict the same; the bytes are 36 at the rate of
-// a large copy. The LDS slice therefore holds the box and nothing besides: no pixel of margin (the corners bound it exactly), the
+// Bound by how many wavefronts are there to compute while others wait for their box: 128 images of 512 x 512 take 58 - 61 us; with the
+// lanes' own stores, 61 - 63 then, without the box's loads 47, without the stores 52, without both 42, with taps that meet no bank conflict
+// the same; the bytes are 36 at the rate of a large copy. The LDS slice therefore holds the box and nothing besides: no pixel of margin (the corners bound it exactly), the
 // repeated row only where it is read, rows of 10 pieces where they fit instead of 11 (a batch turned by up to 30 degrees and scaled by a
 // tenth: 9.4 -> 7.7 KB a wavefront, 20 of them per CU instead of 16; a seventh fewer pieces to load): 63.2 - 64.0 -> 60.9 - 63.1 us on
 // several inputs, in turn. Fewer instructions alone (taps widened inside v_fma_mix_f32: a fifth fewer) measured the same beside it.
